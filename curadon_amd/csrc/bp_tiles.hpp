@@ -7,6 +7,8 @@
 // every pair load stays inside the staged array.
 #pragma once
 
+#include <type_traits>
+
 #include "cmi_internal.hpp"
 
 namespace cmi {
@@ -33,44 +35,128 @@ __device__ __forceinline__ float lerp_pair(const Pair &p, float f) {
     return fmaf(f, p.hi - p.lo, p.lo);
 }
 
-// Sum over angles for one pixel at world position (x, y) (backward_2d.hpp:58-96):
-//   sum_a w_a^WPOW lerp(sino[a], w_a eta_a + D/2),  w_a = DSD / (xi_a + DSO)
-// meta[a] = (-sin, cos, DSD, DSO); px, py = x / du, y / du. `R` covers [A][D + 4].
-template <class SS, int WPOW, class TAB>
-__device__ __forceinline__ float bp2d_pixel(rsrc_t R, TAB meta, int A,
-                                           int D, float x, float y, float px, float py,
-                                           float half_d) {
+// ------------------------------------------------------------------------------------------
+// Fan-beam backprojection of a 64 x NY pixel tile by a workgroup of four wavefronts: wavefront q
+// takes the angles of quarter q, [A q / 4, A (q + 1) / 4), for all pixels of the tile, a thread
+// one column of NY pixels, and the quarters' sums S_q meet in LDS as (S0 + S2) + (S1 + S3).
+// Every path that backprojects a fan beam adds in that order, so a pixel's value does not depend
+// on the path: k_bp2d and the serving kernel here, and k_bp2d_qt, where the quarters' order
+// turns with the pixel (the sum is symmetric under a cyclic shift of the quarters).
+// On gfx950 fma, add and mul of vector registers issue about 1.55 wavefront instructions per clock
+// and CU; min / max / med3, floor, fract, conversions, shifted adds and any instruction that reads
+// a scalar register 0.93, v_rcp_f32 0.48 (issue probe, eight wavefronts per SIMD). With NY = 4
+// rows, a thread shares an angle's constants and its two products with x. Splitting the angles
+// over the wavefronts keeps the number of wavefronts that a thread per pixel would have.
+
+// Projection of one angle of a circular plan, tab[a] = (-sin, cos, DSD, DSO)
+// (backward_2d.hpp:58-96): depth = DSO + (-sin x - cos y), magnification w = DSD / depth, cell
+// coordinate w (cos x - sin y) / du + D/2. The sums are of rounded products (no contraction): a
+// quarter turn of the pixel and the angle exchanges the two products of each and leaves their
+// sum as it was, bit for bit.
+template <int WPOW>
+struct FanAngle {
+    float4 m;
+    float p1, q1;
+    __device__ __forceinline__ FanAngle(float4 m_, float x, float px) : m(m_) {
+#pragma clang fp contract(off)
+        p1 = m.x * x;
+        q1 = m.y * px;
+    }
+    template <class TAB>
+    __device__ __forceinline__ FanAngle(TAB tab, int a, float x, float px)
+        : FanAngle(table4(tab, a), x, px) {}
+    // u: lower-tap cell coordinate (unclamped); wt: weight. px, py = x / du, y / du; c0 = D/2 - .5
+    __device__ __forceinline__ void at(float y, float py, float c0, float &u, float &wt) const {
+#pragma clang fp contract(off)
+        const float depth = (p1 - m.y * y) + m.w;
+        const float eta = q1 + m.x * py;
+        const float w = m.z * __builtin_amdgcn_rcpf(depth);
+        u = __builtin_fmaf(w, eta, c0);
+        wt = WPOW == 2 ? w * w : w;
+    }
+};
+
+// Projection of one ASTRA-like view, tab[3 a ..] (geometry2d.hpp bp_view): depth = n . x + n0,
+// w = L / depth, cell coordinate w (e . x + e0) + c0, weight w^WPOW / |u|. px, py are unused.
+template <int WPOW>
+struct ViewAngle {
+    float4 m0, m1;
+    float idu, d, e;
+    template <class TAB>
+    __device__ __forceinline__ ViewAngle(TAB tab, int a, float x, float)
+        : m0(table4(tab, 3 * a)), m1(table4(tab, 3 * a + 1)), idu(table4(tab, 3 * a + 2).x) {
+        d = fmaf(m0.x, x, m0.z);
+        e = fmaf(m1.x, x, m1.z);
+    }
+    __device__ __forceinline__ void at(float y, float, float, float &u, float &wt) const {
+        const float w = m0.w * __builtin_amdgcn_rcpf(fmaf(m0.y, y, d));
+        u = fmaf(w, fmaf(m1.y, y, e), m1.w);
+        wt = (WPOW == 2 ? w * w : w) * idu;
+    }
+};
+
+// acc[k] += sum over angles [a0, a1) for the pixels (x, y[k]). `R` covers [A][D + 4].
+template <class SS, class ANGLE, int NY, class TAB>
+__device__ __forceinline__ void bp2d_angles(rsrc_t R, TAB tab, int a0, int a1, int D, float x,
+                                            float px, const float (&y)[NY], const float (&py)[NY],
+                                            float c0, float (&acc)[NY]) {
+    constexpr int UA = NY == 1 ? 4 : 2; // angles whose loads are in flight together
     const int Dp = D + 2 * kPadDet;
     const float hi = (float)D;
-    const float c0 = half_d - 0.5f; // D/2 and the texel-centre shift of the lerp, exact
-    float acc = 0.0f;
-    int row = kPadDet;
-    // one angle's sample: weight and lerp fraction, with the tap pair loaded
-    auto sample = [&](const float4 m, int r, float &wt, float &al, Pair &p) {
-        const float depth = fmaf(m.x, x, fmaf(-m.y, y, m.w)); // xi + DSO
-        const float eta = fmaf(m.y, px, m.x * py);
-        const float w = m.z * __builtin_amdgcn_rcpf(depth);
-        const float u = __builtin_amdgcn_fmed3f(fmaf(w, eta, c0), -2.0f, hi);
-        al = __builtin_amdgcn_fractf(u);
-        wt = WPOW == 2 ? w * w : w;
-        p = buf_pair<SS>(R, r + floor_i32(u), 0);
+    int row = a0 * Dp + kPadDet;
+    auto some = [&](int a, auto count) {
+        constexpr int N = decltype(count)::value;
+        float wt[N][NY], al[N][NY];
+        Pair p[N][NY];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const ANGLE g(tab, a + j, x, px); // wave-uniform table entries: scalar loads
+#pragma unroll
+            for (int k = 0; k < NY; ++k) {
+                float u;
+                g.at(y[k], py[k], c0, u, wt[j][k]);
+                u = __builtin_amdgcn_fmed3f(u, -2.0f, hi);
+                al[j][k] = __builtin_amdgcn_fractf(u);
+                p[j][k] = buf_pair<SS>(R, row + j * Dp + floor_i32(u), 0);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+#pragma unroll
+            for (int k = 0; k < NY; ++k)
+                acc[k] = fmaf(lerp_pair(p[j][k], al[j][k]), wt[j][k], acc[k]);
     };
-    int a = 0;
-    for (; a + 3 < A; a += 4, row += 4 * Dp) { // four loads in flight
-        float wt[4], al[4];
-        Pair p[4];
+    int a = a0;
+    for (; a + UA <= a1; a += UA, row += UA * Dp) some(a, std::integral_constant<int, UA>{});
+    for (; a < a1; ++a, row += Dp) some(a, std::integral_constant<int, 1>{});
+}
+
+// The tile's sums over all angles: wavefront q returns those of row q (NY = 4), or wavefront 0
+// those of the one row (NY = 1; the others return 0). All 256 threads of the workgroup call it;
+// ix, iy0 the thread's column and the tile's first row; `red` 4 NY 64 floats of LDS.
+template <class SS, class ANGLE, int NY, class TAB>
+__device__ __forceinline__ float bp2d_tile(rsrc_t R, TAB tab, int A, int D, int nx, int ny, int ix,
+                                           int iy0, float sx, float sy, float ox, float oy,
+                                           float inv_du, float half_d, float *red) {
+    static_assert(NY == 1 || NY == 4, "a wavefront finishes one row");
+    const float x = ((float)ix - (float)nx / 2.0f) * sx + ox + 0.5f;
+    float y[NY], py[NY], acc[NY];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) sample(table4(meta, a + k), row + k * Dp, wt[k], al[k], p[k]);
+    for (int k = 0; k < NY; ++k) {
+        y[k] = ((float)(iy0 + k) - (float)ny / 2.0f) * sy + oy + 0.5f;
+        py[k] = y[k] * inv_du;
+        acc[k] = 0.0f;
+    }
+    const int lane = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int a0 = (int)((int64_t)A * q / 4), a1 = (int)((int64_t)A * (q + 1) / 4);
+    // D/2 and the texel-centre shift of the lerp, exact
+    bp2d_angles<SS, ANGLE, NY>(R, tab, a0, a1, D, x, x * inv_du, y, py, half_d - 0.5f, acc);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) acc = fmaf(fmaf(al[k], p[k].hi - p[k].lo, p[k].lo), wt[k], acc);
-    }
-    for (; a < A; ++a, row += Dp) {
-        float wt, al;
-        Pair p;
-        sample(table4(meta, a), row, wt, al, p);
-        acc = fmaf(fmaf(al, p.hi - p.lo, p.lo), wt, acc);
-    }
-    return acc;
+    for (int k = 0; k < NY; ++k) red[(q * NY + k) * 64 + lane] = acc[k];
+    __syncthreads();
+    if (q >= NY) return 0.0f;
+    const float *r = red + q * 64 + lane;
+    return (r[0] + r[2 * NY * 64]) + (r[NY * 64] + r[3 * NY * 64]);
 }
 
 // Sum over angles for kZB consecutive voxels of one (x, y) column. M[a] is a 3x4 matrix over

@@ -538,63 +538,46 @@ __global__ __launch_bounds__(kFwdRays) void k_fwd2d(const typename SI::raw *__re
 
 // ---------------------------------------------------------------- backprojection ---------
 
-// One thread per pixel, all angles in one pass (backward_2d.hpp:31-99):
-// vol[b][y][x] += (1/du) sum_a w_a^WPOW lerp(sino[b][a], w_a eta_a + D/2),  w_a = DSD/(xi_a + DSO).
-// WPOW = 1 is the reference's weighting; WPOW = 2 the fan-beam FBP distance weight.
-template <class SV, class SS, int WPOW>
+// Quadrant tiles (times the batch) from which k_bp2d_qt backprojects a plan with quarter turns;
+// fewer do not fill the GPU, and k_bp2d, whose workgroups own 64 pixels instead of 4 x 256, gives
+// the same bits sooner. Calls of n^2 images with n angles, us (the host takes 22 of them): n = 256
+// (64 tiles) 23 against 34, 384 (144 tiles) 41 against 47, 512 (256 tiles) 72 against 59, 1024
+// (1024 tiles) 470 against 238.
+constexpr uint64_t kQTMinTiles = 200;
+
+// 64 x 4 tiles (times the batch) from which a workgroup of k_bp2d takes four rows of a plan from
+// views instead of one: 383 x 451 x 501 BF16 (768 tiles) 191 us a forward and backprojection
+// against 203, and smaller images need the workgroups. Circular plans have fewer constants to
+// share and always take one row: 1024^2 x 1024 470 us against 475, 512^2 x 512 72 against 78,
+// 256^2 x 256 23 against 28.
+constexpr uint64_t kViewRowTiles = 512;
+
+// A workgroup per 64 x NY pixel tile, all angles in one pass, a quarter of them per wavefront
+// (backward_2d.hpp:31-99): vol[b][y][x] += f sum_a wt_a lerp(sino[b][a], u_a), ANGLE the plan's
+// projection (bp_tiles.hpp: FanAngle, f = 1/du; ViewAngle, whose weight holds 1/|u_a|, f = 1).
+// Bound by the gathers (64 lanes in about 16 clocks per CU) and VALU issue (15 to 18) alike.
+// Against a thread per pixel for all angles: 256^2 x 256 41 -> 23 us a call, 320^2 x 320 48 -> 28,
+// 1024^2 x 1024 unchanged; 383 x 451 x 501 BF16 from views (whose loop over the angles had one
+// load in flight) 164 -> 30 us.
+template <class SV, class SS, class ANGLE, int NY>
 __global__ __launch_bounds__(kMaxBlock) void k_bp2d(typename SV::raw *__restrict__ vol,
                                                     const typename SS::raw *__restrict__ spad,
-                                                    const float4 *__restrict__ meta, int nx,
+                                                    const float4 *__restrict__ tab, int nx,
                                                     int ny, int D, int A, float sx, float sy,
                                                     float ox, float oy, float inv_du,
-                                                    float half_d) {
-    const int ix = blockIdx.x * blockDim.x + threadIdx.x;
-    const int iy = blockIdx.y * blockDim.y + threadIdx.y;
-    if (ix >= nx || iy >= ny) return;
+                                                    float half_d, float f) {
+    __shared__ float red[4 * NY * 64];
+    const unsigned tx = (unsigned)(nx + 63) / 64; // tiles per row
+    const int wv = threadIdx.x >> 6, iy0 = (int)(blockIdx.x / tx) * NY, iy = iy0 + wv;
+    const int ix = (int)(blockIdx.x % tx) * 64 + (int)(threadIdx.x & 63);
     const size_t b = blockIdx.z;
     const uint32_t sino_elems = (uint32_t)A * (D + 2 * kPadDet);
     const rsrc_t R = make_rsrc(spad + b * sino_elems, bytes_of<SS>(sino_elems));
-    const float x = ((float)ix - (float)nx / 2.0f) * sx + ox + 0.5f;
-    const float y = ((float)iy - (float)ny / 2.0f) * sy + oy + 0.5f;
-    const float acc = bp2d_pixel<SS, WPOW>(R, meta, A, D, x, y, x * inv_du, y * inv_du, half_d);
+    const float acc = bp2d_tile<SS, ANGLE, NY>(R, tab, A, D, nx, ny, ix, iy0, sx, sy, ox, oy,
+                                               inv_du, half_d, red);
+    if (wv >= NY || ix >= nx || iy >= ny) return;
     const size_t i = b * (size_t)nx * ny + (size_t)iy * nx + ix;
-    vol[i] = from_f32<SV>(to_f32<SV>(vol[i]) + acc * inv_du);
-}
-
-// The same for a plan built from ASTRA-like views (geometry2d.hpp bp_view): per view,
-// depth = n . x + n0, w = L / depth, cell coordinate w (e . x + e0) + c0, weight w^WPOW / |u|.
-// vol[b][y][x] += sum_a w_a^WPOW / |u_a| lerp(sino[b][a], cell_a).
-template <class SV, class SS, int WPOW>
-__global__ __launch_bounds__(kMaxBlock) void k_bp2d_vec(typename SV::raw *__restrict__ vol,
-                                                        const typename SS::raw *__restrict__ spad,
-                                                        const float4 *__restrict__ bpv, int nx,
-                                                        int ny, int D, int A, float sx, float sy,
-                                                        float ox, float oy) {
-    const int ix = blockIdx.x * blockDim.x + threadIdx.x;
-    const int iy = blockIdx.y * blockDim.y + threadIdx.y;
-    if (ix >= nx || iy >= ny) return;
-    const size_t b = blockIdx.z;
-    const int Dp = D + 2 * kPadDet;
-    const uint32_t sino_elems = (uint32_t)A * Dp;
-    const rsrc_t R = make_rsrc(spad + b * sino_elems, bytes_of<SS>(sino_elems));
-    const float x = ((float)ix - (float)nx / 2.0f) * sx + ox + 0.5f;
-    const float y = ((float)iy - (float)ny / 2.0f) * sy + oy + 0.5f;
-    const float hi = (float)D;
-    float acc = 0.0f;
-    int row = kPadDet;
-#pragma unroll 4
-    for (int a = 0; a < A; ++a, row += Dp) {
-        const float4 m0 = bpv[3 * a], m1 = bpv[3 * a + 1]; // wave-uniform: scalar loads
-        const float idu = bpv[3 * a + 2].x;
-        const float w = m0.w * __builtin_amdgcn_rcpf(fmaf(m0.x, x, fmaf(m0.y, y, m0.z)));
-        const float eta = fmaf(m1.x, x, fmaf(m1.y, y, m1.z));
-        const float u = __builtin_amdgcn_fmed3f(fmaf(w, eta, m1.w), -2.0f, hi); // c0 - 0.5
-        const float al = __builtin_amdgcn_fractf(u);
-        const Pair p = buf_pair<SS>(R, row + floor_i32(u), 0);
-        acc = fmaf(fmaf(al, p.hi - p.lo, p.lo), (WPOW == 2 ? w * w : w) * idu, acc);
-    }
-    const size_t i = b * (size_t)nx * ny + (size_t)iy * nx + ix;
-    vol[i] = from_f32<SV>(to_f32<SV>(vol[i]) + acc);
+    vol[i] = from_f32<SV>(to_f32<SV>(vol[i]) + acc * f);
 }
 
 // Backprojection by quarter turns, for square images (n even, unit pixels, no offset) whose
@@ -606,142 +589,170 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp2d_vec(typename SV::raw *__rest
 // sample of row a to P, of row a + A/4 to (y, -x), of row a + A/2 to (-x, -y) and of row
 // a + 3A/4 to (-y, x): four pixels per geometry evaluation. In index terms, with h = n/2 and
 // P = (ix, iy) in the quadrant [0, h)^2: (iy, n-1-ix), (n-1-ix, n-1-iy), (n-1-iy, ix).
-// A workgroup owns a 16 x 16 tile of the quadrant. Per chunk of 16 angles, every wavefront
+// A workgroup owns a 16 x 16 tile of the quadrant. Per chunk of 8 angles, every wavefront
 // projects the tile's corners (lanes 4j .. 4j+3 for angle j of the chunk), the four rows of each
 // angle share that footprint (the four rotated tiles project alike), and the workgroup stages
 // the four rows' footprint segments (64 cells) into LDS with 16-byte loads while the previous
 // chunk is sampled from the other buffer. Samples read their tap pair from LDS at immediate
-// offsets, one address per angle for all four rows. The plan checks the symmetry and that every
-// footprint fits a segment; the per-lane clamp keeps every LDS read inside its segment.
-constexpr int kQT = 16;            // tile edge, pixels
-constexpr int kQThreads = kQT * kQT;
-constexpr int kQChunk = 16;        // angles per staged chunk
-constexpr int kQSeg = 64;          // staged cells per row
-static_assert(kQThreads == 256 && kQChunk * 4 * (kQSeg / 4) == 4 * kQThreads,
-              "each thread stages four quads per chunk");
+// offsets, one address per angle for all four rows. The plan checks the symmetry (in the FP32
+// table too) and that every footprint fits a segment.
+// Positions, weights and the order of the sums are those of the per-pixel path (bp_tiles.hpp:
+// FanAngle, quarters of the angles), so the two agree bit for bit: the geometry of an angle is
+// evaluated for P alone, and for the pixel turned k quarters the quarters of the angles come in
+// the order k, k + 1, k + 2, k + 3 (mod 4), under which (S0 + S2) + (S1 + S3) does not change.
+// Two halves of the workgroup (four wavefronts each) take quarters 0 and 2 and quarters 1 and 3
+// of the angles for the same pixels, each with its own LDS buffers, and the second half's sums
+// join through LDS. The kernel is bound by latency (per angle a scalar load, a reciprocal and an
+// LDS read in a row) at VALU 0.7 and LDS 0.8 of their issue rates, so wavefronts count: one half
+// alone with chunks of 16 angles (94 VGPRs, five wavefronts per SIMD; four for want of tiles at
+// 1024^2) took 188 us at 1024^2 x 720 and 4.4 ms at 2048^2 x 4096 FP16, two halves with chunks of
+// 8 (54 VGPRs, eight per SIMD) 174 us and 3.8 ms. The constants through vector loads, which
+// would let their instructions issue at the full rate: 195 us and 4.7 ms. With a weight of w^2
+// per pixel and angle through k_bp2d, 2048^2 x 4096 FP16 took 7.3 ms.
+constexpr int kQT = 16;              // tile edge, pixels
+constexpr int kQHalf = kQT * kQT;    // threads per half
+constexpr int kQThreads = 2 * kQHalf;
+constexpr int kQChunk = 8;           // angles per staged chunk
+constexpr int kQSeg = 64;            // staged cells per row
+constexpr int kQBuf = kQChunk * 4 * kQSeg; // floats per chunk: [angle][row k][cell]
+static_assert(kQHalf == 256 && kQBuf / 4 == 2 * kQHalf, "each thread stages two quads per chunk");
 
 template <class SV, class SS, int WPOW>
 __global__ __launch_bounds__(kQThreads) void k_bp2d_qt(typename SV::raw *__restrict__ vol,
                                                        const typename SS::raw *__restrict__ spad,
                                                        const float4 *__restrict__ meta, int n,
                                                        int D, int A, float inv_du, float half_d) {
-    __shared__ float seg[2][kQChunk * 4 * kQSeg]; // two chunks of [angle][row k][cell]
+    __shared__ float seg[2][2][kQBuf]; // [half][buffer]
     const int h = n / 2, Q = A / 4, Dp = D + 2 * kPadDet;
     const size_t b = blockIdx.z;
     const uint32_t sino_elems = (uint32_t)A * Dp;
     const rsrc_t R = make_rsrc(spad + b * sino_elems, bytes_of<SS>(sino_elems));
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int hf = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int t = threadIdx.x & (kQHalf - 1), lane = t & 63, wv = t >> 6;
     const int bx = blockIdx.x * kQT, by = blockIdx.y * kQT;
     const int ix = bx + (t & (kQT - 1)), iy = by + t / kQT;
-    const float x = (float)ix - (float)h + 0.5f, y = (float)iy - (float)h + 0.5f;
+    // lanes past the quadrant's edge follow its last pixel (their sums are dropped)
+    const float x = (float)min(ix, h - 1) - (float)h + 0.5f;
+    const float y = (float)min(iy, h - 1) - (float)h + 0.5f;
     const float px = x * inv_du, py = y * inv_du;
-    const float hi = (float)D + 2.0f;     // padded coordinates: the row's zero border included
-    const float c2 = half_d - 0.5f + 2.0f; // D/2, the lerp's texel-centre shift and the border
+    const float hi = (float)D;
+    const float c0 = half_d - 0.5f; // D/2 and the lerp's texel-centre shift
     // the tile corner (pixel centre) this lane projects for angle lane >> 2 of a chunk
     const int cxi = (lane & 1) ? min(bx + kQT - 1, h - 1) : bx;
     const int cyi = (lane & 2) ? min(by + kQT - 1, h - 1) : by;
     const float qx = (float)cxi - (float)h + 0.5f, qy = (float)cyi - (float)h + 0.5f;
     const float qpx = qx * inv_du, qpy = qy * inv_du;
-    // staging share: quads q = t & 15 of row k = (t >> 4) & 3 of angles j = wv + 4 m, m < 4
+    // staging share: quads q = t & 15 of row k = (t >> 4) & 3 of angles j = wv + 4 m, m < 2
     const int sq = t & 15, sk = (t >> 4) & 3;
     constexpr int esz = (int)sizeof(typename SS::raw);
+    // the half's angle i, i in [0, 2 Q): quarter hf, then quarter hf + 2
+    auto angle = [&](int i) { return i + (i < Q ? hf : hf + 1) * Q; };
 
-    // Per chunk c, lanes 4 j .. 4 j + 3 of every wavefront hold angle j's segment: s0 (its first
-    // padded cell), c2 - s0 (the sample coordinate's constant in segment coordinates) and the
-    // largest lower-tap coordinate min(D + 2 - s0, kQSeg - 2) (the row's end, or the segment's).
-    struct Seg {
-        int s0;
-        float c2s, hi;
-    };
-    auto footprint = [&](int c) -> Seg {
-        const int a = min(c + (lane >> 2), A - 1);
-        const float4 m = meta[a];
+    // Per chunk of angles from i = c on, lanes 4 j .. 4 j + 3 of every wavefront hold the first
+    // padded cell of angle c + j's segment.
+    auto footprint = [&](int c) -> int {
+        const float4 m = meta[angle(min(c + ((lane >> 2) & (kQChunk - 1)), 2 * Q - 1))];
         const float depth = fmaf(m.x, qx, fmaf(-m.y, qy, m.w));
         const float eta = fmaf(m.y, qpx, m.x * qpy);
         const float w = m.z * __builtin_amdgcn_rcpf(depth);
-        float v = __builtin_amdgcn_fmed3f(fmaf(w, eta, c2), 0.0f, hi);
+        float v = __builtin_amdgcn_fmed3f(fmaf(w, eta, c0), -2.0f, hi);
         v = fminf(v, __shfl_xor(v, 1, 64));
         v = fminf(v, __shfl_xor(v, 2, 64));
-        // at most Dp - kQSeg, so that a segment never runs past its row (the plan requires
-        // Dp >= kQSeg): no staged quad reads another row or straddles the array's end
-        const int s0 = min(max(floor_i32(v) - 1, 0), Dp - kQSeg);
-        return {s0, c2 - (float)s0, fminf(hi - (float)s0, (float)(kQSeg - 2))};
+        // one cell of margin for the corners' rounding; at most Dp - kQSeg, so that a segment
+        // never runs past its row (the plan requires Dp >= kQSeg): no staged quad reads another
+        // row or straddles the array's end
+        return min(max(floor_i32(v) - 1 + kPadDet, 0), Dp - kQSeg);
     };
-    auto load = [&](int c, int s0v, Quad (&qd)[4]) {
+    auto load = [&](int c, int s0v, Quad (&qd)[2]) {
 #pragma unroll
-        for (int mm = 0; mm < 4; ++mm) {
+        for (int mm = 0; mm < 2; ++mm) {
             const int j = wv + 4 * mm;
             const int s0 = __builtin_amdgcn_readlane(s0v, 4 * j);
             // row of angle c + j (past the last angle: the last one's, loaded and unused),
             // turned by k quarters
-            int r = min(c + j, A - 1) + sk * Q;
+            int r = angle(min(c + j, 2 * Q - 1)) + sk * Q;
             r = r >= A ? r - A : r;
             qd[mm] = buf_quad_at<SS>(R, (r * Dp + s0 + 4 * sq) * esz);
         }
     };
-    auto store = [&](int buf, const Quad (&qd)[4]) {
+    auto store = [&](int buf, const Quad (&qd)[2]) {
 #pragma unroll
-        for (int mm = 0; mm < 4; ++mm) {
+        for (int mm = 0; mm < 2; ++mm) {
             const int j = wv + 4 * mm;
-            *reinterpret_cast<float4 *>(&seg[buf][(j * 4 + sk) * kQSeg + 4 * sq]) =
+            *reinterpret_cast<float4 *>(&seg[hf][buf][(j * 4 + sk) * kQSeg + 4 * sq]) =
                 make_float4(qd[mm].v[0], qd[mm].v[1], qd[mm].v[2], qd[mm].v[3]);
         }
     };
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    // angle c + j of a chunk whose segments are in `sg`; TAIL: the angle may lie past the last
-    // one (then it adds nothing)
-    auto sample = [&](int c, int j, const Seg &sg, int bufofs, auto tail) {
-        constexpr bool TAIL = decltype(tail)::value;
-        if (TAIL && c + j >= A) return;
-        const float4 m = meta[c + j]; // wave-uniform: scalar loads
-        const float depth = fmaf(m.x, x, fmaf(-m.y, y, m.w)); // xi + DSO
-        const float eta = fmaf(m.y, px, m.x * py);
-        const float w = m.z * __builtin_amdgcn_rcpf(depth);
-        const float c2s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sg.c2s), 4 * j));
-        const float hj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sg.hi), 4 * j));
-        const float l = __builtin_amdgcn_fmed3f(fmaf(w, eta, c2s), 0.0f, hj);
-        const float al = __builtin_amdgcn_fractf(l);
-        const float wt = WPOW == 2 ? w * w : w;
-        // byte offset of the angle's four rows, opaque in a scalar register so that the rows
-        // stay immediate offsets of one address
-        int jb = bufofs + j * 4 * kQSeg * 4;
+    // angle c + j of a chunk whose segments start at s0v
+    auto sample = [&](int a, int j, int s0v, int bufofs) {
+        const FanAngle<WPOW> g(meta, a, x, px); // wave-uniform: scalar loads
+        float u, wt;
+        g.at(y, py, c0, u, wt);
+        u = __builtin_amdgcn_fmed3f(u, -2.0f, hi);
+        const float al = __builtin_amdgcn_fractf(u);
+        // byte offset of the angle's four rows less that of the segment's first cell, opaque in
+        // a scalar register so that the rows stay immediate offsets of one address
+        int jb = bufofs + j * 4 * kQSeg * 4 - 4 * (__builtin_amdgcn_readlane(s0v, 4 * j) - kPadDet);
         asm("" : "+s"(jb));
         const float *p = reinterpret_cast<const float *>(
-            reinterpret_cast<const char *>(&seg[0][0]) + jb) + floor_i32(l);
+            reinterpret_cast<const char *>(&seg[0][0][0]) + jb) + floor_i32(u);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const float lo = p[k * kQSeg], up = p[k * kQSeg + 1];
             acc[k] = fmaf(fmaf(al, up - lo, lo), wt, acc[k]);
         }
     };
-    using False = std::false_type;
-    using True = std::true_type;
-    Quad qd[4];
-    Seg sg = footprint(0);
-    load(0, sg.s0, qd);
+    float sum[4]; // the half's first quarter
+    auto flush = [&]() {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            sum[k] = acc[k];
+            acc[k] = 0.0f;
+        }
+    };
+    Quad qd[2];
+    int s0 = footprint(0);
+    load(0, s0, qd);
     store(0, qd);
     __syncthreads();
     int cur = 0;
-    for (int c = 0; c < A; c += kQChunk, cur ^= 1) {
+    for (int c = 0; c < 2 * Q; c += kQChunk, cur ^= 1) {
         // next chunk's loads in flight while this one is sampled
         const int cn = c + kQChunk;
-        Seg sn{};
-        if (cn < A) {
+        int sn = 0;
+        if (cn < 2 * Q) {
             sn = footprint(cn);
-            load(cn, sn.s0, qd);
+            load(cn, sn, qd);
         }
-        const int bufofs = cur * kQChunk * 4 * kQSeg * 4;
-        if (cn <= A) {
+        const int bufofs = (2 * hf + cur) * kQBuf * 4;
+        if (cn <= Q || (c >= Q && cn <= 2 * Q)) { // inside a quarter
+            const int a = angle(c);
 #pragma unroll
-            for (int j = 0; j < kQChunk; ++j) sample(c, j, sg, bufofs, False{});
-        } else {
+            for (int j = 0; j < kQChunk; ++j) sample(a + j, j, s0, bufofs);
+            if (cn == Q) flush();
+        } else { // the quarter, or the last one, ends in the chunk
 #pragma unroll
-            for (int j = 0; j < kQChunk; ++j) sample(c, j, sg, bufofs, True{});
+            for (int j = 0; j < kQChunk; ++j)
+                if (c + j < 2 * Q) {
+                    sample(angle(c + j), j, s0, bufofs);
+                    if (c + j + 1 == Q) flush();
+                }
         }
-        if (cn < A) store(cur ^ 1, qd);
-        sg = sn;
+        if (cn < 2 * Q) store(cur ^ 1, qd);
+        s0 = sn;
         __syncthreads();
     }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sum[k] += acc[k];
+    // the second half's sums join the first's ((S0 + S2) + (S1 + S3))
+    if (hf)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) (&seg[0][0][0])[k * kQHalf + t] = sum[k];
+    __syncthreads();
+    if (hf) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sum[k] += (&seg[0][0][0])[k * kQHalf + t];
     if (ix >= h || iy >= h) return;
     const int m1 = n - 1;
     const int px4[4] = {ix, iy, m1 - ix, m1 - iy};
@@ -750,7 +761,7 @@ __global__ __launch_bounds__(kQThreads) void k_bp2d_qt(typename SV::raw *__restr
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const size_t i = (size_t)py4[k] * n + px4[k];
-        vb[i] = from_f32<SV>(to_f32<SV>(vb[i]) + acc[k] * inv_du);
+        vb[i] = from_f32<SV>(to_f32<SV>(vb[i]) + sum[k] * inv_du);
     }
 }
 
@@ -1388,13 +1399,15 @@ void set_plan_shape(cmi_plan2d &p, int device, int vol_prec, const uint64_t vol_
 // Whether the backprojection by quarter turns (k_bp2d_qt) applies: a square image with an even
 // side, unit pixels and no offset (the pixel centres, at (i - n/2) + 1/2 as the reference places
 // them, backward_2d.hpp:58-59, are then symmetric under quarter turns), angles in quadruples
-// a + k A/4 that are quarter turns apart with equal DSO and DSD, a padded detector row at least
-// as long as a staged segment, and every 16 x 16 tile's detector footprint within a staged
-// segment: the projection of a segment of length L at
+// a + k A/4 that are quarter turns apart with equal DSO and DSD, in the FP32 table too (entry
+// for entry the first quarter's sines and cosines exchanged; the zeros of one and the roundoff
+// of the other, below 1e-13, add to half-integers times ones without a trace), a padded detector
+// row at least as long as a staged segment, and every 16 x 16 tile's detector footprint within a
+// staged segment: the projection of a segment of length L at
 // depth >= DSO - r (r the largest pixel-centre radius) spans at most
 // L DSD / (DSO - r) sqrt(1 + (r / (DSO - r))^2) / du cells.
 bool quarter_turns(const fan2d::Scalars &g, const double *angles, const double *DSO,
-                   const double *DSD, int64_t A) {
+                   const double *DSD, int64_t A, const std::vector<float4> &meta) {
     if (g.nx != g.ny || g.nx % 2 != 0 || g.nx < 2 || g.sx != 1.0 || g.sy != 1.0 ||
         g.ox != 0.0 || g.oy != 0.0 || A % 4 != 0 || A < 4 || g.D + 2 * kPad < kQSeg)
         return false;
@@ -1411,6 +1424,14 @@ bool quarter_turns(const fan2d::Scalars &g, const double *angles, const double *
             if (DSO[b] != DSO[a] || DSD[b] != DSD[a]) return false;
             double d = std::remainder(angles[b] - angles[a] - (double)k * M_PI / 2.0, 2.0 * M_PI);
             if (std::fabs(d) > 1e-9) return false;
+            // (-sin, cos) of the angle turned by k quarters
+            const float4 m = meta[a], t = meta[b];
+            const float tx = k == 1 ? -m.y : k == 2 ? -m.x : m.y;
+            const float ty = k == 1 ? m.x : k == 2 ? -m.y : -m.x;
+            auto same = [](float p, float q) {
+                return p == q || (std::fabs(p) < 1e-13f && std::fabs(q) < 1e-13f);
+            };
+            if (!same(t.x, tx) || !same(t.y, ty)) return false;
         }
     }
     const double span = wmax * (kQT - 1) * std::sqrt(2.0) / g.du;
@@ -1649,7 +1670,7 @@ CMI_API cmi_status cmi_plan2d_create(int device, int vol_prec, const uint64_t vo
         geo[a] = fan2d::plan_angle(p->g, angles[a], DSO[a], DSD[a]);
         meta[a] = bp2d_meta(angles[a], DSO[a], DSD[a]);
     }
-    p->quarter = quarter_turns(p->g, angles, DSO, DSD, A);
+    p->quarter = quarter_turns(p->g, angles, DSO, DSD, A, meta);
     return finish_plan2d(std::move(p), geo, meta, {}, plan);
 }
 
@@ -1821,26 +1842,32 @@ CMI_API cmi_status cmi_backward_2d_weighted(const cmi_plan2d *plan, void *volume
         dim3 pb(256), pg((unsigned)((Dp + 255) / 256), (unsigned)A, (unsigned)batch);
         hipLaunchKernelGGL((k_stage_sino2d<SS>), pg, pb, 0, s, (const RS *)sinogram,
                            (RS *)scratch, D, A);
-        dim3 b(64, 4), g((unsigned)((nx + 63) / 64), (unsigned)((ny + 3) / 4), (unsigned)batch);
-        if (plan->d_bpv) {
-            auto kern = weighting == CMI_BP2D_FBP ? k_bp2d_vec<SV, SS, 2> : k_bp2d_vec<SV, SS, 1>;
-            hipLaunchKernelGGL(kern, g, b, 0, s, (typename SV::raw *)volume, (const RS *)scratch,
-                               plan->d_bpv, nx, ny, D, A, (float)plan->g.sx, (float)plan->g.sy,
-                               (float)plan->g.ox, (float)plan->g.oy);
-        } else if (plan->quarter && weighting == CMI_BP2D_REFERENCE) {
-            // (the FBP weighting keeps the per-pixel body, which the serving kernels share, so
-            // that a served FBP volume equals the plain one bit for bit)
-            const unsigned th = (unsigned)((nx / 2 + kQT - 1) / kQT);
-            auto kern = k_bp2d_qt<SV, SS, 1>;
-            hipLaunchKernelGGL(kern, dim3(th, th, (unsigned)batch), dim3(kQThreads), 0, s,
-                               (typename SV::raw *)volume, (const RS *)scratch, plan->d_meta, nx,
-                               D, A, (float)(1.0 / plan->g.du), (float)D / 2.0f);
+        const bool fbp = weighting == CMI_BP2D_FBP;
+        const float inv_du = (float)(1.0 / plan->g.du), half_d = (float)D / 2.0f;
+        const uint64_t th = (uint64_t)(nx / 2 + kQT - 1) / kQT;
+        if (plan->quarter && th * th * batch >= kQTMinTiles) {
+            auto kern = fbp ? k_bp2d_qt<SV, SS, 2> : k_bp2d_qt<SV, SS, 1>;
+            hipLaunchKernelGGL(kern, dim3((unsigned)th, (unsigned)th, (unsigned)batch),
+                               dim3(kQThreads), 0, s, (typename SV::raw *)volume,
+                               (const RS *)scratch, plan->d_meta, nx, D, A, inv_du, half_d);
         } else {
-            auto kern = weighting == CMI_BP2D_FBP ? k_bp2d<SV, SS, 2> : k_bp2d<SV, SS, 1>;
-            hipLaunchKernelGGL(kern, g, b, 0, s, (typename SV::raw *)volume, (const RS *)scratch,
-                               plan->d_meta, nx, ny, D, A, (float)plan->g.sx, (float)plan->g.sy,
-                               (float)plan->g.ox, (float)plan->g.oy, (float)(1.0 / plan->g.du),
-                               (float)D / 2.0f);
+            const unsigned tx = (unsigned)(nx + 63) / 64;
+            auto launch = [&](auto kern, int rows, const float4 *tab, float f) {
+                const unsigned tiles = tx * (unsigned)((ny + rows - 1) / rows);
+                hipLaunchKernelGGL(kern, dim3(tiles, 1, (unsigned)batch), dim3(kMaxBlock), 0, s,
+                                   (typename SV::raw *)volume, (const RS *)scratch, tab, nx, ny,
+                                   D, A, (float)plan->g.sx, (float)plan->g.sy,
+                                   (float)plan->g.ox, (float)plan->g.oy, inv_du, half_d, f);
+            };
+            if (!plan->d_bpv)
+                launch(fbp ? k_bp2d<SV, SS, FanAngle<2>, 1> : k_bp2d<SV, SS, FanAngle<1>, 1>, 1,
+                       plan->d_meta, inv_du);
+            else if ((uint64_t)tx * ((ny + 3) / 4) * batch >= kViewRowTiles)
+                launch(fbp ? k_bp2d<SV, SS, ViewAngle<2>, 4> : k_bp2d<SV, SS, ViewAngle<1>, 4>,
+                       4, plan->d_bpv, 1.0f);
+            else
+                launch(fbp ? k_bp2d<SV, SS, ViewAngle<2>, 1> : k_bp2d<SV, SS, ViewAngle<1>, 1>,
+                       1, plan->d_bpv, 1.0f);
         }
         CMI_HIP_TRY(hipGetLastError());
         return CMI_OK;

@@ -13,7 +13,7 @@
 //   workgroup exits after at most total + grid iterations of the counter, so the launch
 //   drains.
 //
-// Per-tile arithmetic is the plain backprojectors' own (bp2d_pixel / bp3d_column with the
+// Per-tile arithmetic is the plain backprojectors' own (bp2d_tile / bp3d_column with the
 // same scalar inputs), so a voxel's value does not depend on the launch it ran in.
 //
 // Data layout in HBM (per server)
@@ -147,21 +147,22 @@ __global__ __launch_bounds__(64) void k_zero_counter2(unsigned *__restrict__ c) 
 
 // ---------------------------------------------------------------- tiles -------------------
 
-// Fan-beam tile: pixel (ix, iy) as k_bp2d computes it.
+// Fan-beam tile: the 64 x 4 pixels a workgroup of k_bp2d computes. Every thread of the workgroup
+// calls this.
 template <class SV, class SS>
-__device__ __forceinline__ void serve_tile_2d(const DevJob &J, uint32_t t) {
+__device__ __forceinline__ void serve_tile_2d(const DevJob &J, uint32_t t, float *red) {
     const int tx = (int)(t % (uint32_t)J.tiles_x), ty = (int)(t / (uint32_t)J.tiles_x);
-    const int ix = tx * kTile2X + (int)(threadIdx.x % kTile2X);
-    const int iy = ty * kTile2Y + (int)(threadIdx.x / kTile2X);
-    if (ix >= J.nx || iy >= J.ny) return;
+    const int ix = tx * kTile2X + (int)(threadIdx.x & 63);
+    const int iy0 = ty * kTile2Y, iy = iy0 + (int)(threadIdx.x >> 6);
     const rsrc_t R = make_rsrc(J.sino, J.sino_bytes);
     const ctab meta = const_table(J.table);
-    const float x = ((float)ix - (float)J.nx / 2.0f) * J.sx + J.ox + 0.5f;
-    const float y = ((float)iy - (float)J.ny / 2.0f) * J.sy + J.oy + 0.5f;
-    const float px = x * J.inv_du, py = y * J.inv_du;
-    const float acc = J.mode == CMI_BP2D_FBP
-                          ? bp2d_pixel<SS, 2>(R, meta, J.nangles, J.nu, x, y, px, py, J.half_d)
-                          : bp2d_pixel<SS, 1>(R, meta, J.nangles, J.nu, x, y, px, py, J.half_d);
+    const float acc =
+        J.mode == CMI_BP2D_FBP
+            ? bp2d_tile<SS, FanAngle<2>, kTile2Y>(R, meta, J.nangles, J.nu, J.nx, J.ny, ix, iy0,
+                                                  J.sx, J.sy, J.ox, J.oy, J.inv_du, J.half_d, red)
+            : bp2d_tile<SS, FanAngle<1>, kTile2Y>(R, meta, J.nangles, J.nu, J.nx, J.ny, ix, iy0,
+                                                  J.sx, J.sy, J.ox, J.oy, J.inv_du, J.half_d, red);
+    if (ix >= J.nx || iy >= J.ny) return;
     auto *vol = static_cast<typename SV::raw *>(J.volume);
     const size_t i = (size_t)iy * J.nx + ix;
     vol[i] = from_f32<SV>(to_f32<SV>(vol[i]) + acc * J.inv_du);
@@ -257,18 +258,19 @@ __device__ __forceinline__ const DevJob &job_of(const DevJob *__restrict__ jobs,
     return jobs[lo];
 }
 
-// Fan-beam tiles. A kernel of its own: it needs no LDS and few registers, so more workgroups
+// Fan-beam tiles. A kernel of its own: it needs little LDS and few registers, so more workgroups
 // stay resident than for the cone-beam tiles (the 2D body is bound by issue and latency).
 template <class SV, class SS>
 __global__ __launch_bounds__(kThreads) void k_serve_bp2d(const DevJob *__restrict__ jobs,
                                                          int njobs, uint32_t total,
                                                          unsigned *__restrict__ counter) {
     __shared__ unsigned s_tile;
+    __shared__ float red[4 * kTile2Y * 64];
     for (;;) {
-        const uint32_t t = next_tile(counter, &s_tile);
+        const uint32_t t = next_tile(counter, &s_tile); // its barriers also order reuse of `red`
         if (t >= total) return;
         const DevJob &J = job_of(jobs, njobs, t);
-        serve_tile_2d<SV, SS>(J, t - J.first + J.tile_begin);
+        serve_tile_2d<SV, SS>(J, t - J.first + J.tile_begin, red);
     }
 }
 

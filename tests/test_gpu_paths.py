@@ -1,0 +1,83 @@
+"""Edges of the kernels' tiles, chunks and dispatch rules: the sizes at which a path begins, ends or
+hands over to another one, against the FP64 oracle or the other path.
+
+Tolerances are those of test_gpu_fan2d.py / test_gpu_cone3d.py: rel-L2 <= 1e-5 for FP32 storage and
+arithmetic against FP64 (the operators' own errors are 1e-7 to 5e-6).
+"""
+import numpy as np
+import pytest
+import torch
+
+import curadon_amd as cm
+from geoms import as_fan_geometry, fan
+
+pytestmark = pytest.mark.gpu
+
+RTOL_L2 = 1e-5
+
+
+def rel_l2(a, b):
+    a = a.double().cpu().numpy() if isinstance(a, torch.Tensor) else a
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
+
+
+def rand(shape, gpu, seed, dtype=torch.float32):
+    g = torch.Generator().manual_seed(seed)
+    return torch.rand(shape, generator=g).to(device=gpu, dtype=dtype)
+
+
+@pytest.mark.parametrize("mode", ["reference", "fbp"])
+@pytest.mark.parametrize("n,D,A,prec", [
+    (34, 64, 4, torch.float32),    # one angle per quarter; quadrant of 17 pixels: ragged tile
+    (34, 64, 20, torch.float32),   # quarters of 5: two quarter ends in one chunk of 8
+    (64, 91, 36, torch.float32),   # quarters of 9: a chunk across the quarter's end
+    (64, 91, 64, torch.bfloat16),  # quarters of 16: whole chunks
+    (130, 187, 100, torch.float16),
+])
+def test_quarter_turns_equal_pixels(gpu, n, D, A, prec, mode):
+    """The backprojection by quarter turns (batches with enough tiles) and the per-pixel one (a
+    single small image) give the same bits."""
+    geom = as_fan_geometry(fan(n, D, A, 2.0 * n, 3.0 * n), vol_prec=prec, sino_prec=prec)
+    tiles = ((n // 2 + 15) // 16) ** 2
+    assert tiles < 200
+    batch = -(-200 // tiles)
+    y = rand((3, A, D), gpu, 1, prec)
+    many = y.repeat(-(-batch // 3), 1, 1)
+    got = cm.backward(many, geom, mode=mode)
+    for i in range(3):
+        one = cm.backward(y[i].contiguous(), geom, mode=mode)
+        assert torch.equal(got[i], one)
+        assert torch.equal(got[-3 + i], one)
+
+
+@pytest.mark.parametrize("A", [1, 2, 3, 5, 9])
+@pytest.mark.parametrize("ny,nx", [(5, 1), (3, 63), (4, 65)])
+@pytest.mark.parametrize("views", [False, True])
+def test_backward_few_angles_ragged(oracle, gpu, A, ny, nx, views):
+    """Quarters of the angles that are empty or unequal, tiles of 64 pixels with one lane in use,
+    one lane missing and one over."""
+    rec = fan(nx, 70, A, 150.0, 220.0, ny=ny)
+    y = np.random.RandomState(A).rand(A, 70)
+    if views:
+        rec.det_offset, rec.det_rotation, rec.COR, rec.exact_geometry = 1.5, 0.05, 0.75, True
+        geom = cm.FanGeometry(DSD=rec.DSD, DSO=rec.DSO, angles=rec.angles,
+                              vol_shape=rec.vol_shape, det_shape=rec.det_shape, det_offset=1.5,
+                              det_rotation=0.05, COR=0.75, exact_geometry=True)
+    else:
+        geom = as_fan_geometry(rec)
+    for mode, wpow in (("reference", 1), ("fbp", 2)):
+        ref = oracle.bp2d(geom, y, wpow=wpow)
+        got = cm.backward(torch.tensor(y, dtype=torch.float32, device=gpu), geom, mode=mode)
+        assert rel_l2(got, ref) <= RTOL_L2
+
+
+def test_view_rows_batched_equal_single(gpu):
+    """Plans from views: a batch large enough for four rows per thread gives the bits of single
+    images with one row per thread."""
+    geom = cm.FanGeometry(DSD=220.0, DSO=150.0, angles=np.linspace(0, 2, 11), vol_shape=(6, 65),
+                          det_shape=90, det_offset=1.5, exact_geometry=True)
+    y = rand((3, 11, 90), gpu, 5)
+    got = cm.backward(y.repeat(45, 1, 1), geom)    # 135 images x 4 tiles
+    for i in range(3):
+        one = cm.backward(y[i].contiguous(), geom)
+        assert torch.equal(got[i], one) and torch.equal(got[-3 + i], one)
