@@ -193,27 +193,27 @@ __global__ __launch_bounds__(kMaxBlock) void k_stage_panel(const typename S::raw
 
 // ---------------------------------------------------------------- forward -----------------
 
+// Trilinear interpolation of four pairs along the fast axis, at fractions ff, fm, fl: p00 (m, l),
+// p10 (m + 1, l), p01 (m, l + 1), p11 (m + 1, l + 1).
+__device__ __forceinline__ float trilerp(const Pair &p00, const Pair &p10, const Pair &p01,
+                                         const Pair &p11, float ff, float fm, float fl) {
+    const float a00 = lerp_pair(p00, ff), a10 = lerp_pair(p10, ff);
+    const float a01 = lerp_pair(p01, ff), a11 = lerp_pair(p11, ff);
+    const float b0 = fmaf(fm, a10 - a00, a00);
+    const float b1 = fmaf(fm, a11 - a01, a01);
+    return fmaf(fl, b1 - b0, b0);
+}
+
 // Trilinear sample at centred padded coordinates (f, m, l) along the copy's fast, middle and
 // slow axes. `cofs` is the element offset of the copy's centre; sM, sL, sML are the byte strides
 // of one step along the middle axis, the slow axis, and both.
 template <class SI>
 __device__ __forceinline__ float sample3d(rsrc_t R, float f, float m, float l, int Ef, int Em,
                                          int cofs, int sM, int sL, int sML) {
-    const int i_f = floor_i32(f), i_m = floor_i32(m), i_l = floor_i32(l);
-    const float ff = __builtin_amdgcn_fractf(f), fm = __builtin_amdgcn_fractf(m),
-                fl = __builtin_amdgcn_fractf(l);
-    const int o = __mul24(__mul24(i_l, Em) + i_m, Ef) + i_f + cofs;
-    const Pair p00 = buf_pair<SI>(R, o, 0);   // (m,     l)
-    const Pair p10 = buf_pair<SI>(R, o, sM);  // (m + 1, l)
-    const Pair p01 = buf_pair<SI>(R, o, sL);  // (m,     l + 1)
-    const Pair p11 = buf_pair<SI>(R, o, sML); // (m + 1, l + 1)
-    const float a00 = fmaf(ff, p00.hi - p00.lo, p00.lo);
-    const float a10 = fmaf(ff, p10.hi - p10.lo, p10.lo);
-    const float a01 = fmaf(ff, p01.hi - p01.lo, p01.lo);
-    const float a11 = fmaf(ff, p11.hi - p11.lo, p11.lo);
-    const float b0 = fmaf(fm, a10 - a00, a00);
-    const float b1 = fmaf(fm, a11 - a01, a01);
-    return fmaf(fl, b1 - b0, b0);
+    const float i_f = floorf(f), i_m = floorf(m), i_l = floorf(l);
+    const int o = __mul24(__mul24((int)i_l, Em) + (int)i_m, Ef) + (int)i_f + cofs;
+    return trilerp(buf_pair<SI>(R, o, 0), buf_pair<SI>(R, o, sM), buf_pair<SI>(R, o, sL),
+                   buf_pair<SI>(R, o, sML), f - i_f, m - i_m, l - i_l);
 }
 
 // LDS-staged march. The rays of a workgroup (16 x 16 detector pixels of one projection) lie
@@ -225,20 +225,36 @@ __device__ __forceinline__ float sample3d(rsrc_t R, float f, float m, float l, i
 // and every ray takes its samples whose lower tap lies in the slab from there, in its own order
 // j = 0 .. n - 1, slab after slab: positions and trilinear weights are those of a plain per-ray
 // march, and the ray's sum adds one partial sum per slab (at most about 2 kSlab samples each).
-// A sample outside the box (not expected; a safety net), and workgroups whose rays do not all
-// advance the same way along K or whose K is the copy's fast axis, read global memory instead,
-// with the same arithmetic (the latter in blocks of kSumBlock samples).
+// Slabs whose box does not fit, and workgroups whose rays do not all advance the same way along
+// K, whose K is the copy's fast axis, or in which FP32 puts a ray further than kBoxMargin / 2
+// outside the corner rays (a source so far away that its coordinates lose the voxel), read
+// global memory instead, with the same arithmetic (the latter in blocks of kSumBlock samples).
 // A wavefront covers 4 x 16 detector pixels, the 16 along v, and the copy read is the one
 // whose fastest axis v follows (fast[a]), so that a wavefront's rows of a staged box are runs
 // of consecutive voxels.
+//
+// The kernel is bound by VALU issue (1.55 wavefront instructions per clock and CU for fma, add and
+// mul of vector registers, 0.93 for conversions, floors, shifts, compares and whatever reads a
+// scalar register), with LDS at 0.7 of its rate. So:
+// * a sample's LDS address is three fma: the byte strides and the offset are held as FP32
+//   subnormals, n 2^-149, whose bit pattern is the integer n; products with the integral floors
+//   and their sums are exact below 2^23, and the sum's bits are the address (this needs FP32
+//   subnormals, which the compiler keeps unless told otherwise). Fractions are p - floor(p).
+// * the boxes of up to 64 slabs are found at once, one slab per lane, and read from the lanes.
+// * a thread stages quads tid, tid + 256, ... of the box's rows laid end to end: no lane idles in
+//   rows shorter than a power of two, and the LDS address is the quad's number.
+// * a slab's samples run in a loop counted by the wavefront's smallest count, in a scalar
+//   register, and a remainder counted per lane.
+// At 256^3 x 360, 384^2 panel: 15.0 -> 10.1 ms with these and boxes a voxel narrower on every
+// side (62 -> 45 VALU instructions per wavefront's sample, 9 % -> 2 % of the slabs not staged).
 // sino[b][a][iv][iu] = sum_{i=0..nst} trilinear(vol, s + (tmin + i dt) d)  (forward_3d.hpp:87-93)
-constexpr int kSlab = 8;          // slices of lower taps per slab
-// floats of one staged box (16 KiB). A smaller box keeps more workgroups per CU and sends more
-// slabs to the global path: at 256^3 the staged-box capacity in floats gave 2560: 18.3 ms,
-// 3072: 16.7, 3584: 16.3, 4096: 16.3, 4608: 16.5, 5120: 17.5, 5632: 17.6, 6144: 19.1
-// (bit-identical: both paths add the same values in the same order).
-constexpr int kBoxCells = 4096;
-constexpr int kBoxQuads = 8;      // at most 8 x 4 cells per staged row
+constexpr int kSlab = 10;         // slices of lower taps per slab
+// floats of one staged box (20 KiB). A smaller box keeps more workgroups per CU and sends more
+// slabs to the global path. (slices, floats) at 256^3 x 360 on a dense volume: (8, 3072) 11.3 ms,
+// (8, 4096) 11.2, (8, 5120) 11.2, (10, 4096) 11.3, (10, 5120) 10.9, (12, 6144) 11.3; two samples
+// per turn of the loop 11.1 to 11.2, and 64 VGPRs for eight wavefronts per SIMD 14.8 (spills).
+constexpr int kBoxCells = 5120;
+constexpr float kBoxMargin = 0.0625f; // voxels around the corner rays' crossings
 constexpr unsigned kFwdGroup = 32; // projections per group in the workgroup order
 
 template <class SI, class SS>
@@ -250,7 +266,6 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
                                                           int A,
                                                           typename SS::raw *__restrict__ sino) {
     __shared__ float4 box4[kBoxCells / 4];
-    float *box = reinterpret_cast<float *>(box4);
     __shared__ float cl[4][6]; // corner rays in padded index coordinates: point, direction
     __shared__ int red[2][kMaxBlock / 64];
     const int tid = threadIdx.x;
@@ -343,29 +358,47 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
     const int sK = kmid ? Ef : Ef * Em, sQ = kmid ? Ef * Em : Ef;
 
     float acc = 0.0f;
-    int j = 0;
     const int n = p.n;
-    float jf = p.j0;
-    // sample j at the forward's position, from global memory
+    float jf = p.j0;                       // the next sample (exact integers)
+    const float jend = p.j0 + (float)n;    // one past the last
+    // sample jf at the forward's position, from global memory
     auto global_sample = [&]() {
         return sample3d<SI>(R, fmaf(jf, tf, mf), fmaf(jf, tm, mm), fmaf(jf, tl, ml), Ef, Em,
                             cofs, sM, sL, sML);
     };
-    if (!__builtin_amdgcn_readfirstlane((int)slab_ok)) {
-        while (j < n) {
-            const int jend = min(j + kSumBlock, n);
-            float s0 = 0.0f;
-            for (; j < jend; ++j, jf += 1.0f) s0 += global_sample();
-            acc += s0;
+    // crossings of the corner rays with the plane of padded index k along K: the smallest and
+    // largest padded indices along P and Q
+    auto section = [&](float k, float &p0, float &p1, float &q0, float &q1) {
+        p0 = q0 = INFINITY;
+        p1 = q1 = -INFINITY;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float t = (k - cl[c][K]) * __builtin_amdgcn_rcpf(cl[c][3 + K]);
+            const float pc = fmaf(t, cl[c][3 + F], cl[c][F]), qc = fmaf(t, cl[c][3 + Q], cl[c][Q]);
+            p0 = fminf(p0, pc);
+            p1 = fmaxf(p1, pc);
+            q0 = fminf(q0, qc);
+            q1 = fmaxf(q1, qc);
         }
-    } else {
-        // lower-tap K range of the workgroup's samples
-        int klo = 0x7fffffff, khi = -0x7fffffff - 1;
+    };
+    // lower-tap K range of the workgroup's samples
+    int klo = 0x7fffffff, khi = -0x7fffffff - 1;
+    if (slab_ok) {
         if (n > 0) {
-            const int k0 = floor_i32(fmaf(p.j0, tK, mK)) + cK;
-            const int k1 = floor_i32(fmaf(p.j0 + (float)(n - 1), tK, mK)) + cK;
-            klo = min(k0, k1);
-            khi = max(k0, k1);
+            bool in = true;
+            for (int e = 0; e < 2; ++e) { // the first and the last sample
+                const float je = e ? jend - 1.0f : p.j0;
+                const float pk = fmaf(je, tK, mK);
+                const int kk = floor_i32(pk) + cK;
+                klo = min(klo, kk);
+                khi = max(khi, kk);
+                float p0, p1, q0, q1;
+                section(pk + (float)cK, p0, p1, q0, q1);
+                const float pp = fmaf(je, tP, mP) + (float)cP, pq = fmaf(je, tQ, mQ) + (float)cQ;
+                constexpr float tol = 0.5f * kBoxMargin;
+                in = in && pp >= p0 - tol && pp <= p1 + tol && pq >= q0 - tol && pq <= q1 + tol;
+            }
+            if (!in) klo = -0x40000000; // marks the workgroup for the global path
         }
         for (int off = 32; off > 0; off >>= 1) {
             klo = min(klo, __shfl_xor(klo, off, 64));
@@ -378,133 +411,148 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
         __syncthreads();
         klo = min(min(red[0][0], red[0][1]), min(red[0][2], red[0][3]));
         khi = max(max(red[1][0], red[1][1]), max(red[1][2], red[1][3]));
-        const int nslab = khi >= klo ? (khi - klo) / kSlab + 1 : 0;
+        slab_ok = klo != -0x40000000;
+    }
+    if (!__builtin_amdgcn_readfirstlane((int)slab_ok)) {
+        while (jf < jend) {
+            const float je = fminf(jf + (float)kSumBlock, jend);
+            float s0 = 0.0f;
+            for (; jf < je; jf += 1.0f) s0 += global_sample();
+            acc += s0;
+        }
+    } else {
+        const int nslab = __builtin_amdgcn_readfirstlane(khi >= klo ? (khi - klo) / kSlab + 1 : 0);
         const float rtK = n > 0 ? 1.0f / tK : 0.0f;
-        // lanes 8 g + c + 4 e of every wavefront project corner ray c onto plane e of a slab
-        const int cc = tid & 3, ce = (tid >> 2) & 1;
-        const float cKo = cl[cc][K], cKr = __builtin_amdgcn_rcpf(cl[cc][3 + K]);
-        const float cPo = cl[cc][F], cPd = cl[cc][3 + F], cQo = cl[cc][Q], cQd = cl[cc][3 + Q];
+        // lower taps K in [D0, D0 + kSlab - 1] of slab si; slabs follow the rays' direction
+        auto first_slice = [&](int si) {
+            return sgn > 0.0f ? klo + si * kSlab : khi - kSlab + 1 - si * kSlab;
+        };
+        // lane l's plan of slab si0 + l: the box's first indices along P and Q; quads per row and
+        // rows per slice (0: not staged); a little over 2^20 / each, by which a product and a
+        // shift give exact quotients of the numbers of the box's quads and rows
+        int bP0 = 0, bQ0 = 0, bN = 0, bRN = 0, bRQ = 0;
+        auto plan_slabs = [&](int si0) {
+            const float k = (float)first_slice(si0 + (tid & 63));
+            float p0, p1, q0, q1, u0, u1, v0, v1;
+            section(k, p0, p1, q0, q1);
+            section(k + (float)kSlab, u0, u1, v0, v1);
+            constexpr float big = 16384.0f;
+            auto floor_at = [](float v) {
+                return floor_i32(__builtin_amdgcn_fmed3f(v, -big, big));
+            };
+            bP0 = floor_at(fminf(p0, u0) - kBoxMargin);
+            bQ0 = floor_at(fminf(q0, v0) - kBoxMargin);
+            // quads per row and rows per slice: to the upper taps of the largest lower ones
+            const int NQ = (floor_at(fmaxf(p1, u1) + kBoxMargin) + 1 - bP0 + 4) >> 2;
+            const int WQ = floor_at(fmaxf(q1, v1) + kBoxMargin) + 1 - bQ0 + 1;
+            const bool fits = NQ <= kBoxCells / 4 && WQ <= kBoxCells / 4 &&
+                              (kSlab + 1) * NQ * WQ <= kBoxCells / 4;
+            bN = fits ? NQ | WQ << 16 : 0;
+            bRN = (int)(0x1p20f * __builtin_amdgcn_rcpf((float)NQ)) + 1;
+            bRQ = (int)(0x1p20f * __builtin_amdgcn_rcpf((float)WQ)) + 1;
+        };
+        // LDS byte address of the box
+        const int box0 = (int)(uintptr_t)(__attribute__((address_space(3))) float4 *)box4;
         for (int si = 0; si < nslab; ++si) {
-            // lower taps K in [D0, D0 + kSlab - 1]; slabs follow the rays' direction along K
-            const int D0 = sgn > 0.0f ? klo + si * kSlab : khi - kSlab + 1 - si * kSlab;
-            // the box: the corner rays where they cross K = D0 and K = D0 + kSlab
-            const float t = ((float)(D0 + ce * kSlab) - cKo) * cKr;
-            float pmin = fmaf(t, cPd, cPo), qmin = fmaf(t, cQd, cQo);
-            float pmax = pmin, qmax = qmin;
+            if ((si & 63) == 0) plan_slabs(si);
+            const int D0 = first_slice(si);
+            const int P0 = __builtin_amdgcn_readlane(bP0, si & 63);
+            const int Q0 = __builtin_amdgcn_readlane(bQ0, si & 63);
+            const int nn = __builtin_amdgcn_readlane(bN, si & 63);
+            const int NQ = nn & 0xffff, WQ = nn >> 16;
+            if (nn) {
+                const int rn = __builtin_amdgcn_readlane(bRN, si & 63);
+                const int rq = __builtin_amdgcn_readlane(bRQ, si & 63);
+                // quad e of the box is quad e - NQ r of row r = e / NQ, row r - WQ kk of slice
+                // kk = r / WQ
+                const int total = (kSlab + 1) * WQ * NQ;
+                const int g0 = (D0 * sK + Q0 * sQ + P0) * es;
+                Quad v[kBoxCells / 4 / kMaxBlock];
 #pragma unroll
-            for (int off = 1; off < 8; off <<= 1) {
-                pmin = fminf(pmin, __shfl_xor(pmin, off, 64));
-                pmax = fmaxf(pmax, __shfl_xor(pmax, off, 64));
-                qmin = fminf(qmin, __shfl_xor(qmin, off, 64));
-                qmax = fmaxf(qmax, __shfl_xor(qmax, off, 64));
-            }
-            const int P0 = __builtin_amdgcn_readfirstlane((int)floorf(pmin) - 1);
-            const int Q0 = __builtin_amdgcn_readfirstlane((int)floorf(qmin) - 1);
-            const int WP = __builtin_amdgcn_readfirstlane((int)floorf(pmax) + 2 - P0 + 1);
-            const int WQ = __builtin_amdgcn_readfirstlane((int)floorf(qmax) + 2 - Q0 + 1);
-            const int WPp = (WP + 3) & ~3;
-            const int S = WQ * WPp; // floats per staged slice
-            const bool staged = WPp <= 4 * kBoxQuads && WQ <= kBoxCells / ((kSlab + 1) * WPp);
-            if (staged) {
-                // rows (slice kk, row qq) of WP cells, 16 bytes per thread: 32 rows a pass
-                const int rows = (kSlab + 1) * WQ, quad = tid & (kBoxQuads - 1);
-                int r = tid >> 3, kk = r / WQ, qq = r - kk * WQ;
-                for (; r < rows; r += kMaxBlock / kBoxQuads) {
-                    if (4 * quad < WPp) {
-                        const int e = (D0 + kk) * sK + (Q0 + qq) * sQ + P0 + 4 * quad;
-                        const Quad v = buf_quad_at<SI>(R, e * es);
-                        *reinterpret_cast<float4 *>(&box[(kk * WQ + qq) * WPp + 4 * quad]) =
-                            make_float4(v.v[0], v.v[1], v.v[2], v.v[3]);
+                for (int i = 0; i < kBoxCells / 4 / kMaxBlock; ++i) {
+                    const int e = tid + i * kMaxBlock;
+                    if (e < total) {
+                        const int r = (int)(__umul24((unsigned)e, (unsigned)rn) >> 20);
+                        const int kk = (int)(__umul24((unsigned)r, (unsigned)rq) >> 20);
+                        const int qq = r - __mul24(kk, WQ), pq = e - __mul24(r, NQ);
+                        v[i] = buf_quad_at<SI>(R, g0 + (kk * sK + qq * sQ + 4 * pq) * es);
                     }
-                    qq += kMaxBlock / kBoxQuads;
-                    while (qq >= WQ) {
-                        qq -= WQ;
-                        ++kk;
-                    }
+                }
+#pragma unroll
+                for (int i = 0; i < kBoxCells / 4 / kMaxBlock; ++i) {
+                    const int e = tid + i * kMaxBlock;
+                    if (e < total)
+                        box4[e] = make_float4(v[i].v[0], v[i].v[1], v[i].v[2], v[i].v[3]);
                 }
             }
             __syncthreads(); // the box is staged
-            // this ray's samples in the slab: j .. je - 1, where its position along K crosses
-            // the slab's far plane. A sample that the rounding of this estimate puts in the
-            // wrong slab lies outside the box and takes the global path.
+            // one past this ray's last sample in the slab: an estimate from its crossing of the
+            // slab's far plane, put right by the floors of the samples either side of it, so that
+            // a sample is in the slab exactly when its lower tap is
+            const int kofs = cK - D0;
             const float bK = (float)((sgn > 0.0f ? D0 + kSlab : D0) - cK);
-            const int je = j < n ? min(max((int)ceilf(fmaf(bK - mK, rtK, -p.j0)), j), n) : j;
-            const int kofs = cK - D0, pofs = cP - P0, qofs = cQ - Q0;
-            // KM: K is the copy's middle axis (a step in K is the trilinear m step)
-            auto sample_slab = [&](auto km) {
-                constexpr bool KM = decltype(km)::value;
-                const int mstep = KM ? S : WPp, lstep = KM ? WPp : S;
-                auto in_box = [&](int kk, int ip, int iq) {
-                    return staged && (unsigned)kk < (unsigned)kSlab &&
-                           (unsigned)ip <= (unsigned)(WP - 2) && (unsigned)iq <= (unsigned)(WQ - 2);
-                };
-                // strides in bytes, so that a sample's address is two 24-bit products and one
-                // shifted add
-                const int S4 = 4 * S, W4 = 4 * WPp, m4 = 4 * mstep, l4 = 4 * lstep;
-                // the sample at byte offset `ofs` of the box (its lower tap pair)
-                auto box_at = [&](float pK, float pf, float pq, int ofs) {
-                    const char *cb = reinterpret_cast<const char *>(box) + ofs;
-                    const float *c = reinterpret_cast<const float *>(cb);
-                    const float *cm = reinterpret_cast<const float *>(cb + m4);
-                    const float *cl = reinterpret_cast<const float *>(cb + l4);
-                    const float *cml = reinterpret_cast<const float *>(cb + m4 + l4);
-                    const float ff = __builtin_amdgcn_fractf(pf);
-                    const float fm = __builtin_amdgcn_fractf(KM ? pK : pq);
-                    const float fl = __builtin_amdgcn_fractf(KM ? pq : pK);
-                    const float a00 = fmaf(ff, c[1] - c[0], c[0]);
-                    const float a10 = fmaf(ff, cm[1] - cm[0], cm[0]);
-                    const float a01 = fmaf(ff, cl[1] - cl[0], cl[0]);
-                    const float a11 = fmaf(ff, cml[1] - cml[0], cml[0]);
-                    const float b0 = fmaf(fm, a10 - a00, a00);
-                    const float b1 = fmaf(fm, a11 - a01, a01);
-                    return fmaf(fl, b1 - b0, b0);
-                };
-                auto box_sample = [&](float pK, float pf, float pq, int kk, int ip, int iq) {
-                    return box_at(pK, pf, pq, __mul24(kk, S4) + __mul24(iq, W4) + 4 * ip);
-                };
-                // Along a ray every box coordinate is monotonic in jf (jf takes exact integer
-                // values), so a lane whose first and last samples of the slab lie in the box has
-                // all of them there. When every lane of the wavefront is such a lane, it runs the
-                // loop without the per-sample test: the same samples from the same cells, added
-                // in the same order.
-                bool inside = true;
-                if (j < je) {
-                    const float jl = jf + (float)(je - 1 - j);
-                    inside = in_box(floor_i32(fmaf(jf, tK, mK)) + kofs,
-                                    floor_i32(fmaf(jf, tP, mP)) + pofs,
-                                    floor_i32(fmaf(jf, tQ, mQ)) + qofs) &&
-                             in_box(floor_i32(fmaf(jl, tK, mK)) + kofs,
-                                    floor_i32(fmaf(jl, tP, mP)) + pofs,
-                                    floor_i32(fmaf(jl, tQ, mQ)) + qofs);
-                }
-                float part = 0.0f;
-                if (__builtin_amdgcn_ballot_w64(!inside) == 0) {
-                    // counted by jf alone (exact integers); the box offsets of the copy's
-                    // coordinates folded into one wave-uniform byte offset
-                    const float jfe = jf + (float)max(je - j, 0);
-                    const int ofs0 = kofs * S4 + qofs * W4 + 4 * pofs;
-                    for (; jf < jfe; jf += 1.0f) {
-                        const float pK = fmaf(jf, tK, mK);
-                        const float pf = fmaf(jf, tP, mP), pq = fmaf(jf, tQ, mQ);
-                        part += box_at(pK, pf, pq,
-                                       __mul24(floor_i32(pK), S4) + __mul24(floor_i32(pq), W4) +
-                                           4 * floor_i32(pf) + ofs0);
-                    }
-                    j = max(j, je);
-                } else {
-                    for (; j < je; ++j, jf += 1.0f) {
-                        const float pK = fmaf(jf, tK, mK);
-                        const float pf = fmaf(jf, tP, mP), pq = fmaf(jf, tQ, mQ);
-                        const int kk = floor_i32(pK) + kofs;
-                        const int ip = floor_i32(pf) + pofs, iq = floor_i32(pq) + qofs;
-                        if (in_box(kk, ip, iq)) part += box_sample(pK, pf, pq, kk, ip, iq);
-                        else part += global_sample();
-                    }
-                }
-                acc += part;
+            float je = fminf(fmaxf(p.j0 + ceilf(fmaf(bK - mK, rtK, -p.j0)), jf), jend);
+            auto in_slab = [&](float jj) {
+                return (unsigned)(floor_i32(fmaf(jj, tK, mK)) + kofs) < (unsigned)kSlab;
             };
-            if (kmid) sample_slab(std::true_type{});
-            else sample_slab(std::false_type{});
+            if (je < jend && in_slab(je)) je += 1.0f;
+            else if (je > jf && !in_slab(je - 1.0f)) je -= 1.0f;
+            if (nn) {
+                if (je > jf) {
+                    // KM: K is the copy's middle axis (a step in K is the trilinear m step)
+                    auto sample_slab = [&](auto km) {
+                        constexpr bool KM = decltype(km)::value;
+                        const int W4 = 16 * NQ, S4 = W4 * WQ; // bytes per row and per slice
+                        // as subnormals in vector registers
+                        auto sub = [](int i) {
+                            float f = __int_as_float(i < 0 ? -i | (int)0x80000000 : i);
+                            asm("" : "+v"(f));
+                            return f;
+                        };
+                        const float fS = sub(S4), fW = sub(W4), f4 = sub(4);
+                        const float fo =
+                            sub(kofs * S4 + (cQ - Q0) * W4 + (cP - P0) * 4 + box0);
+                        int m4 = KM ? S4 : W4, l4 = KM ? W4 : S4;
+                        asm("" : "+v"(m4), "+v"(l4));
+                        auto sample = [&](float jj) {
+                            const float pK = fmaf(jj, tK, mK), pf = fmaf(jj, tP, mP),
+                                        pq = fmaf(jj, tQ, mQ);
+                            const float iK = floorf(pK), iP = floorf(pf), iQ = floorf(pq);
+                            const int o =
+                                __float_as_int(fmaf(iK, fS, fmaf(iQ, fW, fmaf(iP, f4, fo))));
+                            auto pair = [](int q) {
+                                const auto *c =
+                                    (const __attribute__((address_space(3))) float *)(uintptr_t)
+                                        (unsigned)q;
+                                return Pair{c[0], c[1]};
+                            };
+                            const Pair p00 = pair(o), p10 = pair(o + m4), p01 = pair(o + l4),
+                                       p11 = pair(o + m4 + l4);
+                            const float fK = pK - iK, fQ = pq - iQ;
+                            return trilerp(p00, p10, p01, p11, pf - iP, KM ? fK : fQ,
+                                           KM ? fQ : fK);
+                        };
+                        float part = 0.0f;
+                        // the wavefront's smallest count, over the lanes with any
+                        const int cnt = (int)(je - jf);
+                        int least = __builtin_amdgcn_readfirstlane(cnt);
+                        for (;;) {
+                            const unsigned long long less = __builtin_amdgcn_ballot_w64(cnt < least);
+                            if (less == 0) break;
+                            least = __builtin_amdgcn_readlane(cnt, __builtin_ctzll(less));
+                        }
+                        for (int i = 0; i < least; ++i, jf += 1.0f) part += sample(jf);
+                        for (; jf < je; jf += 1.0f) part += sample(jf);
+                        acc += part;
+                    };
+                    if (kmid) sample_slab(std::true_type{});
+                    else sample_slab(std::false_type{});
+                }
+            } else {
+                float part = 0.0f;
+                for (; jf < je; jf += 1.0f) part += global_sample();
+                acc += part;
+            }
             __syncthreads(); // the box is read before the next slab is staged
         }
     }

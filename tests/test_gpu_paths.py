@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import curadon_amd as cm
-from geoms import as_fan_geometry, fan
+from geoms import as_cone_geometry, as_fan_geometry, cone, fan
 
 pytestmark = pytest.mark.gpu
 
@@ -81,3 +81,27 @@ def test_view_rows_batched_equal_single(gpu):
     for i in range(3):
         one = cm.backward(y[i].contiguous(), geom)
         assert torch.equal(got[i], one) and torch.equal(got[-3 + i], one)
+
+
+@pytest.mark.parametrize("what,rec", [
+    # staged boxes: ragged slabs, one voxel thick along an axis, panels of one tile less and more
+    ("thin x", lambda: cone(1, 17, 15, 6, 60.0, 90.0, nz=21, ny=9)),
+    ("thin z", lambda: cone(23, 16, 17, 6, 60.0, 90.0, nz=1, ny=11)),
+    ("ten slices", lambda: cone(20, 33, 31, 7, 60.0, 90.0, nz=10, ny=30)),
+    # boxes too large to stage: every slab from global memory, or some of them
+    ("coarse panel", lambda: cone(40, 24, 20, 5, 80.0, 120.0, du=(5.0, 5.0))),
+    ("rows too long", lambda: cone(40, 24, 20, 5, 80.0, 120.0, du=(3.0, 1.0))),
+    # rays nearly along the diagonals and within the volume's corners
+    ("near source", lambda: cone(24, 40, 36, 9, 26.0, 60.0, du=(1.5, 1.5))),
+    # FP32 corner rays that lose the voxel: the workgroups march from global memory
+    ("far source", lambda: cone(32, 24, 24, 3, 4.0e6, 4.0e6 + 40.0)),
+    # tilted trajectory: other march axes and copies
+    ("euler", lambda: cone(22, 30, 28, 4, 60.0, 90.0, nz=18, ny=26, angles=np.array(
+        [[0.3, 1.9, 3.0, 5.1], [0.7, 1.4, 0.2, 1.5], [0.1, 0.9, 1.5, 0.4]]))),
+])
+def test_forward_3d_boxes(oracle, gpu, what, rec):
+    rec = rec()
+    geom = as_cone_geometry(rec)
+    vol = np.random.RandomState(4).rand(*rec.vol_shape)
+    got = cm.forward(torch.tensor(vol, dtype=torch.float32, device=gpu), geom)
+    assert rel_l2(got, oracle.fwd3d(geom, vol)) <= RTOL_L2, what
