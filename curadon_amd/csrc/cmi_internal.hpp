@@ -111,6 +111,15 @@ __device__ __forceinline__ int round_i32(float x) {
     return r;
 }
 
+// A workgroup barrier after this wavefront's LDS operations. __syncthreads() alone should wait for
+// them, but where it opens the body of a loop that the compiler has rotated (the barrier's block
+// is then the target of a back edge beside the loop's header), no wait was emitted for the LDS
+// atomics of the turn before, and another wavefront read the cells without them.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
 // ------------------------------------------------------------------ buffer loads -------
 // Raw buffer resources give 32-bit offsets from a scalar base and hardware range checking:
 // a load that lies wholly beyond num_records bytes returns 0 instead of touching memory.

@@ -667,7 +667,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj3d(typename SV::raw *__restric
     // the tile's voxel sums -> the workgroup's 64-bit sums, then the tile (border included)
     // cleared
     auto drain = [&]() {
-        __syncthreads();
+        lds_barrier();
 #pragma unroll 4
         for (int k = 0; k < kATOwn; ++k) {
             const int i = tid + k * kMaxBlock;
@@ -844,7 +844,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj3d(typename SV::raw *__restric
             }
         }
     }
-    __syncthreads();
+    lds_barrier();
 #pragma unroll 4
     for (int k = 0; k < kATOwn; ++k) {
         const int i = tid + k * kMaxBlock;
@@ -956,13 +956,25 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp3d_y(typename SV::raw *__restri
 // the source, bounded by the four lines through the source and that rectangle's corners. The
 // workgroup marches through the volume along the axis K that the tile's central ray follows
 // most closely, in chunks of kBTSlab slices. In each slice the pyramid's section is the
-// quadrilateral where the corner lines cross it; its bounding box (one voxel of margin on each
-// side, clipped to the volume) is walked by the workgroup's threads, x fastest (y when K is x,
-// from a y-fastest copy of the volume), so that a wavefront reads runs of consecutive voxels.
-// Every voxel computes its own (u, v) and adds its taps inside the tile to the tile's cells in
-// LDS. The corner lines need the rays of the pyramid to cross the slices (each corner line's
+// quadrilateral where the corner lines cross it; its bounding box (kBTMargin of a voxel wider on
+// each side, for the FP32 lines; clipped to the volume) is found by the lane that holds the slice. A wavefront takes every
+// fourth slice of a chunk and walks it in steps of 64 voxels, x fastest (y when K is x, from a
+// y-fastest copy of the volume), so that it reads runs of consecutive voxels. All slices of a
+// chunk are walked over the extents of its widest box, their origins moved back where that would
+// leave the volume: voxels outside the pyramid have no cell in the tile and add nothing. So a
+// lane's voxel lies at the same offset from the box's origin in every slice of the chunk, and U,
+// V and W are one sum each of the offset's share (kept in registers, up to kBTSteps steps) and
+// the origin's (evaluated in FP64 by the lane that holds the slice, and read from it).
+// The corner lines need the rays of the pyramid to cross the slices (each corner line's
 // direction has a K component of a quarter of its length, all of one sign); otherwise the
 // whole slice is walked.
+// Bound by VALU issue. Walking the chunk's boxes as one flat list of voxels took 75 VALU and 29
+// SALU instructions per wavefront of voxels (an index walk in three dimensions, tests against the
+// slice's own box, the nine products of the matrix rows); now 38 and 9 with the set-up, and a
+// margin of a sixteenth of a voxel instead of one leaves a quarter of the visits out. Dense
+// volumes, calls: 256^3 x 360 of 384^2 14.2 -> 10.5 ms, 128^3 x 180 of 192^2 1.16 -> 0.78 ms
+// (slices per chunk x steps together 20 x 4: 0.79, 28 x 4: 0.77, 28 x 3: 0.78 and 10.8 ms at 256^3,
+// 20 x 3: 11.0).
 // Fixed point: terms are rounded to units of max|vol| wbound / 2^kBTBits, where wbound >= the
 // weight (1, or 1 / min W^2 for FDK, W > 0 over the volume), so |term| <= 2^kBTBits and a
 // 32-bit LDS cell holds the sum of up to 2^(31 - kBTBits) - 1 terms. A voxel adds at most one
@@ -972,12 +984,13 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp3d_y(typename SV::raw *__restri
 // written once, in the sinogram's storage type.
 constexpr int kBT = 16;                                        // panel tile edge, pixels
 constexpr int kBTP = kBT + 2;                                  // LDS cells per row and rows
-constexpr int kBTSlab = 32;                                    // slices per chunk
+constexpr int kBTSlab = 40;                                    // slices per chunk
 constexpr int kBTBits = 18;                                    // a term's bound: 2^kBTBits
 constexpr int kBTBudget = (1 << (31 - kBTBits)) - 1;           // visits between drains
-// voxels per thread at a time (at 256^3: 1: 12.7 ms, 2: 11.4, 4: 11.7, 8: 13.8)
-constexpr int kBTBatch = 2;
-constexpr int kBTPass = kBTBudget / (kBTBatch * kMaxBlock) * (kBTBatch * kMaxBlock); // per pass
+constexpr int kBTSteps = 3;                                    // steps of a slice walked together
+constexpr float kBTMargin = 0.0625f;                           // voxels around the crossings
+static_assert(kBTSlab % 4 == 0 && kBTSlab / 4 * kBTSteps * kMaxBlock <= kBTBudget,
+              "no drain within a chunk's steps");
 static_assert(kBT * kBT == kMaxBlock, "one tile cell per thread");
 static_assert(kBTSlab <= 64, "one lane per slice of a chunk");
 
@@ -990,8 +1003,6 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
                                                      float wbound, int nx, int ny, int nz, int U,
                                                      int V, int A) {
     __shared__ unsigned int cells[kBTP * kBTP]; // pixel iu0 - 1 + i, iv0 - 1 + j at j kBTP + i
-    __shared__ int4 slab[2][kBTSlab];           // per slice: F range, G range (inclusive)
-    __shared__ int dims[2][2];                  // per chunk: box extents along F and G
     __shared__ float coef[4][4];                // per corner line: F = a + b hK, G = c + d hK
     __shared__ int whole;                       // 1: walk whole slices
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1007,12 +1018,15 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
     float vmax = 0.0f;
     for (int i = lane; i < kMaxParts; i += 64) vmax = fmaxf(vmax, parts[b * kMaxParts + i]);
     for (int off = 32; off > 0; off >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, off, 64));
-    // a voxel value maps to vol ldexp(smant, sexp) units, the FP64 scale 2^18 / (max|vol| wbound)
-    // split into an FP32 mantissa and an exponent (the scale may lie outside the FP32 range)
+    // a voxel value maps to vol s1 s2 units, the scale 2^18 / (max|vol| wbound) in two factors: a
+    // power of two that brings max|vol| to [1, 2) and the rest, which is then in range
     static_assert(kBTBits == 18, "the scale uses 2^18");
-    const double unit_inv = vmax > 0.0f ? 0x1p18 / ((double)vmax * (double)wbound) : 0.0;
-    const int sexp = unit_inv > 0.0 ? ilogb(unit_inv) : 0;
-    const float smant = (float)ldexp(unit_inv, -sexp);
+    const bool some = vmax > 0.0f && vmax < INFINITY;
+    const int vexp = some ? ilogbf(vmax) : 0;
+    const float s1 = ldexpf(1.0f, max(min(-vexp, 127), -126)); // (|vol| below 2^-127: the rest)
+    const double left = ldexp(1.0, -vexp - max(min(-vexp, 127), -126));
+    const float s2 =
+        some ? (float)(0x1p18 * left / (ldexp((double)vmax, -vexp) * (double)wbound)) : 0.0f;
     // march axis: the largest component of the central ray's direction, the cross product of
     // the (U - uc W) and (V - vc W) rows' voxel parts
     int K;
@@ -1075,128 +1089,126 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
                : vol + b * (size_t)nx * ny * nz;
     const int strG = K == 0 ? Wp * Hp : (K == 1 ? nx * ny : nx);
     const int strK = K == 0 ? Hp : (K == 1 ? nx : nx * ny);
-    // matrix rows over (hF, hG, hK, 1)
-    auto row = [&](int r, float &rF, float &rG, float &rK, float &r3) {
-        const float x = m[4 * r], y = m[4 * r + 1], z = m[4 * r + 2];
-        rF = F == 0 ? x : y;
-        rG = G == 1 ? y : z;
-        rK = K == 0 ? x : (K == 1 ? y : z);
-        r3 = m[4 * r + 3];
-    };
-    float uF, uG, uK, u3, vF, vG, vK, v3, wF, wG, wK, w3;
-    row(0, uF, uG, uK, u3);
-    row(1, vF, vG, vK, v3);
-    row(2, wF, wG, wK, w3);
+    // matrix rows over the voxel's index (f, g, k) along (F, G, K), the panel coordinates taken
+    // from the tile's first LDS cell
+    double ru[4], rv[4], rw[4];
+    {
+        auto row = [&](int r, double (&o)[4]) {
+            const double x = m[4 * r], y = m[4 * r + 1], z = m[4 * r + 2];
+            o[0] = F == 0 ? x : y;
+            o[1] = G == 1 ? y : z;
+            o[2] = K == 0 ? x : (K == 1 ? y : z);
+            o[3] = (double)m[4 * r + 3] - o[0] * cF - o[1] * cG - o[2] * cK;
+        };
+        row(0, ru);
+        row(1, rv);
+        row(2, rw);
+        for (int k = 0; k < 4; ++k) {
+            ru[k] -= (double)(iu0 - 1) * rw[k];
+            rv[k] -= (double)(iv0 - 1) * rw[k];
+        }
+    }
     unsigned int *mine = &cells[(tid / kBT + 1) * kBTP + tid % kBT + 1];
     long long own = 0;
     // cells -> registers (border cells, which belong to other tiles, are never read)
     auto drain = [&]() {
-        __syncthreads();
+        lds_barrier();
         own += (long long)(int)*mine;
         *mine = 0u;
         __syncthreads();
     };
+    const float uF = (float)ru[0], uG = (float)ru[1], vF = (float)rv[0], vG = (float)rv[1],
+                wF = (float)rw[0], wG = (float)rw[1];
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     int run = 0; // voxel visits since the last drain
-    int buf = 0;
-    for (int k0 = 0; k0 < nK; k0 += kBTSlab, buf ^= 1) {
-        const int S = min(kBTSlab, nK - k0);
-        if (tid < 64) {
-            int flo = 0, fhi = -1, glo = 0, ghi = -1;
-            if (lane < S) {
-                if (whole) {
-                    fhi = nF - 1;
-                    ghi = nG - 1;
-                } else {
-                    const float hK = (float)(k0 + lane) - cK;
-                    float f0 = INFINITY, f1 = -INFINITY, g0 = INFINITY, g1 = -INFINITY;
-                    for (int c = 0; c < 4; ++c) {
-                        const float f = fmaf(coef[c][1], hK, coef[c][0]);
-                        const float g = fmaf(coef[c][3], hK, coef[c][2]);
-                        f0 = fminf(f0, f);
-                        f1 = fmaxf(f1, f);
-                        g0 = fminf(g0, g);
-                        g1 = fmaxf(g1, g);
-                    }
-                    constexpr float big = 0x1p24f;
-                    flo = max(0, floor_i32(__builtin_amdgcn_fmed3f(f0 + cF, -big, big)) - 1);
-                    fhi = min(nF - 1, floor_i32(__builtin_amdgcn_fmed3f(f1 + cF, -big, big)) + 1);
-                    glo = max(0, floor_i32(__builtin_amdgcn_fmed3f(g0 + cG, -big, big)) - 1);
-                    ghi = min(nG - 1, floor_i32(__builtin_amdgcn_fmed3f(g1 + cG, -big, big)) + 1);
-                }
-                slab[buf][lane] = make_int4(flo, fhi, glo, ghi);
+    for (int k0 = 0; k0 < nK; k0 += kBTSlab) {
+        // lane l holds slice k0 + l: its box, then its walk's origin and shares. Every wavefront
+        // does the same.
+        const int S = min(kBTSlab, nK - k0), k = k0 + min(lane, S - 1);
+        int flo = 0, fhi = nF - 1, glo = 0, ghi = nG - 1;
+        if (!whole) {
+            const float hK = (float)k - cK;
+            float f0 = INFINITY, f1 = -INFINITY, g0 = INFINITY, g1 = -INFINITY;
+            for (int c = 0; c < 4; ++c) {
+                const float f = fmaf(coef[c][1], hK, coef[c][0]);
+                const float g = fmaf(coef[c][3], hK, coef[c][2]);
+                f0 = fminf(f0, f);
+                f1 = fmaxf(f1, f);
+                g0 = fminf(g0, g);
+                g1 = fmaxf(g1, g);
             }
-            int ef = max(fhi - flo + 1, 0), eg = max(ghi - glo + 1, 0);
-            for (int off = 32; off > 0; off >>= 1) {
-                ef = max(ef, __shfl_xor(ef, off, 64));
-                eg = max(eg, __shfl_xor(eg, off, 64));
-            }
-            if (lane == 0) {
-                dims[buf][0] = ef;
-                dims[buf][1] = eg;
-            }
+            auto floor_at = [](float v) {
+                constexpr float big = 0x1p24f;
+                return floor_i32(__builtin_amdgcn_fmed3f(v, -big, big));
+            };
+            flo = max(0, floor_at(f0 + (cF - kBTMargin)) + 1);
+            fhi = min(nF - 1, floor_at(f1 + (cF + kBTMargin)));
+            glo = max(0, floor_at(g0 + (cG - kBTMargin)) + 1);
+            ghi = min(nG - 1, floor_at(g1 + (cG + kBTMargin)));
         }
-        __syncthreads();
-        const int NF = dims[buf][0], NG = dims[buf][1];
-        const int total = NF * NG * S;
+        int ef = max(fhi - flo + 1, 0), eg = max(ghi - glo + 1, 0);
+        if (ef == 0 || eg == 0) ef = eg = 0;
+        for (int off = 32; off > 0; off >>= 1) {
+            ef = max(ef, __shfl_xor(ef, off, 64));
+            eg = max(eg, __shfl_xor(eg, off, 64));
+        }
+        const int NF = __builtin_amdgcn_readfirstlane(ef), NG = __builtin_amdgcn_readfirstlane(eg);
+        const unsigned total = (unsigned)NF * (unsigned)NG;
         if (total == 0) continue;
-        // this thread's element e = tid + n kMaxBlock of the chunk's box, as (dF, dG, dk) with
-        // dF fastest; a step of kMaxBlock elements is (sF, sG, sK)
-        int dF = tid % NF, dG = (tid / NF) % NG, dk = tid / (NF * NG);
-        const int sF = kMaxBlock % NF, sG = (kMaxBlock / NF) % NG, sK = kMaxBlock / (NF * NG);
-        int e = tid;
-        auto advance = [&]() {
-            dF += sF;
-            if (dF >= NF) {
-                dF -= NF;
-                ++dG;
-            }
-            dG += sG;
-            if (dG >= NG) {
-                dG -= NG;
-                ++dk;
-            }
-            dk += sK;
+        flo = max(0, min(flo, nF - NF));
+        glo = max(0, min(glo, nG - NG));
+        const float ul = (float)(ru[0] * flo + ru[1] * glo + ru[2] * k + ru[3]);
+        const float vl = (float)(rv[0] * flo + rv[1] * glo + rv[2] * k + rv[3]);
+        const float wl = (float)(rw[0] * flo + rw[1] * glo + rw[2] * k + rw[3]);
+        const int at = flo + glo * strG + k * strK;
+        const float rNF = 1.0f / (float)NF;
+        auto lane_of = [](float x, int l) {
+            return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
         };
-        for (int base = 0; base < total; base += kBTPass) {
-            const int n = min(kBTPass, total - base);
-            if (run + n > kBTBudget) {
+        // N steps from voxel e0 of every slice on
+        auto steps = [&](unsigned e0, auto count) {
+            constexpr int N = decltype(count)::value;
+            if (run + kBTSlab / 4 * N * kMaxBlock > kBTBudget) {
                 drain();
                 run = 0;
             }
-            run += n;
-            // kBTBatch elements per thread at a time: their loads are issued together. Passes
-            // start at multiples of kBTBatch kMaxBlock elements, so a batch never straddles two.
-            for (; e < base + n; e += kBTBatch * kMaxBlock) {
-                int fq[kBTBatch], gq[kBTBatch], kq[kBTBatch], addr[kBTBatch];
-                bool live[kBTBatch];
+            run += kBTSlab / 4 * N * kMaxBlock;
+            // this lane's voxels, the same in every slice; past the box, the coordinate leaves
+            // the tile
+            float us[N], vs[N], ws[N];
+            int ofs[N];
 #pragma unroll
-                for (int q = 0; q < kBTBatch; ++q) {
-                    const int4 sl = slab[buf][min(dk, S - 1)];
-                    fq[q] = sl.x + dF;
-                    gq[q] = sl.z + dG;
-                    kq[q] = k0 + dk;
-                    live[q] = e + q * kMaxBlock < base + n && fq[q] <= sl.y && gq[q] <= sl.w;
-                    addr[q] = live[q] ? fq[q] + gq[q] * strG + kq[q] * strK : 0;
-                    advance();
-                }
-                float val[kBTBatch];
+            for (int q = 0; q < N; ++q) {
+                const unsigned e = e0 + 64 * q + (unsigned)lane;
+                const bool in = e < total;
+                // e / NF: by the reciprocal, (e + 0.5) / NF lies at least 0.5 / NF from an
+                // integer, far more than the rounding for e < 2^20
+                int dg = total < 1u << 20 ? (int)(((float)e + 0.5f) * rNF)
+                                          : (int)(e / (unsigned)NF);
+                int df = (int)e - dg * NF;
+                if (!in) dg = df = 0;
+                ofs[q] = df + dg * strG;
+                const float xf = (float)df, xg = (float)dg;
+                us[q] = fmaf(uF, xf, uG * xg);
+                vs[q] = in ? fmaf(vF, xf, vG * xg) : 1e30f;
+                ws[q] = fmaf(wF, xf, wG * xg);
+            }
+            for (int l = wv; l < S; l += 4) {
+                const typename SV::raw *slice = src + __builtin_amdgcn_readlane(at, l);
+                float val[N];
 #pragma unroll
-                for (int q = 0; q < kBTBatch; ++q) val[q] = to_f32<SV>(src[addr[q]]);
+                for (int q = 0; q < N; ++q) val[q] = to_f32<SV>(slice[ofs[q]]);
+                const float u0 = lane_of(ul, l), v0 = lane_of(vl, l), w0 = lane_of(wl, l);
 #pragma unroll
-                for (int q = 0; q < kBTBatch; ++q) {
-                    const float vs = live[q] ? ldexpf(val[q] * smant, sexp) : 0.0f;
-                    if (vs == 0.0f) continue;
-                    const float hF = (float)fq[q] - cF, hG = (float)gq[q] - cG,
-                                hK = (float)kq[q] - cK;
-                    const float Uh = fmaf(uF, hF, fmaf(uG, hG, fmaf(uK, hK, u3)));
-                    const float Vh = fmaf(vF, hF, fmaf(vG, hG, fmaf(vK, hK, v3)));
-                    const float Wh = fmaf(wF, hF, fmaf(wG, hG, fmaf(wK, hK, w3)));
-                    const float rw = __builtin_amdgcn_rcpf(Wh);
-                    const float u = Uh * rw, v = Vh * rw;
-                    const int i = floor_i32(u) - (iu0 - 1), j = floor_i32(v) - (iv0 - 1);
-                    if ((unsigned)i > (unsigned)kBT || (unsigned)j > (unsigned)kBT) continue;
+                for (int q = 0; q < N; ++q) {
+                    const float x = val[q] * s1 * s2;
+                    const float r = __builtin_amdgcn_rcpf(ws[q] + w0);
+                    const float u = (us[q] + u0) * r, v = (vs[q] + v0) * r;
+                    const int i = floor_i32(u), j = floor_i32(v);
+                    if ((unsigned)i > (unsigned)kBT || (unsigned)j > (unsigned)kBT || x == 0.0f)
+                        continue;
                     const float fu = __builtin_amdgcn_fractf(u), fv = __builtin_amdgcn_fractf(v);
-                    const float t = FDK ? vs * (rw * rw) : vs;
+                    const float t = FDK ? x * (r * r) : x;
                     const float t1 = t * fu, t0 = t - t1;
                     const float t01 = t0 * fv, t00 = t0 - t01;
                     const float t11 = t1 * fv, t10 = t1 - t11;
@@ -1207,9 +1219,15 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
                     atomicAdd(c + kBTP + 1, (unsigned)round_i32(t11));
                 }
             }
-        }
+        };
+        unsigned e = 0;
+        for (; e + 64 * (kBTSteps - 1) < total; e += 64 * kBTSteps)
+            steps(e, std::integral_constant<int, kBTSteps>{});
+        static_assert(kBTSteps == 3, "the remainder is one or two steps");
+        if (e + 64 < total) steps(e, std::integral_constant<int, 2>{});
+        else if (e < total) steps(e, std::integral_constant<int, 1>{});
     }
-    __syncthreads();
+    lds_barrier();
     own += (long long)(int)*mine;
     const int iu = iu0 + tid % kBT, iv = iv0 + tid / kBT;
     if (iu < U && iv < V) {

@@ -860,7 +860,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj2d_tile(unsigned long long *__
     for (int k = 0; k < kT2Own; ++k) own[k] = 0;
     // cells -> registers, then clear (every thread calls it)
     auto drain = [&]() {
-        __syncthreads();
+        lds_barrier();
 #pragma unroll
         for (int k = 0; k < kT2Own; ++k) {
             const int i = tid + k * kMaxBlock;
@@ -1050,13 +1050,22 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // the source between the lines u = c0 - 1 and u = c0 + kGS (u is a ratio of two functions
 // affine in the pixel). The workgroup marches through the image along the axis K (rows or
 // columns) that the segment's central line follows most closely, in chunks of kGSlab lines;
-// per line the wedge is the interval between the two boundary lines' crossings (one pixel of
-// margin each side, clipped to the image), walked by the workgroup's threads along the line,
-// from the zero-bordered copy whose rows run along it (row-major for rows, transposed for
-// columns), so that a wavefront reads runs of consecutive pixels. Every pixel computes its own
-// u and weight with the backprojector's arithmetic and adds its terms that fall inside the
-// segment to kGS + 2 LDS cells with integer atomics. A segment whose boundary lines meet the
-// lines at grazing angles walks whole lines.
+// per line the wedge is the interval between the two boundary lines' crossings (kGMargin of a
+// pixel wider on each side, for the FP32 lines; clipped to the image). A wavefront takes every fourth line of a chunk and
+// walks it along the line, a lane per pixel, from the zero-bordered copy whose rows run along it
+// (row-major for rows, transposed for columns), so that it reads runs of consecutive pixels. All
+// lines of a chunk are walked over the width of its widest interval, their starts moved back
+// where that would leave the image: pixels outside the wedge have no cell in the segment and add
+// nothing. Depth and detector coordinate are affine in the pixel, so they are one sum each of the
+// lane's share (its pixel number along the line) and the line's (evaluated in FP64 by the lane
+// that holds the line, and read from it). Every pixel adds its terms that fall inside the segment
+// to kGS + 2 LDS cells with integer atomics. A segment whose boundary lines meet the lines at
+// grazing angles walks whole lines.
+// Bound by VALU issue. Walking the chunk's pixels as one flat list, which filled the lanes (0.94
+// against 0.73 at 0.67 pixels per cell) but gave every pixel an index walk, a test against its
+// line's interval and its own affine forms, took 51 VALU and 26 SALU instructions per wavefront of
+// pixels; now 32 and 12 with the set-up. Dense images, calls: 1024^2 x 716 935 -> 750 us, 256^2 x
+// 179 x 4 88 -> 77 us (2, 4, 8 lines in flight: 748, 757, 779 us at 1024^2).
 // Fixed point: terms are rounded to units of max|v| * bound / 2^kGBits, where `bound` is the
 // plan's bound on wt (times 1/du) over the image and all projections, so |term| <= 2^kGBits
 // and a 32-bit LDS cell holds the sum of up to 2^(31 - kGBits) - 1 terms. A pixel adds at most
@@ -1069,10 +1078,10 @@ constexpr int kGC = kGS + 2;                                 // LDS cells: c0 - 
 constexpr int kGSlab = 64;                                   // image lines per chunk
 constexpr int kGBits = 18;                                   // a term's bound: 2^kGBits units
 constexpr int kGBudget = (1 << (31 - kGBits)) - 1;           // pixel visits between drains
-// pixels per thread at a time (at 1024^2: 1: 0.95 ms, 2: 0.91, 4: 0.97, 8: 1.16)
-constexpr int kGBatch = 2;
-constexpr int kGPass = kGBudget / (kGBatch * kMaxBlock) * (kGBatch * kMaxBlock); // per pass
-static_assert(kGS <= kMaxBlock && kGSlab <= 64, "one owned cell per thread, one lane per line");
+constexpr int kGBatch = 4;           // lines per wavefront whose loads are in flight together
+constexpr float kGMargin = 0.0625f;  // pixels around the boundary lines' crossings
+static_assert(kGSlab == 64, "one lane per line");
+static_assert(kGSlab / 4 * kMaxBlock <= kGBudget, "no drain within a chunk's step");
 
 // Largest |v| of each image of a batch, in kAdjParts partial maxima per image.
 template <class SV>
@@ -1095,33 +1104,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_absmax_img2d(const typename SV::r
     }
 }
 
-// One projection's detector coordinate u (lower-tap cell floor(u), clamped to [-2, D] as the
-// backprojector clamps it) and weight wt of the pixel at world (x, y): k_bp2d's arithmetic for
-// circular plans (tab = meta, wt without the 1/du), k_bp2d_vec's for plans from views
-// (tab = three float4 per projection, wt including 1/|u|).
-template <bool VIEWS, int WPOW>
-__device__ __forceinline__ void bpT_geom(const float4 *__restrict__ tab, int a, float x, float y,
-                                         float px, float py, float c0, float hi, float &u,
-                                         float &wt) {
-    if (VIEWS) {
-        const float4 m0 = tab[3 * a], m1 = tab[3 * a + 1];
-        const float idu = tab[3 * a + 2].x;
-        const float w = m0.w * __builtin_amdgcn_rcpf(fmaf(m0.x, x, fmaf(m0.y, y, m0.z)));
-        const float eta = fmaf(m1.x, x, fmaf(m1.y, y, m1.z));
-        u = __builtin_amdgcn_fmed3f(fmaf(w, eta, m1.w), -2.0f, hi);
-        wt = (WPOW == 2 ? w * w : w) * idu;
-    } else {
-        const float4 m = tab[a];
-        const float depth = fmaf(m.x, x, fmaf(-m.y, y, m.w)); // xi + DSO
-        const float eta = fmaf(m.y, px, m.x * py);
-        const float w = m.z * __builtin_amdgcn_rcpf(depth);
-        u = __builtin_amdgcn_fmed3f(fmaf(w, eta, c0), -2.0f, hi);
-        wt = WPOW == 2 ? w * w : w;
-    }
-}
-
 // The line u(x, y) = uc of projection a as l0 x + l1 y + l2 = 0 in world coordinates (FP64),
-// from the same table as bpT_geom: u = w eta + c with w and eta ratios / sums of affine terms.
+// from the backprojector's own table: u = w eta + c with w and eta ratios / sums of affine terms.
 template <bool VIEWS>
 __device__ __forceinline__ void bpT_line(const float4 *__restrict__ tab, int a, double uc,
                                          double inv_du, double c0, double l[3]) {
@@ -1149,19 +1133,18 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
                                                      float sy, float ox, float oy, float inv_du,
                                                      float half_d) {
     __shared__ unsigned int cells[kGC]; // cell c0 - 1 + i at i
-    __shared__ int2 span[2][kGSlab];    // per line of a chunk: pixel range along it (inclusive)
-    __shared__ int width[2];            // per chunk: the widest range
     const int tid = threadIdx.x, lane = tid & 63;
     const int a = (int)(blockIdx.x % (unsigned)A);
     const int c0 = (int)(blockIdx.x / (unsigned)A) * kGS;
     const size_t b = blockIdx.y;
-    const float hi = (float)D, uoff = half_d - 0.5f;
-    // fixed-point scale 2^18 / (max|v| bound) as an FP32 mantissa and an exponent
+    const float uoff = half_d - 0.5f;
+    // fixed-point scale 2^18 / (max|v| bound) in two factors: a power of two that brings max|v|
+    // to [1, 2) and the rest, which is then in range
     static_assert(kGBits == 18, "the scale uses 2^18");
     const float vmax = adj2d_ymax(parts + b * kAdjParts);
-    const double unit_inv = vmax > 0.0f ? 0x1p18 / ((double)vmax * (double)bound) : 0.0;
-    const int sexp = unit_inv > 0.0 ? ilogb(unit_inv) : 0;
-    const float smant = (float)ldexp(unit_inv, -sexp);
+    const bool some = vmax > 0.0f && vmax < INFINITY;
+    const int vexp = some ? ilogbf(vmax) : 0;
+    const double rest = some ? 0x1p18 / (ldexp((double)vmax, -vexp) * (double)bound) : 0.0;
     // pixel index -> world: x = ix sx + bx (the world() map of the backprojector)
     const double bx = (double)ox + 0.5 - (double)((float)nx / 2.0f) * sx;
     const double by = (double)oy + 0.5 - (double)((float)ny / 2.0f) * sy;
@@ -1215,95 +1198,98 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
     for (int i = tid; i < kGC; i += kMaxBlock) cells[i] = 0u;
     long long own = 0;
     auto drain = [&]() {
-        __syncthreads();
+        lds_barrier();
         if (tid < kGS) {
             own += (long long)(int)cells[tid + 1];
             cells[tid + 1] = 0u;
         }
         __syncthreads();
     };
-    int run = 0; // pixel visits since the last drain
-    int buf = 0;
-    for (int k0 = 0; k0 < nK; k0 += kGSlab, buf ^= 1) {
-        const int S = min(kGSlab, nK - k0);
-        if (tid < 64) {
-            int lo = 0, up = -1;
-            if (lane < S) {
-                if (whole) {
-                    up = nF - 1;
-                } else {
-                    const float k = (float)(k0 + lane);
-                    const float g0 = fmaf(f1[0], k, f0[0]), g1 = fmaf(f1[1], k, f0[1]);
-                    constexpr float big = 0x1p24f;
-                    lo = max(0, floor_i32(__builtin_amdgcn_fmed3f(fminf(g0, g1), -big, big)) - 1);
-                    up = min(nF - 1,
-                             floor_i32(__builtin_amdgcn_fmed3f(fmaxf(g0, g1), -big, big)) + 1);
-                }
-                span[buf][lane] = make_int2(lo, up);
-            }
-            int w = max(up - lo + 1, 0);
-            for (int off = 32; off > 0; off >>= 1) w = max(w, __shfl_xor(w, off, 64));
-            if (lane == 0) width[buf] = w;
+    // depth and detector coordinate as affine forms of the pixel (f, k) along (F, K): cf f + ck k
+    // + c1; cell coordinate relative to the segment's first LDS cell, w eta + cu
+    double dc[3], ec[3], L, cu, wmul;
+    {
+        double dx, dy, dz, ex, ey, ez;
+        if (VIEWS) {
+            const float4 m0 = tab[3 * a], m1 = tab[3 * a + 1];
+            dx = m0.x, dy = m0.y, dz = m0.z;
+            ex = m1.x, ey = m1.y, ez = m1.z;
+            L = m0.w, cu = m1.w, wmul = tab[3 * a + 2].x;
+        } else {
+            const float4 m = tab[a];
+            dx = m.x, dy = -m.y, dz = m.w;
+            ex = (double)m.y * inv_du, ey = (double)m.x * inv_du, ez = 0.0;
+            L = m.z, cu = uoff, wmul = inv_du;
         }
-        __syncthreads();
-        const int NW = width[buf];
-        const int total = NW * S;
-        if (total == 0) continue;
-        // element e = tid + n kMaxBlock of the chunk as (dF, dk), dF fastest; a step of
-        // kMaxBlock elements is (sF, sK). Quotients by NW through an FP32 reciprocal: (m + 0.5)
-        // / NW lies at least 0.5 / NW from an integer, far more than the rounding for m < 2^20.
-        const float rNW = 1.0f / (float)NW;
-        int dk = (int)(((float)tid + 0.5f) * rNW), dF = tid - dk * NW;
-        const int sK = (int)(((float)kMaxBlock + 0.5f) * rNW), sF = kMaxBlock - sK * NW;
-        int e = tid;
-        for (int base = 0; base < total; base += kGPass) {
-            const int n = min(kGPass, total - base);
-            if (run + n > kGBudget) {
+        cu -= (double)(c0 - 1);
+        dc[2] = dx * bx + dy * by + dz, ec[2] = ex * bx + ey * by + ez;
+        dx *= sx, ex *= sx, dy *= sy, ey *= sy;
+        dc[0] = rows ? dx : dy, dc[1] = rows ? dy : dx;
+        ec[0] = rows ? ex : ey, ec[1] = rows ? ey : ex;
+    }
+    const float vL = (float)L, vcu = (float)cu;
+    const float s1 = ldexpf(1.0f, max(min(-vexp, 127), -126)); // (max|v| below 2^-127 scales to less)
+    const float s2 = (float)(rest * wmul * ldexp(1.0, -vexp - max(min(-vexp, 127), -126)));
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int run = 0; // pixel visits since the last drain
+    __syncthreads(); // the cells are clear
+    for (int k0 = 0; k0 < nK; k0 += kGSlab) {
+        // lane l holds line k0 + l: the first pixel of its interval, then its walk's start and
+        // shares. Every wavefront does the same.
+        const int S = min(kGSlab, nK - k0), k = k0 + min(lane, S - 1);
+        int lo = 0, up = nF - 1;
+        if (!whole) {
+            const float g0 = fmaf(f1[0], (float)k, f0[0]), g1 = fmaf(f1[1], (float)k, f0[1]);
+            constexpr float big = 0x1p24f;
+            const float gl = fminf(g0, g1) - kGMargin, gu = fmaxf(g0, g1) + kGMargin;
+            lo = max(0, floor_i32(__builtin_amdgcn_fmed3f(gl, -big, big)) + 1);
+            up = min(nF - 1, floor_i32(__builtin_amdgcn_fmed3f(gu, -big, big)));
+        }
+        const int NW = __builtin_amdgcn_readfirstlane(wave_max(up - lo + 1));
+        if (NW <= 0) continue;
+        lo = max(0, min(lo, nF - NW));
+        const float dl = (float)(dc[0] * lo + dc[1] * k + dc[2]);
+        const float el = (float)(ec[0] * lo + ec[1] * k + ec[2]);
+        const int at = lo + k * strK;
+        for (int f = 0; f < NW; f += 64) {
+            if (run + kGSlab / 4 * kMaxBlock > kGBudget) {
                 drain();
                 run = 0;
             }
-            run += n;
-            // kGBatch elements per thread at a time, their loads issued together; passes start
-            // at multiples of kGBatch kMaxBlock elements, so a batch never straddles two
-            for (; e < base + n; e += kGBatch * kMaxBlock) {
-                int fq[kGBatch], kq[kGBatch];
-                bool live[kGBatch];
+            run += kGSlab / 4 * kMaxBlock;
+            // this lane's pixel of every line; past the width, its coordinate leaves the segment
+            const bool in = f + lane < NW;
+            const int df = in ? f + lane : 0;
+            const float dp = (float)(dc[0] * df), ep = in ? (float)(ec[0] * df) : 1e30f;
+            for (int l0 = wv; l0 < S; l0 += 4 * kGBatch) {
                 float val[kGBatch];
 #pragma unroll
                 for (int q = 0; q < kGBatch; ++q) {
-                    const int2 sp = span[buf][min(dk, S - 1)];
-                    fq[q] = sp.x + dF;
-                    kq[q] = k0 + dk;
-                    live[q] = e + q * kMaxBlock < base + n && fq[q] <= sp.y;
-                    val[q] = to_f32<SV>(src[live[q] ? fq[q] + kq[q] * strK : 0]);
-                    dF += sF;
-                    if (dF >= NW) {
-                        dF -= NW;
-                        ++dk;
-                    }
-                    dk += sK;
+                    const int l = min(l0 + 4 * q, S - 1);
+                    val[q] = to_f32<SV>(src[__builtin_amdgcn_readlane(at, l) + df]);
                 }
 #pragma unroll
                 for (int q = 0; q < kGBatch; ++q) {
-                    const float vs = live[q] ? ldexpf(val[q] * smant, sexp) : 0.0f;
-                    if (vs == 0.0f) continue;
-                    const int ix = rows ? fq[q] : kq[q], iy = rows ? kq[q] : fq[q];
-                    const float x = ((float)ix - (float)nx / 2.0f) * sx + ox + 0.5f;
-                    const float y = ((float)iy - (float)ny / 2.0f) * sy + oy + 0.5f;
-                    float u, wt;
-                    bpT_geom<VIEWS, WPOW>(tab, a, x, y, x * inv_du, y * inv_du, uoff, hi, u, wt);
-                    const int i = floor_i32(u) - (c0 - 1);
-                    if ((unsigned)i > (unsigned)kGS) continue;
-                    const float al = __builtin_amdgcn_fractf(u);
-                    const float t = vs * wt * (VIEWS ? 1.0f : inv_du);
-                    const float t1 = t * al, t0 = t - t1;
+                    const int l = l0 + 4 * q;
+                    if (l >= S) break;
+                    const float vs = val[q] * s1 * s2;
+                    const float rd = __builtin_amdgcn_rcpf(
+                        dp + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dl), l)));
+                    const float eta =
+                        ep + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(el), l));
+                    const float w = vL * rd;
+                    const float u = fmaf(w, eta, vcu);
+                    const int i = floor_i32(u);
+                    if ((unsigned)i > (unsigned)kGS || vs == 0.0f) continue;
+                    const float t = vs * (WPOW == 2 ? w * w : w);
+                    const float t1 = t * __builtin_amdgcn_fractf(u), t0 = t - t1;
                     atomicAdd(&cells[i], (unsigned)round_i32(t0));
                     atomicAdd(&cells[i + 1], (unsigned)round_i32(t1));
                 }
             }
         }
     }
-    __syncthreads();
+    lds_barrier();
     if (tid < kGS) {
         own += (long long)(int)cells[tid + 1];
         const int c = c0 + tid;

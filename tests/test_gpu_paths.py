@@ -105,3 +105,47 @@ def test_forward_3d_boxes(oracle, gpu, what, rec):
     vol = np.random.RandomState(4).rand(*rec.vol_shape)
     got = cm.forward(torch.tensor(vol, dtype=torch.float32, device=gpu), geom)
     assert rel_l2(got, oracle.fwd3d(geom, vol)) <= RTOL_L2, what
+
+
+@pytest.mark.parametrize("views", [False, True])
+@pytest.mark.parametrize("ny,nx,D,du", [
+    (3, 2, 5, 1.0),        # lines shorter than a wavefront, a segment wider than the detector
+    (9, 64, 64, 1.5),      # one line's width, one whole segment
+    (67, 150, 129, 1.0),   # chunks of 64 lines and a remainder; a segment of one cell
+    (40, 200, 20, 12.0),   # segments wider than the image: walks of several steps
+])
+def test_backward_transpose_lines(oracle, gpu, views, ny, nx, D, du):
+    """Widths, lines and segments at the edges of the walk's steps, chunks and batches."""
+    n = max(ny, nx)
+    more = {"det_offset": 1.25, "exact_geometry": True} if views else {}
+    geom = cm.FanGeometry(DSD=3.0 * n, DSO=2.0 * n, angles=np.linspace(0, 6, 7),
+                          vol_shape=(ny, nx), det_shape=D, det_spacing=du, **more)
+    v = np.random.RandomState(nx).rand(ny, nx) - 0.3
+    x = torch.tensor(v, dtype=torch.float32, device=gpu)
+    for mode, wpow in (("reference", 1), ("fbp", 2)):
+        got = cm.backward_transpose(x, geom, mode=mode)
+        assert rel_l2(got, oracle.bp2d_T(geom, v, wpow=wpow)) <= RTOL_L2
+    # the scale's two factors over the range of FP32: powers of two scale the result exactly
+    big = cm.backward_transpose(x * 2.0 ** 100, geom, mode="reference")
+    assert torch.equal(big, cm.backward_transpose(x, geom, mode="reference") * 2.0 ** 100)
+
+
+@pytest.mark.parametrize("what,rec", [
+    ("one slice", lambda: cone(21, 30, 17, 5, 60.0, 90.0, nz=1, ny=13)),
+    ("two chunks", lambda: cone(41, 33, 16, 4, 90.0, 130.0, nz=81, ny=7)),   # 40 slices, and one
+    ("one voxel wide", lambda: cone(1, 18, 30, 6, 60.0, 90.0, nz=19, ny=17)),
+    # pixels that see a quarter of the volume each: boxes of many steps, and whole slices
+    ("wide boxes", lambda: cone(30, 6, 6, 3, 80.0, 120.0, du=(10.0, 10.0))),
+    ("whole slices", lambda: cone(30, 5, 5, 3, 45.0, 60.0, du=(40.0, 40.0))),
+])
+def test_backward_transpose_3d_boxes(oracle, gpu, what, rec):
+    rec = rec()
+    geom = as_cone_geometry(rec)
+    v = np.random.RandomState(3).rand(*rec.vol_shape) - 0.3
+    x = torch.tensor(v, dtype=torch.float32, device=gpu)
+    for mode, kw in (("reference", {}), ("matched", {"matched": True}),
+                     ("fdk", {"matched": True, "fdk": True})):
+        got = cm.backward_transpose(x, geom, mode=mode)
+        assert rel_l2(got, oracle.bp3d_T(geom, v, **kw)) <= RTOL_L2, (what, mode)
+    tiny = cm.backward_transpose(x * 2.0 ** -100, geom, mode="matched")
+    assert torch.equal(tiny, cm.backward_transpose(x, geom, mode="matched") * 2.0 ** -100)
