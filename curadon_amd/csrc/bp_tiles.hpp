@@ -14,8 +14,6 @@
 namespace cmi {
 
 constexpr int kPadDet = 2; // zero border of staged sinograms and panels, in cells
-constexpr int kZB = 8;     // z voxels per thread in the 3D backprojector (general geometry)
-constexpr int kYB = 16;    // y voxels per thread in the 3D backprojector (y-invariant U, W)
 
 // Per-angle tables: the bodies take the table pointer type as a template parameter. The plain
 // kernels pass their `const __restrict__` arguments (scalar loads already). The serving kernels
@@ -159,155 +157,99 @@ __device__ __forceinline__ float bp2d_tile(rsrc_t R, TAB tab, int A, int D, int 
     return (r[0] + r[2 * NY * 64]) + (r[NY * 64] + r[3 * NY * 64]);
 }
 
-// Sum over angles for kZB consecutive voxels of one (x, y) column. M[a] is a 3x4 matrix over
-// the centred voxel index h = (x - cx, y - cy, z - cz, 1) giving (U, V, W); (U/W, V/W) is the
-// lower-tap panel coordinate. MATCHED drops voxels behind the source (W <= 0); FDK weights by
-// 1 / W^2. (hx, hy, hz) is the centred index of the column's first voxel. `R` covers
-// [A][V + 4][U + 4].
-template <class SS, bool MATCHED, bool FDK, class TAB>
-__device__ __forceinline__ void bp3d_column(rsrc_t R, TAB M, int A, int U,
-                                           int V, float hx, float hy, float hz,
-                                           float (&acc)[kZB]) {
-    const int Up = U + 2 * kPadDet, Vp = V + 2 * kPadDet;
-    const int panel = Up * Vp;
-    const int sRow = Up * (int)sizeof(typename SS::raw);
-    const float ulim = (float)U, vlim = (float)V;
-    int base = kPadDet * Up + kPadDet;
-    for (int a = 0; a < A; ++a, base += panel) {
-        const TAB m = M + 12 * a; // wave-uniform: scalar loads
-        float Uh = fmaf(m[0], hx, fmaf(m[1], hy, fmaf(m[2], hz, m[3])));
-        float Vh = fmaf(m[4], hx, fmaf(m[5], hy, fmaf(m[6], hz, m[7])));
-        float Wh = fmaf(m[8], hx, fmaf(m[9], hy, fmaf(m[10], hz, m[11])));
-#pragma unroll
-        for (int z = 0; z < kZB; ++z) {
-            const float rw = __builtin_amdgcn_rcpf(Wh);
-            const float u = __builtin_amdgcn_fmed3f(Uh * rw, -2.0f, ulim);
-            const float v = __builtin_amdgcn_fmed3f(Vh * rw, -2.0f, vlim);
-            const float fu = __builtin_amdgcn_fractf(u), fv = __builtin_amdgcn_fractf(v);
-            const int o = base + __mul24((int)floorf(v), Up) + (int)floorf(u);
-            const Pair p0 = buf_pair<SS>(R, o, 0);
-            const Pair p1 = buf_pair<SS>(R, o, sRow);
-            const float r0 = fmaf(fu, p0.hi - p0.lo, p0.lo);
-            const float r1 = fmaf(fu, p1.hi - p1.lo, p1.lo);
-            float s = fmaf(fv, r1 - r0, r0);
-            if (FDK) s *= rw * rw;
-            if (MATCHED) s = Wh > 0.0f ? s : 0.0f;
-            acc[z] += s;
-            Uh += m[2];
-            Vh += m[6];
-            Wh += m[10];
-        }
-    }
-}
-
 // ------------------------------------------------------------------------------------------
-// LDS-staged y runs, for matrices whose U and W rows do not depend on y (M[a][1] == M[a][9] == 0:
-// circular orbits about the y axis, panel turned at most about y). Then a run of voxels along y
-// shares its perspective divide, u tap, u weight and distance weight, and v advances by a
-// constant step.
+// Cone-beam backprojection of a tile of voxels by a workgroup of 256 threads, a run of voxels per
+// thread. M[a] is a 3x4 matrix over the centred voxel index h = (x - cx, y - cy, z - cz, 1) giving
+// (U, V, W); (U/W, V/W) is the lower-tap panel coordinate, clamped to [-2, U] and [-2, V]. The
+// sample is bilinear in the zero-bordered panel. MATCHED drops voxels behind the source (W <= 0);
+// FDK weights by 1 / W^2.
 //
-// A workgroup of 256 threads owns a tile of kTileX x kYB x kTileZ voxels (x, y, z); thread t
-// takes the run of kYB y voxels at (x0 + t % kTileX, z0 + t / kTileX). Angles go in groups of
-// kGroup: every wavefront computes the group's panel footprints from the tile's 8 corners (8
-// lanes per angle; U/W and V/W are linear-fractional, so over a box where W > 0 their extremes
-// are at corners). Each group goes in chunks of kChunk angles: the workgroup stages the
-// chunk's footprints (rows of at most kFootW columns, at most kFootRows rows, from the
-// zero-bordered panel) into LDS and the runs sample from there. A chunk with a footprint that
-// does not fit (or a corner with W <= 0) is sampled from global memory instead, with the same
-// arithmetic.
+// The angles' panel footprints are staged in LDS. Angles go in groups of kGroup: every wavefront
+// computes the group's footprints from the tile's 8 corners (8 lanes per angle; U/W and V/W are
+// linear-fractional, so over a box where W > 0 their extremes are at corners). Per angle the
+// workgroup stages the footprint (rows of at most kFootW columns, at most kFootRows rows, from
+// the zero-bordered panel) into LDS and the runs sample from there. An angle whose footprint does
+// not fit (or with a corner with W <= 0) is sampled from global memory instead, with the same
+// arithmetic, after the others.
 //
-// Per voxel: u = clamp(U/W), v = clamp(fma(y, dv, V0/W)) with dv = M[a][5]/W, lower taps floor(u),
-// floor(v) in the staged panel, bilinear weights fract(u), fract(v); MATCHED drops W <= 0, FDK
-// weights by 1/W^2.
-constexpr int kTileX = 16, kTileZ = 16;
+// A sample's LDS address is two fma: byte strides and the slot's offset are held as FP32 subnormals,
+// n 2^-149, whose bit pattern is the integer n, so that products with the integral floors and their
+// sums are exact below 2^23 and the sum's bits are the address; fractions are p - floor(p). On
+// gfx950 these issue at the full rate, where a conversion to an integer, its offset, the 24-bit
+// product and v_fract_f32 each take almost two slots.
 constexpr int kFootW = 64;                        // staged columns per row
-constexpr int kFootCols = 68;                     // LDS row pitch: 16-byte rows, banks shifted
+// LDS row pitch: 16-byte rows, 12 banks further per row. A wavefront's 8 x 8 columns of voxels (x,
+// z) then meet few conflicts in any direction of view (68 and 16 x 4 columns, whose u and v advance
+// together at 45 degrees: a third of all LDS cycles).
+constexpr int kFootCols = 76;
 constexpr int kFootRows = 60;
-constexpr int kFootSlot = kFootCols * kFootRows;  // floats per staged angle (16 KB)
-// Angles per chunk. One: the 16 KB of LDS and the body's 80 VGPRs keep 6 workgroups (24
-// wavefronts) per CU; four angles per chunk (64 KB) kept two and ran the 384^3 FDK
-// backprojection at half the speed.
-constexpr int kChunk = 1;
-constexpr int kFootFloats = kChunk * kFootSlot;
+constexpr int kFootFloats = kFootCols * kFootRows;
 
-// Per-angle set-up of a run: u tap column (element offset of the lower tap's column relative to
-// `base`), u weight, first v, v step and the sample weight.
-struct RunAngle {
-    int col;
-    float fu, v, dv, w;
-};
-
-template <bool MATCHED, bool FDK, class TAB>
-__device__ __forceinline__ RunAngle run_angle(TAB m, float hx, float hy, float hz,
-                                              float ulim) {
-    const float Uh = fmaf(m[0], hx, fmaf(m[2], hz, m[3]));
-    const float Wh = fmaf(m[8], hx, fmaf(m[10], hz, m[11]));
-    const float Vh = fmaf(m[4], hx, fmaf(m[5], hy, fmaf(m[6], hz, m[7])));
-    const float rw = __builtin_amdgcn_rcpf(Wh);
-    const float u = __builtin_amdgcn_fmed3f(Uh * rw, -2.0f, ulim);
-    RunAngle r;
-    r.col = floor_i32(u);
-    r.fu = __builtin_amdgcn_fractf(u);
-    r.v = Vh * rw;
-    r.dv = m[5] * rw;
-    r.w = FDK ? rw * rw : 1.0f;
-    if (MATCHED) r.w = Wh > 0.0f ? r.w : 0.0f;
-    return r;
-}
-
-// Staged footprints: one workgroup-shared array (16 KB) for every instantiation a kernel
-// uses, so a kernel that dispatches between modes allocates it once.
+// The staged footprint, one workgroup-shared array (18 KB) for every instantiation a kernel uses, so
+// a kernel that dispatches between modes allocates it once.
 static __shared__ __align__(16) float foot_lds[kFootFloats];
 
 // Angles whose footprints one pass of a wavefront evaluates: 8 lanes (the tile's corners) each.
 constexpr int kGroup = 8;
 
-// The kYB samples of one run at one angle from its staged footprint. `bk`: byte offset in
-// foot_lds of the lower tap's column in the slot's row 0; `vbase`: the padded-panel row of that
-// slot row minus kPadDet, so the lower tap's slot row is floor(v) - vbase.
-template <bool WEIGHTED>
-__device__ __forceinline__ void yrun_samples(const RunAngle &r, unsigned bk, int vbase,
-                                             float vlim, float (&acc)[kYB]) {
-#pragma unroll
-    for (int y = 0; y < kYB; ++y) {
-        const float v = __builtin_amdgcn_fmed3f(fmaf((float)y, r.dv, r.v), -2.0f, vlim);
-        const unsigned addr = __umul24((unsigned)(floor_i32(v) - vbase), 4u * kFootCols) + bk;
-        const float *p =
-            reinterpret_cast<const float *>(reinterpret_cast<const char *>(foot_lds) + addr);
-        const float r0 = fmaf(r.fu, p[1] - p[0], p[0]);
-        const float r1 = fmaf(r.fu, p[kFootCols + 1] - p[kFootCols], p[kFootCols]);
-        const float s = fmaf(__builtin_amdgcn_fractf(v), r1 - r0, r0);
-        acc[y] = WEIGHTED ? fmaf(s, r.w, acc[y]) : acc[y] + s;
-    }
+// i 2^-149, opaque in a vector register.
+__device__ __forceinline__ float subnormal(int i) {
+    float f = __int_as_float(i < 0 ? -i | (int)0x80000000 : i);
+    asm("" : "+v"(f));
+    return f;
 }
 
-// (hx, hy, hz): centred index of this thread's run start; (tx, ty, tz): of the tile origin.
-// All 256 threads of the workgroup call it together (lanes without voxels too).
-template <class SS, bool MATCHED, bool FDK, class TAB>
-__device__ __forceinline__ void bp3d_yrun_lds(rsrc_t R, TAB M, int A, int U,
-                                             int V, float hx, float hy, float hz, float tx,
-                                             float ty, float tz, float (&acc)[kYB]) {
+// A staged footprint: the sample at the integral lower taps (iu, iv) lies at the LDS byte address
+// fma(iv, row, fma(iu, col, ofs)), its pair on the next row kFootCols floats further.
+struct Foot {
+    float row, col, ofs; // byte strides and offset, as subnormals
+};
+
+// The four taps of a bilinear sample: rows v and v + 1, columns u and u + 1.
+struct Taps {
+    Pair r0, r1;
+};
+__device__ __forceinline__ Taps foot_taps(unsigned at) {
+    const auto *p = (const __attribute__((address_space(3))) float *)(uintptr_t)at;
+    return {{p[0], p[1]}, {p[kFootCols], p[kFootCols + 1]}};
+}
+__device__ __forceinline__ float bilerp(const Taps &t, float fu, float fv) {
+    const float r0 = lerp_pair(t.r0, fu), r1 = lerp_pair(t.r1, fu);
+    return fmaf(fv, r1 - r0, r0);
+}
+
+// Runs every angle of a tile whose corners lie at (tx, ty, tz) and (tx + ex, ty + ey, tz + ez)
+// (centred indices): from_foot(m, foot) with its footprint staged, then from_panel(m, o), o the
+// element offset of the panel's cell (0, 0), for the angles whose footprint was not (a pass of its
+// own: the two in one loop cost a copy of the runs' sums per angle). YINV: the U and W rows do not
+// depend on y. All 256 threads of the workgroup call it together (lanes without voxels too).
+template <class SS, bool YINV, class TAB, class F1, class F2>
+__device__ __forceinline__ void bp3d_angles(rsrc_t R, TAB M, int A, int U, int V, float tx,
+                                            float ty, float tz, float ex, float ey, float ez,
+                                            F1 &&from_foot, F2 &&from_panel) {
     const int Up = U + 2 * kPadDet, Vp = V + 2 * kPadDet;
     const int panel = Up * Vp;
-    const int sRow = Up * (int)sizeof(typename SS::raw);
     const float ulim = (float)U, vlim = (float)V;
     const int tid = threadIdx.x;
     const int lane = tid & 63, k8 = lane >> 3, c8 = lane & 7;
     // the tile's corner this lane evaluates
-    const float cx = (c8 & 1) ? tx + (float)(kTileX - 1) : tx;
-    const float cy = (c8 & 2) ? ty + (float)(kYB - 1) : ty;
-    const float cz = (c8 & 4) ? tz + (float)(kTileZ - 1) : tz;
-    // staging: thread tid copies quad tid % 16 of footprint row tid / 16 (and rows + 16 ...)
-    const int qrow = tid >> 4, qcol = (tid & 15) << 2;
-    for (int g0 = 0; g0 < A; g0 += kGroup) {
-        const int ng = min(kGroup, A - g0);
-        // footprints: lanes 8k .. 8k+7 take angle g0 + k
+    const float cx = (c8 & 1) ? tx + ex : tx;
+    const float cy = (c8 & 2) ? ty + ey : ty;
+    const float cz = (c8 & 4) ? tz + ez : tz;
+    // The footprints of the angles from g0 on, lanes 8k .. 8k+7 for angle g0 + k: the slot's
+    // padded-panel origin (su, sv) and row count. Returns bit 8k for the angles that fit.
+    auto footprints = [&](int g0, int &su, int &sv, int &rows) -> uint64_t {
         float umin = 0.0f, umax = 0.0f, vmin = 0.0f, vmax = 0.0f;
         int ok = 1;
-        if (k8 < ng) {
+        if (g0 + k8 < A) {
             const TAB m = M + 12 * (g0 + k8);
-            const float Uh = fmaf(m[0], cx, fmaf(m[2], cz, m[3]));
-            const float Wh = fmaf(m[8], cx, fmaf(m[10], cz, m[11]));
+            float Uh = fmaf(m[2], cz, m[3]), Wh = fmaf(m[10], cz, m[11]);
+            if (!YINV) {
+                Uh = fmaf(m[1], cy, Uh);
+                Wh = fmaf(m[9], cy, Wh);
+            }
+            Uh = fmaf(m[0], cx, Uh);
+            Wh = fmaf(m[8], cx, Wh);
             const float Vh = fmaf(m[4], cx, fmaf(m[5], cy, fmaf(m[6], cz, m[7])));
             const float rw = __builtin_amdgcn_rcpf(Wh);
             umin = umax = __builtin_amdgcn_fmed3f(Uh * rw, -2.0f, ulim);
@@ -322,91 +264,195 @@ __device__ __forceinline__ void bp3d_yrun_lds(rsrc_t R, TAB M, int A, int U,
             vmax = fmaxf(vmax, __shfl_xor(vmax, off, 64));
             ok = min(ok, __shfl_xor(ok, off, 64));
         }
-        // every lane now holds its angle's bounds: the slot's padded-panel origin (su0, sv0) and
-        // row count, evaluated once for the group's angles. Lower taps lie within
-        // [floor(min) - 1, floor(max) + 1] (one-texel margin for the rounding of the samples'
-        // u and v against the corners') and the upper tap adds one more row / column.
+        // Lower taps lie within [floor(min) - 1, floor(max) + 1] (one-texel margin for the
+        // rounding of the samples' u and v against the corners') and the upper tap adds one more
+        // row / column.
         const int ulo = floor_i32(umin) - 1 + kPadDet, uhi = floor_i32(umax) + 2 + kPadDet;
         const int vlo = floor_i32(vmin) - 1 + kPadDet, vhi = floor_i32(vmax) + 2 + kPadDet;
-        const int su0 = max(ulo, 0), sv0 = max(vlo, 0);
-        const int srows = min(vhi, Vp - 1) - sv0 + 1;
-        const uint64_t fitm =
-            __ballot(ok && uhi - ulo + 1 <= kFootW && vhi - vlo + 1 <= kFootRows);
-        // not unrolled: eight copies of the sampling code per mode cost registers and
-        // instruction cache (the readlanes take the uniform lane index from an SGPR)
+        su = max(ulo, 0);
+        sv = max(vlo, 0);
+        rows = min(vhi, Vp - 1) - sv + 1;
+        return __ballot(ok && uhi - ulo + 1 <= kFootW && vhi - vlo + 1 <= kFootRows);
+    };
+    // Staging: thread tid copies quad tid % 16 of rows tid / 16 + 16 j. The first kAhead rows of
+    // the next angle are loaded before the current one is sampled.
+    constexpr int kAhead = 2;
+    constexpr unsigned es = sizeof(typename SS::raw);
+    const int qrow = tid >> 4, qcol = (tid & 15) << 2;
+    float *const to = &foot_lds[qrow * kFootCols + qcol];
+    const int lds0 = (int)(uintptr_t)(__attribute__((address_space(3))) float *)foot_lds;
+    const float row = subnormal(4 * kFootCols), col = subnormal(4);
+    bool missed = false;
+    int su0 = 0, sv0 = 0, srows = 0; // of the group's angles, by lane
+    uint64_t fit = 0;
+    bool fits;
+    int su, sv, rows;
+    unsigned g; // byte offset of the thread's first quad
+    RawQuad<SS> next[kAhead];
+    // Loads rows that the footprint does not have too (not stored; beyond the stack they read 0).
+    auto ahead = [&](int a) {
+        if ((a & (kGroup - 1)) == 0) fit = footprints(a, su0, sv0, srows);
+        const int c = 8 * (a & (kGroup - 1));
+        fits = (fit >> c) & 1u;
+        su = __builtin_amdgcn_readlane(su0, c);
+        sv = __builtin_amdgcn_readlane(sv0, c);
+        rows = __builtin_amdgcn_readlane(srows, c);
+        g = (unsigned)(a * panel + (sv + qrow) * Up + su + qcol) * es;
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j)
+            next[j] = buf_raw_quad_at<SS>(R, (int)(g + 16u * j * Up * es));
+    };
+    auto store = [&](int j, const Quad &v) {
+        *reinterpret_cast<float4 *>(to + 16 * j * kFootCols) =
+            make_float4(v.v[0], v.v[1], v.v[2], v.v[3]);
+    };
+    ahead(0);
+    // not unrolled: copies of the sampling code cost registers and instruction cache
 #pragma unroll 1
-        for (int c = 0; c < kGroup; c += kChunk) {
-            if (c >= ng) break;
-            const int na = min(kChunk, ng - c);
-            const int a0 = g0 + c;
-            int ssu[kChunk], ssv[kChunk], srw[kChunk];
-            bool fits = true;
+    for (int a = 0; a < A; ++a) {
+        const bool staged = fits;
+        missed = missed || !staged;
+        const int at0 = lds0 + 4 * ((kPadDet - sv) * kFootCols + (kPadDet - su));
+        if (staged) {
+            __syncthreads(); // the previous angle's samples are read
 #pragma unroll
-            for (int k = 0; k < kChunk; ++k) {
-                ssu[k] = __builtin_amdgcn_readlane(su0, 8 * (c + k));
-                ssv[k] = __builtin_amdgcn_readlane(sv0, 8 * (c + k));
-                srw[k] = __builtin_amdgcn_readlane(srows, 8 * (c + k));
-                if (k < na) fits = fits && ((fitm >> (8 * (c + k))) & 1u);
-            }
-            if (!fits) { // from global memory
-                for (int k = 0; k < na; ++k) {
-                    const TAB m = M + 12 * (a0 + k); // wave-uniform: scalar loads
-                    const RunAngle r = run_angle<MATCHED, FDK>(m, hx, hy, hz, ulim);
-                    const int col = (a0 + k) * panel + kPadDet * Up + kPadDet + r.col;
-#pragma unroll
-                    for (int y = 0; y < kYB; ++y) {
-                        const float v =
-                            __builtin_amdgcn_fmed3f(fmaf((float)y, r.dv, r.v), -2.0f, vlim);
-                        const int o = col + __mul24(floor_i32(v), Up);
-                        const float r0 = lerp_pair(buf_pair<SS>(R, o, 0), r.fu);
-                        const float r1 = lerp_pair(buf_pair<SS>(R, o, sRow), r.fu);
-                        const float s = fmaf(__builtin_amdgcn_fractf(v), r1 - r0, r0);
-                        acc[y] = (MATCHED || FDK) ? fmaf(s, r.w, acc[y]) : acc[y] + s;
-                    }
-                }
-                continue;
-            }
-            __syncthreads(); // the previous chunk's samples are read
-            // staging: thread tid copies quad tid % 16 of rows tid / 16 + 16 j of every slot;
-            // the first rows of the chunk's slots with their loads in flight together, then the
-            // rest (more loads in flight raised the body to 120 VGPRs, four wavefronts a SIMD)
-            {
-                Quad first[kChunk];
-#pragma unroll
-                for (int k = 0; k < kChunk; ++k)
-                    if (k < na && qrow < srw[k])
-                        first[k] = buf_quad<SS>(R, (a0 + k) * panel + (ssv[k] + qrow) * Up +
-                                                       ssu[k] + qcol);
-#pragma unroll
-                for (int k = 0; k < kChunk; ++k)
-                    if (k < na && qrow < srw[k])
-                        *reinterpret_cast<float4 *>(
-                            &foot_lds[k * kFootSlot + qrow * kFootCols + qcol]) =
-                            make_float4(first[k].v[0], first[k].v[1], first[k].v[2],
-                                        first[k].v[3]);
-#pragma unroll
-                for (int k = 0; k < kChunk; ++k) {
-                    if (k >= na) break;
-                    const int g = (a0 + k) * panel + ssv[k] * Up + ssu[k] + qcol;
-                    for (int row = qrow + 16; row < srw[k]; row += 16) {
-                        const Quad v = buf_quad<SS>(R, g + row * Up);
-                        *reinterpret_cast<float4 *>(
-                            &foot_lds[k * kFootSlot + row * kFootCols + qcol]) =
-                            make_float4(v.v[0], v.v[1], v.v[2], v.v[3]);
-                    }
-                }
-            }
+            for (int j = 0; j < kAhead; ++j)
+                if (qrow + 16 * j < rows) store(j, to_quad<SS>(next[j]));
+#pragma unroll 1
+            for (int j = kAhead; qrow + 16 * j < rows; ++j)
+                store(j, buf_quad_at<SS>(R, (int)(g + 16u * j * Up * es)));
+        }
+        if (a + 1 < A) ahead(a + 1);
+        if (staged) {
             __syncthreads();
-#pragma unroll
-            for (int k = 0; k < kChunk; ++k) {
-                if (k >= na) break;
-                const TAB m = M + 12 * (a0 + k); // wave-uniform: scalar loads
-                const RunAngle r = run_angle<MATCHED, FDK>(m, hx, hy, hz, ulim);
-                const unsigned bk = 4u * (unsigned)(k * kFootSlot + r.col + kPadDet - ssu[k]);
-                yrun_samples<MATCHED || FDK>(r, bk, ssv[k] - kPadDet, vlim, acc);
-            }
+            from_foot(M + 12 * a, Foot{row, col, subnormal(at0)});
         }
     }
+    if (!missed) return;
+    for (int g0 = 0; g0 < A; g0 += kGroup) {
+        fit = footprints(g0, su0, sv0, srows);
+#pragma unroll 1
+        for (int c = 0; c < min(kGroup, A - g0); ++c)
+            if (!((fit >> (8 * c)) & 1u))
+                from_panel(M + 12 * (g0 + c), (g0 + c) * panel + kPadDet * Up + kPadDet);
+    }
+}
+
+// A workgroup's tile: kTileX x kRun x kTileZ voxels (x, y, z), a run of kRun y voxels per thread.
+// YINV is for matrices whose U and W rows do not depend on y (M[a][1] == M[a][9] == 0: circular
+// orbits about the y axis, panel turned at most about y): a run then shares its perspective divide,
+// u tap, u weight and distance weight, and v advances by a constant step dv = M[a][5] / W, clamped
+// fma(y, dv, V0 / W). Any other geometry has a divide per voxel, and U, V, W advance by the
+// matrix's y column; shorter runs there, since small volumes (128^3) leave wavefronts wanting.
+constexpr int kTileX = 16, kTileZ = 16;
+template <bool YINV>
+constexpr int kRun = YINV ? 16 : 8;
+
+// The (x, z) offset of this thread's run in the tile: 8 x 8 runs per wavefront.
+__device__ __forceinline__ int tile_x() {
+    return (int)((threadIdx.x & 7u) + ((threadIdx.x >> 3) & 8u));
+}
+__device__ __forceinline__ int tile_z() {
+    return (int)(((threadIdx.x >> 3) & 7u) + ((threadIdx.x >> 4) & 8u));
+}
+
+// acc[y] += sum over the angles for the run of the voxels at centred index (hx, hy + y, hz);
+// (tx, hy, tz) is that of the tile's first voxel. `R` covers [A][V + 4][U + 4].
+// Bound by LDS (two pair reads per voxel and angle, 8 clocks per wavefront and CU, and conflicts)
+// and VALU issue alike. 384^3 x 768 views of 576^2 in half precision, YINV: 19.1 ms with integer
+// addresses (17 VALU slots per voxel and angle instead of 13), pitch 68, 16 x 4 columns per
+// wavefront and a footprint's loads waited for at once; 17.8 with FMA addresses; 16.2 now (LDS busy
+// 91 % of the time, 11 % of that in conflicts; 1.3 VALU instructions a clock and CU).
+// 128^3 x 180 views of 192^2, general: 420 us gathering from global memory (two pairs per voxel at
+// about 18 clocks per gather and CU), 292 staged.
+template <class SS, bool YINV, bool MATCHED, bool FDK, class TAB>
+__device__ __forceinline__ void bp3d_run(rsrc_t R, TAB M, int A, int U, int V, float hx, float hy,
+                                         float hz, float tx, float tz, float (&acc)[kRun<YINV>]) {
+    const float ulim = (float)U, vlim = (float)V;
+    const int Up = U + 2 * kPadDet;
+    const int sRow = Up * (int)sizeof(typename SS::raw);
+    // at_column(iu) gives taps(iv), the taps between columns iu and iu + 1 and rows iv and iv + 1.
+    // kBatch voxels' taps are read before the first is used.
+    constexpr int kBatch = 4;
+    auto run = [&](TAB m, auto &&at_column) {
+        float Uh = fmaf(m[0], hx, fmaf(m[2], hz, m[3]));
+        float Wh = fmaf(m[8], hx, fmaf(m[10], hz, m[11]));
+        float Vh = fmaf(m[4], hx, fmaf(m[5], hy, fmaf(m[6], hz, m[7])));
+        auto weight = [&](float rw) {
+            const float w = FDK ? rw * rw : 1.0f;
+            return MATCHED ? (Wh > 0.0f ? w : 0.0f) : w;
+        };
+        auto add = [&](int y, const Taps &t, float fu, float fv, float w) {
+            const float s = bilerp(t, fu, fv);
+            acc[y] = (MATCHED || FDK) ? fmaf(s, w, acc[y]) : acc[y] + s;
+        };
+        if constexpr (YINV) {
+            const float rw = __builtin_amdgcn_rcpf(Wh);
+            const float u = __builtin_amdgcn_fmed3f(Uh * rw, -2.0f, ulim);
+            const float iu = floorf(u), fu = u - iu;
+            const float v0 = Vh * rw, dv = m[5] * rw, w = weight(rw);
+            auto taps = at_column(iu);
+#pragma unroll
+            for (int y = 0; y < kRun<YINV>; y += kBatch) {
+                float fv[kBatch];
+                Taps t[kBatch];
+#pragma unroll
+                for (int k = 0; k < kBatch; ++k) {
+                    const float v =
+                        __builtin_amdgcn_fmed3f(fmaf((float)(y + k), dv, v0), -2.0f, vlim);
+                    const float iv = floorf(v);
+                    fv[k] = v - iv;
+                    t[k] = taps(iv);
+                }
+#pragma unroll
+                for (int k = 0; k < kBatch; ++k) add(y + k, t[k], fu, fv[k], w);
+            }
+        } else {
+            Uh = fmaf(m[1], hy, Uh);
+            Wh = fmaf(m[9], hy, Wh);
+            float dU = m[1], dV = m[5], dW = m[9];
+            asm("" : "+v"(dU), "+v"(dV), "+v"(dW)); // in vector registers
+#pragma unroll
+            for (int y = 0; y < kRun<YINV>; y += kBatch) {
+                float fu[kBatch], fv[kBatch], w[kBatch];
+                Taps t[kBatch];
+#pragma unroll
+                for (int k = 0; k < kBatch; ++k) {
+                    const float rw = __builtin_amdgcn_rcpf(Wh);
+                    const float u = __builtin_amdgcn_fmed3f(Uh * rw, -2.0f, ulim);
+                    const float v = __builtin_amdgcn_fmed3f(Vh * rw, -2.0f, vlim);
+                    const float iu = floorf(u), iv = floorf(v);
+                    fu[k] = u - iu;
+                    fv[k] = v - iv;
+                    w[k] = weight(rw);
+                    t[k] = at_column(iu)(iv);
+                    Uh += dU;
+                    Vh += dV;
+                    Wh += dW;
+                }
+#pragma unroll
+                for (int k = 0; k < kBatch; ++k) add(y + k, t[k], fu[k], fv[k], w[k]);
+            }
+        }
+    };
+    bp3d_angles<SS, YINV>(
+        R, M, A, U, V, tx, hy, tz, (float)(kTileX - 1), (float)(kRun<YINV> - 1),
+        (float)(kTileZ - 1),
+        [&](TAB m, const Foot &f) {
+            run(m, [&](float iu) {
+                const float ofs = fmaf(iu, f.col, f.ofs);
+                return [=](float iv) { return foot_taps(__float_as_uint(fmaf(iv, f.row, ofs))); };
+            });
+        },
+        [&](TAB m, int base) {
+            run(m, [&](float iu) {
+                const int col = base + (int)iu;
+                return [=](float iv) {
+                    const int o = col + __mul24((int)iv, Up);
+                    return Taps{buf_pair<SS>(R, o, 0), buf_pair<SS>(R, o, sRow)};
+                };
+            });
+        });
 }
 
 } // namespace cmi

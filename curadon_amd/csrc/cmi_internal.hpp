@@ -191,35 +191,45 @@ struct Quad {
     float v[4];
 };
 
-// buf_quad_at takes the byte offset of the first element.
+// The four elements as loaded. A pipeline keeps these in flight: the conversion of 16-bit storage
+// would wait for the load.
 template <class S>
-__device__ __forceinline__ Quad buf_quad_at(rsrc_t r, int byte_offset);
+using RawQuad = unsigned __attribute__((ext_vector_type(sizeof(typename S::raw))));
+
+template <class S>
+__device__ __forceinline__ RawQuad<S> buf_raw_quad_at(rsrc_t r, int byte_offset) {
+    if constexpr (sizeof(typename S::raw) == 4)
+        return __builtin_amdgcn_raw_buffer_load_b128(r, byte_offset, 0, 0);
+    else
+        return __builtin_amdgcn_raw_buffer_load_b64(r, byte_offset, 0, 0);
+}
+
+template <class S>
+__device__ __forceinline__ Quad to_quad(RawQuad<S> v);
 
 template <>
-__device__ __forceinline__ Quad buf_quad_at<F32>(rsrc_t r, int byte_offset) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, byte_offset, 0, 0);
+__device__ __forceinline__ Quad to_quad<F32>(RawQuad<F32> v) {
     const unsigned a = v[0], b = v[1], c = v[2], d = v[3];
     return {{__uint_as_float(a), __uint_as_float(b), __uint_as_float(c), __uint_as_float(d)}};
 }
 template <>
-__device__ __forceinline__ Quad buf_quad_at<F16>(rsrc_t r, int byte_offset) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, byte_offset, 0, 0);
+__device__ __forceinline__ Quad to_quad<F16>(RawQuad<F16> v) {
     const unsigned a = v[0], b = v[1];
     auto h = [](unsigned short x) { return static_cast<float>(__builtin_bit_cast(_Float16, x)); };
     return {{h((unsigned short)(a & 0xffffu)), h((unsigned short)(a >> 16)),
              h((unsigned short)(b & 0xffffu)), h((unsigned short)(b >> 16))}};
 }
 template <>
-__device__ __forceinline__ Quad buf_quad_at<BF16>(rsrc_t r, int byte_offset) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, byte_offset, 0, 0);
+__device__ __forceinline__ Quad to_quad<BF16>(RawQuad<BF16> v) {
     const unsigned a = v[0], b = v[1];
     return {{__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u), __uint_as_float(b << 16),
              __uint_as_float(b & 0xffff0000u)}};
 }
 
+// buf_quad_at takes the byte offset of the first element.
 template <class S>
-__device__ __forceinline__ Quad buf_quad(rsrc_t r, int elem_offset) {
-    return buf_quad_at<S>(r, elem_offset * (int)sizeof(typename S::raw));
+__device__ __forceinline__ Quad buf_quad_at(rsrc_t r, int byte_offset) {
+    return to_quad<S>(buf_raw_quad_at<S>(r, byte_offset));
 }
 
 // Byte size of n elements, for the range check of a resource.

@@ -503,15 +503,9 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
                     auto sample_slab = [&](auto km) {
                         constexpr bool KM = decltype(km)::value;
                         const int W4 = 16 * NQ, S4 = W4 * WQ; // bytes per row and per slice
-                        // as subnormals in vector registers
-                        auto sub = [](int i) {
-                            float f = __int_as_float(i < 0 ? -i | (int)0x80000000 : i);
-                            asm("" : "+v"(f));
-                            return f;
-                        };
-                        const float fS = sub(S4), fW = sub(W4), f4 = sub(4);
+                        const float fS = subnormal(S4), fW = subnormal(W4), f4 = subnormal(4);
                         const float fo =
-                            sub(kofs * S4 + (cQ - Q0) * W4 + (cP - P0) * 4 + box0);
+                            subnormal(kofs * S4 + (cQ - Q0) * W4 + (cP - P0) * 4 + box0);
                         int m4 = KM ? S4 : W4, l4 = KM ? W4 : S4;
                         asm("" : "+v"(m4), "+v"(l4));
                         auto sample = [&](float jj) {
@@ -861,81 +855,49 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj3d(typename SV::raw *__restric
 
 // ---------------------------------------------------------------- backprojection ----------
 
-// One thread per voxel column (ix, iy) and kZB consecutive z; a wavefront covers a 16 x 4 x 8
-// block (bp3d_column). vol += sum over angles.
-template <class SV, class SS, bool MATCHED, bool FDK>
+// Tile of the launch's workgroup over tiles of gridDim.x x gridDim.y x nzt per volume. XCD-aware
+// order: workgroups are dealt to the 8 XCDs in turn, and logical index li gives each XCD a
+// contiguous run of tiles (x fastest), whose panel footprints share L2 (256^3: 2.51
+// -> 2.37 ms).
+struct BpTile {
+    int x, y, z;
+    size_t b;
+};
+__device__ __forceinline__ BpTile bp_tile(int nzt) {
+    const unsigned gx = gridDim.x, gy = gridDim.y, gz = gridDim.z;
+    const unsigned nwg = gx * gy * gz;
+    const unsigned hw = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+    const unsigned n8 = nwg & ~7u;
+    const unsigned li = hw < n8 ? (hw & 7u) * (n8 >> 3) + (hw >> 3) : hw;
+    const unsigned per = gx * gy * (unsigned)nzt;
+    const unsigned l = li % per;
+    return {(int)(l % gx), (int)((l / gx) % gy), (int)(l / (gx * gy)), li / per};
+}
+
+// A workgroup of 256 threads owns a tile of voxels, a run of y voxels per thread, and samples the
+// angles' panel footprints from LDS (bp3d_run). YINV: no angle's U or W row depends on y.
+// vol += sum over angles.
+template <class SV, class SS, bool YINV, bool MATCHED, bool FDK>
 __global__ __launch_bounds__(kMaxBlock) void k_bp3d(typename SV::raw *__restrict__ vol,
                                                     const typename SS::raw *__restrict__ ppad,
                                                     const float *__restrict__ M, int nx, int ny,
                                                     int nz, int U, int V, int A, float cx,
                                                     float cy, float cz) {
-    const int ix = blockIdx.x * blockDim.x + threadIdx.x;
-    const int iy = blockIdx.y * blockDim.y + threadIdx.y;
-    const int nzb = (nz + kZB - 1) / kZB;
-    const int iz0 = (blockIdx.z % nzb) * kZB;
-    const size_t b = blockIdx.z / nzb;
-    if (ix >= nx || iy >= ny) return;
+    constexpr int NY = kRun<YINV>;
+    const BpTile t = bp_tile((nz + kTileZ - 1) / kTileZ);
+    const int ix0 = t.x * kTileX, iy0 = t.y * NY, iz0 = t.z * kTileZ;
+    const int ix = ix0 + tile_x(), iz = iz0 + tile_z();
+    const size_t b = t.b;
     const uint32_t stack = (uint32_t)(U + 2 * kPad) * (V + 2 * kPad) * A;
     const rsrc_t R = make_rsrc(ppad + b * (size_t)stack, bytes_of<SS>(stack));
-    float acc[kZB];
+    float acc[NY];
 #pragma unroll
-    for (int z = 0; z < kZB; ++z) acc[z] = 0.0f;
-    bp3d_column<SS, MATCHED, FDK>(R, M, A, U, V, (float)ix - cx, (float)iy - cy,
-                                  (float)iz0 - cz, acc);
-#pragma unroll
-    for (int z = 0; z < kZB; ++z) {
-        const int iz = iz0 + z;
-        if (iz < nz) {
-            const size_t i = ((b * nz + iz) * ny + iy) * (size_t)nx + ix;
-            vol[i] = from_f32<SV>(to_f32<SV>(vol[i]) + acc[z]);
-        }
-    }
-}
-
-// For matrices whose U and W rows do not depend on y: a workgroup of 256 threads owns a tile of
-// kTileX x kYB x kTileZ voxels, each thread a run of kYB y voxels, and the angles' panel
-// footprints are staged in LDS (bp3d_yrun_lds). vol += sum over angles.
-template <class SV, class SS, bool MATCHED, bool FDK>
-__global__ __launch_bounds__(kMaxBlock) void k_bp3d_y(typename SV::raw *__restrict__ vol,
-                                                      const typename SS::raw *__restrict__ ppad,
-                                                      const float *__restrict__ M, int nx, int ny,
-                                                      int nz, int U, int V, int A, float cx,
-                                                      float cy, float cz) {
-    const int nzt = (nz + kTileZ - 1) / kTileZ;
-    // XCD-aware order: workgroups are dealt to the 8 XCDs in turn, and logical index li gives
-    // each XCD a contiguous run of tiles (x fastest), whose panel footprints share L2
-    // (2.51 -> 2.37 ms at 256^3)
-    int ix0, iy0, iz0;
-    size_t b;
-    {
-        const unsigned gx = gridDim.x, gy = gridDim.y, gz = gridDim.z;
-        const unsigned nwg = gx * gy * gz;
-        const unsigned hw = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-        const unsigned n8 = nwg & ~7u;
-        const unsigned li = hw < n8 ? (hw & 7u) * (n8 >> 3) + (hw >> 3) : hw;
-        const unsigned per = gx * gy * (unsigned)nzt;
-        b = li / per;
-        const unsigned l = li % per;
-        unsigned tx, ty, tz;
-        tx = l % gx;
-        ty = (l / gx) % gy;
-        tz = l / (gx * gy);
-        ix0 = (int)tx * kTileX;
-        iy0 = (int)ty * kYB;
-        iz0 = (int)tz * kTileZ;
-    }
-    const int ix = ix0 + (int)(threadIdx.x % kTileX), iz = iz0 + (int)(threadIdx.x / kTileX);
-    const uint32_t stack = (uint32_t)(U + 2 * kPad) * (V + 2 * kPad) * A;
-    const rsrc_t R = make_rsrc(ppad + b * (size_t)stack, bytes_of<SS>(stack));
-    float acc[kYB];
-#pragma unroll
-    for (int y = 0; y < kYB; ++y) acc[y] = 0.0f;
-    bp3d_yrun_lds<SS, MATCHED, FDK>(R, M, A, U, V, (float)ix - cx, (float)iy0 - cy,
-                                    (float)iz - cz, (float)ix0 - cx, (float)iy0 - cy,
-                                    (float)iz0 - cz, acc);
+    for (int y = 0; y < NY; ++y) acc[y] = 0.0f;
+    bp3d_run<SS, YINV, MATCHED, FDK>(R, M, A, U, V, (float)ix - cx, (float)iy0 - cy,
+                                     (float)iz - cz, (float)ix0 - cx, (float)iz0 - cz, acc);
     if (ix >= nx || iz >= nz) return;
 #pragma unroll
-    for (int y = 0; y < kYB; ++y) {
+    for (int y = 0; y < NY; ++y) {
         const int iy = iy0 + y;
         if (iy < ny) {
             const size_t i = ((b * nz + iz) * ny + iy) * (size_t)nx + ix;
@@ -946,7 +908,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp3d_y(typename SV::raw *__restri
 
 // ------------------------------------------------ transpose of the backprojection -------
 
-// Bᵀ: the transpose of the voxel-driven backprojection (k_bp3d, k_bp3d_y), the gradient of
+// Bᵀ: the transpose of the voxel-driven backprojection (k_bp3d), the gradient of
 // TorchBackprojection. The backprojection adds to voxel h, per projection a, the bilinear
 // interpolation of panel a at (u, v) = (U/W, V/W) from the mode's matrix rows (cells floor(u)
 // + {0, 1} and floor(v) + {0, 1}, weights 1 - fu, fu and 1 - fv, fv; cells outside the panel
@@ -1238,7 +1200,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
 
 // ---------------------------------------------------------------- host helpers -----------
 
-// True when no angle's U or W row depends on y, so k_bp3d_y applies.
+// True when no angle's U or W row depends on y: k_bp3d<YINV>.
 bool y_invariant(const std::vector<float> &m, int64_t A) {
     for (int64_t a = 0; a < A; ++a)
         if (m[12 * a + 1] != 0.0f || m[12 * a + 9] != 0.0f) return false;
@@ -1442,7 +1404,6 @@ cmi_status check_call(const cmi_plan3d *p, const void *vol, int vol_dtype, const
                     "%s: plan precision does not match sinogram precision (%s)", fn,
                     dtype_name(sino_dtype));
     if (batch * (uint64_t)p->A > 65535 ||
-        batch * (uint64_t)((p->g.nz + kZB - 1) / kZB) > 65535 ||
         batch * (uint64_t)(p->g.nz + 2 * kPad) > 65535)
         return fail(CMI_ERR_INVALID_ARGUMENT, "%s: batch too large for one launch", fn);
     CMI_TRY(check_device_ptr(vol, p->device, "volume"));
@@ -1784,25 +1745,20 @@ CMI_API cmi_status cmi_backward_3d(const cmi_plan3d *plan, void *volume, int vol
         const uint64_t n = (uint64_t)Up * Vp * A * batch;
         hipLaunchKernelGGL((k_stage_panel<SS>), dim3((unsigned)((n + 4 * 256 - 1) / (4 * 256))),
                            dim3(256), 0, s, (const RS *)sinogram, (RS *)scratch, U, V, n);
-        if (plan->ycols[mode]) {
+        auto launch = [&](auto yinv) {
+            constexpr bool Y = decltype(yinv)::value;
             const int nzt = (nz + kTileZ - 1) / kTileZ;
-            dim3 bb(kTileX * kTileZ), bg((unsigned)((nx + kTileX - 1) / kTileX),
-                                         (unsigned)((ny + kYB - 1) / kYB), (unsigned)(nzt * batch));
-            auto kern = mode == CMI_BP3D_MATCHED ? k_bp3d_y<SV, SS, true, false>
-                        : mode == CMI_BP3D_FDK   ? k_bp3d_y<SV, SS, true, true>
-                                                 : k_bp3d_y<SV, SS, false, false>;
-            hipLaunchKernelGGL(kern, bg, bb, 0, s, (typename SV::raw *)volume, (const RS *)scratch,
-                               M, nx, ny, nz, U, V, A, cx, cy, cz);
-        } else {
-            const int nzb = (nz + kZB - 1) / kZB;
-            dim3 bb(16, 16), bg((unsigned)((nx + 15) / 16), (unsigned)((ny + 15) / 16),
-                                (unsigned)(nzb * batch));
-            auto kern = mode == CMI_BP3D_MATCHED ? k_bp3d<SV, SS, true, false>
-                        : mode == CMI_BP3D_FDK   ? k_bp3d<SV, SS, true, true>
-                                                 : k_bp3d<SV, SS, false, false>;
-            hipLaunchKernelGGL(kern, bg, bb, 0, s, (typename SV::raw *)volume,
-                               (const RS *)scratch, M, nx, ny, nz, U, V, A, cx, cy, cz);
-        }
+            const dim3 bg((unsigned)((nx + kTileX - 1) / kTileX),
+                          (unsigned)((ny + kRun<Y> - 1) / kRun<Y>), (unsigned)(nzt * batch));
+            auto kern = mode == CMI_BP3D_MATCHED ? k_bp3d<SV, SS, Y, true, false>
+                        : mode == CMI_BP3D_FDK   ? k_bp3d<SV, SS, Y, true, true>
+                                                 : k_bp3d<SV, SS, Y, false, false>;
+            hipLaunchKernelGGL(kern, bg, dim3(kTileX * kTileZ), 0, s,
+                               (typename SV::raw *)volume, (const RS *)scratch, M, nx, ny, nz, U,
+                               V, A, cx, cy, cz);
+        };
+        if (plan->ycols[mode]) launch(std::true_type{});
+        else launch(std::false_type{});
         CMI_HIP_TRY(hipGetLastError());
         return CMI_OK;
     });

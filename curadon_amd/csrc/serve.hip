@@ -13,7 +13,7 @@
 //   workgroup exits after at most total + grid iterations of the counter, so the launch
 //   drains.
 //
-// Per-tile arithmetic is the plain backprojectors' own (bp2d_tile / bp3d_column with the
+// Per-tile arithmetic is the plain backprojectors' own (bp2d_tile / bp3d_run with the
 // same scalar inputs), so a voxel's value does not depend on the launch it ran in.
 //
 // Data layout in HBM (per server)
@@ -38,8 +38,7 @@ namespace {
 constexpr int kRing = 4;       // launches whose job tables may be in flight at once
 constexpr int kThreads = 256;  // threads per workgroup
 constexpr int kTile2X = 64, kTile2Y = 4;   // fan-beam tile: pixels
-constexpr int kTile3X = 16, kTile3Y = 16;  // cone-beam tile: columns of kZB voxels
-// cone-beam tile of y runs: kTileX x kYB x kTileZ voxels (bp_tiles.hpp)
+// cone-beam tile: kTileX x kRun x kTileZ voxels (bp_tiles.hpp)
 
 // Device copy of a job with the derived values the kernel needs.
 struct DevJob {
@@ -59,11 +58,9 @@ struct DevJob {
 uint64_t tiles_of(const cmi_bp_job &j) {
     if (j.kind == CMI_JOB_FAN2D)
         return (uint64_t)((j.nx + kTile2X - 1) / kTile2X) * ((j.ny + kTile2Y - 1) / kTile2Y);
-    if (j.columns == 1)
-        return (uint64_t)((j.nx + kTileX - 1) / kTileX) * ((j.ny + kYB - 1) / kYB) *
-               ((j.nz + kTileZ - 1) / kTileZ);
-    return (uint64_t)((j.nx + kTile3X - 1) / kTile3X) * ((j.ny + kTile3Y - 1) / kTile3Y) *
-           ((j.nz + kZB - 1) / kZB);
+    const uint64_t run = j.columns == 1 ? kRun<true> : kRun<false>;
+    return (uint64_t)((j.nx + kTileX - 1) / kTileX) * ((j.ny + run - 1) / run) *
+           ((j.nz + kTileZ - 1) / kTileZ);
 }
 
 // ---------------------------------------------------------------- staging -----------------
@@ -168,68 +165,35 @@ __device__ __forceinline__ void serve_tile_2d(const DevJob &J, uint32_t t, float
     vol[i] = from_f32<SV>(to_f32<SV>(vol[i]) + acc * J.inv_du);
 }
 
-// Cone-beam tile: the column of kZB voxels k_bp3d gives thread (ix, iy) of z block zb.
-template <class SV, class SS>
+// Cone-beam tile: the tile and runs k_bp3d gives block (tx, ty, tz). Every thread of the workgroup
+// calls this (the LDS staging inside synchronises the workgroup).
+template <class SV, class SS, bool YINV>
 __device__ __forceinline__ void serve_tile_3d(const DevJob &J, uint32_t t) {
-    const uint32_t per_slab = (uint32_t)J.tiles_x * (uint32_t)J.tiles_y;
-    const int zb = (int)(t / per_slab);
-    const uint32_t r = t % per_slab;
-    const int ix = (int)(r % (uint32_t)J.tiles_x) * kTile3X + (int)(threadIdx.x % kTile3X);
-    const int iy = (int)(r / (uint32_t)J.tiles_x) * kTile3Y + (int)(threadIdx.x / kTile3X);
-    if (ix >= J.nx || iy >= J.ny) return;
-    const int iz0 = zb * kZB;
-    const rsrc_t R = make_rsrc(J.sino, J.sino_bytes);
-    float acc[kZB];
-#pragma unroll
-    for (int z = 0; z < kZB; ++z) acc[z] = 0.0f;
-    const float hx = (float)ix - J.cx, hy = (float)iy - J.cy, hz = (float)iz0 - J.cz;
-    if (J.mode == CMI_BP3D_FDK)
-        bp3d_column<SS, true, true>(R, const_table(J.table), J.nangles, J.nu, J.nv, hx, hy, hz, acc);
-    else if (J.mode == CMI_BP3D_MATCHED)
-        bp3d_column<SS, true, false>(R, const_table(J.table), J.nangles, J.nu, J.nv, hx, hy, hz, acc);
-    else
-        bp3d_column<SS, false, false>(R, const_table(J.table), J.nangles, J.nu, J.nv, hx, hy, hz, acc);
-    auto *vol = static_cast<typename SV::raw *>(J.volume);
-#pragma unroll
-    for (int z = 0; z < kZB; ++z) {
-        const int iz = iz0 + z;
-        if (iz < J.nz) {
-            const size_t i = ((size_t)iz * J.ny + iy) * (size_t)J.nx + ix;
-            vol[i] = from_f32<SV>(to_f32<SV>(vol[i]) + acc[z]);
-        }
-    }
-}
-
-// Cone-beam tile of y runs: the tile and runs k_bp3d_y gives block (tx, ty, tz). Every thread
-// of the workgroup calls this (the LDS staging inside synchronises the workgroup).
-template <class SV, class SS>
-__device__ __forceinline__ void serve_tile_3d_y(const DevJob &J, uint32_t t) {
+    constexpr int NY = kRun<YINV>;
     const uint32_t per_slab = (uint32_t)J.tiles_x * (uint32_t)J.tiles_y;
     const int zt = (int)(t / per_slab);
     const uint32_t r = t % per_slab;
     const int ix0 = (int)(r % (uint32_t)J.tiles_x) * kTileX;
-    const int iy0 = (int)(r / (uint32_t)J.tiles_x) * kYB;
+    const int iy0 = (int)(r / (uint32_t)J.tiles_x) * NY;
     const int iz0 = zt * kTileZ;
-    const int ix = ix0 + (int)(threadIdx.x % kTileX), iz = iz0 + (int)(threadIdx.x / kTileX);
+    const int ix = ix0 + tile_x(), iz = iz0 + tile_z();
     const rsrc_t R = make_rsrc(J.sino, J.sino_bytes);
-    float acc[kYB];
+    float acc[NY];
 #pragma unroll
-    for (int y = 0; y < kYB; ++y) acc[y] = 0.0f;
+    for (int y = 0; y < NY; ++y) acc[y] = 0.0f;
     const float hx = (float)ix - J.cx, hy = (float)iy0 - J.cy, hz = (float)iz - J.cz;
     const float tx = (float)ix0 - J.cx, tz = (float)iz0 - J.cz;
+    const ctab M = const_table(J.table);
     if (J.mode == CMI_BP3D_FDK)
-        bp3d_yrun_lds<SS, true, true>(R, const_table(J.table), J.nangles, J.nu, J.nv, hx, hy, hz, tx, hy, tz,
-                                      acc);
+        bp3d_run<SS, YINV, true, true>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, tz, acc);
     else if (J.mode == CMI_BP3D_MATCHED)
-        bp3d_yrun_lds<SS, true, false>(R, const_table(J.table), J.nangles, J.nu, J.nv, hx, hy, hz, tx, hy, tz,
-                                       acc);
+        bp3d_run<SS, YINV, true, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, tz, acc);
     else
-        bp3d_yrun_lds<SS, false, false>(R, const_table(J.table), J.nangles, J.nu, J.nv, hx, hy, hz, tx, hy, tz,
-                                        acc);
+        bp3d_run<SS, YINV, false, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, tz, acc);
     if (ix >= J.nx || iz >= J.nz) return;
     auto *vol = static_cast<typename SV::raw *>(J.volume);
 #pragma unroll
-    for (int y = 0; y < kYB; ++y) {
+    for (int y = 0; y < NY; ++y) {
         const int iy = iy0 + y;
         if (iy < J.ny) {
             const size_t i = ((size_t)iz * J.ny + iy) * (size_t)J.nx + ix;
@@ -274,7 +238,7 @@ __global__ __launch_bounds__(kThreads) void k_serve_bp2d(const DevJob *__restric
     }
 }
 
-// Cone-beam tiles. YRUNS: every job of the launch takes the y-run body (columns == 1), and the
+// Cone-beam tiles. YRUNS: every job of the launch takes the y-invariant body (columns == 1), and the
 // general column body is left out. Five wavefronts per SIMD: the persistent loop around the
 // body's three modes took 97 VGPRs (four wavefronts per SIMD); 96 fit without spills, 80 spilled.
 template <class SV, class SS, bool YRUNS>
@@ -287,8 +251,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) v
         if (t >= total) return;
         const DevJob &J = job_of(jobs, njobs, t);
         const uint32_t lt = t - J.first + J.tile_begin;
-        if (YRUNS || J.columns == 1) serve_tile_3d_y<SV, SS>(J, lt);
-        else serve_tile_3d<SV, SS>(J, lt);
+        if (YRUNS || J.columns == 1) serve_tile_3d<SV, SS, true>(J, lt);
+        else serve_tile_3d<SV, SS, false>(J, lt);
     }
 }
 
@@ -354,7 +318,7 @@ struct cmi_server {
     int device = 0;
     uint32_t max_jobs = 0;
     uint32_t grid = 0;   // resident workgroups of the cone-beam serving kernel (any job)
-    uint32_t grid3y = 0; // resident workgroups of the cone-beam serving kernel (y runs only)
+    uint32_t grid3y = 0; // resident workgroups of the cone-beam serving kernel (y-invariant jobs only)
     uint32_t grid2d = 0; // resident workgroups of the fan-beam serving kernel
     DevJob *d_jobs = nullptr;
     unsigned *d_counter = nullptr;
@@ -551,7 +515,7 @@ CMI_API cmi_status cmi_serve_backproject(cmi_server *p, const cmi_bp_job *jobs, 
     // launch-tile numbering (the two kinds run in separate launches)
     DevJob *h = p->h_jobs + (size_t)slot * p->max_jobs;
     uint32_t n2 = 0, total2 = 0, total3 = 0;
-    bool yruns = true; // every cone-beam job takes the y-run body
+    bool yruns = true; // every cone-beam job takes the y-invariant body
     for (uint32_t i = 0; i < njobs; ++i) {
         n2 += jobs[i].kind == CMI_JOB_FAN2D ? 1u : 0u;
         if (jobs[i].kind != CMI_JOB_FAN2D && jobs[i].columns != 1) yruns = false;
@@ -572,12 +536,10 @@ CMI_API cmi_status cmi_serve_backproject(cmi_server *p, const cmi_bp_job *jobs, 
         if (fan) {
             d.tiles_x = (d.nx + kTile2X - 1) / kTile2X;
             d.tiles_y = (d.ny + kTile2Y - 1) / kTile2Y;
-        } else if (d.columns == 1) {
-            d.tiles_x = (d.nx + kTileX - 1) / kTileX;
-            d.tiles_y = (d.ny + kYB - 1) / kYB;
         } else {
-            d.tiles_x = (d.nx + kTile3X - 1) / kTile3X;
-            d.tiles_y = (d.ny + kTile3Y - 1) / kTile3Y;
+            const int run = d.columns == 1 ? kRun<true> : kRun<false>;
+            d.tiles_x = (d.nx + kTileX - 1) / kTileX;
+            d.tiles_y = (d.ny + run - 1) / run;
         }
         uint32_t &first = fan ? total2 : total3;
         d.first = first;

@@ -149,3 +149,35 @@ def test_backward_transpose_3d_boxes(oracle, gpu, what, rec):
         assert rel_l2(got, oracle.bp3d_T(geom, v, **kw)) <= RTOL_L2, (what, mode)
     tiny = cm.backward_transpose(x * 2.0 ** -100, geom, mode="matched")
     assert torch.equal(tiny, cm.backward_transpose(x, geom, mode="matched") * 2.0 ** -100)
+
+
+TILTED = np.array([[0.3, 1.9, 3.0, 5.1, 5.9], [0.7, 1.4, 0.2, 1.5, 1.1], [0.1, 0.9, 1.5, 0.4, 0.2]])
+
+
+@pytest.mark.parametrize("what,rec", [
+    # circular orbits: runs of 16 y voxels
+    ("one angle", lambda: cone(17, 20, 18, 1, 60.0, 90.0, nz=15, ny=5)),
+    ("one group", lambda: cone(16, 24, 26, 8, 60.0, 90.0, nz=33, ny=16)),
+    ("a group and one", lambda: cone(33, 50, 44, 9, 80.0, 120.0, nz=16, ny=17)),
+    # footprints of 30 to 60 rows, and wider or higher than the staged ones (some or all angles)
+    ("many rows", lambda: cone(20, 70, 90, 6, 60.0, 90.0, du=(0.45, 0.6))),
+    ("too wide", lambda: cone(20, 130, 40, 6, 60.0, 90.0, du=(0.3, 1.0))),
+    ("too high", lambda: cone(20, 40, 160, 6, 60.0, 90.0, du=(1.0, 0.25))),
+    ("some too wide", lambda: cone(20, 90, 40, 12, 33.0, 66.0, du=(0.6, 1.0))),
+    # a ragged tile's corners lie behind the source, its voxels do not
+    ("corners behind", lambda: cone(17, 40, 40, 12, 20.0, 44.0)),
+    # tilted orbits: runs of 8 y voxels, a divide per voxel
+    ("tilted", lambda: cone(17, 30, 28, 5, 60.0, 90.0, nz=18, ny=9, angles=TILTED)),
+    ("tilted, too wide", lambda: cone(19, 150, 150, 5, 60.0, 90.0, du=(0.25, 0.25),
+                                      angles=TILTED)),
+    ("tilted, corners behind", lambda: cone(17, 40, 40, 5, 20.0, 44.0, ny=17, angles=TILTED)),
+])
+def test_backward_3d_footprints(oracle, gpu, what, rec):
+    rec = rec()
+    geom = as_cone_geometry(rec)
+    y = np.random.RandomState(6).rand(rec.nangles, *rec.det_shape)
+    x = torch.tensor(y, dtype=torch.float32, device=gpu)
+    for mode, kw in (("reference", {}), ("matched", {"matched": True}),
+                     ("fdk", {"matched": True, "fdk": True})):
+        got = cm.backward(x, geom, mode=mode)
+        assert rel_l2(got, oracle.bp3d(geom, y, **kw)) <= RTOL_L2, (what, mode)
