@@ -338,26 +338,29 @@ __device__ __forceinline__ void bp3d_angles(rsrc_t R, TAB M, int A, int U, int V
     }
 }
 
-// A workgroup's tile: kTileX x kRun x kTileZ voxels (x, y, z), a run of kRun y voxels per thread.
+// A workgroup's tile: kTileX x kTileY x kTileZ voxels (x, y, z), a run of kRun y voxels per thread.
 // YINV is for matrices whose U and W rows do not depend on y (M[a][1] == M[a][9] == 0: circular
 // orbits about the y axis, panel turned at most about y): a run then shares its perspective divide,
 // u tap, u weight and distance weight, and v advances by a constant step dv = M[a][5] / W, clamped
 // fma(y, dv, V0 / W). Any other geometry has a divide per voxel, and U, V, W advance by the
-// matrix's y column; shorter runs there, since small volumes (128^3) leave wavefronts wanting.
-constexpr int kTileX = 16, kTileZ = 16;
+// matrix's y column; half as many voxels there, since small volumes (128^3) leave wavefronts
+// wanting.
+constexpr int kTileX = 16, kTileY = 16;
+template <bool YINV>
+constexpr int kTileZ = YINV ? 16 : 8;
 template <bool YINV>
 constexpr int kRun = YINV ? 16 : 8;
 
-// The (x, z) offset of this thread's run in the tile: 8 x 8 runs per wavefront.
-__device__ __forceinline__ int tile_x() {
-    return (int)((threadIdx.x & 7u) + ((threadIdx.x >> 3) & 8u));
-}
-__device__ __forceinline__ int tile_z() {
-    return (int)(((threadIdx.x >> 3) & 7u) + ((threadIdx.x >> 4) & 8u));
+// This thread's run in the tile: offset of its first voxel. A wavefront has 8 x 8 runs (x, z).
+template <bool YINV>
+__device__ __forceinline__ int3 tile_run() {
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    return make_int3((l & 7) + 8 * (w & 1), YINV ? 0 : 8 * (w >> 1),
+                     (l >> 3) + (YINV ? 8 * (w >> 1) : 0));
 }
 
 // acc[y] += sum over the angles for the run of the voxels at centred index (hx, hy + y, hz);
-// (tx, hy, tz) is that of the tile's first voxel. `R` covers [A][V + 4][U + 4].
+// (tx, ty, tz) is that of the tile's first voxel. `R` covers [A][V + 4][U + 4].
 // Bound by LDS (two pair reads per voxel and angle, 8 clocks per wavefront and CU, and conflicts)
 // and VALU issue alike. 384^3 x 768 views of 576^2 in half precision, YINV: 19.1 ms with integer
 // addresses (17 VALU slots per voxel and angle instead of 13), pitch 68, 16 x 4 columns per
@@ -367,7 +370,8 @@ __device__ __forceinline__ int tile_z() {
 // about 18 clocks per gather and CU), 292 staged.
 template <class SS, bool YINV, bool MATCHED, bool FDK, class TAB>
 __device__ __forceinline__ void bp3d_run(rsrc_t R, TAB M, int A, int U, int V, float hx, float hy,
-                                         float hz, float tx, float tz, float (&acc)[kRun<YINV>]) {
+                                         float hz, float tx, float ty, float tz,
+                                         float (&acc)[kRun<YINV>]) {
     const float ulim = (float)U, vlim = (float)V;
     const int Up = U + 2 * kPadDet;
     const int sRow = Up * (int)sizeof(typename SS::raw);
@@ -436,8 +440,8 @@ __device__ __forceinline__ void bp3d_run(rsrc_t R, TAB M, int A, int U, int V, f
         }
     };
     bp3d_angles<SS, YINV>(
-        R, M, A, U, V, tx, hy, tz, (float)(kTileX - 1), (float)(kRun<YINV> - 1),
-        (float)(kTileZ - 1),
+        R, M, A, U, V, tx, ty, tz, (float)(kTileX - 1), (float)(kTileY - 1),
+        (float)(kTileZ<YINV> - 1),
         [&](TAB m, const Foot &f) {
             run(m, [&](float iu) {
                 const float ofs = fmaf(iu, f.col, f.ofs);

@@ -884,9 +884,10 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp3d(typename SV::raw *__restrict
                                                     int nz, int U, int V, int A, float cx,
                                                     float cy, float cz) {
     constexpr int NY = kRun<YINV>;
-    const BpTile t = bp_tile((nz + kTileZ - 1) / kTileZ);
-    const int ix0 = t.x * kTileX, iy0 = t.y * NY, iz0 = t.z * kTileZ;
-    const int ix = ix0 + tile_x(), iz = iz0 + tile_z();
+    const BpTile t = bp_tile((nz + kTileZ<YINV> - 1) / kTileZ<YINV>);
+    const int tx = t.x * kTileX, ty = t.y * kTileY, tz = t.z * kTileZ<YINV>;
+    const int3 o = tile_run<YINV>();
+    const int ix = tx + o.x, iy0 = ty + o.y, iz = tz + o.z;
     const size_t b = t.b;
     const uint32_t stack = (uint32_t)(U + 2 * kPad) * (V + 2 * kPad) * A;
     const rsrc_t R = make_rsrc(ppad + b * (size_t)stack, bytes_of<SS>(stack));
@@ -894,7 +895,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp3d(typename SV::raw *__restrict
 #pragma unroll
     for (int y = 0; y < NY; ++y) acc[y] = 0.0f;
     bp3d_run<SS, YINV, MATCHED, FDK>(R, M, A, U, V, (float)ix - cx, (float)iy0 - cy,
-                                     (float)iz - cz, (float)ix0 - cx, (float)iz0 - cz, acc);
+                                     (float)iz - cz, (float)tx - cx, (float)ty - cy,
+                                     (float)tz - cz, acc);
     if (ix >= nx || iz >= nz) return;
 #pragma unroll
     for (int y = 0; y < NY; ++y) {
@@ -1747,13 +1749,13 @@ CMI_API cmi_status cmi_backward_3d(const cmi_plan3d *plan, void *volume, int vol
                            dim3(256), 0, s, (const RS *)sinogram, (RS *)scratch, U, V, n);
         auto launch = [&](auto yinv) {
             constexpr bool Y = decltype(yinv)::value;
-            const int nzt = (nz + kTileZ - 1) / kTileZ;
+            const int nzt = (nz + kTileZ<Y> - 1) / kTileZ<Y>;
             const dim3 bg((unsigned)((nx + kTileX - 1) / kTileX),
-                          (unsigned)((ny + kRun<Y> - 1) / kRun<Y>), (unsigned)(nzt * batch));
+                          (unsigned)((ny + kTileY - 1) / kTileY), (unsigned)(nzt * batch));
             auto kern = mode == CMI_BP3D_MATCHED ? k_bp3d<SV, SS, Y, true, false>
                         : mode == CMI_BP3D_FDK   ? k_bp3d<SV, SS, Y, true, true>
                                                  : k_bp3d<SV, SS, Y, false, false>;
-            hipLaunchKernelGGL(kern, bg, dim3(kTileX * kTileZ), 0, s,
+            hipLaunchKernelGGL(kern, bg, dim3(kMaxBlock), 0, s,
                                (typename SV::raw *)volume, (const RS *)scratch, M, nx, ny, nz, U,
                                V, A, cx, cy, cz);
         };

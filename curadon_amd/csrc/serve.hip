@@ -38,7 +38,7 @@ namespace {
 constexpr int kRing = 4;       // launches whose job tables may be in flight at once
 constexpr int kThreads = 256;  // threads per workgroup
 constexpr int kTile2X = 64, kTile2Y = 4;   // fan-beam tile: pixels
-// cone-beam tile: kTileX x kRun x kTileZ voxels (bp_tiles.hpp)
+// cone-beam tile: kTileX x kTileY x kTileZ voxels (bp_tiles.hpp)
 
 // Device copy of a job with the derived values the kernel needs.
 struct DevJob {
@@ -58,9 +58,9 @@ struct DevJob {
 uint64_t tiles_of(const cmi_bp_job &j) {
     if (j.kind == CMI_JOB_FAN2D)
         return (uint64_t)((j.nx + kTile2X - 1) / kTile2X) * ((j.ny + kTile2Y - 1) / kTile2Y);
-    const uint64_t run = j.columns == 1 ? kRun<true> : kRun<false>;
-    return (uint64_t)((j.nx + kTileX - 1) / kTileX) * ((j.ny + run - 1) / run) *
-           ((j.nz + kTileZ - 1) / kTileZ);
+    const uint64_t tz = j.columns == 1 ? kTileZ<true> : kTileZ<false>;
+    return (uint64_t)((j.nx + kTileX - 1) / kTileX) * ((j.ny + kTileY - 1) / kTileY) *
+           ((j.nz + tz - 1) / tz);
 }
 
 // ---------------------------------------------------------------- staging -----------------
@@ -173,23 +173,24 @@ __device__ __forceinline__ void serve_tile_3d(const DevJob &J, uint32_t t) {
     const uint32_t per_slab = (uint32_t)J.tiles_x * (uint32_t)J.tiles_y;
     const int zt = (int)(t / per_slab);
     const uint32_t r = t % per_slab;
-    const int ix0 = (int)(r % (uint32_t)J.tiles_x) * kTileX;
-    const int iy0 = (int)(r / (uint32_t)J.tiles_x) * NY;
-    const int iz0 = zt * kTileZ;
-    const int ix = ix0 + tile_x(), iz = iz0 + tile_z();
+    const int x0 = (int)(r % (uint32_t)J.tiles_x) * kTileX;
+    const int y0 = (int)(r / (uint32_t)J.tiles_x) * kTileY;
+    const int z0 = zt * kTileZ<YINV>;
+    const int3 o = tile_run<YINV>();
+    const int ix = x0 + o.x, iy0 = y0 + o.y, iz = z0 + o.z;
     const rsrc_t R = make_rsrc(J.sino, J.sino_bytes);
     float acc[NY];
 #pragma unroll
     for (int y = 0; y < NY; ++y) acc[y] = 0.0f;
     const float hx = (float)ix - J.cx, hy = (float)iy0 - J.cy, hz = (float)iz - J.cz;
-    const float tx = (float)ix0 - J.cx, tz = (float)iz0 - J.cz;
+    const float tx = (float)x0 - J.cx, ty = (float)y0 - J.cy, tz = (float)z0 - J.cz;
     const ctab M = const_table(J.table);
     if (J.mode == CMI_BP3D_FDK)
-        bp3d_run<SS, YINV, true, true>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, tz, acc);
+        bp3d_run<SS, YINV, true, true>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, ty, tz, acc);
     else if (J.mode == CMI_BP3D_MATCHED)
-        bp3d_run<SS, YINV, true, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, tz, acc);
+        bp3d_run<SS, YINV, true, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, ty, tz, acc);
     else
-        bp3d_run<SS, YINV, false, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, tz, acc);
+        bp3d_run<SS, YINV, false, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, ty, tz, acc);
     if (ix >= J.nx || iz >= J.nz) return;
     auto *vol = static_cast<typename SV::raw *>(J.volume);
 #pragma unroll
@@ -537,9 +538,8 @@ CMI_API cmi_status cmi_serve_backproject(cmi_server *p, const cmi_bp_job *jobs, 
             d.tiles_x = (d.nx + kTile2X - 1) / kTile2X;
             d.tiles_y = (d.ny + kTile2Y - 1) / kTile2Y;
         } else {
-            const int run = d.columns == 1 ? kRun<true> : kRun<false>;
             d.tiles_x = (d.nx + kTileX - 1) / kTileX;
-            d.tiles_y = (d.ny + run - 1) / run;
+            d.tiles_y = (d.ny + kTileY - 1) / kTileY;
         }
         uint32_t &first = fan ? total2 : total3;
         d.first = first;

@@ -44,7 +44,7 @@ from .reconstruction import (cosine_weights_cone, cosine_weights_fan, fft_length
 # 2.1e12 voxel-angles/s at 384^3 against 2.35e12 pixel-angles/s at 2048^2).
 CONE_COST = 1.15
 PIXELS_PER_TILE_2D = 64 * 4
-# voxels per tile of the cone-beam kernel: runs of 16 y voxels / of 8 (16 x 16 runs)
+# voxels per tile of the cone-beam kernel: y-invariant matrices (16 x 16 x 16) / others (16 x 16 x 8)
 VOXELS_PER_TILE_3D = {True: 16 * 16 * 16, False: 16 * 16 * 8}
 
 
