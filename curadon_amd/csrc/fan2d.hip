@@ -801,42 +801,68 @@ __device__ __forceinline__ float adj2d_ymax(const float *__restrict__ parts) {
     return m;
 }
 
-// Matched adjoint (exact transpose of k_fwd2d), tile-driven. A workgroup owns a kT2 x kT2 texel
-// tile and a group of angles. Per angle, the candidate rays are those through the tile's
-// footprint box (every texel's [t - .5, t + 1.5) box, in the ray search frame, projected onto
-// the detector through its corners); the candidates of kAdjAngles angles form one list, and
-// each thread takes one ray, keeps its parameters in registers and walks the kT2 + 1 dominant
-// rows whose samples reach the tile. A sample on row pd (lower tap) with column c adds y q.x
-// times its forward weights to the texels (pd, floor c), (pd, floor c + 1), (pd + 1, ...)
-// (fan2d.hip header), in fixed point with integer LDS atomics: gfx950 runs them about 45 times
-// faster than FP32 LDS atomic adds, and integer sums are exact, so the result does not depend on
-// the order of the additions. A term is rounded to units of max|y q.x| / 2^19 (so |term| <=
-// 2^19) and added to a 32-bit LDS cell: half the LDS atomic traffic of 64-bit cells, which
-// bounds this kernel. A candidate ray adds at most two terms to a cell (one sample per dominant
-// row, and a cell takes the lower-row weights of one sample and the upper-row weights of the
-// sample before), so a run of passes whose candidates number c adds at most 2 c 2^19 to a cell:
-// each thread moves its share of the cells into 64-bit registers and clears them before that
-// bound could pass 2^31 - 1 (runs of at most 2047 candidates), which keeps every 32-bit sum
-// exact. y- and x-dominant rays add to separate tiles whose rows run along their dominant axis,
-// padded by one row and column on each side: the four taps of a sample are then four immediate
-// offsets from one LDS address and need no bounds checks. Each tile then adds its sums, in units
-// of max|y q.x| / 2^30, to a 64-bit image with integer global atomics (several angle groups
-// share a tile), and k_adj2d_finish adds that image to the volume.
-constexpr int kT2 = 32;       // texel tile edge
-constexpr int kAdjAngles = 8; // angles whose candidate rays are staged together
+// Matched adjoint (exact transpose of k_fwd2d), tile-driven. A workgroup owns a tile of texels, a
+// group of angles and the rays of one dominant axis: kT2Rows rows across that axis (row: constant
+// dominant coordinate) by kT2Cols columns along the other. Per angle, the candidate rays are those
+// through the tile's footprint box (every texel's [t - .5, t + 1.5) box, in the ray search frame,
+// projected onto the detector through its corners); the candidates of kAdjAngles angles form one
+// list, and each thread takes one ray, keeps its parameters in registers and walks the rows on
+// which its samples reach the tile. Angles all of whose candidates have the other dominant axis are
+// left out; the tiles are wide since a ray of slope m leaves kT2Cols columns' width only for the
+// share m kT2Rows / (kT2Cols + m kT2Rows) of its wavefront's rows (32 x 32 texels: lane use 0.62).
+//
+// A sample on row t (lower tap) with column c adds wl = y q.x (1 - frac md) times (1 - frac c,
+// frac c) to row t and wh = y q.x frac md times the same to row t + 1 (fan2d.hip header). Row t so
+// gets two terms of a ray, from its samples t - 1 and t, whose columns differ by the slope's |m|
+// <= 1: three cells from the floor of the smaller one, p, on. With f = frac p, A the weight of the
+// sample at p and B the other's (constant along the ray), g1 = min(f + |m|, 1) and g2 = max(f +
+// |m| - 1, 0), they get A + B - b, b - B g2 and B g2, b = A f + B g1. The first sample's own row
+// and the row after the last sample get one term each, apart.
+// Terms are fixed point with integer LDS atomics: gfx950 runs them about 45 times faster than FP32
+// LDS atomic adds, and integer sums are exact, so the result does not depend on the order of the
+// additions. A, B and the terms are rounded to units of max|y q.x| / 2^19 (so |A + B| <= 2^19)
+// and added to a 32-bit LDS cell: half the LDS traffic of 64-bit cells. A candidate ray adds at
+// most one term to a cell, within 2^19 + 2, so a run of passes whose candidates number c keeps a
+// cell within c (2^19 + 2): each thread moves its share of the cells into 64-bit registers and
+// clears them before that could pass 2^31 - 1, which keeps every 32-bit sum exact. Each tile
+// then adds its sums, in units of max|y q.x| / 2^30, to a 64-bit image with integer global atomics
+// (the two axes' tiles and several angle groups share a texel), and k_adj2d_finish adds that image
+// to the volume.
+//
+// Bound by LDS atomics (three per row and ray, two clocks per wavefront and CU each, and conflicts)
+// and VALU issue (16 slots: 12 full, 4 half rate) alike: the LDS address is one FMA on subnormals
+// (bp_tiles.hpp). 16 images of 512^2, 512 angles of 724 cells: 2.79 ms with four atomics per
+// sample, 32 x 32 texels of both axes and the candidates' lists worked out on scalars; 2.01 with the
+// rows and tiles above (VALU 1.2 instructions a clock and CU, LDS busy 61 %), 1.65 with the lists
+// by lane (1.4 and 77 %, 46 % of that in conflicts). 24 x 96 texels: 1.66, 16 x 128: 1.71,
+// 48 x 64: 1.83.
+constexpr int kT2Rows = 32, kT2Cols = 64;
+constexpr int kAdjAngles = 16; // angles whose candidate rays form one list: 4 lanes each
 // Candidate order within an angle: phase p holds the rays p, p + kAdjPh, p + 2 kAdjPh, ..., so
 // the lanes of a wavefront take rays kAdjPh cells apart and add to different LDS cells more
-// often (padding the phases to equal size leaves holes, which are skipped). At 1024^2: kAdjPh
-// 1 (adjacent rays): 1.23 ms, 2: 1.15, 3: 1.21, 4: 1.27; bit-identical.
+// often (padding the phases to equal size leaves holes, which are skipped). At the size above: kAdjPh 1
+// (adjacent rays): 2.04 ms, 2: 1.65, 3: 1.72, 4: 1.91; bit-identical.
 constexpr int kAdjPh = 2;
-static_assert(kAdjAngles <= 16, "lanes 4 s .. 4 s + 3 of a wavefront project angle s");
-constexpr int kT2Pad = kT2 + 2;   // padded rows and columns
-constexpr int kT2Pitch = kT2 + 3; // odd pitch in words
-constexpr int kT2Cells = 2 * kT2Pad * kT2Pitch;
+// Columns before and after the tile's that take what a ray adds next to it: rows are walked while
+// p is in [-2, kT2Cols), rounded outwards by kT2Margin rows, and a row has cells floor(p) to + 2.
+constexpr int kT2Side = 3;
+constexpr float kT2Margin = 0.01f;
+constexpr int kT2Pitch = kT2Cols + 2 * kT2Side + 1; // odd, in words
+constexpr int kT2Cells = kT2Rows * kT2Pitch;
 constexpr int kT2Own = (kT2Cells + kMaxBlock - 1) / kMaxBlock; // cells per thread
 constexpr int kAdjBits = 19;        // a term's bound: 2^kAdjBits units
-// candidates per 32-bit accumulation run: 2 kAdjBudget 2^kAdjBits <= 2^31 - 2^20
-constexpr int kAdjBudget = (1 << (31 - kAdjBits - 1)) - 1;
+// candidates per 32-bit accumulation run
+constexpr int kAdjBudget = (1 << (31 - kAdjBits)) - 2;
+static_assert((int64_t)kAdjBudget * ((1 << kAdjBits) + 2) < (1ll << 31), "32-bit sums are exact");
+
+// Tiles of one image: those of the y-dominant rays, then those of the x-dominant ones.
+__host__ __device__ inline unsigned adj2d_tiles(unsigned across, unsigned along) {
+    return ((across + kT2Rows - 1) / kT2Rows) * ((along + kT2Cols - 1) / kT2Cols);
+}
+
+__device__ __forceinline__ void lds_add(__attribute__((address_space(3))) unsigned *p, unsigned v) {
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 
 template <class SS>
 __global__ __launch_bounds__(kMaxBlock) void k_adj2d_tile(unsigned long long *__restrict__ accimg,
@@ -846,14 +872,11 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj2d_tile(unsigned long long *__
                                                          const float4 *__restrict__ ns,
                                                          const float *__restrict__ parts, int nx,
                                                          int ny, int D, int A, int G) {
-    // tile[0]: y-dominant rays, rows along y; tile[1]: x-dominant rays, rows along x. Padded
-    // by one row and column before and after, so every tap of a kept sample lands in the array.
     // 32-bit cells while the angles are added; 64-bit cells (the same memory) for the totals.
     __shared__ union {
-        unsigned int c32[2][kT2Pad * kT2Pitch];
-        unsigned long long c64[2][kT2Pad * kT2Pitch];
+        unsigned int c32[kT2Cells];
+        unsigned long long c64[kT2Cells];
     } sh;
-    auto &tile = sh.c32;
     const int tid = threadIdx.x;
     long long own[kT2Own]; // this thread's cells tid + k kMaxBlock, moved out of LDS
 #pragma unroll
@@ -865,41 +888,54 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj2d_tile(unsigned long long *__
         for (int k = 0; k < kT2Own; ++k) {
             const int i = tid + k * kMaxBlock;
             if (i < kT2Cells) {
-                own[k] += (int)(&tile[0][0])[i];
-                (&tile[0][0])[i] = 0u;
+                own[k] += (int)sh.c32[i];
+                sh.c32[i] = 0u;
             }
         }
         __syncthreads();
     };
     int run = 0; // candidates added since the last drain
     // XCD-aware order: workgroups are dealt to the 8 XCDs in turn, and logical index li gives
-    // each XCD a contiguous run of tiles of one angle group (x fastest), whose candidate rays
-    // share L2 (1.15 -> 1.08 ms at 1024^2; angle groups fastest: 1.17 ms)
-    int g, tx0, ty0;
+    // each XCD a contiguous run of tiles of one angle group, whose candidate rays share L2 (with
+    // square tiles 1.15 -> 1.08 ms at 1024^2; angle groups fastest: 1.17 ms)
+    bool ydom;
+    int g, d0, c0; // angle group; the tile's first texel along the dominant axis and along the other
     size_t b;
     {
-        const unsigned gx = gridDim.x, gy = gridDim.y, gz = gridDim.z;
-        const unsigned nwg = gx * gy * gz;
-        const unsigned hw = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+        const unsigned gx = gridDim.x, nwg = gx * gridDim.z;
+        const unsigned hw = blockIdx.x + gx * blockIdx.z;
         const unsigned n8 = nwg & ~7u;
         const unsigned li = hw < n8 ? (hw & 7u) * (n8 >> 3) + (hw >> 3) : hw;
-        const unsigned per = gx * gy * (unsigned)G;
+        const unsigned per = gx * (unsigned)G;
         b = li / per;
-        const unsigned l = li % per;
-        tx0 = (int)(l % gx) * kT2;
-        ty0 = (int)((l / gx) % gy) * kT2;
-        g = (int)(l / (gx * gy));
+        g = (int)(li % per / gx);
+        unsigned t = li % gx;
+        const unsigned ty = adj2d_tiles(ny, nx);
+        ydom = t < ty;
+        if (!ydom) t -= ty;
+        const unsigned wide = (unsigned)((ydom ? nx : ny) + kT2Cols - 1) / kT2Cols;
+        d0 = (int)(t / wide) * kT2Rows;
+        c0 = (int)(t % wide) * kT2Cols;
     }
     const int a0 = (int)((int64_t)g * A / G), a1 = (int)((int64_t)(g + 1) * A / G);
-    for (int i = tid; i < kT2Cells; i += kMaxBlock) (&tile[0][0])[i] = 0u;
-    __syncthreads(); // the tiles are clear before any wave adds to them
+    for (int i = tid; i < kT2Cells; i += kMaxBlock) sh.c32[i] = 0u;
+    __syncthreads(); // the tile is clear before any wave adds to it
     const float ymax = adj2d_ymax(parts + b * kAdjParts);
     const float yscale = ymax > 0.0f ? (float)(1 << kAdjBits) / ymax : 0.0f;
-    // the tile's first texel in the ray table's centred padded frame
-    const int px0 = tx0 + kPad - (nx + 2 * kPad) / 2, py0 = ty0 + kPad - (ny + 2 * kPad) / 2;
-    // footprint box corner this lane projects (lanes 0..3 of every wavefront)
-    const float qx = (tid & 1) ? (float)tx0 + (float)kT2 + 0.5f : (float)tx0 - 0.5f;
-    const float qy = (tid & 2) ? (float)ty0 + (float)kT2 + 0.5f : (float)ty0 - 0.5f;
+    // the tile's first row and column in the ray table's centred padded frame
+    const int fx = kPad - (nx + 2 * kPad) / 2, fy = kPad - (ny + 2 * kPad) / 2;
+    const int rowf = d0 + (ydom ? fy : fx), colf = c0 + (ydom ? fx : fy);
+    const float cmin = (float)(colf - 2), cmax = (float)(colf + kT2Cols);
+    // byte strides and the address of row 0, column 0 of that frame, as subnormals
+    const int lds0 = (int)(uintptr_t)(__attribute__((address_space(3))) unsigned *)sh.c32;
+    const float col = subnormal(4), pitch = subnormal(4 * kT2Pitch);
+    const float ofs = subnormal(lds0 + 4 * (kT2Side - colf));
+    // Footprint box corner this lane projects. The box ends with the image: a corner beyond it could
+    // lie behind the source.
+    const int c1 = min(c0 + kT2Cols, ydom ? nx : ny), d1 = min(d0 + kT2Rows, ydom ? ny : nx);
+    const float qc = (tid & 1) ? (float)c1 + 0.5f : (float)c0 - 0.5f;
+    const float qd = (tid & 2) ? (float)d1 + 0.5f : (float)d0 - 0.5f;
+    const float qx = ydom ? qc : qd, qy = ydom ? qd : qc;
     const typename SS::raw *sb = sino + b * (size_t)A * D;
     // kAdjAngles angles at a time: their candidate rays form one list, one ray per thread
     for (int ag = a0; ag < a1; ag += kAdjAngles) {
@@ -907,34 +943,49 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj2d_tile(unsigned long long *__
         // candidate range per angle: lanes 4 s .. 4 s + 3 of every wavefront project the four
         // corners of the footprint box for angle ag + s
         const int slot = (tid & 63) >> 2;
-        float kk = 0.0f;
+        float kmin = 0.0f, kmax = 0.0f, ox = 0.0f, oy = 0.0f, ux = 0.0f, uy = 0.0f;
         if (slot < na) {
             const float *gp = ageo + 6 * (ag + slot);
             const float wx = qx - gp[0], wy = qy - gp[1];
-            kk = -(wx * gp[3] - wy * gp[2]) / (wx * gp[5] - wy * gp[4]);
+            ox = gp[2], oy = gp[3], ux = gp[4], uy = gp[5];
+            const float depth = wx * uy - wy * ux;
+            kmin = kmax = -(wx * oy - wy * ox) / depth;
+            // a corner that is not in front of the source bounds nothing
+            if (!(depth * (ox * uy - oy * ux) > 0.0f)) kmin = -1e9f, kmax = 1e9f;
         }
-        float kmin = kk, kmax = kk;
         for (int off = 1; off < 4; off <<= 1) {
             kmin = fminf(kmin, __shfl_xor(kmin, off, 64));
             kmax = fmaxf(kmax, __shfl_xor(kmax, off, 64));
         }
-        int k0s[kAdjAngles], offs[kAdjAngles], cnts[kAdjAngles];
-        int total = 0;
-#pragma unroll
-        for (int q = 0; q < kAdjAngles; ++q) {
-            const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(kmin), 4 * q));
-            const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(kmax), 4 * q));
-            int cnt = 0, k0 = 0;
-            // an angle whose box misses the detector (or gives NaN) has no candidates
-            if (q < na && hi >= -1.0f && lo <= (float)D) {
-                k0 = max((int)floorf(lo - 0.01f), 0);
-                cnt = max(min((int)ceilf(hi + 0.01f), D - 1) - k0 + 1, 0);
-            }
-            k0s[q] = k0;
-            offs[q] = total;
-            cnts[q] = cnt;
-            total += kAdjPh * ((cnt + kAdjPh - 1) / kAdjPh);
+        // Both end rays clearly closer to the other axis, and to the same end of it: so are all
+        // rays between them.
+        bool other;
+        {
+            const float lo = fmaxf(kmin - 0.01f, 0.0f), hi = fminf(kmax + 0.01f, (float)(D - 1));
+            const float x0 = fmaf(lo - 1.0f, ux, ox), y0 = fmaf(lo - 1.0f, uy, oy);
+            const float x1 = fmaf(hi + 1.0f, ux, ox), y1 = fmaf(hi + 1.0f, uy, oy);
+            const float m0 = ydom ? x0 : y0, n0 = ydom ? y0 : x0;
+            const float m1 = ydom ? x1 : y1, n1 = ydom ? y1 : x1;
+            other = fabsf(m0) > 1.001f * fabsf(n0) && fabsf(m1) > 1.001f * fabsf(n1) &&
+                    (m0 > 0.0f) == (m1 > 0.0f);
         }
+        // By lane: the slot's angle's first candidate and their number (an angle whose box misses
+        // the detector has none), the padded numbers' sum up to the slot
+        int kfirst = 0, count = 0;
+        if (slot < na && !other && kmax >= -1.0f && kmin <= (float)D) {
+            kfirst = max((int)floorf(kmin - 0.01f), 0);
+            count = max(min((int)ceilf(kmax + 0.01f), D - 1) - kfirst + 1, 0);
+        }
+        int upto = kAdjPh * ((count + kAdjPh - 1) / kAdjPh);
+        const int padded = upto;
+#pragma unroll
+        for (int off = 4; off < 64; off <<= 1) {
+            const int v = __shfl_up(upto, off, 64);
+            upto += (tid & 63) >= off ? v : 0;
+        }
+        const int total = __builtin_amdgcn_readlane(upto, 63);
+        const int start = upto - padded;
+        int q0 = 0; // the last angle with start <= the wavefront's first ray
         // one candidate ray per thread, its parameters in registers; `total` and the pass
         // sizes are the same for the whole workgroup
         for (int base = 0; base < total; base += kMaxBlock) {
@@ -945,56 +996,88 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj2d_tile(unsigned long long *__
             }
             run += pass;
             const int ri = base + tid;
-            if (ri >= total) continue;
-            int q = 0;
+            const int wave0 = __builtin_amdgcn_readfirstlane(base + (tid & ~63));
+            if (wave0 >= total) continue;
+            while (q0 + 1 < kAdjAngles && __builtin_amdgcn_readlane(start, 4 * (q0 + 1)) <= wave0)
+                ++q0;
+            int q = q0, pp = ri - __builtin_amdgcn_readlane(start, 4 * q0);
+            int k0 = __builtin_amdgcn_readlane(kfirst, 4 * q0);
+            int cnt = __builtin_amdgcn_readlane(count, 4 * q0);
+            for (int u = q0 + 1; u < kAdjAngles; ++u) {
+                const int from = __builtin_amdgcn_readlane(start, 4 * u);
+                if (from >= wave0 + 64) break;
+                const int ku = __builtin_amdgcn_readlane(kfirst, 4 * u);
+                const int cu = __builtin_amdgcn_readlane(count, 4 * u);
+                if (ri >= from) q = u, pp = ri - from, k0 = ku, cnt = cu;
+            }
+            const int pm = (cnt + kAdjPh - 1) / kAdjPh;
+            int ph = 0;
 #pragma unroll
-            for (int u = 0; u < kAdjAngles; ++u)
-                if (ri >= offs[u]) q = u;
-            const int pm = (cnts[q] + kAdjPh - 1) / kAdjPh;
-            const int pp = ri - offs[q];
-            const int rl = (pp % pm) * kAdjPh + pp / pm;
-            if (pm == 0 || rl >= cnts[q]) continue;
-            const size_t r = (size_t)(ag + q) * D + k0s[q] + rl;
+            for (int u = 1; u < kAdjPh; ++u)
+                if (pp >= pm) ph = u, pp -= pm;
+            const int rl = pp * kAdjPh + ph;
+            if (rl >= cnt) continue;
+            const size_t r = (size_t)(ag + q) * D + k0 + rl;
             const float4 qn = ns[r];
-            const int n = __float_as_int(qn.y);
-            if (n <= 0) continue;
-            const float yv = to_f32<SS>(sb[r]) * qn.x * yscale; // |yv| <= 2^kAdjBits
-            if (yv == 0.0f) continue;
             const float4 e = ev[r];
-            const bool ydom = fabsf(e.w) == 1.0f;
+            const int n = __float_as_int(qn.y);
+            const float yv = to_f32<SS>(sb[r]) * qn.x * yscale; // |yv| <= 2^kAdjBits
+            if (n <= 0 || yv == 0.0f || (fabsf(e.w) == 1.0f) != ydom) continue;
             const float md = ydom ? e.y : e.x, sd = ydom ? e.w : e.z;
             const float mc = ydom ? e.x : e.y, vc = ydom ? e.z : e.w;
-            const int r0 = (int)floorf(md);
-            const float fb = md - (float)r0;
+            const float f0 = floorf(md), fb = md - f0;
             const float wl = yv * (1.0f - fb), wh = yv * fb; // rows pd, pd + 1
-            const int s = sd > 0.0f ? 1 : -1;
-            const int jlo = (int)qn.z, jhi = jlo + n - 1;
-            const int d0 = ydom ? py0 : px0, c0 = ydom ? px0 : py0;
-            // Step t is the sample whose dominant lower tap is pd = d0 - 1 + t (tile row t - 1):
-            // jf = s (pd - r0). Keep the steps with jf in [jlo, jhi] that reach the tile's rows.
-            const int ta = s > 0 ? jlo + r0 - d0 + 1 : r0 - jhi - d0 + 1;
-            const int t_lo = max(ta, 0), t_hi = min(ta + n - 1, kT2);
-            // Step t adds wl [1 - fa, fa] to tile row t - 1 and wh [1 - fa, fa] to row t at the
-            // columns lc, lc + 1: padded rows t, t + 1 and columns lc + 1, lc + 2, four
-            // immediate offsets from one address. Steps with lc outside [-1, kT2) miss the tile.
-            unsigned int *row = &tile[ydom ? 0 : 1][t_lo * kT2Pitch + 1];
-            float jf = (float)(s * (d0 - 1 + t_lo - r0));
-            const float fs = (float)s;
-            for (int t = t_lo; t <= t_hi; ++t) {
-                const float c = fmaf(jf, vc, mc);
-                jf += fs;
-                const int lc = floor_i32(c) - c0; // the lower tap's column in the tile
-                if ((unsigned)(lc + 1) <= (unsigned)kT2) {
-                    const float fa = __builtin_amdgcn_fractf(c);
-                    const float v1 = wl * fa, v0 = wl - v1, u1 = wh * fa, u0 = wh - u1;
-                    unsigned int *q = row + lc;
-                    atomicAdd(q, (unsigned int)round_i32(v0));
-                    atomicAdd(q + 1, (unsigned int)round_i32(v1));
-                    atomicAdd(q + kT2Pitch, (unsigned int)round_i32(u0));
-                    atomicAdd(q + kT2Pitch + 1, (unsigned int)round_i32(u1));
-                }
-                row += kT2Pitch;
+            const int r0 = (int)f0, jlo = (int)qn.z;
+            // the ray's samples are on the tile's rows (lower tap) first to first + n - 1; sample
+            // `row` has step s (row + rowf - r0) and column fma(that, vc, mc)
+            const float slope = sd > 0.0f ? vc : -vc; // of the column per row
+            const int first = (sd > 0.0f ? r0 + jlo : r0 - (jlo + n - 1)) - rowf;
+            const float m = fabsf(vc);
+            // p = fma(k, slope, mc) on row k - kd
+            const bool up = slope >= 0.0f;
+            const int kd = rowf - r0 - (up ? 1 : 0);
+            // rows with both terms whose cells reach the tile
+            const float inv = __builtin_amdgcn_rcpf(up ? fmaxf(m, 1e-6f) : fminf(-m, -1e-6f));
+            const float e0 = (cmin - mc) * inv, e1 = (cmax - mc) * inv;
+            const float klo = fminf(e0, e1) - kT2Margin, khi = fmaxf(e0, e1) + kT2Margin;
+            const int rlo = max(max(first + 1, 0), (int)ceilf(fmaxf(klo, -1e9f)) - kd);
+            const int rhi = min(min(first + n - 1, kT2Rows - 1), (int)floorf(fminf(khi, 1e9f)) - kd);
+            if (rlo <= rhi) {
+                const float wb = up ? wl : wh, wa = up ? wh : wl;
+                const int all = round_i32(yv);
+                const float m1 = m - 1.0f;
+                float k = (float)(rlo + kd);
+                float at0 = fmaf((float)rlo, pitch, ofs);
+                const float end = fmaf((float)rhi, pitch, ofs);
+                do {
+                    const float p = fmaf(k, slope, mc);
+                    const float fl = floorf(p), f = p - fl;
+                    const float g1 = __builtin_amdgcn_fmed3f(f + m, 0.0f, 1.0f);
+                    const float g2 = __builtin_amdgcn_fmed3f(f + m1, 0.0f, 1.0f);
+                    const int x2 = round_i32(wb * g2);
+                    const int b2 = round_i32(fmaf(wb, g1, wa * f));
+                    auto *const at = (__attribute__((address_space(3))) unsigned *)(uintptr_t)
+                        __float_as_uint(fmaf(fl, col, at0));
+                    lds_add(at, (unsigned)(all - b2));
+                    lds_add(at + 1, (unsigned)(b2 - x2));
+                    lds_add(at + 2, (unsigned)x2);
+                    k += 1.0f;
+                    at0 += pitch;
+                } while (at0 <= end);
             }
+            // rows with one term
+            auto one = [&](int row, int sample, float w) {
+                if ((unsigned)row >= (unsigned)kT2Rows) return;
+                const float c = fmaf((float)(sample + rowf - r0), slope, mc);
+                const float fl = floorf(c);
+                if (!(fl >= cmin && fl <= cmax)) return;
+                const int x1 = round_i32(w * (c - fl));
+                unsigned *const at = &sh.c32[row * kT2Pitch + kT2Side + ((int)fl - colf)];
+                atomicAdd(at, (unsigned)(round_i32(w) - x1));
+                atomicAdd(at + 1, (unsigned)x1);
+            };
+            one(first, first, wl);
+            one(first + n, first + n - 1, wh);
         }
     }
     drain();
@@ -1002,15 +1085,15 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj2d_tile(unsigned long long *__
 #pragma unroll
     for (int k = 0; k < kT2Own; ++k) {
         const int i = tid + k * kMaxBlock;
-        if (i < kT2Cells) (&sh.c64[0][0])[i] = (unsigned long long)(own[k] * (1ll << (30 - kAdjBits)));
+        if (i < kT2Cells) sh.c64[i] = (unsigned long long)(own[k] * (1ll << (30 - kAdjBits)));
     }
     __syncthreads();
     unsigned long long *out = accimg + b * (size_t)nx * ny;
-    for (int i = tid; i < kT2 * kT2; i += kMaxBlock) {
-        const int lx = i % kT2, ly = i / kT2;
-        const int X = tx0 + lx, Y = ty0 + ly;
-        const unsigned long long v =
-            sh.c64[0][(ly + 1) * kT2Pitch + lx + 1] + sh.c64[1][(lx + 1) * kT2Pitch + ly + 1];
+    for (int i = tid; i < kT2Rows * kT2Cols; i += kMaxBlock) {
+        // x fastest
+        const int lc = ydom ? i % kT2Cols : i / kT2Rows, ld = ydom ? i / kT2Cols : i % kT2Rows;
+        const int X = ydom ? c0 + lc : d0 + ld, Y = ydom ? d0 + ld : c0 + lc;
+        const unsigned long long v = sh.c64[ld * kT2Pitch + kT2Side + lc];
         if (X < nx && Y < ny && v != 0ull) atomicAdd(&out[(size_t)Y * nx + X], v);
     }
 }
@@ -1955,13 +2038,13 @@ CMI_API cmi_status cmi_adjoint_2d(const cmi_plan2d *plan, void *volume, int vol_
         hipLaunchKernelGGL((k_adj2d_absmax<SS>), dim3(kAdjParts, (unsigned)batch),
                            dim3(kMaxBlock), 0, s, (const typename SS::raw *)sinogram, plan->d_ns,
                            rays, parts);
-        // angle groups: enough workgroups to fill the GPU many times over (about 96 per CU; at
-        // 1024^2 a target of 8192 workgroups gave 1.09 ms, 16384: 1.06, 24576: 1.04, 32768: 1.05)
-        const unsigned tx = (unsigned)((nx + kT2 - 1) / kT2), ty = (unsigned)((ny + kT2 - 1) / kT2);
-        const uint64_t tiles = (uint64_t)tx * ty * batch;
+        // angle groups: enough workgroups to fill the GPU many times over (about 96 per CU; with
+        // tiles of 32 x 32 at 1024^2 a target of 8192 workgroups gave 1.09 ms, 16384: 1.06, 24576: 1.04, 32768: 1.05)
+        const unsigned tiles = adj2d_tiles(ny, nx) + adj2d_tiles(nx, ny);
+        const uint64_t all = (uint64_t)tiles * batch;
         const int G = (int)std::max<uint64_t>(
-            1, std::min<uint64_t>((uint64_t)A, (24576 + tiles - 1) / tiles));
-        hipLaunchKernelGGL((k_adj2d_tile<SS>), dim3(tx, ty, (unsigned)(G * batch)),
+            1, std::min<uint64_t>((uint64_t)A, (24576 + all - 1) / all));
+        hipLaunchKernelGGL((k_adj2d_tile<SS>), dim3(tiles, 1, (unsigned)(G * batch)),
                            dim3(kMaxBlock), 0, s, accimg, (const typename SS::raw *)sinogram,
                            plan->d_ageo, plan->d_ev, plan->d_ns, parts, nx, ny, D, A, G);
         const size_t one = (size_t)nx * ny;

@@ -181,3 +181,26 @@ def test_backward_3d_footprints(oracle, gpu, what, rec):
                      ("fdk", {"matched": True, "fdk": True})):
         got = cm.backward(x, geom, mode=mode)
         assert rel_l2(got, oracle.bp3d(geom, y, **kw)) <= RTOL_L2, (what, mode)
+
+
+@pytest.mark.parametrize("what,rec", [
+    ("one pixel", lambda: fan(1, 9, 5, 6.0, 9.0)),
+    ("one tile", lambda: fan(64, 99, 17, 128.0, 192.0, ny=32)),      # 64 x 32: one of each axis
+    ("one over", lambda: fan(65, 99, 16, 128.0, 192.0, ny=33)),      # lists of 16 angles: one whole
+    ("one less", lambda: fan(31, 99, 33, 128.0, 192.0, ny=63)),      # two and one angle
+    # rays along the axes and the diagonals, of slope 0 and 1
+    ("axes", lambda: fan(50, 80, 8, 100.0, 150.0, arc=2 * np.pi, ny=70)),
+    # fans of more than 90 degrees: rays of both axes and both directions in one angle and tile
+    ("wide fan", lambda: fan(40, 220, 11, 30.0, 60.0, du=1.5)),
+    ("coarse cells", lambda: fan(90, 13, 21, 150.0, 220.0, du=12.0)),
+    ("fine cells", lambda: fan(20, 700, 9, 50.0, 75.0, du=0.06)),     # many rays per texel
+    ("spacings", lambda: fan(48, 90, 13, 120.0, 170.0, spacing=(0.7, 1.3), offset=(2.5, -1.5))),
+])
+def test_adjoint_tiles(oracle, gpu, what, rec):
+    """Rows with two terms and with one, tiles of either dominant axis, lists of angles of which
+    some have no ray of the tile's axis."""
+    rec = rec()
+    geom = as_fan_geometry(rec)
+    y = np.random.RandomState(8).rand(rec.nangles, rec.det_shape) - 0.3
+    got = cm.adjoint(torch.tensor(y, dtype=torch.float32, device=gpu), geom)
+    assert rel_l2(got, oracle.adj2d(rec, y)) <= RTOL_L2, what
