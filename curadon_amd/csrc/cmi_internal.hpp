@@ -111,6 +111,11 @@ __device__ __forceinline__ int round_i32(float x) {
     return r;
 }
 
+// *p += v for an LDS cell whose address was computed as a number.
+__device__ __forceinline__ void lds_add(__attribute__((address_space(3))) unsigned *p, unsigned v) {
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // A workgroup barrier after this wavefront's LDS operations. __syncthreads() alone should wait for
 // them, but where it opens the body of a loop that the compiler has rotated (the barrier's block
 // is then the target of a back edge beside the loop's header), no wait was emitted for the LDS

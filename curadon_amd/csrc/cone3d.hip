@@ -597,11 +597,11 @@ __global__ __launch_bounds__(kMaxBlock) void k_absmax_parts(const typename S::ra
     }
 }
 
-// Matched adjoint, tile-driven: a workgroup owns a kAT^3 voxel tile with accumulators in LDS.
-// For each angle it projects the tile's box, grown by one voxel on each side (the samples
-// whose trilinear footprint reaches the tile), through the geometry-matched matrices onto the
-// panel; the rays through the covered pixels (plus one pixel of margin) are the candidates. Each
-// candidate walks only its samples inside the grown box, at the forward's FP32 positions, and
+// Matched adjoint, tile-driven: a workgroup owns a kAT^3 voxel tile with accumulators in LDS and a
+// group of angles. For each angle it projects the tile's box, grown by one voxel on each side (the
+// samples whose trilinear footprint reaches the tile), through the geometry-matched matrices onto
+// the panel; the rays through the covered pixels (plus one pixel of margin) are the candidates.
+// Each candidate walks only its samples inside the grown box, at the forward's FP32 positions, and
 // adds y * w to the tile voxels its footprint covers. The accumulators are fixed point in units
 // of max|y| / 2^19: a contribution y * w is rounded to that grid (|term| <= 2^19) and added to a
 // 32-bit LDS cell with an integer LDS atomic, which gfx950 executes about 45 times faster than an
@@ -616,27 +616,53 @@ __global__ __launch_bounds__(kMaxBlock) void k_absmax_parts(const typename S::ra
 // adds at most 2 (Du + 2)(Dv + 2) terms to a voxel (2 per candidate where that is smaller).
 // The workgroup keeps a running bound of these and, before it could pass 2^31 / 2^19, moves
 // the 32-bit sums of its 16^3 voxels into 64-bit sums and clears the tile. The 64-bit sums live
-// in a global array of which each workgroup owns one tile's worth (written by the first drain,
-// read and written only by the thread that owns the voxel), not in registers: sixteen 64-bit
-// registers per thread held the kernel at four wavefronts per SIMD, and without them it keeps
-// six (48.0 -> 43.3 ms at 256^3, bit-identical).
-// The tile is added to the volume once, in its storage type.
+// in a global array with one tile's worth per tile, not in registers: sixteen 64-bit registers per
+// thread held the kernel at four wavefronts per SIMD, and without them it keeps six (48.0 -> 43.3
+// ms at 256^3, bit-identical). A tile's only workgroup (gridDim.z == batch x tiles) writes them
+// first and adds the tile to the volume once, in its storage type; where several angle groups
+// share a tile, they add to them with integer atomics (cleared before) and k_adj3d_finish adds
+// the sums, which are the same, to the volume.
+//
+// Bound by LDS atomics (eight per sample, two clocks per wavefront and CU each and almost as many
+// in conflicts) and VALU issue (24 full, 12 half rate slots: LDS addresses by FMA on subnormals,
+// bp_tiles.hpp, and no test per sample, kAT3Margin). 97 x 120 x 133 voxels, 90 views of 150 x 171:
+// 2.16 ms with one workgroup per tile (504: 1.5 wavefronts per SIMD), 1.60 with the samples' loop
+// as it is now, 0.73 with angle groups (LDS busy 77 %, 47 % of that in conflicts).
 constexpr int kAT = 16;
 // candidate rays of one wavefront are kPh pixels apart in u and v (at 256^3, six wavefronts per
 // SIMD, tiles in XCD order: kPh 1: 47.1 ms, 2: 38.2; tiles in launch order: 2: 38.7, 3: 42.5,
 // 4: 43.7, 5: 45.5, 6: 46.1)
 constexpr int kPh = 2;
+// Samples are walked over the steps whose positions lie in the grown box, widened by this share
+// of a step for rounding: the lower corner of a sample lies in [-2, kAT + 1) on each axis.
+constexpr float kAT3Margin = 0.01f;
 // LDS tile: padded by one voxel before and after on each axis, so that every tap of a sample
 // whose lower corner lies in [-1, kAT) on each axis lands in the array (taps outside the tile
 // are added to the border and dropped): the eight taps are then immediate offsets from one LDS
-// address. Odd row and slice pitches (in words) spread voxels that differ only in y or z over
-// different banks, as the lanes of one atomic instruction hit voxels at various depths.
-constexpr int kATP = kAT + 2, kATRow = kATP + 1, kATSlice = kATP * kATRow + 1;
-constexpr int kATCells = kATP * kATSlice;
+// address. A corner one further out on x or y lands in the border of the row or slice beside,
+// one further on z in kATGuard cells before or after the slices. The odd slice pitch spreads
+// voxels that differ only in z over different banks.
+constexpr int kATP = kAT + 2, kATRow = kATP, kATSlice = kATP * kATRow + 1;
+constexpr int kATGuard = kATSlice + kATRow + 2;
+constexpr int kATCells = kATP * kATSlice + 2 * kATGuard;
 constexpr int kATOwn = kAT * kAT * kAT / kMaxBlock; // tile voxels per thread
 static_assert(kAT * kAT * kAT % kMaxBlock == 0, "whole voxels per thread");
 constexpr int kAdj3Bits = 19;                             // a term's bound: 2^kAdj3Bits units
 constexpr int kAdj3Budget = (1 << (31 - kAdj3Bits)) - 16; // terms per voxel between drains
+// Workgroups of k_adj3d that angle groups are made for: tiles differ in their rays (those near the
+// source have many), so that many more than the 1536 which the GPU holds at once pay. Workgroups
+// at most, 97 x 120 x 133 x 90 views / 160^3 x 180 / 192^3 x 180 / 256^3 x 360: none 1.60 / 5.34 /
+// 8.54 / 33.2 ms, 3072: 0.82 / - / 8.18 / 33.2, 6144: 0.78 / 4.79 / 7.67 / 32.3, 12288: 0.73 / 4.16
+// / 7.00 / 34.9, 24576: 0.73 / 3.92 / 6.74 / 32.6.
+constexpr uint64_t kAdj3Workgroups = 24576;
+
+// vol[o] += a voxel's sum of fixed-point terms.
+template <class SV>
+__device__ __forceinline__ void adj3d_add(typename SV::raw *__restrict__ vol, size_t o,
+                                          long long total, float ymax) {
+    const float add = (float)((double)total * ((double)ymax * 0x1p-19));
+    vol[o] = from_f32<SV>(to_f32<SV>(vol[o]) + add);
+}
 
 template <class SV, class SS>
 __global__ __launch_bounds__(kMaxBlock) void k_adj3d(typename SV::raw *__restrict__ vol,
@@ -645,40 +671,17 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj3d(typename SV::raw *__restric
                                                      const float4 *__restrict__ rs,
                                                      const float *__restrict__ M,
                                                      const float *__restrict__ parts, int nx,
-                                                     int ny, int nz, int U, int V, int A,
+                                                     int ny, int nz, int U, int V, int A, int G,
                                                      long long *__restrict__ totals) {
-    __shared__ unsigned int tile[kATCells];
+    __shared__ unsigned int cells[kATCells];
+    unsigned int *const tile = cells + kATGuard;
     const int tid = threadIdx.x;
-    // this workgroup's 64-bit voxel sums so far, in global memory it alone uses; none before
-    // the first drain
-    long long *own = totals + ((size_t)blockIdx.x +
-                               gridDim.x * ((size_t)blockIdx.y + gridDim.y * (size_t)blockIdx.z)) *
-                                  (kAT * kAT * kAT);
-    bool first = true;
-    auto cell_of = [](int j) {
-        return (j / (kAT * kAT) + 1) * kATSlice + ((j / kAT) % kAT + 1) * kATRow + j % kAT + 1;
-    };
-    // the tile's voxel sums -> the workgroup's 64-bit sums, then the tile (border included)
-    // cleared
-    auto drain = [&]() {
-        lds_barrier();
-#pragma unroll 4
-        for (int k = 0; k < kATOwn; ++k) {
-            const int i = tid + k * kMaxBlock;
-            const long long v = (int)tile[cell_of(i)];
-            own[i] = first ? v : own[i] + v;
-        }
-        first = false;
-        __syncthreads();
-        for (int i = tid; i < kATCells; i += kMaxBlock) tile[i] = 0u;
-        __syncthreads();
-    };
-    int bound = 0; // terms a voxel may have received since the last drain
     const int ntz = (nz + kAT - 1) / kAT;
     // XCD-aware order: workgroups are dealt to the 8 XCDs in turn, and logical index li gives
-    // each XCD a contiguous run of tiles (x fastest), whose candidate rays share L2
-    int x0, y0, z0;
-    size_t b;
+    // each XCD a contiguous run of tiles (x fastest) of an angle group, whose candidate rays
+    // share L2
+    int x0, y0, z0, g;
+    size_t b, slot; // volume; the tile's place among all
     {
         const unsigned gx = gridDim.x, gy = gridDim.y, gz = gridDim.z;
         const unsigned nwg = gx * gy * gz;
@@ -686,83 +689,112 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj3d(typename SV::raw *__restric
         const unsigned n8 = nwg & ~7u;
         const unsigned li = hw < n8 ? (hw & 7u) * (n8 >> 3) + (hw >> 3) : hw;
         const unsigned per = gx * gy * (unsigned)ntz;
-        b = li / per;
+        g = (int)(li / per % (unsigned)G);
+        b = li / per / (unsigned)G;
         const unsigned l = li % per;
+        slot = b * per + l;
         x0 = (int)(l % gx) * kAT;
         y0 = (int)((l / gx) % gy) * kAT;
         z0 = (int)(l / (gx * gy)) * kAT;
     }
-    // fixed-point scale: max|y| of this volume's projections maps to 2^30
+    const int a0 = (int)((int64_t)g * A / G), a1 = (int)((int64_t)(g + 1) * A / G);
+    // the tile's 64-bit voxel sums; G == 1: in global memory that this workgroup alone uses, none
+    // before the first drain
+    long long *own = totals + slot * (kAT * kAT * kAT);
+    bool first = true;
+    auto cell_of = [](int j) {
+        return (j / (kAT * kAT) + 1) * kATSlice + ((j / kAT) % kAT + 1) * kATRow + j % kAT + 1;
+    };
+    auto share = [&](int i, long long v) {
+        if (v != 0) atomicAdd((unsigned long long *)&own[i], (unsigned long long)v);
+    };
+    // the tile's voxel sums -> the 64-bit sums, then the tile (border included) cleared
+    auto drain = [&]() {
+        lds_barrier();
+#pragma unroll 4
+        for (int k = 0; k < kATOwn; ++k) {
+            const int i = tid + k * kMaxBlock;
+            const long long v = (int)tile[cell_of(i)];
+            if (G > 1) share(i, v);
+            else own[i] = first ? v : own[i] + v;
+        }
+        first = false;
+        __syncthreads();
+        for (int i = tid; i < kATCells; i += kMaxBlock) cells[i] = 0u;
+        __syncthreads();
+    };
+    int bound = 0; // terms a voxel may have received since the last drain
+    // fixed-point scale: max|y| of this volume's projections maps to 2^19
     float ymax = 0.0f;
     for (int i = tid & 63; i < kMaxParts; i += 64) ymax = fmaxf(ymax, parts[b * kMaxParts + i]);
     for (int off = 32; off > 0; off >>= 1) ymax = fmaxf(ymax, __shfl_xor(ymax, off, 64));
     const float yscale = ymax > 0.0f ? (float)(1 << kAdj3Bits) / ymax : 0.0f;
-    for (int i = tid; i < kATCells; i += kMaxBlock) tile[i] = 0u;
+    for (int i = tid; i < kATCells; i += kMaxBlock) cells[i] = 0u;
     const int Wp = nx + 2 * kPad, Hp = ny + 2 * kPad, Dp = nz + 2 * kPad;
     // centred padded coordinate p -> voxel index floor(p) + c
     const int cx = Wp / 2 - kPad, cy = Hp / 2 - kPad, cz = Dp / 2 - kPad;
-    // centred padded coordinate p -> padded tile index floor(p) + o
-    const int ox = cx - x0 + 1, oy = cy - y0 + 1, oz = cz - z0 + 1;
+    // byte strides and the address of floor(p) = (0, 0, 0), as subnormals
+    const float fcol = subnormal(4), frow = subnormal(4 * kATRow), fslice = subnormal(4 * kATSlice);
+    const float fofs = subnormal((int)(uintptr_t)(__attribute__((address_space(3))) unsigned *)tile +
+                                 4 * ((cx - x0 + 1) + (cy - y0 + 1) * kATRow +
+                                      (cz - z0 + 1) * kATSlice));
     // samples reaching the tile: floor(p) + c in [t0 - 1, t0 + kAT - 1] on each axis
     const float lox = (float)(x0 - 1 - cx), loy = (float)(y0 - 1 - cy), loz = (float)(z0 - 1 - cz);
     const float hix = lox + (float)(kAT + 1), hiy = loy + (float)(kAT + 1),
                 hiz = loz + (float)(kAT + 1);
     // the grown box's corner this lane projects (centred voxel index of the matrices)
-    const int c8 = tid & 7;
+    const int c8 = tid & 7, k8 = (tid & 63) >> 3;
     const float qx = (float)((c8 & 1) ? x0 + kAT : x0 - 1) - (float)((nx - 1) / 2.0);
     const float qy = (float)((c8 & 2) ? y0 + kAT : y0 - 1) - (float)((ny - 1) / 2.0);
     const float qz = (float)((c8 & 4) ? z0 + kAT : z0 - 1) - (float)((nz - 1) / 2.0);
     const typename SS::raw *sb = sino + b * (size_t)A * V * U;
+    // By lane, for the angle of its eight lanes: the candidates' first column and row, their
+    // numbers, and the most terms that the angle adds to a voxel
+    int cu0 = 0, cv0 = 0, cnu = 0, cnv = 0, cterms = 0;
     __syncthreads();
-    for (int a = 0; a < A; ++a) {
-        const float *m = M + 12 * a; // wave-uniform: scalar loads
-        const float Uh = fmaf(m[0], qx, fmaf(m[1], qy, fmaf(m[2], qz, m[3])));
-        const float Vh = fmaf(m[4], qx, fmaf(m[5], qy, fmaf(m[6], qz, m[7])));
-        const float Wh = fmaf(m[8], qx, fmaf(m[9], qy, fmaf(m[10], qz, m[11])));
-        const float rw = __builtin_amdgcn_rcpf(Wh);
-        float umin = Uh * rw, umax = umin, vmin = Vh * rw, vmax = vmin;
-        float uabs = fabsf(umin), vabs = fabsf(vmin), wmin = Wh;
-        int ok = Wh > 0.0f ? 1 : 0;
+    for (int a = a0; a < a1; ++a) {
+        const int sel = 8 * ((a - a0) & 7);
+        if (sel == 0) {
+            const float *m = M + 12 * min(a + k8, A - 1);
+            const float Uh = fmaf(m[0], qx, fmaf(m[1], qy, fmaf(m[2], qz, m[3])));
+            const float Vh = fmaf(m[4], qx, fmaf(m[5], qy, fmaf(m[6], qz, m[7])));
+            const float Wh = fmaf(m[8], qx, fmaf(m[9], qy, fmaf(m[10], qz, m[11])));
+            const float rw = __builtin_amdgcn_rcpf(Wh);
+            float u0 = Uh * rw, u1 = u0, v0 = Vh * rw, v1 = v0, wm = Wh;
+            int ok = Wh > 0.0f ? 1 : 0;
 #pragma unroll
-        for (int off = 1; off < 8; off <<= 1) {
-            umin = fminf(umin, __shfl_xor(umin, off, 64));
-            umax = fmaxf(umax, __shfl_xor(umax, off, 64));
-            vmin = fminf(vmin, __shfl_xor(vmin, off, 64));
-            vmax = fmaxf(vmax, __shfl_xor(vmax, off, 64));
-            ok = min(ok, __shfl_xor(ok, off, 64));
-            uabs = fmaxf(uabs, __shfl_xor(uabs, off, 64));
-            vabs = fmaxf(vabs, __shfl_xor(vabs, off, 64));
-            wmin = fminf(wmin, __shfl_xor(wmin, off, 64));
+            for (int off = 1; off < 8; off <<= 1) {
+                u0 = fminf(u0, __shfl_xor(u0, off, 64));
+                u1 = fmaxf(u1, __shfl_xor(u1, off, 64));
+                v0 = fminf(v0, __shfl_xor(v0, off, 64));
+                v1 = fmaxf(v1, __shfl_xor(v1, off, 64));
+                ok = min(ok, __shfl_xor(ok, off, 64));
+                wm = fminf(wm, __shfl_xor(wm, off, 64));
+            }
+            // no bound where a corner is not in front of the source: all rays, and 2^30 terms
+            cu0 = cv0 = 0, cnu = U, cnv = V, cterms = 1 << 30;
+            if (ok) {
+                const float ua = fmaxf(fabsf(u0), fabsf(u1)), va = fmaxf(fabsf(v0), fabsf(v1));
+                const float su = fabsf(m[0]) + fabsf(m[1]) + fabsf(m[2]);
+                const float sv = fabsf(m[4]) + fabsf(m[5]) + fabsf(m[6]);
+                const float sw = fabsf(m[8]) + fabsf(m[9]) + fabsf(m[10]);
+                // 1 % margin for the approximate reciprocals; the +2 covers the pixel count of an
+                // interval (floor + 1) and rays that FP32 positions put one pixel further
+                const float du = 2.02f * (su + ua * sw) / wm, dv = 2.02f * (sv + va * sw) / wm;
+                if (du < 1024.0f && dv < 1024.0f) cterms = 2 * ((int)du + 2) * ((int)dv + 2);
+                if (u1 < -2.0f || u0 > (float)(U + 1) || v1 < -2.0f || v0 > (float)(V + 1)) {
+                    cnu = 0;
+                } else {
+                    cu0 = max(0, (int)ceilf(u0) - 1);
+                    cnu = min(U - 1, (int)floorf(u1) + 1) - cu0 + 1;
+                    cv0 = max(0, (int)ceilf(v0) - 1);
+                    cnv = min(V - 1, (int)floorf(v1) + 1) - cv0 + 1;
+                }
+            }
         }
-        // every lane group holds the same values; take lane 0's
-        int iu0 = 0, iu1 = U - 1, iv0 = 0, iv1 = V - 1;
-        // this angle's terms per voxel, at most (no bound where a corner is not in front of
-        // the source); 2^30 stands for unbounded
-        int per_angle = 1 << 30;
-        if (__builtin_amdgcn_readfirstlane(ok)) {
-            const float ua = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(uabs)));
-            const float va = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(vabs)));
-            const float wm = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(wmin)));
-            const float su = fabsf(m[0]) + fabsf(m[1]) + fabsf(m[2]);
-            const float sv = fabsf(m[4]) + fabsf(m[5]) + fabsf(m[6]);
-            const float sw = fabsf(m[8]) + fabsf(m[9]) + fabsf(m[10]);
-            // 1 % margin for the approximate reciprocals; the +2 covers the pixel count of an
-            // interval (floor + 1) and rays that FP32 positions put one pixel further
-            const float du = 2.02f * (su + ua * sw) / wm, dv = 2.02f * (sv + va * sw) / wm;
-            if (du < 1024.0f && dv < 1024.0f)
-                per_angle = 2 * ((int)du + 2) * ((int)dv + 2);
-            const float u0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(umin)));
-            const float u1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(umax)));
-            const float v0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(vmin)));
-            const float v1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(vmax)));
-            if (u1 < -2.0f || u0 > (float)(U + 1) || v1 < -2.0f || v0 > (float)(V + 1)) continue;
-            iu0 = max(0, (int)ceilf(u0) - 1);
-            iu1 = min(U - 1, (int)floorf(u1) + 1);
-            iv0 = max(0, (int)ceilf(v0) - 1);
-            iv1 = min(V - 1, (int)floorf(v1) + 1);
-        }
-        const int niu = iu1 - iu0 + 1, niv = iv1 - iv0 + 1;
+        const int niu = __builtin_amdgcn_readlane(cnu, sel), niv = __builtin_amdgcn_readlane(cnv, sel);
         if (niu <= 0 || niv <= 0) continue;
+        const int iu0 = __builtin_amdgcn_readlane(cu0, sel), iv0 = __builtin_amdgcn_readlane(cv0, sel);
         // Candidates in phase order: phase (pu, pv) in [0, kPh)^2 holds the rays
         // (pu + kPh qu, pv + kPh qv), so the consecutive candidates of a wavefront are kPh
         // pixels apart in u and v and their samples' taps rarely meet in one atomic instruction
@@ -770,9 +802,10 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj3d(typename SV::raw *__restric
         // size leaves holes past the rectangle's edge, which are skipped.
         const int nqu = (niu + kPh - 1) / kPh, nqv = (niv + kPh - 1) / kPh;
         const int nq = nqu * nqv, nc = kPh * kPh * nq;
+        const float rnqu = __builtin_amdgcn_rcpf((float)nqu);
         // passes of kMaxBlock candidates, the same for the whole workgroup; a pass adds at most
-        // two terms per candidate to a voxel, and the angle at most per_angle in all
-        int allowance = per_angle;
+        // two terms per candidate to a voxel, and the angle at most cterms in all
+        int allowance = __builtin_amdgcn_readlane(cterms, sel);
         for (int cb = 0; cb < nc; cb += kMaxBlock) {
             const int inc = min(2 * min(kMaxBlock, nc - cb), allowance);
             allowance -= inc;
@@ -783,20 +816,26 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj3d(typename SV::raw *__restric
             bound += inc;
             const int c = cb + tid;
             if (c >= nc) continue;
-            const int ph = c / nq, rq = c - ph * nq;
-            const int qv = rq / nqu, qu = rq - qv * nqu;
+            int ph = 0, rq = c;
+#pragma unroll
+            for (int u = 1; u < kPh * kPh; ++u)
+                if (rq >= nq) ph = u, rq -= nq;
+            // rq / nqu, off by one at most before the correction
+            int qv = (int)((float)rq * rnqu), qu = rq - qv * nqu;
+            if (qu < 0) --qv, qu += nqu;
+            if (qu >= nqu) ++qv, qu -= nqu;
             const int lu = (ph % kPh) + kPh * qu, lv = (ph / kPh) + kPh * qv;
             if (lu >= niu || lv >= niv) continue;
             const int iu = iu0 + lu, iv = iv0 + lv;
             const size_t r = ((size_t)a * V + iv) * U + iu;
             const float4 s4 = rs[r];
-            const int n = __float_as_int(s4.w);
-            if (n <= 0) continue;
-            const float y = to_f32<SS>(sb[r]) * yscale; // |y| <= 2^30
-            if (y == 0.0f) continue;
             const float4 m4 = rm[r];
-            // jf range with p in [lo, hi) on every axis, one sample of margin each side
-            float jlo = m4.w, jhi = m4.w + (float)(n - 1);
+            const float y = to_f32<SS>(sb[r]) * yscale; // |y| <= 2^19
+            const int n = __float_as_int(s4.w);
+            if (n <= 0 || y == 0.0f) continue;
+            // jf range with p in [lo, hi) on every axis
+            const float jlast = m4.w + (float)(n - 1);
+            float jlo = m4.w, jhi = jlast;
             const float st[3] = {s4.x, s4.y, s4.z}, mm[3] = {m4.x, m4.y, m4.z};
             const float lo[3] = {lox, loy, loz}, hi[3] = {hix, hiy, hiz};
             bool empty = false;
@@ -805,52 +844,83 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj3d(typename SV::raw *__restric
                 if (st[d] != 0.0f) {
                     const float r0 = __builtin_amdgcn_rcpf(st[d]);
                     const float t1 = (lo[d] - mm[d]) * r0, t2 = (hi[d] - mm[d]) * r0;
-                    jlo = fmaxf(jlo, fminf(t1, t2) - 1.0f);
-                    jhi = fminf(jhi, fmaxf(t1, t2) + 1.0f);
+                    jlo = fmaxf(jlo, fminf(t1, t2) - kAT3Margin);
+                    jhi = fminf(jhi, fmaxf(t1, t2) + kAT3Margin);
                 } else if (mm[d] < lo[d] || mm[d] >= hi[d]) {
                     empty = true;
                 }
             }
             if (empty) continue;
-            const float jend = fminf(floorf(jhi), m4.w + (float)(n - 1));
-            for (float jf = fmaxf(ceilf(jlo), m4.w); jf <= jend; jf += 1.0f) {
+            const float jend = floorf(jhi);
+            for (float jf = ceilf(jlo); jf <= jend; jf += 1.0f) {
                 // the forward's own positions (k_fwd3d)
                 const float px = fmaf(jf, s4.x, m4.x), py = fmaf(jf, s4.y, m4.y),
                             pz = fmaf(jf, s4.z, m4.z);
-                // padded tile indices of the lower corner, kept if in [0, kAT] on each axis
-                const int lx = floor_i32(px) + ox, ly = floor_i32(py) + oy,
-                          lz = floor_i32(pz) + oz;
-                if ((unsigned)lx > (unsigned)kAT || (unsigned)ly > (unsigned)kAT ||
-                    (unsigned)lz > (unsigned)kAT)
-                    continue;
-                const float fx = __builtin_amdgcn_fractf(px), fy = __builtin_amdgcn_fractf(py),
-                            fz = __builtin_amdgcn_fractf(pz);
+                const float ix = floorf(px), iy = floorf(py), iz = floorf(pz);
+                const float fx = px - ix, fy = py - iy, fz = pz - iz;
                 // the eight trilinear weights times y, as differences of products
                 const float x1 = y * fx, x0w = y - x1;
                 const float y01 = x0w * fy, y00 = x0w - y01, y11 = x1 * fy, y10 = x1 - y11;
-                const float w[8] = {y00 - y00 * fz, y10 - y10 * fz, y01 - y01 * fz,
-                                    y11 - y11 * fz, y00 * fz, y10 * fz, y01 * fz, y11 * fz};
-                unsigned int *t = &tile[__mul24(lz, kATSlice) + __mul24(ly, kATRow) + lx];
+                const float z00 = y00 * fz, z10 = y10 * fz, z01 = y01 * fz, z11 = y11 * fz;
+                const float w[8] = {y00 - z00, y10 - z10, y01 - z01, y11 - z11,
+                                    z00,       z10,       z01,       z11};
+                auto *const t = (__attribute__((address_space(3))) unsigned *)(uintptr_t)
+                    __float_as_uint(fmaf(iz, fslice, fmaf(iy, frow, fmaf(ix, fcol, fofs))));
 #pragma unroll
                 for (int k = 0; k < 8; ++k)
-                    atomicAdd(t + (k >> 2) * kATSlice + ((k >> 1) & 1) * kATRow + (k & 1),
-                              (unsigned int)round_i32(w[k]));
+                    lds_add(t + (k >> 2) * kATSlice + ((k >> 1) & 1) * kATRow + (k & 1),
+                            (unsigned int)round_i32(w[k]));
             }
         }
     }
     lds_barrier();
+    if (G > 1) {
+#pragma unroll 4
+        for (int k = 0; k < kATOwn; ++k) {
+            const int i = tid + k * kMaxBlock;
+            share(i, (int)tile[cell_of(i)]);
+        }
+        return;
+    }
 #pragma unroll 4
     for (int k = 0; k < kATOwn; ++k) {
         const int i = tid + k * kMaxBlock;
         const long long total = (first ? 0ll : own[i]) + (int)tile[cell_of(i)];
         const int lx = i % kAT, ly = (i / kAT) % kAT, lz = i / (kAT * kAT);
         const int X = x0 + lx, Y = y0 + ly, Z = z0 + lz;
-        if (X < nx && Y < ny && Z < nz) {
-            const size_t o = ((b * nz + Z) * ny + Y) * (size_t)nx + X;
-            const float add = (float)((double)total * ((double)ymax * 0x1p-19));
-            vol[o] = from_f32<SV>(to_f32<SV>(vol[o]) + add);
-        }
+        if (X < nx && Y < ny && Z < nz)
+            adj3d_add<SV>(vol, ((b * nz + Z) * ny + Y) * (size_t)nx + X, total, ymax);
     }
+}
+
+// vol += the tiles' sums (k_adj3d with several angle groups). A workgroup per tile, as dealt there.
+template <class SV>
+__global__ __launch_bounds__(kMaxBlock) void k_adj3d_finish(typename SV::raw *__restrict__ vol,
+                                                            const float *__restrict__ parts,
+                                                            int nx, int ny, int nz,
+                                                            const long long *__restrict__ totals) {
+    const int ntz = (nz + kAT - 1) / kAT;
+    const int x0 = (int)blockIdx.x * kAT, y0 = (int)blockIdx.y * kAT,
+              z0 = (int)(blockIdx.z % ntz) * kAT;
+    const size_t b = blockIdx.z / ntz;
+    const size_t slot = blockIdx.x + gridDim.x * ((size_t)blockIdx.y +
+                                                  gridDim.y * (size_t)blockIdx.z);
+    float ymax = 0.0f;
+    for (int i = threadIdx.x & 63; i < kMaxParts; i += 64)
+        ymax = fmaxf(ymax, parts[b * kMaxParts + i]);
+    for (int off = 32; off > 0; off >>= 1) ymax = fmaxf(ymax, __shfl_xor(ymax, off, 64));
+#pragma unroll 4
+    for (int k = 0; k < kATOwn; ++k) {
+        const int i = threadIdx.x + k * kMaxBlock;
+        const int X = x0 + i % kAT, Y = y0 + (i / kAT) % kAT, Z = z0 + i / (kAT * kAT);
+        if (X < nx && Y < ny && Z < nz)
+            adj3d_add<SV>(vol, ((b * nz + Z) * ny + Y) * (size_t)nx + X,
+                          totals[slot * (kAT * kAT * kAT) + i], ymax);
+    }
+}
+
+__global__ __launch_bounds__(kMaxBlock) void k_clear_sums(long long *__restrict__ p) {
+    p[(size_t)blockIdx.x * kMaxBlock + threadIdx.x] = 0;
 }
 
 // ---------------------------------------------------------------- backprojection ----------
@@ -1783,7 +1853,7 @@ CMI_API cmi_status cmi_adjoint_3d(const cmi_plan3d *plan, void *volume, int vol_
               A = (int)plan->A;
     const size_t rays = (size_t)A * U * V;
     // scratch: the march table [2][rays], [batch][kMaxParts] partial maxima of |y|, then (256-byte
-    // aligned) the tiles' 64-bit sums, one tile of kAT^3 per workgroup
+    // aligned) the tiles' 64-bit sums
     const size_t ntiles = (size_t)((nx + kAT - 1) / kAT) * ((ny + kAT - 1) / kAT) *
                           ((nz + kAT - 1) / kAT) * batch;
     float4 *table = nullptr;
@@ -1803,12 +1873,22 @@ CMI_API cmi_status cmi_adjoint_3d(const cmi_plan3d *plan, void *volume, int vol_
         hipLaunchKernelGGL((k_absmax_parts<SS>), dim3(kMaxParts, (unsigned)batch),
                            dim3(kMaxBlock), 0, s, (const typename SS::raw *)sinogram, rays, parts);
         const int ntz = (nz + kAT - 1) / kAT;
-        dim3 ab(kMaxBlock), ag((unsigned)((nx + kAT - 1) / kAT), (unsigned)((ny + kAT - 1) / kAT),
-                               (unsigned)(ntz * batch));
-        hipLaunchKernelGGL((k_adj3d<SV, SS>), ag, ab, 0, s, (typename SV::raw *)volume,
+        const dim3 tiles((unsigned)((nx + kAT - 1) / kAT), (unsigned)((ny + kAT - 1) / kAT),
+                         (unsigned)(ntz * batch));
+        const int G = (int)std::max<uint64_t>(
+            1, std::min<uint64_t>({(uint64_t)A, (kAdj3Workgroups + ntiles - 1) / ntiles,
+                                   65535 / (uint64_t)tiles.z}));
+        if (G > 1)
+            hipLaunchKernelGGL(k_clear_sums, dim3((unsigned)(ntiles * kATOwn)), dim3(kMaxBlock), 0,
+                               s, totals);
+        hipLaunchKernelGGL((k_adj3d<SV, SS>), dim3(tiles.x, tiles.y, tiles.z * G),
+                           dim3(kMaxBlock), 0, s, (typename SV::raw *)volume,
                            (const typename SS::raw *)sinogram, (const float4 *)table,
                            (const float4 *)(table + rays), plan->d_mmat, parts, nx, ny, nz,
-                           U, V, A, totals);
+                           U, V, A, G, totals);
+        if (G > 1)
+            hipLaunchKernelGGL((k_adj3d_finish<SV>), tiles, dim3(kMaxBlock), 0, s,
+                               (typename SV::raw *)volume, parts, nx, ny, nz, totals);
         CMI_HIP_TRY(hipGetLastError());
         return CMI_OK;
     });

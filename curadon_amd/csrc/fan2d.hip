@@ -860,10 +860,6 @@ __host__ __device__ inline unsigned adj2d_tiles(unsigned across, unsigned along)
     return ((across + kT2Rows - 1) / kT2Rows) * ((along + kT2Cols - 1) / kT2Cols);
 }
 
-__device__ __forceinline__ void lds_add(__attribute__((address_space(3))) unsigned *p, unsigned v) {
-    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 template <class SS>
 __global__ __launch_bounds__(kMaxBlock) void k_adj2d_tile(unsigned long long *__restrict__ accimg,
                                                          const typename SS::raw *__restrict__ sino,

@@ -204,3 +204,33 @@ def test_adjoint_tiles(oracle, gpu, what, rec):
     y = np.random.RandomState(8).rand(rec.nangles, rec.det_shape) - 0.3
     got = cm.adjoint(torch.tensor(y, dtype=torch.float32, device=gpu), geom)
     assert rel_l2(got, oracle.adj2d(rec, y)) <= RTOL_L2, what
+
+
+@pytest.mark.parametrize("what,rec", [
+    ("ragged tiles", lambda: cone(17, 30, 28, 5, 60.0, 90.0, nz=33, ny=15)),
+    ("one voxel", lambda: cone(1, 5, 5, 3, 6.0, 9.0)),
+    ("thin y", lambda: cone(40, 50, 9, 18, 90.0, 130.0, nz=16, ny=1)),    # groups of one angle
+    # hundreds of rays through a voxel: the 32-bit sums are moved within an angle
+    ("fine panel", lambda: cone(5, 230, 220, 3, 15.0, 22.0, du=(0.06, 0.06))),
+    ("tilted", lambda: cone(20, 30, 28, 5, 60.0, 90.0, nz=18, ny=35, angles=TILTED)),
+    # corners of a tile's box behind the source: all rays are candidates
+    ("near source", lambda: cone(17, 40, 40, 12, 20.0, 44.0)),
+])
+def test_adjoint_3d_tiles(oracle, gpu, what, rec):
+    rec = rec()
+    geom = as_cone_geometry(rec)
+    y = np.random.RandomState(9).rand(rec.nangles, *rec.det_shape) - 0.3
+    got = cm.adjoint(torch.tensor(y, dtype=torch.float32, device=gpu), geom)
+    assert rel_l2(got, oracle.adj3d(rec, y)) <= RTOL_L2, what
+
+
+def test_adjoint_3d_angle_groups(gpu):
+    """A tile's only workgroup (a batch of many tiles) and angle groups that share a tile (one
+    volume) give the same bits."""
+    geom = as_cone_geometry(cone(256, 60, 9, 7, 520.0, 780.0, du=(8.0, 2.0), nz=2, ny=16))
+    y = rand((2, 7, 9, 60), gpu, 12) - 0.3
+    batch = 1600                                   # x 16 tiles
+    many = cm.adjoint(y.repeat(batch // 2, 1, 1, 1), geom)
+    for i in range(2):
+        one = cm.adjoint(y[i].contiguous(), geom)
+        assert torch.equal(many[i], one) and torch.equal(many[batch - 2 + i], one)
