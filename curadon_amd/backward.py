@@ -22,18 +22,20 @@ def backward(sinogram, volume=None, geom=None, *, volume_out=None, mode="referen
     if isinstance(geom, FanGeometry):
         if mode not in ("reference", "fbp"):
             raise ValueError(f"fan-beam backward: unknown mode {mode!r}")
+        plan = geom.plan  # once per call: every access compares all attributes
         if volume is None:
             volume = torch.zeros(tuple(sinogram.shape[:-2]) + tuple(int(v) for v in geom.vol_shape),
-                                 dtype=_C.dtype_of_code(geom.plan.vol_prec),
+                                 dtype=_C.dtype_of_code(plan.vol_prec),
                                  device=sinogram.device)
-        _C.backward_2d(volume, sinogram, geom.plan, weighting=mode)
+        _C.backward_2d(volume, sinogram, plan, weighting=mode)
         return volume
     if isinstance(geom, ConeGeometry):
+        plan = geom.plan
         if volume is None:
             volume = torch.zeros(tuple(sinogram.shape[:-3]) + tuple(int(v) for v in geom.vol_shape),
-                                 dtype=_C.dtype_of_code(geom.plan.vol_prec),
+                                 dtype=_C.dtype_of_code(plan.vol_prec),
                                  device=sinogram.device)
-        _C.backward_3d_plan(volume, sinogram, geom.plan, mode=mode)
+        _C.backward_3d_plan(volume, sinogram, plan, mode=mode)
         return volume
     raise ValueError("Unknown geometry type")
 
@@ -42,18 +44,20 @@ def adjoint(sinogram, volume=None, geom=None, *, volume_out=None):
     """Matched adjoint A^T of ``forward`` (exact transpose), accumulated into ``volume``."""
     volume, geom = _split(volume, geom, None, volume_out, "volume")
     if isinstance(geom, FanGeometry):
+        plan = geom.plan
         if volume is None:
             volume = torch.zeros(tuple(sinogram.shape[:-2]) + tuple(int(v) for v in geom.vol_shape),
-                                 dtype=_C.dtype_of_code(geom.plan.vol_prec),
+                                 dtype=_C.dtype_of_code(plan.vol_prec),
                                  device=sinogram.device)
-        _C.adjoint_2d(volume, sinogram, geom.plan)
+        _C.adjoint_2d(volume, sinogram, plan)
         return volume
     if isinstance(geom, ConeGeometry):
+        plan = geom.plan
         if volume is None:
             volume = torch.zeros(tuple(sinogram.shape[:-3]) + tuple(int(v) for v in geom.vol_shape),
-                                 dtype=_C.dtype_of_code(geom.plan.vol_prec),
+                                 dtype=_C.dtype_of_code(plan.vol_prec),
                                  device=sinogram.device)
-        _C.adjoint_3d_plan(volume, sinogram, geom.plan)
+        _C.adjoint_3d_plan(volume, sinogram, plan)
         return volume
     raise ValueError("Unknown geometry type")
 
@@ -66,17 +70,19 @@ def backward_transpose(volume, geom, sinogram=None, *, mode="reference"):
     if isinstance(geom, FanGeometry):
         if mode not in ("reference", "fbp"):
             raise ValueError(f"fan-beam backward_transpose: unknown mode {mode!r}")
+        plan = geom.plan
         if sinogram is None:
             sinogram = torch.empty(tuple(volume.shape[:-2]) + tuple(geom.sinogram_shape()),
-                                   dtype=_C.dtype_of_code(geom.plan.det_prec),
+                                   dtype=_C.dtype_of_code(plan.det_prec),
                                    device=volume.device)
-        _C.backward_2d_transpose(volume, sinogram, geom.plan, weighting=mode)
+        _C.backward_2d_transpose(volume, sinogram, plan, weighting=mode)
         return sinogram
     if isinstance(geom, ConeGeometry):
+        plan = geom.plan
         if sinogram is None:
             sinogram = torch.empty(tuple(volume.shape[:-3]) + tuple(geom.sinogram_shape()),
-                                   dtype=_C.dtype_of_code(geom.plan.det_prec),
+                                   dtype=_C.dtype_of_code(plan.det_prec),
                                    device=volume.device)
-        _C.backward_3d_transpose(volume, sinogram, geom.plan, mode=mode)
+        _C.backward_3d_transpose(volume, sinogram, plan, mode=mode)
         return sinogram
     raise ValueError("Unknown geometry type")

@@ -37,18 +37,17 @@ def _split(first, second, geom_kw, out_kw, out_name):
 
 def forward(volume, sinogram=None, geom=None, *, sinogram_out=None):
     sinogram, geom = _split(sinogram, geom, None, sinogram_out, "sinogram")
+    if not isinstance(geom, _GEOMS):
+        raise ValueError("Unknown geometry type")
+    plan = geom.plan  # once per call: every access compares all attributes
     if isinstance(geom, FanGeometry):
         if sinogram is None:
             sinogram = torch.empty(tuple(volume.shape[:-2]) + geom.sinogram_shape(),
-                                   dtype=_C.dtype_of_code(geom.plan.det_prec),
-                                   device=volume.device)
-        _C.forward_2d(volume, sinogram, geom.plan)
+                                   dtype=_C.dtype_of_code(plan.det_prec), device=volume.device)
+        _C.forward_2d(volume, sinogram, plan)
         return sinogram
-    if isinstance(geom, ConeGeometry):
-        if sinogram is None:
-            sinogram = torch.empty(tuple(volume.shape[:-3]) + geom.sinogram_shape(),
-                                   dtype=_C.dtype_of_code(geom.plan.det_prec),
-                                   device=volume.device)
-        _C.forward_3d_plan(volume, sinogram, geom.plan)
-        return sinogram
-    raise ValueError("Unknown geometry type")
+    if sinogram is None:
+        sinogram = torch.empty(tuple(volume.shape[:-3]) + geom.sinogram_shape(),
+                               dtype=_C.dtype_of_code(plan.det_prec), device=volume.device)
+    _C.forward_3d_plan(volume, sinogram, plan)
+    return sinogram

@@ -44,10 +44,10 @@ def _rot_rpy(roll, pitch, yaw):
                      [-sp, cp * sy, cp * cy]])
 
 
-def _fp(a) -> bytes:
-    """Bytes of an array-like as FP64, for plan fingerprints."""
+def _fp(a) -> Tuple[tuple, bytes]:
+    """Shape and bytes of an array-like as FP64, for plan fingerprints."""
     a = np.asarray(a, dtype=np.float64)
-    return bytes(repr(a.shape), "ascii") + a.tobytes()
+    return a.shape, a.tobytes()
 
 
 def is_convertible_to_float(val: Any):
