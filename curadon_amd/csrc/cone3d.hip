@@ -1009,6 +1009,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp3d(typename SV::raw *__restrict
 // volumes, calls: 256^3 x 360 of 384^2 14.2 -> 10.5 ms, 128^3 x 180 of 192^2 1.16 -> 0.78 ms
 // (slices per chunk x steps together 20 x 4: 0.79, 28 x 4: 0.77, 28 x 3: 0.78 and 10.8 ms at 256^3,
 // 20 x 3: 11.0).
+// The matrix rows in LDS and the cells' addresses by FMA on subnormals then freed 20 VGPRs (84 kept
+// five wavefronts per SIMD, 63 keep eight): the kernel at 128^3 x 180 670 -> 569 us.
 // Fixed point: terms are rounded to units of max|vol| wbound / 2^kBTBits, where wbound >= the
 // weight (1, or 1 / min W^2 for FDK, W > 0 over the volume), so |term| <= 2^kBTBits and a
 // 32-bit LDS cell holds the sum of up to 2^(31 - kBTBits) - 1 terms. A voxel adds at most one
@@ -1038,6 +1040,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
                                                      int V, int A) {
     __shared__ unsigned int cells[kBTP * kBTP]; // pixel iu0 - 1 + i, iv0 - 1 + j at j kBTP + i
     __shared__ float coef[4][4];                // per corner line: F = a + b hK, G = c + d hK
+    __shared__ double rows[3][4];               // matrix rows, see below
     __shared__ int whole;                       // 1: walk whole slices
     const int tid = threadIdx.x, lane = tid & 63;
     const int a = (int)(blockIdx.x % (unsigned)A), ti = (int)(blockIdx.x / (unsigned)A);
@@ -1110,11 +1113,29 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
             whole = !(okm == ~0ull && (posm == 0ull || posm == ~0ull));
     }
     for (int i = tid; i < kBTP * kBTP; i += kMaxBlock) cells[i] = 0u;
-    __syncthreads();
     const int nK = K == 0 ? nx : (K == 1 ? ny : nz);
     const int nF = F == 0 ? nx : ny, nG = G == 1 ? ny : nz;
     const float cK = K == 0 ? cx : (K == 1 ? cy : cz);
     const float cF = F == 0 ? cx : cy, cG = G == 1 ? cy : cz;
+    // matrix rows over the voxel's index (f, g, k) along (F, G, K), the panel coordinates taken
+    // from the tile's middle LDS cell (kept in LDS: 24 registers of the walk otherwise)
+    constexpr int kMid = kBTP / 2 - 1;
+    static_assert(2 * kMid == kBT, "lower taps lie within kMid cells of the middle one");
+    if (tid < 3) {
+        auto row = [&](int r, double (&o)[4]) {
+            const double x = m[4 * r], y = m[4 * r + 1], z = m[4 * r + 2];
+            o[0] = F == 0 ? x : y;
+            o[1] = G == 1 ? y : z;
+            o[2] = K == 0 ? x : (K == 1 ? y : z);
+            o[3] = (double)m[4 * r + 3] - o[0] * cF - o[1] * cG - o[2] * cK;
+        };
+        double o[4], w[4];
+        row(tid, o);
+        row(2, w);
+        const double mid = tid == 0 ? (double)(iu0 - 1 + kMid) : (double)(iv0 - 1 + kMid);
+        for (int k = 0; k < 4; ++k) rows[tid][k] = tid < 2 ? o[k] - mid * w[k] : o[k];
+    }
+    __syncthreads();
     // voxel (f, g, k) along (F, G, K) lies at src[f + g strG + k strK]: the volume, or for K = x
     // the y-fastest copy [z + 2][x + 2][y + 2]
     const int Wp = nx + 2 * kPad, Hp = ny + 2 * kPad;
@@ -1123,25 +1144,6 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
                : vol + b * (size_t)nx * ny * nz;
     const int strG = K == 0 ? Wp * Hp : (K == 1 ? nx * ny : nx);
     const int strK = K == 0 ? Hp : (K == 1 ? nx : nx * ny);
-    // matrix rows over the voxel's index (f, g, k) along (F, G, K), the panel coordinates taken
-    // from the tile's first LDS cell
-    double ru[4], rv[4], rw[4];
-    {
-        auto row = [&](int r, double (&o)[4]) {
-            const double x = m[4 * r], y = m[4 * r + 1], z = m[4 * r + 2];
-            o[0] = F == 0 ? x : y;
-            o[1] = G == 1 ? y : z;
-            o[2] = K == 0 ? x : (K == 1 ? y : z);
-            o[3] = (double)m[4 * r + 3] - o[0] * cF - o[1] * cG - o[2] * cK;
-        };
-        row(0, ru);
-        row(1, rv);
-        row(2, rw);
-        for (int k = 0; k < 4; ++k) {
-            ru[k] -= (double)(iu0 - 1) * rw[k];
-            rv[k] -= (double)(iv0 - 1) * rw[k];
-        }
-    }
     unsigned int *mine = &cells[(tid / kBT + 1) * kBTP + tid % kBT + 1];
     long long own = 0;
     // cells -> registers (border cells, which belong to other tiles, are never read)
@@ -1151,8 +1153,12 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
         *mine = 0u;
         __syncthreads();
     };
-    const float uF = (float)ru[0], uG = (float)ru[1], vF = (float)rv[0], vG = (float)rv[1],
-                wF = (float)rw[0], wG = (float)rw[1];
+    const float uF = (float)rows[0][0], uG = (float)rows[0][1], vF = (float)rows[1][0],
+                vG = (float)rows[1][1], wF = (float)rows[2][0], wG = (float)rows[2][1];
+    // byte strides and the middle cell's address, as subnormals
+    const float ccol = subnormal(4), crow = subnormal(4 * kBTP);
+    const float cofs = subnormal((int)(uintptr_t)(__attribute__((address_space(3))) unsigned *)cells +
+                                 4 * (kMid * kBTP + kMid));
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     int run = 0; // voxel visits since the last drain
     for (int k0 = 0; k0 < nK; k0 += kBTSlab) {
@@ -1191,9 +1197,10 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
         if (total == 0) continue;
         flo = max(0, min(flo, nF - NF));
         glo = max(0, min(glo, nG - NG));
-        const float ul = (float)(ru[0] * flo + ru[1] * glo + ru[2] * k + ru[3]);
-        const float vl = (float)(rv[0] * flo + rv[1] * glo + rv[2] * k + rv[3]);
-        const float wl = (float)(rw[0] * flo + rw[1] * glo + rw[2] * k + rw[3]);
+        auto at_origin = [&](int r) {
+            return (float)(rows[r][0] * flo + rows[r][1] * glo + rows[r][2] * k + rows[r][3]);
+        };
+        const float ul = at_origin(0), vl = at_origin(1), wl = at_origin(2);
         const int at = flo + glo * strG + k * strK;
         const float rNF = 1.0f / (float)NF;
         auto lane_of = [](float x, int l) {
@@ -1238,19 +1245,20 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT3d(typename SS::raw *__restric
                     const float x = val[q] * s1 * s2;
                     const float r = __builtin_amdgcn_rcpf(ws[q] + w0);
                     const float u = (us[q] + u0) * r, v = (vs[q] + v0) * r;
-                    const int i = floor_i32(u), j = floor_i32(v);
-                    if ((unsigned)i > (unsigned)kBT || (unsigned)j > (unsigned)kBT || x == 0.0f)
+                    const float i = floorf(u), j = floorf(v);
+                    if (!(fabsf(i) <= (float)kMid && fabsf(j) <= (float)kMid) || x == 0.0f)
                         continue;
-                    const float fu = __builtin_amdgcn_fractf(u), fv = __builtin_amdgcn_fractf(v);
+                    const float fu = u - i, fv = v - j;
                     const float t = FDK ? x * (r * r) : x;
                     const float t1 = t * fu, t0 = t - t1;
                     const float t01 = t0 * fv, t00 = t0 - t01;
                     const float t11 = t1 * fv, t10 = t1 - t11;
-                    unsigned int *c = &cells[j * kBTP + i];
-                    atomicAdd(c, (unsigned)round_i32(t00));
-                    atomicAdd(c + 1, (unsigned)round_i32(t10));
-                    atomicAdd(c + kBTP, (unsigned)round_i32(t01));
-                    atomicAdd(c + kBTP + 1, (unsigned)round_i32(t11));
+                    auto *const c = (__attribute__((address_space(3))) unsigned *)(uintptr_t)
+                        __float_as_uint(fmaf(j, crow, fmaf(i, ccol, cofs)));
+                    lds_add(c, (unsigned)round_i32(t00));
+                    lds_add(c + 1, (unsigned)round_i32(t10));
+                    lds_add(c + kBTP, (unsigned)round_i32(t01));
+                    lds_add(c + kBTP + 1, (unsigned)round_i32(t11));
                 }
             }
         };
