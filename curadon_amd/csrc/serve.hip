@@ -240,8 +240,9 @@ __global__ __launch_bounds__(kThreads) void k_serve_bp2d(const DevJob *__restric
 }
 
 // Cone-beam tiles. YRUNS: every job of the launch takes the y-invariant body (columns == 1), and the
-// general column body is left out. Five wavefronts per SIMD: the persistent loop around the
-// body's three modes took 97 VGPRs (four wavefronts per SIMD); 96 fit without spills, 80 spilled.
+// general body is left out. Five wavefronts per SIMD (94 VGPRs; without the bound the persistent
+// loop around the body's three modes took 97, four wavefronts). Six, with 79, take the same time: 411
+// us for eight small jobs.
 template <class SV, class SS, bool YRUNS>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_serve_bp3d(const DevJob *__restrict__ jobs,
                                                          int njobs, uint32_t total,

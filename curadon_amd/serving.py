@@ -40,11 +40,12 @@ from .reconstruction import (cosine_weights_cone, cosine_weights_fan, fft_length
                              filter_rows_weighted)
 
 # Relative cost of one voxel-angle of the cone-beam backprojector to one pixel-angle of the
-# fan-beam one (2 x 2 taps from LDS-staged footprints against 2 taps from the sinogram; measured
-# 2.1e12 voxel-angles/s at 384^3 against 2.35e12 pixel-angles/s at 2048^2).
+# fan-beam one (2 x 2 taps from LDS-staged footprints against 2 taps from the sinogram; set at
+# 2.1e12 voxel-angles/s at 384^3 against 2.35e12 pixel-angles/s at 2048^2; the former are 2.7e12
+# now).
 CONE_COST = 1.15
 PIXELS_PER_TILE_2D = 64 * 4
-# voxels per tile of the cone-beam kernel: y-invariant matrices (16 x 16 x 16) / others (16 x 16 x 8)
+# voxels per tile of the cone-beam kernel: matrices free of y / others
 VOXELS_PER_TILE_3D = {True: 16 * 16 * 16, False: 16 * 16 * 8}
 
 

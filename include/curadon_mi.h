@@ -412,7 +412,7 @@ typedef enum cmi_job_kind { CMI_JOB_FAN2D = 0, CMI_JOB_CONE3D = 1 } cmi_job_kind
  *   table   device copy of cmi_fan2d_bp_table / cmi_cone3d_bp_matrices output
  *   volume  [ny][nx] / [nz][ny][nx], accumulated into
  *   mode    fan: cmi_bp2d_weighting; cone: cmi_bp3d_mode (the mode the matrices were made for)
- *   columns cone only: 0 = z columns (any geometry), 1 = y runs (y_invariant matrices only)
+ *   columns cone only: 0 = any geometry, 1 = matrices free of y (y_invariant only)
  *   fan only: sx, sy pixel spacing, ox, oy volume offset, inv_du = 1 / detector spacing
  * No counterpart in the reference, which runs one operator call per image.
  */
@@ -441,7 +441,7 @@ CMI_API cmi_status cmi_server_destroy(cmi_server *server);
 
 /* Workgroups of the cone-beam serving kernel for jobs of either tile layout that the device
  * holds resident at once (the persistent grid of a launch with at least that many cone-beam
- * tiles). Launches whose cone-beam jobs all take y runs, and the fan-beam tiles, use kernels of
+ * tiles). Launches whose cone-beam jobs all have columns = 1, and the fan-beam tiles, use kernels of
  * their own with their own resident counts. */
 CMI_API cmi_status cmi_server_get_capacity(const cmi_server *server, uint32_t *workgroups);
 
