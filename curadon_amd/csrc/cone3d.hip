@@ -991,7 +991,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp3d(typename SV::raw *__restrict
 // workgroup marches through the volume along the axis K that the tile's central ray follows
 // most closely, in chunks of kBTSlab slices. In each slice the pyramid's section is the
 // quadrilateral where the corner lines cross it; its bounding box (kBTMargin of a voxel wider on
-// each side, for the FP32 lines; clipped to the volume) is found by the lane that holds the slice. A wavefront takes every
+// each side, for the FP32 lines; clipped to the volume) is found by the lane that holds the slice.
+// A wavefront takes every
 // fourth slice of a chunk and walks it in steps of 64 voxels, x fastest (y when K is x, from a
 // y-fastest copy of the volume), so that it reads runs of consecutive voxels. All slices of a
 // chunk are walked over the extents of its widest box, their origins moved back where that would

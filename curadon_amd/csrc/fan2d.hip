@@ -525,7 +525,8 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
 // Six wavefronts per SIMD (80 VGPRs, 40 bytes of scratch with FP32 images): 0.498 ms at 1024^2, five
 // 0.511.
 template <class SI, class SS>
-__global__ __launch_bounds__(kFwdRays) __attribute__((amdgpu_waves_per_eu(6))) void k_fwd2d(const typename SI::raw *__restrict__ scratch,
+__global__ __launch_bounds__(kFwdRays) __attribute__((amdgpu_waves_per_eu(6)))
+void k_fwd2d(const typename SI::raw *__restrict__ scratch,
                                               int Wp, int Hp, const float4 *__restrict__ ev,
                                               const float4 *__restrict__ ns,
                                               typename SS::raw *__restrict__ sino, int D, int A) {
@@ -1162,8 +1163,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // affine in the pixel). The workgroup marches through the image along the axis K (rows or
 // columns) that the segment's central line follows most closely, in chunks of kGSlab lines;
 // per line the wedge is the interval between the two boundary lines' crossings (kGMargin of a
-// pixel wider on each side, for the FP32 lines; clipped to the image). A wavefront takes every fourth line of a chunk and
-// walks it along the line, a lane per pixel, from the zero-bordered copy whose rows run along it
+// pixel wider on each side, for the FP32 lines; clipped to the image). A wavefront takes every
+// fourth line of a chunk and walks it along the line, a lane per pixel, from the zero-bordered copy whose rows run along it
 // (row-major for rows, transposed for columns), so that it reads runs of consecutive pixels. All
 // lines of a chunk are walked over the width of its widest interval, their starts moved back
 // where that would leave the image: pixels outside the wedge have no cell in the segment and add
@@ -1719,8 +1720,8 @@ cmi_status fan2d_forward_enqueue(const cmi_plan2d *plan, const void *volume, int
         // block_x * block_y (at most kFwdRays) adjacent cells of one angle per workgroup
         const unsigned nt = std::min<unsigned>(plan->block_x * plan->block_y, kFwdRays);
         dim3 fb(nt), fg((unsigned)((D + nt - 1) / nt), (unsigned)A, (unsigned)batch);
-        hipLaunchKernelGGL((k_fwd2d<SI, SS>), fg, fb, 0, s, (const RI *)scratch, Wp, Hp, plan->d_ev, plan->d_ns,
-                           (typename SS::raw *)sinogram, D, A);
+        hipLaunchKernelGGL((k_fwd2d<SI, SS>), fg, fb, 0, s, (const RI *)scratch, Wp, Hp,
+                           plan->d_ev, plan->d_ns, (typename SS::raw *)sinogram, D, A);
         CMI_HIP_TRY(hipGetLastError());
         return CMI_OK;
     });
@@ -2067,7 +2068,8 @@ CMI_API cmi_status cmi_adjoint_2d(const cmi_plan2d *plan, void *volume, int vol_
                            dim3(kMaxBlock), 0, s, (const typename SS::raw *)sinogram, plan->d_ns,
                            rays, parts);
         // angle groups: enough workgroups to fill the GPU many times over (about 96 per CU; with
-        // tiles of 32 x 32 at 1024^2 a target of 8192 workgroups gave 1.09 ms, 16384: 1.06, 24576: 1.04, 32768: 1.05)
+        // tiles of 32 x 32 at 1024^2 a target of 8192 workgroups gave 1.09 ms, 16384: 1.06, 24576:
+        // 1.04, 32768: 1.05)
         const unsigned tiles = adj2d_tiles(ny, nx) + adj2d_tiles(nx, ny);
         const uint64_t all = (uint64_t)tiles * batch;
         const int G = (int)std::max<uint64_t>(

@@ -234,3 +234,21 @@ def test_adjoint_3d_angle_groups(gpu):
     for i in range(2):
         one = cm.adjoint(y[i].contiguous(), geom)
         assert torch.equal(many[i], one) and torch.equal(many[batch - 2 + i], one)
+
+
+@pytest.mark.parametrize("ny,nx", [(1, 40), (12, 33), (15, 64), (27, 90), (28, 29), (59, 31), (150, 140)])
+@pytest.mark.parametrize("D,du", [
+    (70, 0.4),     # many cells per texel: narrow bands, four groups of threads with rows to spare
+    (300, 0.9),    # bands of about 25 quads
+    (200, 1.55),   # more than 32 quads: two groups of threads, nine rows each
+    (130, 3.0),    # bands too wide for LDS
+])
+def test_forward_bands(oracle, gpu, ny, nx, D, du):
+    """Images whose rows (with the border) end before, at and after a band and a group of rows, in
+    both dominant axes; angles on and between the axes."""
+    n = max(ny, nx)
+    rec = fan(nx, D, 9, 2.0 * n, 3.0 * n, du=du, ny=ny)
+    geom = as_fan_geometry(rec)
+    img = np.random.RandomState(D + ny).rand(ny, nx)
+    got = cm.forward(torch.tensor(img, dtype=torch.float32, device=gpu), geom)
+    assert rel_l2(got, oracle.fwd2d(rec, img)) <= RTOL_L2
