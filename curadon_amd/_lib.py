@@ -146,6 +146,8 @@ SIGNATURES = {
                                      C.c_float, _vp, _i32, _vp]),
     "cmi_filter_pack": (_i32, [_i32, _vp, _u64, _u64, _vp, _u64, _u64, _vp, _vp]),
     "cmi_filter_unpack": (_i32, [_i32, _vp, _u64, _u64, _u64, _vp, _vp]),
+    "cmi_cosine_weights": (_i32, [_i32, _vp, C.c_double, _u64, _u64, C.c_double, C.c_double, _vp,
+                                  _vp]),
     "cmi_bp_job_tiles": (_i32, [C.POINTER(BPJob), _u64p]),
     "cmi_server_create": (_i32, [_i32, C.c_uint32, C.POINTER(_vp)]),
     "cmi_server_destroy": (_i32, [_vp]),
@@ -728,6 +730,24 @@ def filter_unpack(src, dst):
         raise ValueError("filter_unpack: tensors on different devices")
     check(_lib.cmi_filter_unpack(dst.device.index or 0, src.data_ptr(), rows, D, src.shape[1],
                                  dst.data_ptr(), torch.cuda.current_stream(dst.device).cuda_stream))
+
+
+def cosine_weights(dsd, dv, du, dst):
+    """dst (rows, D) FP32 := dsd / sqrt(dsd^2 + u^2 + v^2) at the cells' centres; dsd is a number or
+    an FP64 device tensor of a distance per row (cmi_cosine_weights). Enqueued on the current
+    stream."""
+    _require_device_tensor(dst, "destination")
+    if dst.dtype != torch.float32 or dst.dim() != 2 or not dst.is_contiguous():
+        raise TypeError("destination must be a contiguous FP32 matrix")
+    rows = None
+    if isinstance(dsd, torch.Tensor):
+        if (dsd.dtype != torch.float64 or dsd.shape != dst.shape[:1] or not dsd.is_contiguous() or
+                dsd.device != dst.device):
+            raise TypeError("distances must be FP64, one per row, on the destination's device")
+        rows, dsd = dsd.data_ptr(), 0.0
+    check(_lib.cmi_cosine_weights(dst.device.index or 0, rows, dsd, dst.shape[0], dst.shape[1], dv,
+                                  du, dst.data_ptr(),
+                                  torch.cuda.current_stream(dst.device).cuda_stream))
 
 
 def stage_projections(src, dst, row_scale=None, scale=1.0):

@@ -28,6 +28,7 @@ import functools
 import threading
 import math
 
+import numpy as np
 import torch
 
 from .geometry import ConeGeometry, FanGeometry
@@ -206,11 +207,31 @@ def filter_rows_weighted(p: torch.Tensor, cw: torch.Tensor, n_det: int, window="
     return out
 
 
+def _uniform(a: np.ndarray):
+    """The value that all entries of an array share, or None."""
+    return float(a[0]) if (a == a[0]).all() else None
+
+
+def _native_weights(device, rows, cells) -> bool:
+    # the kernel's range; other devices and sizes evaluate the same operations with torch
+    return (device is not None and torch.device(device).type == "cuda" and
+            0 < rows <= 1 << 24 and 0 < cells <= 1 << 24)
+
+
 def cosine_weights_fan(geom: FanGeometry, device=None) -> torch.Tensor:
     """(A, D) cosine pre-weights DSD / sqrt(DSD^2 + u^2), u the cell centre on the detector.
     Evaluated in FP64 on `device` (correctly rounded operations: the same values on any
     device) and returned as FP32."""
     D = geom.det_shape
+    if (isinstance(geom.DSD, np.ndarray) and geom.DSD.ndim == 1 and
+            _native_weights(device, geom.DSD.size, D)):
+        from . import _lib
+        dsd = _uniform(geom.DSD)
+        if dsd is None:
+            dsd = torch.as_tensor(geom.DSD, dtype=torch.float64).to(device)
+        cw = torch.empty((geom.DSD.size, D), dtype=torch.float32, device=device)
+        _lib.cosine_weights(dsd, 0.0, float(geom.det_spacing), cw)
+        return cw
     u = (torch.arange(D, dtype=torch.float64, device=device) - (D - 1) / 2) * geom.det_spacing
     dsd = torch.as_tensor(geom.DSD, dtype=torch.float64).to(device)[:, None]
     return (dsd / torch.sqrt(dsd * dsd + (u * u)[None, :])).to(torch.float32)
@@ -220,6 +241,11 @@ def cosine_weights_cone(geom: ConeGeometry, device=None) -> torch.Tensor:
     """(V, U) cosine pre-weights DSD / sqrt(DSD^2 + u^2 + v^2), FP64 on `device`, as FP32."""
     V, U = (int(v) for v in geom.det_shape)
     dv, du = (float(v) for v in geom.det_spacing)
+    if _native_weights(device, V, U):
+        from . import _lib
+        cw = torch.empty((V, U), dtype=torch.float32, device=device)
+        _lib.cosine_weights(float(geom.DSD), dv, du, cw)
+        return cw
     u = (torch.arange(U, dtype=torch.float64, device=device) - (U - 1) / 2) * du
     v = (torch.arange(V, dtype=torch.float64, device=device) - (V - 1) / 2) * dv
     r2 = (v * v)[:, None] + (u * u)[None, :]
@@ -232,9 +258,9 @@ def _native_filter(sinogram: torch.Tensor, dt) -> bool:
     return sinogram.is_cuda and dt == torch.float32 and sinogram.dtype == torch.float32
 
 
-def fbp_filter(sinogram: torch.Tensor, geom, window="ram-lak", frequency_scaling=1.0):
-    """Cosine-weighted, ramp-filtered and scaled projections (FP32), ready for the weighted
-    backprojection (`backward(..., mode="fbp")` for fan beam, mode="fdk" for cone beam)."""
+def _filtered(sinogram: torch.Tensor, geom, window, frequency_scaling):
+    """Cosine-weighted and ramp-filtered projections, and the scale that they still need: a number,
+    or a column of one per angle."""
     dev = sinogram.device
     dt = torch.float64 if sinogram.dtype == torch.float64 else torch.float32
     if (isinstance(geom, FanGeometry) and not geom.is_centred_circular()) or (
@@ -245,22 +271,34 @@ def fbp_filter(sinogram: torch.Tensor, geom, window="ram-lak", frequency_scaling
             "backward / adjoint, or a centred circular geometry")
     if isinstance(geom, FanGeometry):
         cw = cosine_weights_fan(geom, dev).to(dt)
-        scale = (math.pi / geom.nangles) * torch.as_tensor(
-            geom.DSO / geom.DSD, dtype=dt, device=dev)[:, None]
+        ratio = geom.DSO / geom.DSD
+        one = _uniform(ratio)
+        if one is None:
+            scale = (math.pi / geom.nangles) * torch.as_tensor(ratio, dtype=dt, device=dev)[:, None]
+        else:  # a number needs no copy to the device; rounded as the tensor's product is
+            num = np.float64 if dt == torch.float64 else np.float32
+            scale = float(num(math.pi / geom.nangles) * num(one))
         if _native_filter(sinogram, dt):
             return filter_rows_weighted(sinogram, cw, geom.det_shape, window,
-                                        frequency_scaling) * scale
+                                        frequency_scaling), scale
         H = ramp_response(geom.det_shape, window, frequency_scaling, dev)
-        return filter_rows(sinogram.to(dt) * cw, H) * scale
+        return filter_rows(sinogram.to(dt) * cw, H), scale
     if isinstance(geom, ConeGeometry):
         cw = cosine_weights_cone(geom, dev).to(dt)
         scale = (math.pi / geom.nangles) * geom.DSD / (float(geom.det_spacing[1]) * geom.DSO)
         if _native_filter(sinogram, dt):
             return filter_rows_weighted(sinogram, cw, int(geom.det_shape[1]), window,
-                                        frequency_scaling) * scale
+                                        frequency_scaling), scale
         H = ramp_response(int(geom.det_shape[1]), window, frequency_scaling, dev)
-        return filter_rows(sinogram.to(dt) * cw, H) * scale
+        return filter_rows(sinogram.to(dt) * cw, H), scale
     raise ValueError("Unknown geometry type")
+
+
+def fbp_filter(sinogram: torch.Tensor, geom, window="ram-lak", frequency_scaling=1.0):
+    """Cosine-weighted, ramp-filtered and scaled projections (FP32), ready for the weighted
+    backprojection (`backward(..., mode="fbp")` for fan beam, mode="fdk" for cone beam)."""
+    q, scale = _filtered(sinogram, geom, window, frequency_scaling)
+    return q * scale
 
 
 def fbp(sinogram: torch.Tensor, geom, window="ram-lak", frequency_scaling=1.0, volume=None):
@@ -271,8 +309,12 @@ def fbp(sinogram: torch.Tensor, geom, window="ram-lak", frequency_scaling=1.0, v
     on its own, storing the filtered ones in FP16 ~2e-5."""
     from . import _lib
     from .backward import backward
-    q = fbp_filter(sinogram, geom, window, frequency_scaling)
-    q = q.to(_lib.dtype_of_code(geom.plan.det_prec)).contiguous()
+    # scaled in FP32 (FP64) and cast in one pass over the projections (384^3 from 768 views of
+    # 576^2, FP16: 19.2 ms instead of 19.6 for scale, then cast); the backprojection records no
+    # gradient, and out= takes no tensor that does
+    q, scale = _filtered(sinogram.detach(), geom, window, frequency_scaling)
+    out = torch.empty(0, dtype=_lib.dtype_of_code(geom.plan.det_prec), device=q.device)
+    q = torch.mul(q, scale, out=out).contiguous()
     mode = "fbp" if isinstance(geom, FanGeometry) else "fdk"
     return backward(q, volume, geom, mode=mode)
 

@@ -395,6 +395,16 @@ CMI_API cmi_status cmi_filter_pack(int device, const float *src, uint64_t rows, 
 CMI_API cmi_status cmi_filter_unpack(int device, const float *src, uint64_t rows, uint64_t D,
                                      uint64_t L, float *dst, void *stream);
 
+/*
+ * Cosine pre-weights of a filtered backprojection, evaluated in FP64 and rounded to FP32:
+ *   dst[r][i] = d / sqrt(d^2 + u^2 + v^2), u = (i - (D - 1) / 2) du, v = (r - (rows - 1) / 2) dv,
+ * d = dsd_rows[r], or dsd where dsd_rows is null. A fan beam's rows are its angles (dv = 0, a
+ * distance each), a cone beam's its panel rows. No counterpart in the reference, whose example
+ * filters parallel-beam weights only (examples/fbp.py:51-56). Device memory, enqueued on `stream`.
+ */
+CMI_API cmi_status cmi_cosine_weights(int device, const double *dsd_rows, double dsd, uint64_t rows,
+                                      uint64_t D, double dv, double du, float *dst, void *stream);
+
 /* Job kinds of the serving backprojector. */
 typedef enum cmi_job_kind { CMI_JOB_FAN2D = 0, CMI_JOB_CONE3D = 1 } cmi_job_kind;
 

@@ -252,3 +252,39 @@ def test_forward_bands(oracle, gpu, ny, nx, D, du):
     img = np.random.RandomState(D + ny).rand(ny, nx)
     got = cm.forward(torch.tensor(img, dtype=torch.float32, device=gpu), geom)
     assert rel_l2(got, oracle.fwd2d(rec, img)) <= RTOL_L2
+
+
+@pytest.mark.parametrize("prec", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lead,grad", [((), False), ((2,), True)])
+@pytest.mark.parametrize("rec", [lambda: fan(33, 51, 7, 70.0, 100.0, ny=21),
+                                 lambda: cone(17, 20, 18, 6, 60.0, 90.0, nz=15, ny=5)])
+def test_fbp_equals_its_steps(gpu, rec, lead, grad, prec):
+    """The filtered projections scaled and cast in one pass are those of `fbp_filter`, rounded."""
+    rec = rec()
+    as_geom = as_fan_geometry if isinstance(rec.det_shape, int) else as_cone_geometry
+    geom = as_geom(rec, vol_prec=prec, sino_prec=prec)
+    mode = "fbp" if isinstance(geom, cm.FanGeometry) else "fdk"
+    for src in (torch.float32, torch.float64):
+        y = rand(lead + tuple(geom.sinogram_shape()), gpu, 3, src).requires_grad_(grad)
+        got = cm.fbp(y, geom)
+        steps = cm.backward(cm.fbp_filter(y, geom).detach().to(prec), geom, mode=mode)
+        assert torch.equal(got, steps) and got.dtype == prec and not got.requires_grad
+
+
+@pytest.mark.parametrize("A,D", [(1, 1), (3, 256), (5, 257), (65537, 2)])
+@pytest.mark.parametrize("one", [True, False])
+def test_cosine_weights_equal_host(gpu, A, D, one):
+    """The kernel's weights are the host's, bit for bit, as is the scale of equal distances."""
+    from curadon_amd import reconstruction as R
+    dso = 100.0 + 0.1 * (np.zeros(A) if one else np.arange(A) % 97)
+    geom = cm.FanGeometry(DSD=1.37 * dso, DSO=dso, angles=np.linspace(0, 6, A), vol_shape=(8, 8),
+                          det_shape=D, det_spacing=0.731)
+    host = R.cosine_weights_fan(geom, "cpu")
+    assert torch.equal(R.cosine_weights_fan(geom, gpu).cpu(), host)
+    c = cm.ConeGeometry(DSD=137.1, DSO=100.3, angles=np.linspace(0, 6, 3), vol_shape=(8, 8, 8),
+                        det_shape=(A, D), det_spacing=(0.31, 0.731))
+    assert torch.equal(R.cosine_weights_cone(c, gpu).cpu(), R.cosine_weights_cone(c, "cpu"))
+    y = rand((A, D), gpu, 7)
+    q, scale = R._filtered(y, geom, "ram-lak", 1.0)
+    column = (np.pi / A) * torch.as_tensor(dso / (1.37 * dso), dtype=torch.float32, device=gpu)
+    assert torch.equal(q * scale, q * column[:, None])
