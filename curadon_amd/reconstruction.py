@@ -272,7 +272,8 @@ def _filtered(sinogram: torch.Tensor, geom, window, frequency_scaling):
     if isinstance(geom, FanGeometry):
         cw = cosine_weights_fan(geom, dev).to(dt)
         ratio = geom.DSO / geom.DSD
-        one = _uniform(ratio)
+        # rows that are not the angles go on meeting a column, which broadcasts or refuses them
+        one = _uniform(ratio) if sinogram.shape[-2:-1] == (geom.nangles,) else None
         if one is None:
             scale = (math.pi / geom.nangles) * torch.as_tensor(ratio, dtype=dt, device=dev)[:, None]
         else:  # a number needs no copy to the device; rounded as the tensor's product is

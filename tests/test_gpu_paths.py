@@ -288,3 +288,16 @@ def test_cosine_weights_equal_host(gpu, A, D, one):
     q, scale = R._filtered(y, geom, "ram-lak", 1.0)
     column = (np.pi / A) * torch.as_tensor(dso / (1.37 * dso), dtype=torch.float32, device=gpu)
     assert torch.equal(q * scale, q * column[:, None])
+
+
+def test_fbp_filter_rows_that_are_not_the_angles(gpu):
+    """Equal distances change nothing in which shapes are refused and how others broadcast."""
+    A, D = 6, 20
+    for dso in (np.full(A, 50.0), 50.0 + np.arange(A)):
+        geom = cm.FanGeometry(DSD=1.5 * dso, DSO=dso, angles=np.linspace(0, 5, A),
+                              vol_shape=(8, 8), det_shape=D)
+        y = rand((2, A, D), gpu, 9)
+        with pytest.raises(RuntimeError):
+            cm.fbp_filter(y.reshape(2 * A, D), geom)
+        assert cm.fbp_filter(y[:, :, None, :], geom).shape == (2, A, A, D)
+        assert cm.fbp_filter(y, geom).shape == (2, A, D)
