@@ -301,7 +301,6 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
     const int ta = s > 0 ? r0 + jlo : r0 - jhi; // first row of this lane
     const int tz = ta + n - 1;                  // last row
     const int k = (int)threadIdx.x;
-    if (k == 0) *flag = 0; // ordered before every use by block_min's barriers
     // pass-wide: rows [tr0, tr1], the latest first row and earliest last row of any lane, the
     // first and last active lane, whether every lane of the workgroup is in the pass, and whether
     // any is in the other
@@ -535,11 +534,11 @@ void k_fwd2d(const typename SI::raw *__restrict__ scratch,
         float band[kBandRows * kPitch];
         float4 ext[2];
         int red[8 * kMaxWaves];
-        int flag;
+        int flag[2]; // one per pass: no barrier follows a pass's read where nothing is staged
     } sh;
     float *band = sh.band;
     float4 *ext = sh.ext;
-    int *red = sh.red, *flag = &sh.flag;
+    int *red = sh.red;
     const int nthreads = blockDim.x;
     // The launch's linear workgroup index taken with angles fastest: consecutive workgroups
     // (dealt to the 8 XCDs in turn) hold the same cells at successive angles, so every XCD
@@ -556,16 +555,18 @@ void k_fwd2d(const typename SI::raw *__restrict__ scratch,
     const int one = Wp * Hp;
     const rsrc_t R = make_rsrc(scratch + b * 2 * (size_t)one, bytes_of<SI>(2 * (uint64_t)one));
     const int c0x = Wp / 2, c0y = Hp / 2;
-    // the zero cells; ordered before their first read by the barriers at the start of a pass
+    // the zero cells and the flags; ordered before their first use by the barriers at the start of
+    // a pass
     for (int i = threadIdx.x; i < 2 * kBandRows; i += nthreads)
         band[(i >> 1) * kPitch + kPitch - 2 + (i & 1)] = 0.0f;
+    if (threadIdx.x < 2) sh.flag[threadIdx.x] = 0;
     const float scale = valid ? ns[r].x : 0.0f;
     bool others = false; // whether a lane's ray is x dominant
     float acc = march_band<SI, true>(R, ev + r, ns + r, valid, Wp, c0y * Wp + c0x, band,
-                                             red, ext, flag, nthreads, others);
+                                             red, ext, &sh.flag[0], nthreads, others);
     if (others)
         acc += march_band<SI, false>(R, ev + r, ns + r, valid, Hp, one + c0x * Hp + c0y,
-                                             band, red, ext, flag, nthreads, others);
+                                             band, red, ext, &sh.flag[1], nthreads, others);
     if (valid) sino[b * (size_t)A * D + r] = from_f32<SS>(acc * scale);
 }
 

@@ -1,0 +1,42 @@
+"""Geometries and sizes at the far ends of what the operators accept: sources close to the image and
+far from it, rays along an axis, tall panels, infinities. Against the FP64 oracle.
+
+Tolerances are those of test_gpu_fan2d.py / test_gpu_cone3d.py unless a test derives its own.
+"""
+import numpy as np
+import pytest
+import torch
+
+import curadon_amd as cm
+from geoms import as_fan_geometry, fan
+
+pytestmark = pytest.mark.gpu
+
+RTOL_L2 = 1e-5
+
+
+def rel_l2(a, b):
+    a = a.double().cpu().numpy() if isinstance(a, torch.Tensor) else a
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
+
+
+@pytest.mark.parametrize("rec", [
+    lambda: fan(64, 48, 12, 36.0, 60.0, du=4.0),           # a workgroup of one wavefront
+    lambda: fan(64, 64, 12, 46.0, 70.0, du=4.0),
+    lambda: fan(64, 128, 13, 36.0, 60.0, du=2.5),          # of two
+    lambda: fan(256, 128, 12, 190.0, 290.0, du=12.0),
+    lambda: fan(300, 100, 9, 60.0, 90.0, du=8.0, ny=40),   # the source inside the image's circle
+    lambda: fan(40, 300, 9, 60.0, 90.0, du=4.0, ny=300),
+])
+def test_forward_wide_fan(oracle, gpu, rec):
+    """Fans of more than 90 degrees within one workgroup of the forward: rays of one dominant axis
+    go both ways, some of them outside the workgroup's first and last, and rays of the other axis
+    follow in a second pass. Such a pass reads the image from global memory."""
+    rec = rec()
+    geom = as_fan_geometry(rec)
+    img = np.random.RandomState(11).rand(*rec.vol_shape)
+    x = torch.tensor(img, dtype=torch.float32, device=gpu)
+    got = cm.forward(x, geom)
+    assert rel_l2(got, oracle.fwd2d(rec, img)) <= RTOL_L2
+    for _ in range(3):
+        assert torch.equal(cm.forward(x, geom), got)
