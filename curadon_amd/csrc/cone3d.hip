@@ -225,10 +225,16 @@ __device__ __forceinline__ float sample3d(rsrc_t R, float f, float m, float l, i
 // and every ray takes its samples whose lower tap lies in the slab from there, in its own order
 // j = 0 .. n - 1, slab after slab: positions and trilinear weights are those of a plain per-ray
 // march, and the ray's sum adds one partial sum per slab (at most about 2 kSlab samples each).
-// Slabs whose box does not fit, and workgroups whose rays do not all advance the same way along
-// K, whose K is the copy's fast axis, or in which FP32 puts a ray further than kBoxMargin / 2
-// outside the corner rays (a source so far away that its coordinates lose the voxel), read
-// global memory instead, with the same arithmetic (the latter in blocks of kSumBlock samples).
+// Slabs whose box does not fit, and workgroups whose rays do not all advance the same way along K
+// or whose K is the copy's fast axis, read global memory instead, with the same arithmetic (the
+// latter in blocks of kSumBlock samples).
+// Every sample of a staged slab lies in its box, at any distance of the source: the corner rays are
+// held as their crossings of the volume's middle plane and their slopes along K, both evaluated in
+// FP64, and a box that fits has slopes below 25 over at most 2050 slices either way, so FP32 puts
+// the crossings less than 0.01 voxels off; the samples' own positions, from FP64 midpoints, are
+// less than 0.001 off. kBoxMargin covers both. (With the rays from their source in FP32, sources
+// from 10^6 voxels on lost a margin's width: workgroups had to march from global memory, and of
+// those that did not, some still read past their boxes.)
 // A wavefront covers 4 x 16 detector pixels, the 16 along v, and the copy read is the one
 // whose fastest axis v follows (fast[a]), so that a wavefront's rows of a staged box are runs
 // of consecutive voxels.
@@ -266,7 +272,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
                                                           int A,
                                                           typename SS::raw *__restrict__ sino) {
     __shared__ float4 box4[kBoxCells / 4];
-    __shared__ float cl[4][6]; // corner rays in padded index coordinates: point, direction
+    __shared__ float cdir[4][3];     // corner rays: direction
+    __shared__ float4 cross[4];      // on centred slice k of K: P = x + y k, Q = z + w k
     __shared__ int red[2][kMaxBlock / 64];
     const int tid = threadIdx.x;
     // XCD-aware order. Workgroups are dealt to the 8 XCDs in turn, so dispatch slot hw runs
@@ -307,15 +314,13 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
     const int a = (int)tz % A;
     const size_t b = tz / A;
     const int Wp = nx + 2 * kPad, Hp = ny + 2 * kPad, Dp = nz + 2 * kPad;
+    // the corner ray of lanes 0..3
+    const double cu = (double)((tid & 1) ? min(iu0 + 15, U - 1) : iu0);
+    const double cv = (double)((tid & 2) ? min(iv0 + 15, V - 1) : iv0);
     if (tid < 4) {
         const FwdGeom &g = geo[a];
-        const int cu = (tid & 1) ? min(iu0 + 15, U - 1) : iu0;
-        const int cv = (tid & 2) ? min(iv0 + 15, V - 1) : iv0;
-        for (int d = 0; d < 3; ++d) {
-            const double q = g.org[d] + (double)cu * g.du[d] + (double)cv * g.dv[d];
-            cl[tid][d] = (float)(g.src[d] + (double)kPad);
-            cl[tid][3 + d] = (float)(q - g.src[d]);
-        }
+        for (int d = 0; d < 3; ++d)
+            cdir[tid][d] = (float)(g.org[d] + cu * g.du[d] + cv * g.dv[d] - g.src[d]);
     }
     March3 p{};
     if (live) p = march_params(geo[a], nx, ny, nz, iu, iv, Wp, Hp, Dp);
@@ -340,12 +345,12 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
     __syncthreads(); // corner rays
     // march axis K: the largest component of the corner rays' summed direction
     float ds[3];
-    for (int d = 0; d < 3; ++d) ds[d] = cl[0][3 + d] + cl[1][3 + d] + cl[2][3 + d] + cl[3][3 + d];
+    for (int d = 0; d < 3; ++d) ds[d] = cdir[0][d] + cdir[1][d] + cdir[2][d] + cdir[3][d];
     const int K = fabsf(ds[0]) >= fabsf(ds[1]) ? (fabsf(ds[0]) >= fabsf(ds[2]) ? 0 : 2)
                                                : (fabsf(ds[1]) >= fabsf(ds[2]) ? 1 : 2);
     const float sgn = ds[K] > 0.0f ? 1.0f : -1.0f;
     bool slab_ok = K != F;
-    for (int c = 0; c < 4; ++c) slab_ok = slab_ok && cl[c][3 + K] * sgn > 0.0f;
+    for (int c = 0; c < 4; ++c) slab_ok = slab_ok && cdir[c][K] * sgn > 0.0f;
     const int Q = 3 - K - F; // the third axis (when K != F)
     // padded index = centred coordinate + E / 2 on each axis
     const int cK = pick(Wp, Hp, Dp, K) / 2, cP = Ef / 2, cQ = pick(Wp, Hp, Dp, Q) / 2;
@@ -366,39 +371,37 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
         return sample3d<SI>(R, fmaf(jf, tf, mf), fmaf(jf, tm, mm), fmaf(jf, tl, ml), Ef, Em,
                             cofs, sM, sL, sML);
     };
-    // crossings of the corner rays with the plane of padded index k along K: the smallest and
-    // largest padded indices along P and Q
+    // crossings of the corner rays with centred slice k along K: the smallest and largest padded
+    // indices along P and Q
     auto section = [&](float k, float &p0, float &p1, float &q0, float &q1) {
         p0 = q0 = INFINITY;
         p1 = q1 = -INFINITY;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const float t = (k - cl[c][K]) * __builtin_amdgcn_rcpf(cl[c][3 + K]);
-            const float pc = fmaf(t, cl[c][3 + F], cl[c][F]), qc = fmaf(t, cl[c][3 + Q], cl[c][Q]);
+            const float4 l = cross[c];
+            const float pc = fmaf(k, l.y, l.x), qc = fmaf(k, l.w, l.z);
             p0 = fminf(p0, pc);
             p1 = fmaxf(p1, pc);
             q0 = fminf(q0, qc);
             q1 = fmaxf(q1, qc);
         }
+        p0 += (float)cP, p1 += (float)cP, q0 += (float)cQ, q1 += (float)cQ;
     };
     // lower-tap K range of the workgroup's samples
     int klo = 0x7fffffff, khi = -0x7fffffff - 1;
     if (slab_ok) {
+        if (tid < 4) {
+            double pc, sp, qc, sq;
+            cone3d::line_on_planes(geo[a], cu, cv, K, F, (double)(cK - kPad), pc, sp);
+            cone3d::line_on_planes(geo[a], cu, cv, K, Q, (double)(cK - kPad), qc, sq);
+            cross[tid] = make_float4((float)(pc + (double)(kPad - cP)), (float)sp,
+                                     (float)(qc + (double)(kPad - cQ)), (float)sq);
+        }
         if (n > 0) {
-            bool in = true;
-            for (int e = 0; e < 2; ++e) { // the first and the last sample
-                const float je = e ? jend - 1.0f : p.j0;
-                const float pk = fmaf(je, tK, mK);
-                const int kk = floor_i32(pk) + cK;
-                klo = min(klo, kk);
-                khi = max(khi, kk);
-                float p0, p1, q0, q1;
-                section(pk + (float)cK, p0, p1, q0, q1);
-                const float pp = fmaf(je, tP, mP) + (float)cP, pq = fmaf(je, tQ, mQ) + (float)cQ;
-                constexpr float tol = 0.5f * kBoxMargin;
-                in = in && pp >= p0 - tol && pp <= p1 + tol && pq >= q0 - tol && pq <= q1 + tol;
-            }
-            if (!in) klo = -0x40000000; // marks the workgroup for the global path
+            const int k0 = floor_i32(fmaf(p.j0, tK, mK)) + cK;
+            const int k1 = floor_i32(fmaf(jend - 1.0f, tK, mK)) + cK;
+            klo = min(k0, k1);
+            khi = max(k0, k1);
         }
         for (int off = 32; off > 0; off >>= 1) {
             klo = min(klo, __shfl_xor(klo, off, 64));
@@ -411,7 +414,6 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
         __syncthreads();
         klo = min(min(red[0][0], red[0][1]), min(red[0][2], red[0][3]));
         khi = max(max(red[1][0], red[1][1]), max(red[1][2], red[1][3]));
-        slab_ok = klo != -0x40000000;
     }
     if (!__builtin_amdgcn_readfirstlane((int)slab_ok)) {
         while (jf < jend) {
@@ -432,7 +434,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_fwd3d(const typename SI::raw *__r
         // shift give exact quotients of the numbers of the box's quads and rows
         int bP0 = 0, bQ0 = 0, bN = 0, bRN = 0, bRQ = 0;
         auto plan_slabs = [&](int si0) {
-            const float k = (float)first_slice(si0 + (tid & 63));
+            const float k = (float)(first_slice(si0 + (tid & 63)) - cK);
             float p0, p1, q0, q1, u0, u1, v0, v1;
             section(k, p0, p1, q0, q1);
             section(k + (float)kSlab, u0, u1, v0, v1);

@@ -197,6 +197,17 @@ __host__ __device__ inline Ray3 setup_ray3(const FwdGeom &a, int64_t nx, int64_t
     return r;
 }
 
+// The line from the source through panel position (iu, iv) on the planes across axis K: its
+// coordinate along axis d on plane k (voxel coordinates) is at + (k - k0) slope. Evaluated at a
+// plane k0 inside the volume, both are of the volume's size however far away the source is.
+__host__ __device__ inline void line_on_planes(const FwdGeom &a, double iu, double iv, int K, int d,
+                                               double k0, double &at, double &slope) {
+    const double eK = a.org[K] + iu * a.du[K] + iv * a.dv[K] - a.src[K];
+    const double ed = a.org[d] + iu * a.du[d] + iv * a.dv[d] - a.src[d];
+    slope = ed / eK;
+    at = a.src[d] + (k0 - a.src[K]) * slope;
+}
+
 } // namespace cmi::cone3d
 
 #pragma float_control(pop)
