@@ -1066,10 +1066,14 @@ __global__ __launch_bounds__(kMaxBlock) void k_adj2d_tile(unsigned long long *__
             // p = fma(k, slope, mc) on row k - kd
             const bool up = slope >= 0.0f;
             const int kd = rowf - r0 - (up ? 1 : 0);
-            // rows with both terms whose cells reach the tile
-            const float inv = __builtin_amdgcn_rcpf(up ? fmaxf(m, 1e-6f) : fminf(-m, -1e-6f));
+            // rows with both terms whose cells reach the tile. Below a slope of 2^-21 a ray moves
+            // less than a quarter of a column over any image (at most 2^20 rows): it is walked at
+            // that slope, rounded outwards by all of that.
+            constexpr float flat = 0x1p-21f;
+            const float margin = m < flat ? 0.25f / flat : kT2Margin;
+            const float inv = __builtin_amdgcn_rcpf(up ? fmaxf(m, flat) : fminf(-m, -flat));
             const float e0 = (cmin - mc) * inv, e1 = (cmax - mc) * inv;
-            const float klo = fminf(e0, e1) - kT2Margin, khi = fmaxf(e0, e1) + kT2Margin;
+            const float klo = fminf(e0, e1) - margin, khi = fmaxf(e0, e1) + margin;
             const int rlo = max(max(first + 1, 0), (int)ceilf(fmaxf(klo, -1e9f)) - kd);
             const int rhi = min(min(first + n - 1, kT2Rows - 1), (int)floorf(fminf(khi, 1e9f)) - kd);
             if (rlo <= rhi) {

@@ -54,3 +54,22 @@ def test_forward_3d_far_sources(oracle, gpu, dso):
     ref = oracle.fwd3d(geom, vol)
     assert rel_l2(got, ref) <= RTOL_L2
     assert np.abs(got.double().cpu().numpy() - ref).max() <= MAXABS * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("dso,gap", [(2.0e6, 4e-4), (8.0e5, 3e-4), (5.0e7, 1e-4), (5.0e8, 2e-5)])
+@pytest.mark.parametrize("cell", [0, 1])
+def test_adjoint_rays_along_tile_edges(oracle, gpu, dso, gap, cell):
+    """A ray almost along each axis, `gap` of a texel before (and after) the first texel of a tile
+    of 64 columns: all of its rows add that share to the texels before, which are another tile's.
+    Terms are rounded to 2^-19 of the largest (0.95e-6 each, three to a texel and ray, two rays) and
+    positions to 2e-6 (FP32 at 40 texels from the centre): 1e-5, 6e-6 of the largest sum."""
+    rec = fan(1200, 2, 2, dso, 2.0 * dso, du=2.0 * (1.0 - 2.0 * gap), offset=(-40.0, -40.0),
+              arc=np.pi)                    # world (0, 0) lies between texels 639 and 640 then
+    geom = as_fan_geometry(rec)
+    y = np.zeros((2, 2))
+    y[:, cell] = 1.0
+    ref = oracle.adj2d(rec, y)
+    got = cm.adjoint(torch.tensor(y, dtype=torch.float32, device=gpu), geom)
+    small = (ref > 0.2 * gap) & (ref < 5 * gap)
+    assert small.sum() > 1000               # texels that take the small share alone
+    assert np.abs(got.double().cpu().numpy() - ref).max() <= 6e-6 * np.abs(ref).max()
