@@ -172,9 +172,10 @@ __device__ __forceinline__ float bp2d_tile(rsrc_t R, TAB tab, int A, int D, int 
 // not fit (or with a corner with W <= 0) is sampled from global memory instead, with the same
 // arithmetic, after the others.
 //
-// A sample's LDS address is two fma: byte strides and the slot's offset are held as FP32 subnormals,
-// n 2^-149, whose bit pattern is the integer n, so that products with the integral floors and their
-// sums are exact below 2^23 and the sum's bits are the address; fractions are p - floor(p). On
+// A sample's LDS address is two fma: byte strides and the slot's offset are held as FP32 numbers n
+// 2^-149. Such a number's bit pattern is the integer n below 2^24, and multiples of 4 are exact below
+// 2^26, so that products with the integral floors and their sums are exact (the panels' rows reach
+// 2^16, at 304 bytes each) and the sum's bits are the address; fractions are p - floor(p). On
 // gfx950 these issue at the full rate, where a conversion to an integer, its offset, the 24-bit
 // product and v_fract_f32 each take almost two slots.
 constexpr int kFootW = 64;                        // staged columns per row
@@ -184,6 +185,8 @@ constexpr int kFootW = 64;                        // staged columns per row
 constexpr int kFootCols = 76;
 constexpr int kFootRows = 60;
 constexpr int kFootFloats = kFootCols * kFootRows;
+// addresses before the slot's offset: rows and columns of panels of up to 2^16 cells a side
+static_assert(4ll * (kFootCols + 1) * (65536 + 2 * kPadDet) < 1ll << 26, "exact as n 2^-149");
 
 // The staged footprint, one workgroup-shared array (18 KB) for every instantiation a kernel uses, so
 // a kernel that dispatches between modes allocates it once.
@@ -192,7 +195,7 @@ static __shared__ __align__(16) float foot_lds[kFootFloats];
 // Angles whose footprints one pass of a wavefront evaluates: 8 lanes (the tile's corners) each.
 constexpr int kGroup = 8;
 
-// i 2^-149, opaque in a vector register.
+// i 2^-149 for |i| < 2^24, opaque in a vector register.
 __device__ __forceinline__ float subnormal(int i) {
     float f = __int_as_float(i < 0 ? -i | (int)0x80000000 : i);
     asm("" : "+v"(f));
@@ -202,7 +205,7 @@ __device__ __forceinline__ float subnormal(int i) {
 // A staged footprint: the sample at the integral lower taps (iu, iv) lies at the LDS byte address
 // fma(iv, row, fma(iu, col, ofs)), its pair on the next row kFootCols floats further.
 struct Foot {
-    float row, col, ofs; // byte strides and offset, as subnormals
+    float row, col, ofs; // byte strides and offset, times 2^-149
 };
 
 // The four taps of a bilinear sample: rows v and v + 1, columns u and u + 1.
@@ -325,7 +328,7 @@ __device__ __forceinline__ void bp3d_angles(rsrc_t R, TAB M, int A, int U, int V
         if (a + 1 < A) ahead(a + 1);
         if (staged) {
             __syncthreads();
-            from_foot(M + 12 * a, Foot{row, col, subnormal(at0)});
+            from_foot(M + 12 * a, Foot{row, col, __builtin_amdgcn_ldexpf((float)at0, -149)});
         }
     }
     if (!missed) return;

@@ -73,3 +73,39 @@ def test_adjoint_rays_along_tile_edges(oracle, gpu, dso, gap, cell):
     small = (ref > 0.2 * gap) & (ref < 5 * gap)
     assert small.sum() > 1000               # texels that take the small share alone
     assert np.abs(got.double().cpu().numpy() - ref).max() <= 6e-6 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("columns", [0, 1])
+@pytest.mark.parametrize("v0", [100, 27600, 55300, 65300])
+def test_served_tall_panels(gpu, columns, v0):
+    """Rows far down a tall panel are sampled as the same rows of a short one: the staged
+    footprints' LDS addresses hold for every panel the server accepts. Positions are quarters of a
+    pixel and every weight is exact, so both give the same bits."""
+    from curadon_amd import _lib
+    A, U, V, n = 3, 40, 65536, 24
+    gen = torch.Generator().manual_seed(v0)
+    rows = torch.randint(0, 256, (A, 200, U), generator=gen).float()
+
+    def served(first, height):
+        panel = torch.zeros((A, height + 4, U + 4))
+        panel[:, 2 + first:202 + first, 2:-2] = rows
+        panel = panel.to(gpu)
+        # (U, V, W) = (x + .25 + 12 + a, y + z + .5 + first + 90 - a, 1)
+        M = torch.zeros((A, 3, 4))
+        M[:, 0, 0], M[:, 0, 3] = 1.0, torch.arange(A) + 17.25
+        M[:, 1, 1], M[:, 1, 2], M[:, 1, 3] = 1.0, 1.0, first + 90.5 - torch.arange(A)
+        M[:, 2, 3] = 1.0
+        M = M.to(gpu)
+        vol = torch.zeros((n, n, n), device=gpu)
+        job = _lib.BPJob(kind=_lib.JOB_CONE3D, mode=0, columns=columns, sino=panel.data_ptr(),
+                         table=M.data_ptr(), volume=vol.data_ptr(), nx=n, ny=n, nz=n, nu=U,
+                         nv=height, nangles=A)
+        job.tile_end = _lib.bp_job_tiles(job)
+        server = _lib.Server(gpu.index or 0, 4)
+        server.backproject([job], torch.float32, torch.float32)
+        torch.cuda.synchronize()
+        return vol
+
+    tall, short = served(v0, V), served(0, 200)
+    assert float(short.min()) > 0.0
+    assert torch.equal(tall, short)
