@@ -381,7 +381,10 @@ __device__ __forceinline__ void bp3d_run(rsrc_t R, TAB M, int A, int U, int V, f
     // at_column(iu) gives taps(iv), the taps between columns iu and iu + 1 and rows iv and iv + 1.
     // kBatch voxels' taps are read before the first is used.
     constexpr int kBatch = 4;
-    auto run = [&](TAB m, auto &&at_column) {
+    // DROP: a voxel behind the source has no sample at all (a weight of 0 would let infinities and
+    // NaN of the panel through). Staged tiles lie before the source.
+    auto run = [&](TAB m, auto drop, auto &&at_column) {
+        constexpr bool DROP = decltype(drop)::value;
         float Uh = fmaf(m[0], hx, fmaf(m[2], hz, m[3]));
         float Wh = fmaf(m[8], hx, fmaf(m[10], hz, m[11]));
         float Vh = fmaf(m[4], hx, fmaf(m[5], hy, fmaf(m[6], hz, m[7])));
@@ -390,7 +393,8 @@ __device__ __forceinline__ void bp3d_run(rsrc_t R, TAB M, int A, int U, int V, f
             return MATCHED ? (Wh > 0.0f ? w : 0.0f) : w;
         };
         auto add = [&](int y, const Taps &t, float fu, float fv, float w) {
-            const float s = bilerp(t, fu, fv);
+            float s = bilerp(t, fu, fv);
+            if (DROP && MATCHED) s = w > 0.0f ? s : 0.0f;
             acc[y] = (MATCHED || FDK) ? fmaf(s, w, acc[y]) : acc[y] + s;
         };
         if constexpr (YINV) {
@@ -446,13 +450,13 @@ __device__ __forceinline__ void bp3d_run(rsrc_t R, TAB M, int A, int U, int V, f
         R, M, A, U, V, tx, ty, tz, (float)(kTileX - 1), (float)(kTileY - 1),
         (float)(kTileZ<YINV> - 1),
         [&](TAB m, const Foot &f) {
-            run(m, [&](float iu) {
+            run(m, std::false_type{}, [&](float iu) {
                 const float ofs = fmaf(iu, f.col, f.ofs);
                 return [=](float iv) { return foot_taps(__float_as_uint(fmaf(iv, f.row, ofs))); };
             });
         },
         [&](TAB m, int base) {
-            run(m, [&](float iu) {
+            run(m, std::bool_constant<!YINV>{}, [&](float iu) {
                 const int col = base + (int)iu;
                 return [=](float iv) {
                     const int o = col + __mul24((int)iv, Up);

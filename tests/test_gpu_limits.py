@@ -109,3 +109,23 @@ def test_served_tall_panels(gpu, columns, v0):
     tall, short = served(v0, V), served(0, 200)
     assert float(short.min()) > 0.0
     assert torch.equal(tall, short)
+
+
+@pytest.mark.parametrize("mode", ["matched", "fdk"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_backward_3d_nothing_behind_the_source(gpu, mode, value):
+    """Voxels behind the source (W <= 0, tilted orbit) take nothing from a projection, whatever its
+    pixels hold."""
+    rec = cone(26, 40, 36, 1, 5.0, 30.0, angles=np.array([[0.5], [0.6], [0.3]]))
+    geom = as_cone_geometry(rec)
+    M = np.asarray(geom.bp_matrices(mode), dtype=np.float64).reshape(3, 4)
+    n = rec.vol_shape
+    z, y, x = np.meshgrid(*[np.arange(int(k)) - (int(k) - 1) / 2 for k in n], indexing="ij")
+    W = M[2, 0] * x + M[2, 1] * y + M[2, 2] * z + M[2, 3]
+    assert abs(M[2, 1]) > 1e-3                       # not the layout of a circular orbit
+    behind = torch.tensor(W < -1e-4 * np.abs(W).max(), device=gpu)
+    assert 1000 < int(behind.sum()) < behind.numel() - 1000
+    sino = torch.full(tuple(geom.sinogram_shape()), value, device=gpu)
+    got = cm.backward(sino, geom, mode=mode)
+    assert not bool(got[~behind].isfinite().all())   # what lies before it does take them
+    assert bool((got[behind] == 0).all())
