@@ -66,6 +66,9 @@ struct cmi_plan2d {
     // for circular plans, with the view's 1 / |u| for plans from views); infinite when a
     // source lies inside the image's bounding box
     double bt_bound[2] = {INFINITY, INFINITY};
+    // detector cells per pixel at the image's centre, mean over the projections (0 where a
+    // projection's source lies inside the image's bounding box)
+    double cells_per_pixel = 0.0;
 };
 
 namespace {
@@ -1162,9 +1165,9 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // al; cells outside the row read zero), times 1/du (circular plans; the view's 1/|u| is part of
 // wt for plans from views). So sino[a][c] = sum_p (those weights) v[p], with k_bp2d's FP32
 // positions and weights.
-// A workgroup owns a segment of kGS detector cells of one projection and gathers it. The pixels
-// whose terms reach the segment's cells are those with u in [c0 - 1, c0 + kGS): a wedge from
-// the source between the lines u = c0 - 1 and u = c0 + kGS (u is a ratio of two functions
+// A workgroup owns a segment of GS detector cells of one projection and gathers it. The pixels
+// whose terms reach the segment's cells are those with u in [c0 - 1, c0 + GS): a wedge from
+// the source between the lines u = c0 - 1 and u = c0 + GS (u is a ratio of two functions
 // affine in the pixel). The workgroup marches through the image along the axis K (rows or
 // columns) that the segment's central line follows most closely, in chunks of kGSlab lines;
 // per line the wedge is the interval between the two boundary lines' crossings (kGMargin of a
@@ -1173,10 +1176,10 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // (row-major for rows, transposed for columns), so that it reads runs of consecutive pixels. All
 // lines of a chunk are walked over the width of its widest interval, their starts moved back
 // where that would leave the image: pixels outside the wedge have no cell in the segment and add
-// nothing. Depth and detector coordinate are affine in the pixel, so they are one sum each of the
-// lane's share (its pixel number along the line) and the line's (evaluated in FP64 by the lane
-// that holds the line, and read from it). Every pixel adds its terms that fall inside the segment
-// to kGS + 2 LDS cells with integer atomics. A segment whose boundary lines meet the lines at
+// nothing. Depth d and d u, u the cell coordinate from the segment's start on, are affine in the
+// pixel, so they are one sum each of the lane's share (its pixel number along the line) and the
+// line's (evaluated in FP64 by the lane that holds the line, and read from it). Every pixel adds its terms that fall inside the segment
+// to GS + 2 LDS cells with integer atomics. A segment whose boundary lines meet the lines at
 // grazing angles walks whole lines.
 // Bound by VALU issue. Walking the chunk's pixels as one flat list, which filled the lanes (0.94
 // against 0.73 at 0.67 pixels per cell) but gave every pixel an index walk, a test against its
@@ -1187,11 +1190,20 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // plan's bound on wt (times 1/du) over the image and all projections, so |term| <= 2^kGBits
 // and a 32-bit LDS cell holds the sum of up to 2^(31 - kGBits) - 1 terms. A pixel adds at most
 // one term to a cell, so the cells are moved into 64-bit registers (one per thread of the first
-// kGS) and cleared before the pixel visits since the last such drain could pass that count.
+// GS) and cleared before the pixel visits since the last such drain could pass that count.
 // Integer sums are exact: the result does not depend on the order of the additions. Each
 // segment is written once, in the sinogram's storage type.
-constexpr int kGS = 64;                                      // detector cells per segment
-constexpr int kGC = kGS + 2;                                 // LDS cells: c0 - 1 .. c0 + kGS
+// Detector cells per segment: kGSFine where a pixel has at least kGFine cells, so that the walk's
+// lines are still about a wavefront wide, or kGFineFew where that leaves fewer than kGFineMany
+// workgroups an image; else kGS, which gives more workgroups and, at one pixel per cell, lines that
+// just fit a wavefront. 512^2 x 180, calls, us with kGS and with kGSFine (walking the chunk's pixels
+// as one flat list: third): 10 cells per pixel 351, 115 (161), 4 cells 168, 86 (110), 2 cells 102,
+// 96 (97), 1 cell 84, 140 (93); 200^2 x 181 (543 workgroups) of 2 cells 39, 42 (41), 128^2 x 180
+// (540) of 4 cells 39, 39 (40). kGS 64: 5 % more at one cell per pixel of parallel rays, 2 % less at
+// 1.5.
+constexpr int kGS = 62, kGSFine = 256;
+constexpr double kGFine = 1.75, kGFineFew = 4.0;
+constexpr uint64_t kGFineMany = 1024;
 constexpr int kGSlab = 64;                                   // image lines per chunk
 constexpr int kGBits = 18;                                   // a term's bound: 2^kGBits units
 constexpr int kGBudget = (1 << (31 - kGBits)) - 1;           // pixel visits between drains
@@ -1199,6 +1211,7 @@ constexpr int kGBatch = 4;           // lines per wavefront whose loads are in f
 constexpr float kGMargin = 0.0625f;  // pixels around the boundary lines' crossings
 static_assert(kGSlab == 64, "one lane per line");
 static_assert(kGSlab / 4 * kMaxBlock <= kGBudget, "no drain within a chunk's step");
+static_assert(kGSFine <= kMaxBlock, "one owned cell per thread");
 
 // Largest |v| of each image of a batch, in kAdjParts partial maxima per image.
 template <class SV>
@@ -1241,7 +1254,7 @@ __device__ __forceinline__ void bpT_line(const float4 *__restrict__ tab, int a, 
     }
 }
 
-template <class SV, class SS, int WPOW, bool VIEWS>
+template <class SV, class SS, int WPOW, bool VIEWS, int GS>
 __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restrict__ sino,
                                                      const typename SV::raw *__restrict__ staged,
                                                      const float4 *__restrict__ tab,
@@ -1249,10 +1262,10 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
                                                      int nx, int ny, int D, int A, float sx,
                                                      float sy, float ox, float oy, float inv_du,
                                                      float half_d) {
-    __shared__ unsigned int cells[kGC]; // cell c0 - 1 + i at i
+    __shared__ unsigned int cells[GS + 2]; // cell c0 - 1 + i at i
     const int tid = threadIdx.x, lane = tid & 63;
     const int a = (int)(blockIdx.x % (unsigned)A);
-    const int c0 = (int)(blockIdx.x / (unsigned)A) * kGS;
+    const int c0 = (int)(blockIdx.x / (unsigned)A) * GS;
     const size_t b = blockIdx.y;
     const float uoff = half_d - 0.5f;
     // fixed-point scale 2^18 / (max|v| bound) in two factors: a power of two that brings max|v|
@@ -1277,7 +1290,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
     int rows;
     {
         double n[3];
-        index_line((double)c0 + 0.5 * kGS, n);
+        index_line((double)c0 + 0.5 * GS, n);
         rows = fabs(n[0]) >= fabs(n[1]) ? 1 : 0;
         rows = __builtin_amdgcn_readfirstlane(rows);
     }
@@ -1294,7 +1307,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
     double sgn[2];
     for (int e = 0; e < 2; ++e) {
         double n[3];
-        index_line(e ? (double)(c0 + kGS) : (double)(c0 - 1), n);
+        index_line(e ? (double)(c0 + GS) : (double)(c0 - 1), n);
         const double nF_ = rows ? n[0] : n[1], nK_ = rows ? n[1] : n[0];
         sgn[e] = nF_;
         if (!(fabs(nF_) >= 0.25 * sqrt(nF_ * nF_ + nK_ * nK_)) || nF_ == 0.0) {
@@ -1312,21 +1325,22 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
                                   (rows ? (size_t)0 : (size_t)Wp * Hp) +
                                   (size_t)kPad * (rows ? Wp : Hp) + kPad;
     const int strK = rows ? Wp : Hp;
-    for (int i = tid; i < kGC; i += kMaxBlock) cells[i] = 0u;
+    for (int i = tid; i < GS + 2; i += kMaxBlock) cells[i] = 0u;
     long long own = 0;
     auto drain = [&]() {
         lds_barrier();
-        if (tid < kGS) {
+        if (tid < GS) {
             own += (long long)(int)cells[tid + 1];
             cells[tid + 1] = 0u;
         }
         __syncthreads();
     };
-    // depth and detector coordinate as affine forms of the pixel (f, k) along (F, K): cf f + ck k
-    // + c1; cell coordinate relative to the segment's first LDS cell, w eta + cu
-    double dc[3], ec[3], L, cu, wmul;
+    // depth d and e = d u as affine forms of the pixel (f, k) along (F, K), cf f + ck k + c1; u the
+    // cell coordinate from the segment's first LDS cell on, so that FP32 rounds no larger numbers
+    // than those
+    double dc[3], ec[3], L, wmul;
     {
-        double dx, dy, dz, ex, ey, ez;
+        double dx, dy, dz, ex, ey, ez, cu;
         if (VIEWS) {
             const float4 m0 = tab[3 * a], m1 = tab[3 * a + 1];
             dx = m0.x, dy = m0.y, dz = m0.z;
@@ -1339,12 +1353,13 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
             L = m.z, cu = uoff, wmul = inv_du;
         }
         cu -= (double)(c0 - 1);
+        ex = L * ex + cu * dx, ey = L * ey + cu * dy, ez = L * ez + cu * dz;
         dc[2] = dx * bx + dy * by + dz, ec[2] = ex * bx + ey * by + ez;
         dx *= sx, ex *= sx, dy *= sy, ey *= sy;
         dc[0] = rows ? dx : dy, dc[1] = rows ? dy : dx;
         ec[0] = rows ? ex : ey, ec[1] = rows ? ey : ex;
     }
-    const float vL = (float)L, vcu = (float)cu;
+    const float vL = (float)L;
     const float s1 = ldexpf(1.0f, max(min(-vexp, 127), -126)); // (max|v| below 2^-127 scales to less)
     const float s2 = (float)(rest * wmul * ldexp(1.0, -vexp - max(min(-vexp, 127), -126)));
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1392,12 +1407,11 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
                     const float vs = val[q] * s1 * s2;
                     const float rd = __builtin_amdgcn_rcpf(
                         dp + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dl), l)));
-                    const float eta =
-                        ep + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(el), l));
-                    const float w = vL * rd;
-                    const float u = fmaf(w, eta, vcu);
+                    const float u = rd *
+                        (ep + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(el), l)));
                     const int i = floor_i32(u);
-                    if ((unsigned)i > (unsigned)kGS || vs == 0.0f) continue;
+                    if ((unsigned)i > (unsigned)GS || vs == 0.0f) continue;
+                    const float w = vL * rd;
                     const float t = vs * (WPOW == 2 ? w * w : w);
                     const float t1 = t * __builtin_amdgcn_fractf(u), t0 = t - t1;
                     atomicAdd(&cells[i], (unsigned)round_i32(t0));
@@ -1407,7 +1421,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
         }
     }
     lds_barrier();
-    if (tid < kGS) {
+    if (tid < GS) {
         own += (long long)(int)cells[tid + 1];
         const int c = c0 + tid;
         if (c < D) {
@@ -1557,30 +1571,34 @@ cmi_status finish_plan2d(std::unique_ptr<cmi_plan2d> p, const std::vector<AngleG
                               (ny - 1.0 - ny / 2.0) * p->g.sy + p->g.oy + 0.5};
         double b1 = 0.0, b2 = 0.0;
         bool ok = true;
+        // depth, magnification and 1 / |u| of projection a at (x, y)
+        auto at = [&](int64_t a, double x, double y, double &w, double &scale) {
+            double depth, L;
+            if (!meta.empty()) {
+                const float4 m = meta[a];
+                depth = (double)m.x * x - (double)m.y * y + (double)m.w;
+                L = m.z;
+                scale = 1.0 / p->g.du;
+            } else {
+                const float4 m0 = bpv[3 * a];
+                depth = (double)m0.x * x + (double)m0.y * y + (double)m0.z;
+                L = m0.w;
+                scale = bpv[3 * a + 2].x;
+            }
+            w = std::fabs(L) / depth;
+            return depth > 0.0;
+        };
+        double w, scale, cells = 0.0;
         for (int64_t a = 0; a < A && ok; ++a) {
-            for (int c = 0; c < 4; ++c) {
-                const double x = xs[c & 1], y = ys[c >> 1];
-                double depth, L, scale;
-                if (!meta.empty()) {
-                    const float4 m = meta[a];
-                    depth = (double)m.x * x - (double)m.y * y + (double)m.w;
-                    L = m.z;
-                    scale = 1.0 / p->g.du;
-                } else {
-                    const float4 m0 = bpv[3 * a];
-                    depth = (double)m0.x * x + (double)m0.y * y + (double)m0.z;
-                    L = m0.w;
-                    scale = bpv[3 * a + 2].x;
-                }
-                if (!(depth > 0.0)) {
-                    ok = false;
-                    break;
-                }
-                const double w = std::fabs(L) / depth;
+            for (int c = 0; c < 4 && ok; ++c) {
+                ok = at(a, xs[c & 1], ys[c >> 1], w, scale);
                 b1 = std::max(b1, w * scale);
                 b2 = std::max(b2, w * w * scale);
             }
+            (void)at(a, 0.5 * (xs[0] + xs[1]), 0.5 * (ys[0] + ys[1]), w, scale);
+            cells += w * scale;
         }
+        if (ok) p->cells_per_pixel = cells / (double)A * std::sqrt(p->g.sx * p->g.sy);
         if (ok && b1 > 0.0 && std::isfinite(b2)) {
             p->bt_bound[0] = 1.01 * b1;
             p->bt_bound[1] = 1.01 * b2;
@@ -2008,7 +2026,12 @@ CMI_API cmi_status cmi_backward_2d_transpose(const cmi_plan2d *plan, void *sinog
     const int nx = (int)plan->g.nx, ny = (int)plan->g.ny, D = (int)plan->g.D, A = (int)plan->A;
     const size_t img = (size_t)nx * ny;
     const int Wp = nx + 2 * kPad, Hp = ny + 2 * kPad;
-    const uint64_t nseg = (uint64_t)(D + kGS - 1) / kGS;
+    // (not by the batch: an image's bits do not depend on the others)
+    const bool fine = plan->cells_per_pixel >=
+                      ((uint64_t)A * ((D + kGSFine - 1) / kGSFine) >= kGFineMany ? kGFine
+                                                                                 : kGFineFew);
+    const int gs = fine ? kGSFine : kGS;
+    const uint64_t nseg = (uint64_t)(D + gs - 1) / gs;
     if ((uint64_t)A * nseg * kMaxBlock >= (1ull << 32) || batch > 65535)
         return fail(CMI_ERR_INVALID_ARGUMENT,
                     "backward_2d_transpose: too many projections, cells or images for one "
@@ -2032,8 +2055,13 @@ CMI_API cmi_status cmi_backward_2d_transpose(const cmi_plan2d *plan, void *sinog
                            dim3(kMaxBlock), 0, s, (const RV *)volume, img, parts);
         const bool views = plan->d_bpv != nullptr;
         const bool fbp = weighting == CMI_BP2D_FBP;
-        auto kern = views ? (fbp ? k_bpT2d<SV, SS, 2, true> : k_bpT2d<SV, SS, 1, true>)
-                          : (fbp ? k_bpT2d<SV, SS, 2, false> : k_bpT2d<SV, SS, 1, false>);
+        auto pick = [&](auto cells) {
+            constexpr int GS = decltype(cells)::value;
+            return views ? (fbp ? k_bpT2d<SV, SS, 2, true, GS> : k_bpT2d<SV, SS, 1, true, GS>)
+                         : (fbp ? k_bpT2d<SV, SS, 2, false, GS> : k_bpT2d<SV, SS, 1, false, GS>);
+        };
+        auto kern = fine ? pick(std::integral_constant<int, kGSFine>{})
+                         : pick(std::integral_constant<int, kGS>{});
         // projections fastest: neighbouring workgroups gather overlapping wedges
         hipLaunchKernelGGL(kern, dim3((unsigned)(A * nseg), (unsigned)batch), dim3(kMaxBlock),
                            0, s, (typename SS::raw *)sinogram, (const RV *)scratch,

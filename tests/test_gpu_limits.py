@@ -129,3 +129,31 @@ def test_backward_3d_nothing_behind_the_source(gpu, mode, value):
     got = cm.backward(sino, geom, mode=mode)
     assert not bool(got[~behind].isfinite().all())   # what lies before it does take them
     assert bool((got[behind] == 0).all())
+
+
+@pytest.mark.parametrize("views", [False, True])
+@pytest.mark.parametrize("ny,nx,A,D,du", [
+    (40, 30, 7, 255, 0.25),     # a segment of 256 cells, less one
+    (40, 30, 7, 257, 0.25),     # and one cell over
+    (70, 66, 7, 1100, 0.1),     # lines of a few pixels in segments of ten cells a pixel
+    (20, 150, 7, 600, 0.24),    # either side of the lines between the segments' sizes
+    (20, 150, 7, 600, 0.26),
+    (20, 150, 400, 600, 0.5),
+    (150, 20, 400, 400, 0.65),
+])
+def test_backward_transpose_fine_cells(oracle, gpu, views, ny, nx, A, D, du):
+    """FP32 rounds a position of up to D / 2 cells by 2^-24 of that at most in each of its about
+    four operations, and a position's error is its weights' (0.58 in the mean square)."""
+    n = max(ny, nx)
+    more = {"det_offset": 0.25, "exact_geometry": True} if views else {}
+    geom = cm.FanGeometry(DSD=3.0 * n, DSO=2.0 * n, angles=np.linspace(0, 6, A),
+                          vol_shape=(ny, nx), det_shape=D, det_spacing=1.5 * du, **more)
+    v = np.random.RandomState(nx).rand(ny, nx)
+    x = torch.tensor(v, dtype=torch.float32, device=gpu)
+    tol = max(RTOL_L2, 4 * (D / 2) * 2.0 ** -24 / 0.58)
+    for mode, wpow in (("reference", 1), ("fbp", 2)):
+        got = cm.backward_transpose(x, geom, mode=mode)
+        assert rel_l2(got, oracle.bp2d_T(geom, v, wpow=wpow)) <= tol
+    three = cm.backward_transpose(torch.stack([x, 2.0 * x, x.flip(0)]), geom)
+    one = cm.backward_transpose(x, geom)
+    assert torch.equal(three[0], one) and torch.equal(three[1], 2.0 * one)
