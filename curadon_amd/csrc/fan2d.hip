@@ -77,11 +77,6 @@ constexpr int kPad = 2;        // zero border of the staged image copies, in tex
 constexpr int kMaxBlock = 256; // threads per workgroup every kernel here is compiled for
 static_assert(kPad == kPadDet, "sinograms are staged with the backprojector's border");
 
-// Per-angle constants of the backprojector: (-sin, cos, DSD, DSO) (backward_2d.hpp:58-62).
-float4 bp2d_meta(double angle, double dso, double dsd) {
-    return make_float4((float)-std::sin(angle), (float)std::cos(angle), (float)dsd, (float)dso);
-}
-
 // ---------------------------------------------------------------- ray table ----------------
 
 __global__ __launch_bounds__(kMaxBlock) void k_ray_table(const AngleGeom *__restrict__ geo, int A,
@@ -1513,18 +1508,58 @@ void set_plan_shape(cmi_plan2d &p, int device, int vol_prec, const uint64_t vol_
     p.A = (int64_t)nangles;
 }
 
+// Whether angles a + k A / 4 are quarter turns of angle a with equal distances, to 1e-9: FP32 tables
+// hold no more.
+bool quarter_apart(const double *angles, const double *DSO, const double *DSD, int64_t A,
+                   int64_t a) {
+    const int64_t Q = A / 4;
+    for (int64_t k = 1; k < 4; ++k) {
+        const int64_t b = a + k * Q;
+        if (DSO[b] != DSO[a] || DSD[b] != DSD[a]) return false;
+        const double d =
+            std::remainder(angles[b] - angles[a] - (double)k * M_PI / 2.0, 2.0 * M_PI);
+        if (!(std::fabs(d) <= 1e-9)) return false;
+    }
+    return true;
+}
+
+// The backprojector's table of circular plans: (-sin, cos, DSD, DSO) per angle
+// (backward_2d.hpp:58-62). Where all angles come in quadruples of quarter turns,
+// so do its entries, exactly (angles written with some ten digits would round apart now and then):
+// the first quarter's sines and cosines exchanged. Entries that agree, or of which both are zero but
+// for roundoff (below 1e-13: added to half-integers times ones, they leave no trace), stay.
+void bp2d_table(const double *angles, const double *DSO, const double *DSD, int64_t A, float *t) {
+    bool turns = A % 4 == 0;
+    for (int64_t a = 0; a < A; ++a) {
+        t[4 * a] = (float)-std::sin(angles[a]);
+        t[4 * a + 1] = (float)std::cos(angles[a]);
+        t[4 * a + 2] = (float)DSD[a];
+        t[4 * a + 3] = (float)DSO[a];
+        turns = turns && (a >= A / 4 || quarter_apart(angles, DSO, DSD, A, a));
+    }
+    if (!turns) return;
+    auto turn = [](float &p, float q) {
+        if (!(p == q || (std::fabs(p) < 1e-13f && std::fabs(q) < 1e-13f))) p = q;
+    };
+    for (int64_t a = 0; a < A / 4; ++a)
+        for (int64_t k = 1; k < 4; ++k) { // (-sin, cos) of the angle turned by k quarters
+            float *m = t + 4 * (a + k * (A / 4));
+            const float x = t[4 * a], y = t[4 * a + 1];
+            turn(m[0], k == 1 ? -y : k == 2 ? -x : y);
+            turn(m[1], k == 1 ? x : k == 2 ? -y : -x);
+        }
+}
+
 // Whether the backprojection by quarter turns (k_bp2d_qt) applies: a square image with an even
 // side, unit pixels and no offset (the pixel centres, at (i - n/2) + 1/2 as the reference places
 // them, backward_2d.hpp:58-59, are then symmetric under quarter turns), angles in quadruples
-// a + k A/4 that are quarter turns apart with equal DSO and DSD, in the FP32 table too (entry
-// for entry the first quarter's sines and cosines exchanged; the zeros of one and the roundoff
-// of the other, below 1e-13, add to half-integers times ones without a trace), a padded detector
-// row at least as long as a staged segment, and every 16 x 16 tile's detector footprint within a
-// staged segment: the projection of a segment of length L at
-// depth >= DSO - r (r the largest pixel-centre radius) spans at most
+// a + k A/4 that are quarter turns apart with equal DSO and DSD (their table entries then are,
+// exactly: bp2d_table), a padded detector row at least as long as a staged segment, and every
+// 16 x 16 tile's detector footprint within a staged segment: the projection of a segment of length
+// L at depth >= DSO - r (r the largest pixel-centre radius) spans at most
 // L DSD / (DSO - r) sqrt(1 + (r / (DSO - r))^2) / du cells.
 bool quarter_turns(const fan2d::Scalars &g, const double *angles, const double *DSO,
-                   const double *DSD, int64_t A, const std::vector<float4> &meta) {
+                   const double *DSD, int64_t A) {
     if (g.nx != g.ny || g.nx % 2 != 0 || g.nx < 2 || g.sx != 1.0 || g.sy != 1.0 ||
         g.ox != 0.0 || g.oy != 0.0 || A % 4 != 0 || A < 4 || g.D + 2 * kPad < kQSeg)
         return false;
@@ -1536,20 +1571,7 @@ bool quarter_turns(const fan2d::Scalars &g, const double *angles, const double *
         const double ratio = r / (DSO[a] - r);
         wmax = std::max(wmax, DSD[a] / (DSO[a] - r) * std::sqrt(1.0 + ratio * ratio));
         if (a >= Q) continue;
-        for (int64_t k = 1; k < 4; ++k) {
-            const int64_t b = a + k * Q;
-            if (DSO[b] != DSO[a] || DSD[b] != DSD[a]) return false;
-            double d = std::remainder(angles[b] - angles[a] - (double)k * M_PI / 2.0, 2.0 * M_PI);
-            if (std::fabs(d) > 1e-9) return false;
-            // (-sin, cos) of the angle turned by k quarters
-            const float4 m = meta[a], t = meta[b];
-            const float tx = k == 1 ? -m.y : k == 2 ? -m.x : m.y;
-            const float ty = k == 1 ? m.x : k == 2 ? -m.y : -m.x;
-            auto same = [](float p, float q) {
-                return p == q || (std::fabs(p) < 1e-13f && std::fabs(q) < 1e-13f);
-            };
-            if (!same(t.x, tx) || !same(t.y, ty)) return false;
-        }
+        if (!quarter_apart(angles, DSO, DSD, A, a)) return false;
     }
     const double span = wmax * (kQT - 1) * std::sqrt(2.0) / g.du;
     return span + 4.0 <= (double)kQSeg;
@@ -1786,12 +1808,10 @@ CMI_API cmi_status cmi_plan2d_create(int device, int vol_prec, const uint64_t vo
 
     const int64_t A = p->A;
     std::vector<AngleGeom> geo(A);
+    for (int64_t a = 0; a < A; ++a) geo[a] = fan2d::plan_angle(p->g, angles[a], DSO[a], DSD[a]);
+    p->quarter = quarter_turns(p->g, angles, DSO, DSD, A);
     std::vector<float4> meta(A);
-    for (int64_t a = 0; a < A; ++a) {
-        geo[a] = fan2d::plan_angle(p->g, angles[a], DSO[a], DSD[a]);
-        meta[a] = bp2d_meta(angles[a], DSO[a], DSD[a]);
-    }
-    p->quarter = quarter_turns(p->g, angles, DSO, DSD, A, meta);
+    bp2d_table(angles, DSO, DSD, A, &meta[0].x);
     return finish_plan2d(std::move(p), geo, meta, {}, plan);
 }
 
@@ -1855,13 +1875,7 @@ CMI_API cmi_status cmi_fan2d_bp_table(uint64_t nangles, const double *angles, co
     clear_error();
     if (!angles || !DSO || !DSD || !table)
         return fail(CMI_ERR_INVALID_ARGUMENT, "fan2d_bp_table: null argument");
-    for (uint64_t a = 0; a < nangles; ++a) {
-        const float4 m = bp2d_meta(angles[a], DSO[a], DSD[a]);
-        table[4 * a + 0] = m.x;
-        table[4 * a + 1] = m.y;
-        table[4 * a + 2] = m.z;
-        table[4 * a + 3] = m.w;
-    }
+    bp2d_table(angles, DSO, DSD, (int64_t)nangles, table);
     return CMI_OK;
 }
 

@@ -349,7 +349,8 @@ CMI_API cmi_status cmi_backward_3d_transpose(const cmi_plan3d *plan, void *sinog
  * Host helpers that build the backprojection tables a serving job carries, from the same
  * geometry arguments as the plans (no counterpart in the reference, whose backprojectors
  * rebuild them per call: backward_2d.hpp:58-62, backward_3d.hpp:110-178).
- *   cmi_fan2d_bp_table: table[4a..4a+3] = (-sin a, cos a, DSD[a], DSO[a]) in FP32.
+ *   cmi_fan2d_bp_table: table[4a..4a+3] = (-sin a, cos a, DSD[a], DSO[a]) in FP32; where all
+ *   angles come in quadruples of quarter turns (to 1e-9), so do their entries, exactly.
  *   cmi_cone3d_bp_matrices: 12 floats per angle, the 3x4 matrix of `mode` (cmi_bp3d_mode)
  *   that cmi_backward_3d uses for the same description; *y_invariant (if not null) is set to
  *   1 when no angle's U or W row depends on y (circular orbits about the y axis, untilted

@@ -157,3 +157,18 @@ def test_backward_transpose_fine_cells(oracle, gpu, views, ny, nx, A, D, du):
     three = cm.backward_transpose(torch.stack([x, 2.0 * x, x.flip(0)]), geom)
     one = cm.backward_transpose(x, geom)
     assert torch.equal(three[0], one) and torch.equal(three[1], 2.0 * one)
+
+
+@pytest.mark.parametrize("mode,wpow", [("reference", 1), ("fbp", 2)])
+def test_backward_quarter_turns_of_rounded_angles(oracle, gpu, mode, wpow):
+    """Angles written with ten digits: by quarter turns (a batch) and by pixels (one image), the same
+    bits, and the oracle's values."""
+    rec = fan(64, 91, 200, 128.0, 192.0)
+    rec.angles = np.round(rec.angles, 10)
+    geom = as_fan_geometry(rec)
+    y = np.random.RandomState(5).rand(200, 91)
+    x = torch.tensor(y, dtype=torch.float32, device=gpu)
+    one = cm.backward(x, geom, mode=mode)
+    assert rel_l2(one, oracle.bp2d(rec, y, wpow=wpow)) <= RTOL_L2
+    many = cm.backward(x.expand(60, 200, 91).contiguous(), geom, mode=mode)
+    assert torch.equal(many[0], one) and torch.equal(many[59], one)
