@@ -42,8 +42,8 @@ __device__ __forceinline__ float lerp_pair(const Pair &p, float f) {
 // turns with the pixel (the sum is symmetric under a cyclic shift of the quarters).
 // On gfx950 fma, add and mul of vector registers issue about 1.55 wavefront instructions per clock
 // and CU; min / max / med3, floor, fract, conversions, shifted adds and any instruction that reads
-// a scalar register 0.93, v_rcp_f32 0.48 (issue probe, eight wavefronts per SIMD). With NY = 4
-// rows, a thread shares an angle's constants and its two products with x. Splitting the angles
+// a scalar register 0.93, v_rcp_f32 0.48 (issue probe, eight wavefronts per SIMD). With
+// several rows, a thread shares an angle's constants and its two products with x. Splitting the angles
 // over the wavefronts keeps the number of wavefronts that a thread per pixel would have.
 
 // Projection of one angle of a circular plan, tab[a] = (-sin, cos, DSD, DSO)
@@ -129,14 +129,14 @@ __device__ __forceinline__ void bp2d_angles(rsrc_t R, TAB tab, int a0, int a1, i
     for (; a < a1; ++a, row += Dp) some(a, std::integral_constant<int, 1>{});
 }
 
-// The tile's sums over all angles: wavefront q returns those of row q (NY = 4), or wavefront 0
-// those of the one row (NY = 1; the others return 0). All 256 threads of the workgroup call it;
+// The tile's sums over all angles: wavefront q returns those of row q, q < NY (the others return
+// 0). All 256 threads of the workgroup call it;
 // ix, iy0 the thread's column and the tile's first row; `red` 4 NY 64 floats of LDS.
 template <class SS, class ANGLE, int NY, class TAB>
 __device__ __forceinline__ float bp2d_tile(rsrc_t R, TAB tab, int A, int D, int nx, int ny, int ix,
                                            int iy0, float sx, float sy, float ox, float oy,
                                            float inv_du, float half_d, float *red) {
-    static_assert(NY == 1 || NY == 4, "a wavefront finishes one row");
+    static_assert(NY <= 4, "a wavefront finishes one row");
     const float x = ((float)ix - (float)nx / 2.0f) * sx + ox + 0.5f;
     float y[NY], py[NY], acc[NY];
 #pragma unroll

@@ -577,12 +577,16 @@ void k_fwd2d(const typename SI::raw *__restrict__ scratch,
 // (1024 tiles) 470 against 238.
 constexpr uint64_t kQTMinTiles = 200;
 
-// 64 x 4 tiles (times the batch) from which a workgroup of k_bp2d takes four rows of a plan from
-// views instead of one: 383 x 451 x 501 BF16 (768 tiles) 191 us a forward and backprojection
-// against 203, and smaller images need the workgroups. Circular plans have fewer constants to
-// share and always take one row: 1024^2 x 1024 470 us against 475, 512^2 x 512 72 against 78,
-// 256^2 x 256 23 against 28.
-constexpr uint64_t kViewRowTiles = 512;
+// A workgroup of k_bp2d takes one row of 64 pixels, which gives the most workgroups, or two where a
+// pixel has at least kRowsFine cells and that leaves kRowTiles workgroups (64 x 2 tiles times the
+// batch): the gathers of a wavefront then span many lines, which two rows of one angle share. Both
+// give the same bits. Calls with one, two and four rows, us: 1024^2 x 181, 5 cells a pixel 116, 99,
+// 99 (a thread per pixel, rows together: 105), 3.3 cells 109, 99, 100 (104), 2 cells 93, 96, 98
+// (94); 768^2 x 181, 5 cells 77, 64, 72 (76), 2 cells 56, 58, 66 (70); from views x 501, 4 cells a
+// pixel: 1024^2 268, 248, 241, 384^2 (1152 tiles) 59, 53, 59, 256^2 (512 tiles) 32, 42, 48; 1 cell:
+// 1024^2 237, 238, 236, 680^2 119, 124, 128, 448^2 58, 69, 70, 383 x 451 55, 56, 53.
+constexpr double kRowsFine = 2.5;
+constexpr uint64_t kRowTiles = 1024;
 
 // A workgroup per 64 x NY pixel tile, all angles in one pass, a quarter of them per wavefront
 // (backward_2d.hpp:31-99): vol[b][y][x] += f sum_a wt_a lerp(sino[b][a], u_a), ANGLE the plan's
@@ -590,7 +594,7 @@ constexpr uint64_t kViewRowTiles = 512;
 // Bound by the gathers (64 lanes in about 16 clocks per CU) and VALU issue (15 to 18) alike.
 // Against a thread per pixel for all angles: 256^2 x 256 41 -> 23 us a call, 320^2 x 320 48 -> 28,
 // 1024^2 x 1024 unchanged; 383 x 451 x 501 BF16 from views (whose loop over the angles had one
-// load in flight) 164 -> 30 us.
+// load in flight) 167 -> 55 us.
 template <class SV, class SS, class ANGLE, int NY>
 __global__ __launch_bounds__(kMaxBlock) void k_bp2d(typename SV::raw *__restrict__ vol,
                                                     const typename SS::raw *__restrict__ spad,
@@ -1994,15 +1998,19 @@ CMI_API cmi_status cmi_backward_2d_weighted(const cmi_plan2d *plan, void *volume
                                    D, A, (float)plan->g.sx, (float)plan->g.sy,
                                    (float)plan->g.ox, (float)plan->g.oy, inv_du, half_d, f);
             };
-            if (!plan->d_bpv)
-                launch(fbp ? k_bp2d<SV, SS, FanAngle<2>, 1> : k_bp2d<SV, SS, FanAngle<1>, 1>, 1,
-                       plan->d_meta, inv_du);
-            else if ((uint64_t)tx * ((ny + 3) / 4) * batch >= kViewRowTiles)
-                launch(fbp ? k_bp2d<SV, SS, ViewAngle<2>, 4> : k_bp2d<SV, SS, ViewAngle<1>, 4>,
-                       4, plan->d_bpv, 1.0f);
-            else
-                launch(fbp ? k_bp2d<SV, SS, ViewAngle<2>, 1> : k_bp2d<SV, SS, ViewAngle<1>, 1>,
-                       1, plan->d_bpv, 1.0f);
+            const bool two = plan->cells_per_pixel >= kRowsFine &&
+                             (uint64_t)tx * ((ny + 1) / 2) * batch >= kRowTiles;
+            auto kernel = [&](auto rows) {
+                constexpr int NY = decltype(rows)::value;
+                if (plan->d_bpv)
+                    launch(fbp ? k_bp2d<SV, SS, ViewAngle<2>, NY> : k_bp2d<SV, SS, ViewAngle<1>, NY>,
+                           NY, plan->d_bpv, 1.0f);
+                else
+                    launch(fbp ? k_bp2d<SV, SS, FanAngle<2>, NY> : k_bp2d<SV, SS, FanAngle<1>, NY>,
+                           NY, plan->d_meta, inv_du);
+            };
+            if (two) kernel(std::integral_constant<int, 2>{});
+            else kernel(std::integral_constant<int, 1>{});
         }
         CMI_HIP_TRY(hipGetLastError());
         return CMI_OK;

@@ -172,3 +172,25 @@ def test_backward_quarter_turns_of_rounded_angles(oracle, gpu, mode, wpow):
     assert rel_l2(one, oracle.bp2d(rec, y, wpow=wpow)) <= RTOL_L2
     many = cm.backward(x.expand(60, 200, 91).contiguous(), geom, mode=mode)
     assert torch.equal(many[0], one) and torch.equal(many[59], one)
+
+
+@pytest.mark.parametrize("views", [False, True])
+@pytest.mark.parametrize("ny,nx,A", [(1, 65, 5), (3, 64, 9), (6, 130, 8), (7, 63, 2)])
+def test_backward_fine_cells_rows(oracle, gpu, views, ny, nx, A):
+    """Fine cells: a batch with enough tiles takes two rows per thread, one image one; the same
+    bits, rows left over at the image's edge among them. The oracle's tolerance as for the
+    transpose: positions of up to D / 2 cells, four operations of 2^-24 each."""
+    more = {"det_offset": 0.25, "exact_geometry": True} if views else {}
+    D = 6 * nx
+    geom = cm.FanGeometry(DSD=3.0 * nx, DSO=2.0 * nx, angles=np.linspace(0, 5, A),
+                          vol_shape=(ny, nx), det_shape=D, det_spacing=0.4, **more)
+    y = np.random.RandomState(nx).rand(3, A, D)
+    x = torch.tensor(y, dtype=torch.float32, device=gpu)
+    tiles = ((nx + 63) // 64) * ((ny + 1) // 2)
+    many = x.repeat(-(-1024 // (3 * tiles)), 1, 1).contiguous()
+    for mode, wpow in (("reference", 1), ("fbp", 2)):
+        got = cm.backward(many, geom, mode=mode)
+        for i in range(3):
+            one = cm.backward(x[i].contiguous(), geom, mode=mode)
+            assert rel_l2(one, oracle.bp2d(geom, y[i], wpow=wpow)) <= 4 * (D / 2) * 2.0 ** -24 / 0.58
+            assert torch.equal(got[i], one) and torch.equal(got[-3 + i], one)
