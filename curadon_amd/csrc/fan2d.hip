@@ -177,7 +177,7 @@ struct BandSums {
 // holds adjacent detector cells of one angle and walks the dominant rows tau in increasing
 // order: on row tau every lane whose dominant axis is the pass's takes its sample
 // jf = s (tau - floor(md)), if jf lies in its range [q.z, q.z + N - 1], so all lanes read the
-// same two rows. The rows come in bands of at most kBandMax: the workgroup stages a band's rows
+// same two rows. The rows come in bands (HalfBands, WholeBands): the workgroup stages a band's rows
 // and the one below of the copy whose rows run along the dominant axis, over the
 // columns its samples in the band touch, into LDS (rows of kPitch floats, filled with
 // 4-element row loads) and interpolates from there. The last two cells of every row are kept
@@ -195,26 +195,43 @@ struct BandSums {
 // the launch shape).
 //
 // Bound by LDS (two pair reads of four clocks per wavefront, row and CU) and VALU issue (eight full
-// and three half rate slots) alike, so it wants wavefronts: bands of whole groups (19.5 KB) kept 16
-// per CU, half groups keep 24. The staging plans are made a lane per band and the check that the
-// rays stay beside the extreme ones once per pass (both were made per band, a third of all VALU
-// instructions). 1024^2 x 1024 angles of 1448 cells: 0.52 -> 0.50 ms; 16 images of 512^2, 512
-// angles of 724 cells: 1.38 -> 1.28 ms (LDS busy 79 %); 383 x 451 x 501 angles of 701 cells in
-// BF16: 0.126 -> 0.110 ms. Groups of 15 rows, a band each, would take 0.47 and 1.18 ms (28
-// wavefronts), but round 16-bit images' sums more often.
+// and three half rate slots) alike. The staging plans are made a lane per band and the check that
+// the rays stay beside the extreme ones once per pass (both were made per band, a third of all VALU
+// instructions). A group comes as one band (19.5 KB, 16 wavefronts per CU) or, where the copies
+// exceed an XCD's 4 MB of L2 and the loads take long, as two (12.2 KB, 24 wavefronts; twice the
+// barriers). Calls with half and whole groups, us (bands of whole groups planned one by one: third):
+// parallel rays 1024^2 x 360 of 0.67 pixels 308, 452 (451), 1024^2 x 60 189, 204 (207), x 500 408,
+// 427 (433), 1024^2 x 500 in BF16 373, 391 (502), 1024^2 x 180 of 1.2 pixels 391, 428 (440); but
+// 512^2 x 180 of 0.5 pixels 110, 97 (98), 400^2 x 500 of 0.7 114, 106 (107), 512^2 x 500 of 1.2 210,
+// 193 (191), 128^2 x 180 of 0.5 38, 33 (34), 200^2 x 180 of 0.7 in BF16 50, 47 (58); fine cells, whose
+// bands are narrow, want whole groups in large images too: 1024^2 x 180 of 0.3 310, 287 (308).
+// Groups of 15 rows, a band each, would be faster still (28 wavefronts), but round 16-bit images'
+// sums more often.
+constexpr uint64_t kHalfBytes = 4u << 20;
+constexpr double kHalfCells = 2.0; // cells per pixel
 
-// Rows of a summation group, and its two bands: rows [0, kBandMax) and [kBandMax, kGroup).
-constexpr int kGroup = 31, kBandMax = 16;
-// Staged rows of a band: its rows and the one below, 17 at most, as shares of K rows of 2 or 4
-// groups of threads (K = 9 or 5; the rows past the seventeenth are not read).
-constexpr int kBandRows = 20;
-__host__ __device__ constexpr int band_share(int lg) { return lg == 1 ? 9 : 5; }
-static_assert(2 * band_share(1) > kBandMax && 4 * band_share(2) > kBandMax &&
-              2 * band_share(1) <= kBandRows && 4 * band_share(2) <= kBandRows, "shares fit");
+constexpr int kGroup = 31; // rows of a summation group
+
+// How a group's rows come: kPer bands of at most kMax rows, band bn from row(bn) on. A band and the
+// row below it are staged as shares of share(lg) rows of 2^lg groups of threads, lg = 1 or 2 (kRows
+// rows in all; those past the band's own are not read), the first kAhead of a share ahead.
+struct HalfBands { // rows [0, 16) and [16, 31) of a group
+    static constexpr int kPer = 2, kMax = 16, kRows = 20, kAhead = 5;
+    __host__ __device__ static constexpr int share(int lg) { return lg == 1 ? 9 : 5; }
+    __host__ __device__ static constexpr int row(int bn) {
+        return (bn >> 1) * kGroup + (bn & 1) * kMax;
+    }
+};
+struct WholeBands {
+    static constexpr int kPer = 1, kMax = kGroup, kRows = 32, kAhead = 8;
+    __host__ __device__ static constexpr int share(int lg) { return lg == 1 ? 16 : 8; }
+    __host__ __device__ static constexpr int row(int bn) { return bn * kGroup; }
+};
 // LDS row pitch in floats: a multiple of 4 (16-byte row stores) and below 255, so that one
 // address reaches a tap pair and the pair below it with two ds_read2_b32 immediate offsets.
-// 152 (12.2 KB per band) keeps thirteen workgroups per CU: 128 rays at up to about 0.95 texels per
-// cell plus a band's slope and the tap margins fit; wider bands take the global path.
+// 152 (12.2 KB per half group, 19.5 KB per group) keeps thirteen or eight workgroups per CU: 128
+// rays at up to about 0.95 or 0.9 texels per cell plus a band's slope and the tap margins fit; wider
+// bands take the global path.
 constexpr int kPitch = 152;
 constexpr int kFwdRays = 128;          // rays (threads) per workgroup of the forward
 constexpr int kMaxWaves = kFwdRays / 64;
@@ -273,7 +290,7 @@ __device__ __forceinline__ float ray_at(const RayRow &r, int t) {
     return fmaf((float)(r.s * (t - r.r0)), r.vc, r.mc);
 }
 
-template <class SI, bool YDOM>
+template <class SI, bool YDOM, class B>
 __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__ ev,
                                             const float4 *__restrict__ ns, bool valid,
                                             int rstride, int cofs, float *band, int *red,
@@ -342,9 +359,9 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
     float acc = 0.0f;
     // The staging plans of 64 bands at a time, a lane each: band first + lane needs columns c_lo ..
     // c_lo + W - 1 (its extreme rays' at its first and last row), Q quads. It is staged when W fits
-    // a row and at least two groups of Q threads exist. G' groups of Q threads, G' = 2^lg the
-    // largest power of two with G' Q <= nthreads: thread g Q + q (g < G') takes quad q of the K =
-    // kBandRows / G' consecutive rows g K .. g K + K - 1. A row then lies at a wave-uniform byte
+    // a row and at least two groups of Q threads exist: G' = 2^lg groups, four if 4 Q <= nthreads
+    // and two otherwise. Thread g Q + q (g < G') takes quad q of the K = B::share(lg) consecutive
+    // rows g K .. g K + K - 1. A row then lies at a wave-uniform byte
     // offset from the thread's first row in the copy (one add; the offset stays in the load's
     // range-checked vector offset, so rows outside the copy read zeros) and at a constant one in
     // LDS (the store's immediate offset), and no row needs a bound. Quotients come from a float
@@ -352,7 +369,6 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
     // 1/(2 Q) > 2^-8 away from the next integer.
     int plan_lo = 0, plan_q = 0; // c_lo; Q + (lg << 8), 0 where the band is not staged
     float plan_rq = 0.0f;        // 1 / Q
-    auto band_row = [](int bn) { return (bn >> 1) * kGroup + (bn & 1) * kBandMax; };
     int first = INT_MIN / 2; // band of lane 0's plan
     struct Stage {
         int t0, c_lo, q;
@@ -366,7 +382,7 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
         if (bn >= first + 64) {
             first = bn;
             const int mine = first + (int)(threadIdx.x & 63);
-            const int lo = max(tr0, band_row(mine)), hi = min(tr1, band_row(mine + 1) - 1);
+            const int lo = max(tr0, B::row(mine)), hi = min(tr1, B::row(mine + 1) - 1);
             const RayRow e0 = ray_row<YDOM>(ext[0]), e1 = ray_row<YDOM>(ext[1]);
             const float ca = ray_at(e0, lo), cb = ray_at(e0, hi);
             const float cc = ray_at(e1, lo), cd = ray_at(e1, hi);
@@ -383,14 +399,14 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
         }
         const int i = bn - first;
         Stage P{};
-        P.t0 = band_row(bn);
+        P.t0 = B::row(bn);
         P.q = __builtin_amdgcn_readlane(plan_q, i);
         if (P.q) {
             P.c_lo = __builtin_amdgcn_readlane(plan_lo, i);
             const float rq =
                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(plan_rq), i));
             const int Q = P.q & 255, lg = P.q >> 8;
-            P.K = band_share(lg);
+            P.K = B::share(lg);
             const int g = (int)(ftid * rq);
             P.mine = g < (1 << lg);
             const int q4 = ((int)threadIdx.x - g * Q) << 2;
@@ -408,16 +424,18 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
     };
     // The first kAhead rows of a thread's share of band i + 1 are loaded while band i is sampled
     // (registers `pre`), so their latency hides behind the sampling.
-    constexpr int kAhead = 5;
-    static_assert(band_share(2) == kAhead && band_share(1) <= 2 * kAhead, "rows of a share");
+    constexpr int kAhead = B::kAhead;
+    static_assert(B::share(2) == kAhead && B::share(1) <= 2 * kAhead, "rows of a share");
+    static_assert(2 * B::share(1) > B::kMax && 4 * B::share(2) > B::kMax &&
+                  2 * B::share(1) <= B::kRows && 4 * B::share(2) <= B::kRows, "shares fit");
     RawQuad<SI> pre[kAhead];
     auto load_ahead = [&](const Stage &P) {
         if (P.q && P.mine)
 #pragma unroll
             for (int u = 0; u < kAhead; ++u) pre[u] = buf_raw_quad_at<SI>(R, P.gb + u * rowb);
     };
-    int bn = 2 * floor_div(tr0, kGroup);
-    if (band_row(bn + 1) <= tr0) ++bn;
+    int bn = B::kPer * floor_div(tr0, kGroup);
+    if (B::kPer > 1 && B::row(bn + 1) <= tr0) ++bn;
     Stage P = plan_band(bn);
     load_ahead(P);
     BandSums sums;
@@ -428,7 +446,7 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
 #pragma unroll
                 for (int u = 0; u < kAhead; ++u) store_row(P, u, pre[u]);
                 if (P.K > kAhead) {
-                    constexpr int kRest = band_share(1) - kAhead;
+                    constexpr int kRest = B::share(1) - kAhead;
                     RawQuad<SI> v[kRest];
 #pragma unroll
                     for (int u = 0; u < kRest; ++u)
@@ -441,7 +459,7 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
         }
         ++bn;
         Stage N{};
-        N.t0 = band_row(bn);
+        N.t0 = B::row(bn);
         if (N.t0 <= tr1) {
             N = plan_band(bn);
             load_ahead(N);
@@ -459,10 +477,10 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
             int t = b_lo;
             // up to four rows' taps are read before the first is used
             auto batch = [&](auto rows, auto &&address) {
-                constexpr int B = decltype(rows)::value;
-                float c[B], x[B][4];
+                constexpr int N4 = decltype(rows)::value;
+                float c[N4], x[N4][4];
 #pragma unroll
-                for (int u = 0; u < B; ++u) {
+                for (int u = 0; u < N4; ++u) {
                     c[u] = fmaf(u == 0 ? jf : jf + (float)u * sf, vc, mc);
                     const float *p = address(u, floor_i32(c[u]));
                     x[u][0] = p[0];
@@ -471,11 +489,11 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
                     x[u][3] = p[kPitch + 1];
                 }
 #pragma unroll
-                for (int u = 0; u < B; ++u)
+                for (int u = 0; u < N4; ++u)
                     sums.add(x[u][0], x[u][1], x[u][2], x[u][3], __builtin_amdgcn_fractf(c[u]));
-                t += B;
-                jf += (float)B * sf;
-                rowa += B * kPitch;
+                t += N4;
+                jf += (float)N4 * sf;
+                rowa += N4 * kPitch;
             };
             if (full) { // every lane has a sample on every row of the band
                 auto at = [&](int u, int i) { return rowa + u * kPitch + i; };
@@ -506,7 +524,7 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
                 sums.add(a.lo, a.hi, b.lo, b.hi, __builtin_amdgcn_fractf(c));
             }
         }
-        if ((bn & 1) == 0 || N.t0 > tr1) { // the group's last band
+        if (bn % B::kPer == 0 || N.t0 > tr1) { // the group's last band
             acc += sums.total(fb);
             sums = BandSums{};
         }
@@ -517,11 +535,11 @@ __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__
 }
 
 // One workgroup = nthreads <= kFwdRays adjacent detector cells of one angle, one thread per
-// ray; LDS holds one band of kBandRows x kPitch floats (9.7 KB).
+// ray; LDS holds one band of B::kRows x kPitch floats.
 // sino[b][a][k] = scale * sum_{j<N} bilinear(img, e + j v)   (forward_2d.hpp:63-78)
-// Six wavefronts per SIMD (80 VGPRs, 40 bytes of scratch with FP32 images): 0.498 ms at 1024^2, five
-// 0.511.
-template <class SI, class SS>
+// Half groups: six wavefronts per SIMD (80 VGPRs, 40 bytes of scratch with FP32 images): 0.498 ms at
+// 1024^2 x 1024, five 0.511. Whole groups: four, by their LDS.
+template <class SI, class SS, class B>
 __global__ __launch_bounds__(kFwdRays) __attribute__((amdgpu_waves_per_eu(6)))
 void k_fwd2d(const typename SI::raw *__restrict__ scratch,
                                               int Wp, int Hp, const float4 *__restrict__ ev,
@@ -529,7 +547,7 @@ void k_fwd2d(const typename SI::raw *__restrict__ scratch,
                                               typename SS::raw *__restrict__ sino, int D, int A) {
     // one LDS object with the band first, so that cell addresses need no base offset
     __shared__ struct {
-        float band[kBandRows * kPitch];
+        float band[B::kRows * kPitch];
         float4 ext[2];
         int red[8 * kMaxWaves];
         int flag[2]; // one per pass: no barrier follows a pass's read where nothing is staged
@@ -555,15 +573,15 @@ void k_fwd2d(const typename SI::raw *__restrict__ scratch,
     const int c0x = Wp / 2, c0y = Hp / 2;
     // the zero cells and the flags; ordered before their first use by the barriers at the start of
     // a pass
-    for (int i = threadIdx.x; i < 2 * kBandRows; i += nthreads)
+    for (int i = threadIdx.x; i < 2 * B::kRows; i += nthreads)
         band[(i >> 1) * kPitch + kPitch - 2 + (i & 1)] = 0.0f;
     if (threadIdx.x < 2) sh.flag[threadIdx.x] = 0;
     const float scale = valid ? ns[r].x : 0.0f;
     bool others = false; // whether a lane's ray is x dominant
-    float acc = march_band<SI, true>(R, ev + r, ns + r, valid, Wp, c0y * Wp + c0x, band,
+    float acc = march_band<SI, true, B>(R, ev + r, ns + r, valid, Wp, c0y * Wp + c0x, band,
                                              red, ext, &sh.flag[0], nthreads, others);
     if (others)
-        acc += march_band<SI, false>(R, ev + r, ns + r, valid, Hp, one + c0x * Hp + c0y,
+        acc += march_band<SI, false, B>(R, ev + r, ns + r, valid, Hp, one + c0x * Hp + c0y,
                                              band, red, ext, &sh.flag[1], nthreads, others);
     if (valid) sino[b * (size_t)A * D + r] = from_f32<SS>(acc * scale);
 }
@@ -1769,7 +1787,10 @@ cmi_status fan2d_forward_enqueue(const cmi_plan2d *plan, const void *volume, int
         // block_x * block_y (at most kFwdRays) adjacent cells of one angle per workgroup
         const unsigned nt = std::min<unsigned>(plan->block_x * plan->block_y, kFwdRays);
         dim3 fb(nt), fg((unsigned)((D + nt - 1) / nt), (unsigned)A, (unsigned)batch);
-        hipLaunchKernelGGL((k_fwd2d<SI, SS>), fg, fb, 0, s, (const RI *)scratch, Wp, Hp,
+        const bool half = plan->cells_per_pixel < kHalfCells &&
+                          2 * (uint64_t)Wp * Hp * sizeof(RI) >= kHalfBytes;
+        auto kern = half ? k_fwd2d<SI, SS, HalfBands> : k_fwd2d<SI, SS, WholeBands>;
+        hipLaunchKernelGGL(kern, fg, fb, 0, s, (const RI *)scratch, Wp, Hp,
                            plan->d_ev, plan->d_ns, (typename SS::raw *)sinogram, D, A);
         CMI_HIP_TRY(hipGetLastError());
         return CMI_OK;

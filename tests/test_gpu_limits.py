@@ -194,3 +194,25 @@ def test_backward_fine_cells_rows(oracle, gpu, views, ny, nx, A):
             one = cm.backward(x[i].contiguous(), geom, mode=mode)
             assert rel_l2(one, oracle.bp2d(geom, y[i], wpow=wpow)) <= 4 * (D / 2) * 2.0 ** -24 / 0.58
             assert torch.equal(got[i], one) and torch.equal(got[-3 + i], one)
+
+
+@pytest.mark.parametrize("prec", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("ny", [1, 11, 12, 13, 15, 27, 28, 43, 44, 59, 74, 75])
+@pytest.mark.parametrize("turned", [False, True])
+@pytest.mark.parametrize("D,du", [(70, 0.55), (300, 0.9), (200, 1.55), (130, 3.0)])
+def test_forward_half_bands(oracle, gpu, prec, ny, turned, D, du):
+    """Images of at least 4 MB in their two copies, whose groups of 31 rows come in two bands: image
+    rows (with the border) that end before, at and after a band and a group, in either dominant
+    axis, narrow and wide bands. FP32 sinograms of images in either type."""
+    nx = 4096 * 1024 // (8 if prec == torch.float32 else 4) // (ny + 4) + 1
+    rec = fan(nx, D, 5, 2.0 * nx, 3.0 * nx, du=1.5 * du, ny=ny, arc=0.4)
+    rec.angles = rec.angles - 0.15
+    img = np.random.RandomState(D + ny).rand(ny, nx)
+    if turned:
+        rec.vol_shape, img, rec.angles = rec.vol_shape[::-1].copy(), img.T.copy(), rec.angles + np.pi / 2
+    geom = as_fan_geometry(rec, vol_prec=prec, sino_prec=torch.float32)
+    x = torch.tensor(img, dtype=prec, device=gpu)
+    got = cm.forward(x, geom)
+    ref = oracle.fwd2d(rec, x.double().cpu().numpy())
+    assert np.abs(ref).max() > 0.1
+    assert rel_l2(got, ref) <= RTOL_L2
