@@ -98,7 +98,9 @@ template <class SS, class ANGLE, int NY, class TAB>
 __device__ __forceinline__ void bp2d_angles(rsrc_t R, TAB tab, int a0, int a1, int D, float x,
                                             float px, const float (&y)[NY], const float (&py)[NY],
                                             float c0, float (&acc)[NY]) {
-    constexpr int UA = NY == 1 ? 4 : 2; // angles whose loads are in flight together
+    // angles whose loads are in flight together (one row: 4 took 55 us for 383 x 451 x 501 from views
+    // in BF16, 8 take 51)
+    constexpr int UA = NY == 1 ? 8 : 2;
     const int Dp = D + 2 * kPadDet;
     const float hi = (float)D;
     int row = a0 * Dp + kPadDet;
@@ -126,6 +128,10 @@ __device__ __forceinline__ void bp2d_angles(rsrc_t R, TAB tab, int a0, int a1, i
     };
     int a = a0;
     for (; a + UA <= a1; a += UA, row += UA * Dp) some(a, std::integral_constant<int, UA>{});
+    if (UA > 4 && a + 4 <= a1) {
+        some(a, std::integral_constant<int, 4>{});
+        a += 4, row += 4 * Dp;
+    }
     for (; a < a1; ++a, row += Dp) some(a, std::integral_constant<int, 1>{});
 }
 

@@ -197,18 +197,20 @@ struct BandSums {
 // Bound by LDS (two pair reads of four clocks per wavefront, row and CU) and VALU issue (eight full
 // and three half rate slots) alike. The staging plans are made a lane per band and the check that
 // the rays stay beside the extreme ones once per pass (both were made per band, a third of all VALU
-// instructions). A group comes as one band (19.5 KB, 16 wavefronts per CU) or, where the copies
-// exceed an XCD's 4 MB of L2 and the loads take long, as two (12.2 KB, 24 wavefronts; twice the
-// barriers). Calls with half and whole groups, us (bands of whole groups planned one by one: third):
-// parallel rays 1024^2 x 360 of 0.67 pixels 308, 452 (451), 1024^2 x 60 189, 204 (207), x 500 408,
-// 427 (433), 1024^2 x 500 in BF16 373, 391 (502), 1024^2 x 180 of 1.2 pixels 391, 428 (440); but
-// 512^2 x 180 of 0.5 pixels 110, 97 (98), 400^2 x 500 of 0.7 114, 106 (107), 512^2 x 500 of 1.2 210,
-// 193 (191), 128^2 x 180 of 0.5 38, 33 (34), 200^2 x 180 of 0.7 in BF16 50, 47 (58); fine cells, whose
-// bands are narrow, want whole groups in large images too: 1024^2 x 180 of 0.3 310, 287 (308).
+// instructions). A group comes as one band (19.5 KB, 16 wavefronts per CU) or as two (12.2 KB, 24
+// wavefronts, twice the barriers): where the copies exceed an XCD's 4 MB of L2, so that loads take
+// long, or kHalfGroups workgroups keep the GPU full for long, unless cells are fine and bands narrow.
+// Calls with half and whole groups, us (bands of whole groups planned one by one: third): 1024^2 x
+// 360 of 0.67 pixels, parallel rays 308, 452 (451), 1024^2 x 60 of 0.7 189, 204 (207), x 500 408, 427
+// (433), in BF16 373, 391 (502), 1024^2 x 180 of 1.2 391, 428 (440); 16 images of 512^2 x 512 of 0.86
+// 1573, 1684 (1721), of 0.67 1668, 1658 (1747), of 256^2 x 180 of 0.78 217, 225 (234); but 512^2 x 180
+// of 0.5 110, 97 (98), 400^2 x 500 of 0.7 114, 106 (107), 512^2 x 500 of 1.2 210, 193 (191), 128^2 x
+// 180 of 0.5 38, 33 (34), 200^2 x 180 of 0.7 in BF16 50, 47 (58); fine cells: 1024^2 x 180 of 0.3 310,
+// 287 (308), 16 images of 512^2 x 512 of 0.5 2101, 2012 (2143).
 // Groups of 15 rows, a band each, would be faster still (28 wavefronts), but round 16-bit images'
 // sums more often.
-constexpr uint64_t kHalfBytes = 4u << 20;
-constexpr double kHalfCells = 2.0; // cells per pixel
+constexpr uint64_t kHalfBytes = 4u << 20, kHalfGroups = 8192;
+constexpr double kHalfCells = 1.6; // cells per pixel
 
 constexpr int kGroup = 31; // rows of a summation group
 
@@ -602,7 +604,8 @@ constexpr uint64_t kQTMinTiles = 200;
 // 99 (a thread per pixel, rows together: 105), 3.3 cells 109, 99, 100 (104), 2 cells 93, 96, 98
 // (94); 768^2 x 181, 5 cells 77, 64, 72 (76), 2 cells 56, 58, 66 (70); from views x 501, 4 cells a
 // pixel: 1024^2 268, 248, 241, 384^2 (1152 tiles) 59, 53, 59, 256^2 (512 tiles) 32, 42, 48; 1 cell:
-// 1024^2 237, 238, 236, 680^2 119, 124, 128, 448^2 58, 69, 70, 383 x 451 55, 56, 53.
+// 1024^2 237, 238, 236, 680^2 119, 124, 128, 448^2 58, 69, 70, 383 x 451 51, 56, 53 (four rows pay
+// only where the workgroups happen to fill the CUs evenly).
 constexpr double kRowsFine = 2.5;
 constexpr uint64_t kRowTiles = 1024;
 
@@ -612,7 +615,7 @@ constexpr uint64_t kRowTiles = 1024;
 // Bound by the gathers (64 lanes in about 16 clocks per CU) and VALU issue (15 to 18) alike.
 // Against a thread per pixel for all angles: 256^2 x 256 41 -> 23 us a call, 320^2 x 320 48 -> 28,
 // 1024^2 x 1024 unchanged; 383 x 451 x 501 BF16 from views (whose loop over the angles had one
-// load in flight) 167 -> 55 us.
+// load in flight) 167 -> 51 us.
 template <class SV, class SS, class ANGLE, int NY>
 __global__ __launch_bounds__(kMaxBlock) void k_bp2d(typename SV::raw *__restrict__ vol,
                                                     const typename SS::raw *__restrict__ spad,
@@ -1788,7 +1791,8 @@ cmi_status fan2d_forward_enqueue(const cmi_plan2d *plan, const void *volume, int
         const unsigned nt = std::min<unsigned>(plan->block_x * plan->block_y, kFwdRays);
         dim3 fb(nt), fg((unsigned)((D + nt - 1) / nt), (unsigned)A, (unsigned)batch);
         const bool half = plan->cells_per_pixel < kHalfCells &&
-                          2 * (uint64_t)Wp * Hp * sizeof(RI) >= kHalfBytes;
+                          (2 * (uint64_t)Wp * Hp * sizeof(RI) >= kHalfBytes ||
+                           (uint64_t)fg.x * A * batch >= kHalfGroups);
         auto kern = half ? k_fwd2d<SI, SS, HalfBands> : k_fwd2d<SI, SS, WholeBands>;
         hipLaunchKernelGGL(kern, fg, fb, 0, s, (const RI *)scratch, Wp, Hp,
                            plan->d_ev, plan->d_ns, (typename SS::raw *)sinogram, D, A);
