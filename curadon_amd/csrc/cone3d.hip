@@ -651,11 +651,24 @@ constexpr int kATOwn = kAT * kAT * kAT / kMaxBlock; // tile voxels per thread
 static_assert(kAT * kAT * kAT % kMaxBlock == 0, "whole voxels per thread");
 constexpr int kAdj3Bits = 19;                             // a term's bound: 2^kAdj3Bits units
 constexpr int kAdj3Budget = (1 << (31 - kAdj3Bits)) - 16; // terms per voxel between drains
-// Workgroups of k_adj3d that angle groups are made for: tiles differ in their rays (those near the
-// source have many), so that many more than the 1536 which the GPU holds at once pay. Workgroups
-// at most, 97 x 120 x 133 x 90 views / 160^3 x 180 / 192^3 x 180 / 256^3 x 360: none 1.60 / 5.34 /
-// 8.54 / 33.2 ms, 3072: 0.82 / - / 8.18 / 33.2, 6144: 0.78 / 4.79 / 7.67 / 32.3, 12288: 0.73 / 4.16
-// / 7.00 / 34.9, 24576: 0.73 / 3.92 / 6.74 / 32.6.
+// Angle groups per tile. A group costs its workgroup's clearing of the LDS tile and 4096 64-bit
+// atomics, as much as some thousand samples, so it is given kAdj3Samples of them (a tile's share of
+// the plan's); or, as long as that leaves fewer than kAdj3Fill workgroups, kAdj3Least. Tiles differ in
+// their rays (those near the source have many), so that many more than the 1536 workgroups which the
+// GPU holds at once pay: to kAdj3Workgroups. us, with 1 / 2 / 4 / 8 / 16 / 32 / 64 groups, and what
+// this rule takes: 97 x 120 x 133 x 90 views (504 tiles) 1315 / 948 / 880 / 698 / 702 / 684 / 753, 49;
+// 128^3 x 40 views (512) of 192^2 487 / 423 / 399 / 358 / 357 / 459 / 521, 21; of 96^2 214 / 174 / 179 /
+// 173 / 240 / 413 / 490, 5; of 48^2 166 / 128 / 138 / 154 / 188 / 275 / 319, 2; 48^3 x 60 of 18^2 (27)
+// 240 / 138 / 79 / 54 / 43 / 44 / 57, 14.
+// Where the tiles fill the GPU and the angles are few, a group is a sector of the circle, whose tiles
+// near the source are neighbours in the order and fall to one or two XCDs: one group there. us, with
+// 1 / 2 / 4 / 8 / 16 groups: 128^3 (512 tiles) of 640^2, 4 views 492 / 693 / 566 / 632 / 572, 12 views
+// 1509 / 1934 / 2136 / 2142 / 1605, 24 views 2990 / 3681 / 3801 / 3393 / 3298; of 384^2, 12 views 482 /
+// 604 / 567 / 598 / 484, 24 views 954 / 1118 / 1099 / 899 / 876; 192^3 (1728) x 12 of 288^2 373 / 376 /
+// 376 / 495 / 616, x 24 of 960^2 8621 / 9602 / 10264 / 8793 / 8898; but 96^3 (216) x 12 of 288^2 393 /
+// 307 / 299 / 288 / 241.
+constexpr uint64_t kAdj3Samples = 10000, kAdj3Least = 1500, kAdj3Fill = 1024;
+constexpr uint64_t kAdj3FullTiles = 512, kAdj3FewAngles = 24, kAdj3TilesPerAngle = 32;
 constexpr uint64_t kAdj3Workgroups = 24576;
 
 // vol[o] += a voxel's sum of fixed-point terms.
@@ -1886,9 +1899,17 @@ CMI_API cmi_status cmi_adjoint_3d(const cmi_plan3d *plan, void *volume, int vol_
         const int ntz = (nz + kAT - 1) / kAT;
         const dim3 tiles((unsigned)((nx + kAT - 1) / kAT), (unsigned)((ny + kAT - 1) / kAT),
                          (unsigned)(ntz * batch));
-        const int G = (int)std::max<uint64_t>(
-            1, std::min<uint64_t>({(uint64_t)A, (kAdj3Workgroups + ntiles - 1) / ntiles,
-                                   65535 / (uint64_t)tiles.z}));
+        const uint64_t samples = plan->total_samples * batch / ntiles; // per tile
+        const int G =
+            ntiles >= kAdj3FullTiles &&
+                    (uint64_t)A <= std::min(kAdj3FewAngles, ntiles / kAdj3TilesPerAngle)
+                ? 1
+                : (int)std::max<uint64_t>(
+                      1, std::min<uint64_t>({(uint64_t)A, (kAdj3Workgroups + ntiles - 1) / ntiles,
+                                             65535 / (uint64_t)tiles.z,
+                                             std::max(samples / kAdj3Samples,
+                                                      std::min(kAdj3Fill / ntiles,
+                                                               samples / kAdj3Least))}));
         if (G > 1)
             hipLaunchKernelGGL(k_clear_sums, dim3((unsigned)(ntiles * kATOwn)), dim3(kMaxBlock), 0,
                                s, totals);

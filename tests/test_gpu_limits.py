@@ -216,3 +216,16 @@ def test_forward_half_bands(oracle, gpu, prec, ny, turned, D, du):
     ref = oracle.fwd2d(rec, x.double().cpu().numpy())
     assert np.abs(ref).max() > 0.1
     assert rel_l2(got, ref) <= RTOL_L2
+
+
+@pytest.mark.parametrize("A", [16, 17, 24])
+@pytest.mark.parametrize("batch", [511, 512, 768])
+def test_adjoint_3d_few_angles(gpu, A, batch):
+    """Volumes of one tile in batches around the number of tiles from which few angles stay one
+    group: the same bits as in a batch of three, whose tiles have groups of their own."""
+    geom = as_cone_geometry(cone(16, 24, 20, A, 40.0, 60.0, du=(1.0, 1.0)))
+    y = torch.tensor(np.random.RandomState(A).rand(3, A, 20, 24) - 0.3, dtype=torch.float32, device=gpu)
+    few = cm.adjoint(y, geom)
+    many = cm.adjoint(y.repeat((batch + 2) // 3, 1, 1, 1)[:batch].contiguous(), geom)
+    for i in range(batch):
+        assert torch.equal(many[i], few[i % 3])
