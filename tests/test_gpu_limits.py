@@ -229,3 +229,34 @@ def test_adjoint_3d_few_angles(gpu, A, batch):
     many = cm.adjoint(y.repeat((batch + 2) // 3, 1, 1, 1)[:batch].contiguous(), geom)
     for i in range(batch):
         assert torch.equal(many[i], few[i % 3])
+
+
+@pytest.mark.parametrize("rec", [
+    lambda: cone(40, 120, 90, 7, 80.0, 120.0, nz=1, ny=30),           # panels far beyond the volume
+    lambda: cone(40, 120, 90, 7, 80.0, 120.0, nz=30, ny=1),
+    lambda: cone(1, 120, 90, 7, 80.0, 120.0, nz=30, ny=30),
+    lambda: cone(20, 100, 100, 7, 80.0, 120.0, det_offset=(31.0, -23.0), nz=13, ny=17),
+    lambda: cone(20, 100, 100, 5, 40.0, 60.0, du=(0.31, 0.29), nz=4,
+                 angles=np.array([[0.3, 1.9, 3.0, 5.1, 5.9], [0.7, 1.4, 0.2, 1.5, 1.1],
+                                  [0.1, 0.9, 1.5, 0.4, 0.2]])),
+])
+def test_backward_transpose_3d_tiles_beside_the_volume(oracle, gpu, rec):
+    """Panel tiles whose rays pass the volume on any side, next to tiles that see one edge of it:
+    the latter keep every voxel, the former are zero.
+
+    A pixel of these fine panels holds few terms, each rounded to units of 2^-18 max|v| wbound
+    (wbound = 1, or 1 / min W^2 for FDK): 0.29 units rms, against terms of rms|v| / 3 (two linear
+    weights of rms 1 / sqrt(3)). Twice that."""
+    rec = rec()
+    geom = as_cone_geometry(rec)
+    v = np.random.RandomState(5).rand(*rec.vol_shape) - 0.3
+    x = torch.tensor(v, dtype=torch.float32, device=gpu)
+    wmin = 1.0 - np.linalg.norm(rec.vol_shape) / 2.0 / rec.DSO
+    unit = 0.29 * 2.0 ** -18 * np.abs(v).max() / (np.sqrt(np.mean(v * v)) / 3.0)
+    for mode, kw, wbound in (("reference", {}, 1.0), ("matched", {"matched": True}, 1.0),
+                             ("fdk", {"matched": True, "fdk": True}, 1.0 / wmin ** 2)):
+        got = cm.backward_transpose(x, geom, mode=mode)
+        want = oracle.bp3d_T(geom, v, **kw)
+        assert rel_l2(got, want) <= 2.0 * unit * wbound, mode
+        beside = want == 0.0
+        assert beside.any() and not got.cpu().numpy()[beside].any()
