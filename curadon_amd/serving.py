@@ -39,11 +39,11 @@ from .geometry import ConeGeometry, FanGeometry
 from .reconstruction import (cosine_weights_cone, cosine_weights_fan, fft_length,
                              filter_rows_weighted)
 
-# Relative cost of one voxel-angle of the cone-beam backprojector to one pixel-angle of the
-# fan-beam one (2 x 2 taps from LDS-staged footprints against 2 taps from the sinogram; set at
-# 2.1e12 voxel-angles/s at 384^3 against 2.35e12 pixel-angles/s at 2048^2; the former are 2.7e12
-# now).
-CONE_COST = 1.15
+# Relative cost of one voxel-angle of the cone-beam tiles to one pixel-angle of the fan-beam ones.
+# Launches of jobs of one kind, 1e12 per second, 16-bit / FP32 storage: cone 96^3 2.11 / 2.12,
+# 256^3 2.20 / 2.04, 384^3 2.33 / 2.16; fan 256^2 1.93 / 1.89, 1024^2 2.15 / 2.08, 2048^2 2.26 / 2.15.
+# The ratios of like sizes lie between 0.89 and 1.02.
+CONE_COST = 1.0
 PIXELS_PER_TILE_2D = 64 * 4
 # voxels per tile of the cone-beam kernel: matrices free of y / others
 VOXELS_PER_TILE_3D = {True: 16 * 16 * 16, False: 16 * 16 * 8}
