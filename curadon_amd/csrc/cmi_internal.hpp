@@ -142,25 +142,6 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void *base, uint32_t bytes) {
                                              kBufferFlags);
 }
 
-template <class S>
-__device__ __forceinline__ float buf_load(rsrc_t r, int elem_offset);
-
-template <>
-__device__ __forceinline__ float buf_load<F32>(rsrc_t r, int elem_offset) {
-    return __builtin_bit_cast(float,
-                              __builtin_amdgcn_raw_buffer_load_b32(r, elem_offset * 4, 0, 0));
-}
-template <>
-__device__ __forceinline__ float buf_load<F16>(rsrc_t r, int elem_offset) {
-    const unsigned short u = __builtin_amdgcn_raw_buffer_load_b16(r, elem_offset * 2, 0, 0);
-    return static_cast<float>(__builtin_bit_cast(_Float16, u));
-}
-template <>
-__device__ __forceinline__ float buf_load<BF16>(rsrc_t r, int elem_offset) {
-    const unsigned short u = __builtin_amdgcn_raw_buffer_load_b16(r, elem_offset * 2, 0, 0);
-    return __builtin_bit_cast(float, (uint32_t)u << 16);
-}
-
 // Two adjacent elements (offsets o and o + 1) in FP32, with one load: 8 bytes for F32 pairs,
 // 4 bytes for 16-bit pairs. The load need not be aligned to its size (an F32 pair sits at any
 // dword, a 16-bit pair at any 2-byte boundary): the ROCm driver runs gfx9-family shaders in

@@ -15,7 +15,7 @@
 //
 // Forward rays take their discrete quantities (hit, step count) from an FP64 set-up in the
 // kernel, identical to the host oracle's, then march in FP32 from the ray's midpoint in
-// volume-centred padded coordinates, summing in blocks of 32 samples.
+// volume-centred padded coordinates, summing by slabs of slices (or blocks of 32 samples).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -20,8 +20,10 @@
 // is +-1 along the ray's dominant axis, so with jf = j - N/2, md the midpoint's dominant
 // coordinate and s the step's sign, sample jf's dominant lower tap is the integer
 // floor(md) + s jf with weight fract(md) (exact, one row per sample); its other coordinate is
-// c = fma(jf, v_other, m_other) in FP32, lower tap floor(c), weight fract(c). The forward and
-// the adjoint both use exactly this, so they are each other's transpose.
+// c = fma(jf, v_other, m_other) in FP32, lower tap floor(c), weight fract(c). The forward uses
+// exactly this. The adjoint, its transpose up to rounding, takes a ray's samples in pairs on
+// neighbouring rows: the one with the smaller column as here, the other at that column plus the
+// slope.
 //   per call     for each image b of the batch, one block of 2 * (nx+4) * (ny+4) elements:
 //                pad  [ny+4][nx+4]               image with a 2-texel zero border
 //                padT [nx+4][ny+4]               the same, transposed
@@ -271,12 +273,8 @@ __device__ __forceinline__ int floor_div(int a, int b) {
     return a >= 0 ? a / b : -((-a + b - 1) / b);
 }
 
-// One pass (YDOM: rays whose dominant axis is y, row-major copy; else x, transposed copy).
-// All threads of the workgroup call it together; returns the lane's sum, 0 if not in the pass.
-//   rstride      elements per row of the copy (rows run along the dominant axis)
-//   cofs         element offset of the copy's centre (centred coordinate 0, 0)
-// Dominant row range and column of a ray at row t: sample jf = s (t - floor(md)), column
-// coordinate fma(jf, vc, mc). Used for the workgroup's extreme rays.
+// Column of a ray at row t: sample jf = s (t - floor(md)), coordinate fma(jf, vc, mc). Used for the
+// workgroup's extreme rays.
 struct RayRow {
     float mc, vc;
     int r0, s;
@@ -292,6 +290,10 @@ __device__ __forceinline__ float ray_at(const RayRow &r, int t) {
     return fmaf((float)(r.s * (t - r.r0)), r.vc, r.mc);
 }
 
+// One pass (YDOM: rays whose dominant axis is y, row-major copy; else x, transposed copy).
+// All threads of the workgroup call it together; returns the lane's sum, 0 if not in the pass.
+//   rstride      elements per row of the copy (rows run along the dominant axis)
+//   cofs         element offset of the copy's centre (centred coordinate 0, 0)
 template <class SI, bool YDOM, class B>
 __device__ __forceinline__ float march_band(rsrc_t R, const float4 *__restrict__ ev,
                                             const float4 *__restrict__ ns, bool valid,
@@ -1179,12 +1181,12 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 
 // ------------------------------------------------ transpose of the backprojection -------
 
-// Bᵀ: the transpose of the voxel-driven backprojection (k_bp2d / k_bp2d_vec), the gradient of
+// Bᵀ: the transpose of the voxel-driven backprojection (k_bp2d), the gradient of
 // TorchBackprojection. The backprojection gives pixel p, per projection a, wt_a(p) times the
 // linear interpolation of row a at u_a(p) (cells floor(u) and floor(u) + 1, weights 1 - al and
 // al; cells outside the row read zero), times 1/du (circular plans; the view's 1/|u| is part of
-// wt for plans from views). So sino[a][c] = sum_p (those weights) v[p], with k_bp2d's FP32
-// positions and weights.
+// wt for plans from views). So sino[a][c] = sum_p (those weights) v[p]; positions and weights agree
+// with k_bp2d's up to FP32 rounding (they come from FP64 sums per line, see below).
 // A workgroup owns a segment of GS detector cells of one projection and gathers it. The pixels
 // whose terms reach the segment's cells are those with u in [c0 - 1, c0 + GS): a wedge from
 // the source between the lines u = c0 - 1 and u = c0 + GS (u is a ratio of two functions
@@ -1192,14 +1194,15 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // columns) that the segment's central line follows most closely, in chunks of kGSlab lines;
 // per line the wedge is the interval between the two boundary lines' crossings (kGMargin of a
 // pixel wider on each side, for the FP32 lines; clipped to the image). A wavefront takes every
-// fourth line of a chunk and walks it along the line, a lane per pixel, from the zero-bordered copy whose rows run along it
-// (row-major for rows, transposed for columns), so that it reads runs of consecutive pixels. All
+// fourth line of a chunk and walks it along the line, a lane per pixel, from the zero-bordered copy
+// whose rows run along it (row-major for rows, transposed for columns), so that it reads runs of
+// consecutive pixels. All
 // lines of a chunk are walked over the width of its widest interval, their starts moved back
 // where that would leave the image: pixels outside the wedge have no cell in the segment and add
 // nothing. Depth d and d u, u the cell coordinate from the segment's start on, are affine in the
 // pixel, so they are one sum each of the lane's share (its pixel number along the line) and the
-// line's (evaluated in FP64 by the lane that holds the line, and read from it). Every pixel adds its terms that fall inside the segment
-// to GS + 2 LDS cells with integer atomics. A segment whose boundary lines meet the lines at
+// line's (evaluated in FP64 by the lane that holds the line, and read from it). Every pixel adds its
+// terms that fall inside the segment to GS + 2 LDS cells with integer atomics. A segment whose boundary lines meet the lines at
 // grazing angles walks whole lines.
 // Bound by VALU issue. Walking the chunk's pixels as one flat list, which filled the lanes (0.94
 // against 0.73 at 0.67 pixels per cell) but gave every pixel an index walk, a test against its
