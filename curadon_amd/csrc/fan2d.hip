@@ -661,13 +661,13 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp2d(typename SV::raw *__restrict
 // the order k, k + 1, k + 2, k + 3 (mod 4), under which (S0 + S2) + (S1 + S3) does not change.
 // Two halves of the workgroup (four wavefronts each) take quarters 0 and 2 and quarters 1 and 3
 // of the angles for the same pixels, each with its own LDS buffers, and the second half's sums
-// join through LDS. The kernel is bound by latency (per angle a scalar load, a reciprocal and an
-// LDS read in a row) at VALU 0.7 and LDS 0.8 of their issue rates, so wavefronts count: one half
-// alone with chunks of 16 angles (94 VGPRs, five wavefronts per SIMD; four for want of tiles at
-// 1024^2) took 188 us at 1024^2 x 720 and 4.4 ms at 2048^2 x 4096 FP16, two halves with chunks of
-// 8 (54 VGPRs, eight per SIMD) 174 us and 3.8 ms. The constants through vector loads, which
-// would let their instructions issue at the full rate: 195 us and 4.7 ms. With a weight of w^2
-// per pixel and angle through k_bp2d, 2048^2 x 4096 FP16 took 7.3 ms.
+// join through LDS. No pipe is full (VALU 1.16 of 1.55 instructions a clock and CU, LDS busy 0.7 of
+// the time): per angle a scalar load, a reciprocal and an LDS read follow each other, so wavefronts
+// count: one half alone with chunks of 16 angles (94 VGPRs, five wavefronts per SIMD; four for want
+// of tiles at 1024^2) took 188 us at 1024^2 x 720 and 4.4 ms at 2048^2 x 4096 FP16, two halves with
+// chunks of 8 (54 VGPRs, eight per SIMD) 174 us and 3.8 ms. The constants through vector loads,
+// which would let their instructions issue at the full rate: 195 us and 4.7 ms. With a weight of
+// w^2 per pixel and angle through k_bp2d, 2048^2 x 4096 FP16 took 7.3 ms.
 constexpr int kQT = 16;              // tile edge, pixels
 constexpr int kQHalf = kQT * kQT;    // threads per half
 constexpr int kQThreads = 2 * kQHalf;
@@ -1202,8 +1202,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // nothing. Depth d and d u, u the cell coordinate from the segment's start on, are affine in the
 // pixel, so they are one sum each of the lane's share (its pixel number along the line) and the
 // line's (evaluated in FP64 by the lane that holds the line, and read from it). Every pixel adds its
-// terms that fall inside the segment to GS + 2 LDS cells with integer atomics. A segment whose boundary lines meet the lines at
-// grazing angles walks whole lines.
+// terms that fall inside the segment to GS + 2 LDS cells with integer atomics. A segment whose
+// boundary lines meet the lines at grazing angles walks whole lines.
 // Bound by VALU issue. Walking the chunk's pixels as one flat list, which filled the lanes (0.94
 // against 0.73 at 0.67 pixels per cell) but gave every pixel an index walk, a test against its
 // line's interval and its own affine forms, took 51 VALU and 26 SALU instructions per wavefront of
