@@ -1218,7 +1218,11 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // pixel, so they are one sum each of the lane's share (its pixel number along the line) and the
 // line's (evaluated in FP64 by the lane that holds the line, and read from it). Every pixel adds its
 // terms that fall inside the segment to GS + 2 LDS cells with integer atomics. A segment whose
-// boundary lines meet the lines at grazing angles walks whole lines.
+// boundary lines meet the lines at grazing angles walks whole lines. Where the widest interval is at
+// most half a wavefront, in thin images and at an image's corners, a wavefront walks several lines
+// at a time; a segment whose wedge passes beside the image walks nothing. Calls before / with both:
+// 5 images of 1 x 512 x 90 56 / 35 us, 5 of 33 x 512 x 180 133 / 105, 512^2 x 180 of 0.5 pixels a
+// cell 97 / 85, 1024^2 x 360 of 0.67 490 / 433.
 // Bound by VALU issue. Walking the chunk's pixels as one flat list, which filled the lanes (0.94
 // against 0.73 at 0.67 pixels per cell) but gave every pixel an index walk, a test against its
 // line's interval and its own affine forms, took 51 VALU and 26 SALU instructions per wavefront of
@@ -1235,10 +1239,9 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // lines are still about a wavefront wide, or kGFineFew where that leaves fewer than kGFineMany
 // workgroups an image; else kGS, which gives more workgroups and, at one pixel per cell, lines that
 // just fit a wavefront. 512^2 x 180, calls, us with kGS and with kGSFine (walking the chunk's pixels
-// as one flat list: third): 10 cells per pixel 351, 115 (161), 4 cells 168, 86 (110), 2 cells 102,
-// 96 (97), 1 cell 84, 140 (93); 200^2 x 181 (543 workgroups) of 2 cells 39, 42 (41), 128^2 x 180
-// (540) of 4 cells 39, 39 (40). kGS 64: 5 % more at one cell per pixel of parallel rays, 2 % less at
-// 1.5.
+// as one flat list: third): 10 cells per pixel 141, 87 (161), 4 cells 103, 78 (110), 2 cells 82, 85
+// (97), 1 cell 77, 120 (93); 200^2 x 181 (543 workgroups) of 2 cells 39, 37 (41), 128^2 x 180 (540)
+// of 4 cells 38, 39 (40). kGS 64: 5 % more at one cell per pixel of parallel rays, 2 % less at 1.5.
 constexpr int kGS = 62, kGSFine = 256;
 constexpr double kGFine = 1.75, kGFineFew = 4.0;
 constexpr uint64_t kGFineMany = 1024;
@@ -1401,9 +1404,31 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
     const float s1 = ldexpf(1.0f, max(min(-vexp, 127), -126)); // (max|v| below 2^-127 scales to less)
     const float s2 = (float)(rest * wmul * ldexp(1.0, -vexp - max(min(-vexp, 127), -126)));
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // a pixel of value val, depth d and e = d u adds its terms in the segment to the cells
+    auto visit = [&](float val, float d, float e) {
+        const float vs = val * s1 * s2;
+        const float rd = __builtin_amdgcn_rcpf(d), u = rd * e;
+        const int i = floor_i32(u);
+        if ((unsigned)i > (unsigned)GS || vs == 0.0f) return;
+        const float w = vL * rd;
+        const float t = vs * (WPOW == 2 ? w * w : w);
+        const float t1 = t * __builtin_amdgcn_fractf(u), t0 = t - t1;
+        atomicAdd(&cells[i], (unsigned)round_i32(t0));
+        atomicAdd(&cells[i + 1], (unsigned)round_i32(t1));
+    };
     int run = 0; // pixel visits since the last drain
     __syncthreads(); // the cells are clear
-    for (int k0 = 0; k0 < nK; k0 += kGSlab) {
+    // nothing to walk if both boundary lines pass the image on one side (a pixel away and more) at
+    // its first and at its last line
+    bool beside = false;
+    if (!whole) {
+        const float e0 = fmaf(f1[0], (float)(nK - 1), f0[0]);
+        const float e1 = fmaf(f1[1], (float)(nK - 1), f0[1]);
+        beside = fmaxf(fmaxf(f0[0], f0[1]), fmaxf(e0, e1)) < -1.0f ||
+                 fminf(fminf(f0[0], f0[1]), fminf(e0, e1)) > (float)nF;
+    }
+    const int todo = __builtin_amdgcn_readfirstlane(beside ? 0 : nK);
+    for (int k0 = 0; k0 < todo; k0 += kGSlab) {
         // lane l holds line k0 + l: the first pixel of its interval, then its walk's start and
         // shares. Every wavefront does the same.
         const int S = min(kGSlab, nK - k0), k = k0 + min(lane, S - 1);
@@ -1421,6 +1446,24 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
         const float dl = (float)(dc[0] * lo + dc[1] * k + dc[2]);
         const float el = (float)(ec[0] * lo + ec[1] * k + ec[2]);
         const int at = lo + k * strK;
+        if (NW <= 32) { // several lines to a wavefront
+            if (run + kGSlab / 4 * kMaxBlock > kGBudget) {
+                drain();
+                run = 0;
+            }
+            run += kGSlab / 4 * kMaxBlock;
+            const int sh = NW > 1 ? 32 - __builtin_clz((unsigned)NW - 1) : 0; // lanes a line: 2^sh
+            const int f = lane & ((1 << sh) - 1), per = 64 >> sh;
+            const bool in = f < NW;
+            const int df = in ? f : 0;
+            const float dp = (float)(dc[0] * df), ep = (float)(ec[0] * df);
+            for (int l0 = wv * per; l0 < S; l0 += 4 * per) {
+                const int m = l0 + (lane >> sh), l = min(m, S - 1);
+                const float val = to_f32<SV>(src[__shfl(at, l, 64) + df]);
+                visit(in && m < S ? val : 0.0f, dp + __shfl(dl, l, 64), ep + __shfl(el, l, 64));
+            }
+            continue;
+        }
         for (int f = 0; f < NW; f += 64) {
             if (run + kGSlab / 4 * kMaxBlock > kGBudget) {
                 drain();
@@ -1442,18 +1485,9 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
                 for (int q = 0; q < kGBatch; ++q) {
                     const int l = l0 + 4 * q;
                     if (l >= S) break;
-                    const float vs = val[q] * s1 * s2;
-                    const float rd = __builtin_amdgcn_rcpf(
-                        dp + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dl), l)));
-                    const float u = rd *
-                        (ep + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(el), l)));
-                    const int i = floor_i32(u);
-                    if ((unsigned)i > (unsigned)GS || vs == 0.0f) continue;
-                    const float w = vL * rd;
-                    const float t = vs * (WPOW == 2 ? w * w : w);
-                    const float t1 = t * __builtin_amdgcn_fractf(u), t0 = t - t1;
-                    atomicAdd(&cells[i], (unsigned)round_i32(t0));
-                    atomicAdd(&cells[i + 1], (unsigned)round_i32(t1));
+                    visit(val[q],
+                          dp + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dl), l)),
+                          ep + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(el), l)));
                 }
             }
         }

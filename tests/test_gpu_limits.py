@@ -260,3 +260,34 @@ def test_backward_transpose_3d_tiles_beside_the_volume(oracle, gpu, rec):
         assert rel_l2(got, want) <= 2.0 * unit * wbound, mode
         beside = want == 0.0
         assert beside.any() and not got.cpu().numpy()[beside].any()
+
+
+@pytest.mark.parametrize("views", [False, True])
+@pytest.mark.parametrize("ny,nx,D,du", [
+    (70, 1, 300, 1.5), (1, 70, 300, 1.5), (130, 7, 400, 1.5), (65, 2, 90, 4.0),
+    (40, 31, 100, 1.5), (40, 32, 100, 1.5), (40, 33, 100, 1.5), (33, 40, 40, 9.0),
+    (20, 20, 500, 1.5),                    # segments that see no pixel on both sides
+])
+def test_backward_transpose_thin_images(oracle, gpu, views, ny, nx, D, du):
+    """Lines of up to 32 pixels, several to a wavefront, widths around that, and detectors far
+    beyond the image on both sides.
+
+    Terms are rounded to units of 2^-18 max|v| bound, 0.29 units rms, against terms of rms|v| w /
+    sqrt(3) (w >= 0.6 bound with the source at twice the image's size): twice that, and the rounding
+    of positions as above."""
+    n = max(ny, nx)
+    more = {"det_offset": 0.25, "exact_geometry": True} if views else {}
+    geom = cm.FanGeometry(DSD=3.0 * n, DSO=2.0 * n, angles=np.linspace(0, 6, 9),
+                          vol_shape=(ny, nx), det_shape=D, det_spacing=du, **more)
+    v = np.random.RandomState(ny + nx).rand(ny, nx) - 0.3
+    x = torch.tensor(v, dtype=torch.float32, device=gpu)
+    units = 0.29 * 2.0 ** -18 * np.abs(v).max() / (np.sqrt(np.mean(v * v)) / 3 ** 0.5)
+    for mode, wpow in (("reference", 1), ("fbp", 2)):
+        got = cm.backward_transpose(x, geom, mode=mode)
+        want = oracle.bp2d_T(geom, v, wpow=wpow)
+        assert rel_l2(got, want) <= 2.0 * units / 0.6 ** wpow + 4 * (D / 2) * 2.0 ** -24 / 0.58, mode
+        hit = np.pad(want != 0.0, ((0, 0), (1, 1)))
+        beside = ~(hit[:, :-2] | hit[:, 1:-1] | hit[:, 2:])
+        assert not got.cpu().numpy()[beside].any()
+        both = cm.backward_transpose(torch.stack([x, 2.0 * x]), geom, mode=mode)
+        assert torch.equal(both[0], got) and torch.equal(both[1], 2.0 * got)
