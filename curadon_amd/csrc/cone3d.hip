@@ -981,7 +981,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_bp3d(typename SV::raw *__restrict
     for (int y = 0; y < NY; ++y) acc[y] = 0.0f;
     bp3d_run<SS, YINV, MATCHED, FDK>(R, M, A, U, V, (float)ix - cx, (float)iy0 - cy,
                                      (float)iz - cz, (float)tx - cx, (float)ty - cy,
-                                     (float)tz - cz, acc);
+                                     (float)tz - cz, __builtin_amdgcn_readfirstlane(ny - iy0),
+                                     acc);
     if (ix >= nx || iz >= nz) return;
 #pragma unroll
     for (int y = 0; y < NY; ++y) {

@@ -207,12 +207,16 @@ __device__ __forceinline__ void serve_tile_3d(const DevJob &J, uint32_t t) {
     const float hx = (float)ix - J.cx, hy = (float)iy0 - J.cy, hz = (float)iz - J.cz;
     const float tx = (float)x0 - J.cx, ty = (float)y0 - J.cy, tz = (float)z0 - J.cz;
     const ctab M = const_table(J.table);
+    const int count = __builtin_amdgcn_readfirstlane(J.ny - iy0);
     if (J.mode == CMI_BP3D_FDK)
-        bp3d_run<SS, YINV, true, true>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, ty, tz, acc);
+        bp3d_run<SS, YINV, true, true>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, ty, tz, count,
+                                       acc);
     else if (J.mode == CMI_BP3D_MATCHED)
-        bp3d_run<SS, YINV, true, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, ty, tz, acc);
+        bp3d_run<SS, YINV, true, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, ty, tz, count,
+                                        acc);
     else
-        bp3d_run<SS, YINV, false, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, ty, tz, acc);
+        bp3d_run<SS, YINV, false, false>(R, M, J.nangles, J.nu, J.nv, hx, hy, hz, tx, ty, tz, count,
+                                         acc);
     if (ix >= J.nx || iz >= J.nz) return;
     auto *vol = static_cast<typename SV::raw *>(J.volume);
 #pragma unroll

@@ -291,3 +291,18 @@ def test_backward_transpose_thin_images(oracle, gpu, views, ny, nx, D, du):
         assert not got.cpu().numpy()[beside].any()
         both = cm.backward_transpose(torch.stack([x, 2.0 * x]), geom, mode=mode)
         assert torch.equal(both[0], got) and torch.equal(both[1], 2.0 * got)
+
+
+@pytest.mark.parametrize("ny", [1, 3, 4, 5, 8, 9, 12, 13, 17, 20, 21])
+def test_backward_3d_thin_runs(oracle, gpu, ny):
+    """Tilted orbits: runs of 8 y voxels in batches of four, of which the volume ends within any."""
+    rec = cone(18, 36, 34, 5, 60.0, 90.0, nz=9, ny=ny,
+               angles=np.array([[0.3, 1.9, 3.0, 5.1, 5.9], [0.7, 1.4, 0.2, 1.5, 1.1],
+                                [0.1, 0.9, 1.5, 0.4, 0.2]]))
+    geom = as_cone_geometry(rec)
+    y = np.random.RandomState(ny).rand(rec.nangles, *rec.det_shape)
+    x = torch.tensor(y, dtype=torch.float32, device=gpu)
+    for mode, kw in (("reference", {}), ("matched", {"matched": True}),
+                     ("fdk", {"matched": True, "fdk": True})):
+        got = cm.backward(x, geom, mode=mode)
+        assert rel_l2(got, oracle.bp3d(geom, y, **kw)) <= RTOL_L2, mode
