@@ -929,6 +929,19 @@ constexpr int kAdjBits = 19;        // a term's bound: 2^kAdjBits units
 constexpr int kAdjBudget = (1 << (31 - kAdjBits)) - 2;
 static_assert((int64_t)kAdjBudget * ((1 << kAdjBits) + 2) < (1ll << 31), "32-bit sums are exact");
 
+// Angle groups per tile. A group costs its workgroup's clearing of the tile and up to 2048 64-bit
+// atomics, so it is given kAdjSamples samples (a tile's share of the plan's) or, as long as that
+// leaves fewer than kAdjFill workgroups, kAdjLeast; at most kAdjWorkgroups workgroups (with tiles of 32
+// x 32 at 1024^2 a limit of 8192 gave 1.09 ms, 16384: 1.06, 24576: 1.04, 32768: 1.05). Calls with 1 /
+// 3 / 6 / 12 / 24 / 60 / 180 groups, us, and what this rule takes (by the number of workgroups alone,
+// and with tiles of 32 x 32 before: last two): 512^2 x 180 of 1.5 pixels 107 / 67 / 65 / 60 / 76 / 120 /
+// 285, 16 (168, 209), of 0.15 616 / 630 / 787 / 642 / 565 / 478 / 519, 63 (497, 621); 200^2 x 60 of 0.6 78 /
+// 46 / 38 / 34 / 34 / 37, 11 (43, 39); 64^2 x 360 of 0.6 391 / 204 / 126 / 72 / 46 / 35 / 35, 96 (45, 37);
+// 5 images of 1 x 100 x 360 of 0.6 113 / 56 / 48 / 36 / 35 / 35 / 48 (75, 60); 1024^2 x 720 of 0.6 960 /
+// 1057 / 1260 / 746 / 737 / 811 / 1235, 24 (739, 1210).
+constexpr uint64_t kAdjSamples = 20000, kAdjLeast = 5000, kAdjFill = 4096, kAdjWorkgroups = 24576;
+constexpr uint64_t kAdjRay = 16; // samples that a ray's set-up counts for
+
 // Tiles of one image: those of the y-dominant rays, then those of the x-dominant ones.
 __host__ __device__ inline unsigned adj2d_tiles(unsigned across, unsigned along) {
     return ((across + kT2Rows - 1) / kT2Rows) * ((along + kT2Cols - 1) / kT2Cols);
@@ -2199,13 +2212,13 @@ CMI_API cmi_status cmi_adjoint_2d(const cmi_plan2d *plan, void *volume, int vol_
         hipLaunchKernelGGL((k_adj2d_absmax<SS>), dim3(kAdjParts, (unsigned)batch),
                            dim3(kMaxBlock), 0, s, (const typename SS::raw *)sinogram, plan->d_ns,
                            rays, parts);
-        // angle groups: enough workgroups to fill the GPU many times over (about 96 per CU; with
-        // tiles of 32 x 32 at 1024^2 a target of 8192 workgroups gave 1.09 ms, 16384: 1.06, 24576:
-        // 1.04, 32768: 1.05)
         const unsigned tiles = adj2d_tiles(ny, nx) + adj2d_tiles(nx, ny);
         const uint64_t all = (uint64_t)tiles * batch;
+        const uint64_t samples = (plan->total_samples + kAdjRay * rays) * batch / all; // per tile
         const int G = (int)std::max<uint64_t>(
-            1, std::min<uint64_t>((uint64_t)A, (24576 + all - 1) / all));
+            1, std::min<uint64_t>(
+                   {(uint64_t)A, (kAdjWorkgroups + all - 1) / all,
+                    std::max(samples / kAdjSamples, std::min(kAdjFill / all, samples / kAdjLeast))}));
         hipLaunchKernelGGL((k_adj2d_tile<SS>), dim3(tiles, 1, (unsigned)(G * batch)),
                            dim3(kMaxBlock), 0, s, accimg, (const typename SS::raw *)sinogram,
                            plan->d_ageo, plan->d_ev, plan->d_ns, parts, nx, ny, D, A, G);
