@@ -660,6 +660,10 @@ constexpr int kAdj3Budget = (1 << (31 - kAdj3Bits)) - 16; // terms per voxel bet
 // 128^3 x 40 views (512) of 192^2 487 / 423 / 399 / 358 / 357 / 459 / 521, 21; of 96^2 214 / 174 / 179 /
 // 173 / 240 / 413 / 490, 5; of 48^2 166 / 128 / 138 / 154 / 188 / 275 / 319, 2; 48^3 x 60 of 18^2 (27)
 // 240 / 138 / 79 / 54 / 43 / 44 / 57, 14.
+// Groups need two launches more, about 9 us: tiles whose work, an angle counting for kAdj3Angle
+// samples, is below kAdj3Alone have one. us, with 1 / 2 / 4 groups: 16^3 x 5 views of 12^2 36 / 47 / 48,
+// x 9 51 / 47 / 47, x 2 of 30^2 43 / 48 / 48, x 3 59 / 52 / 48; 90^3 (216) x 5 of 67^2 46 / 50 / 56, x 9
+// 61 / 57 / 62; 5^3 x 9 of 4^2 37 / 47 / 47, x 20 60 / 48 / 48.
 // Where the tiles fill the GPU and the angles are few, a group is a sector of the circle, whose tiles
 // near the source are neighbours in the order and fall to one or two XCDs: one group there. us, with
 // 1 / 2 / 4 / 8 / 16 groups: 128^3 (512 tiles) of 640^2, 4 views 492 / 693 / 566 / 632 / 572, 12 views
@@ -669,6 +673,7 @@ constexpr int kAdj3Budget = (1 << (31 - kAdj3Bits)) - 16; // terms per voxel bet
 // 307 / 299 / 288 / 241.
 constexpr uint64_t kAdj3Samples = 10000, kAdj3Least = 1500, kAdj3Fill = 1024;
 constexpr uint64_t kAdj3FullTiles = 512, kAdj3FewAngles = 24, kAdj3TilesPerAngle = 32;
+constexpr uint64_t kAdj3Angle = 3000, kAdj3Alone = 40000;
 constexpr uint64_t kAdj3Workgroups = 24576;
 
 // vol[o] += a voxel's sum of fixed-point terms.
@@ -1917,8 +1922,9 @@ CMI_API cmi_status cmi_adjoint_3d(const cmi_plan3d *plan, void *volume, int vol_
                          (unsigned)(ntz * batch));
         const uint64_t samples = plan->total_samples * batch / ntiles; // per tile
         const int G =
-            ntiles >= kAdj3FullTiles &&
-                    (uint64_t)A <= std::min(kAdj3FewAngles, ntiles / kAdj3TilesPerAngle)
+            samples + kAdj3Angle * A < kAdj3Alone ||
+                    (ntiles >= kAdj3FullTiles &&
+                     (uint64_t)A <= std::min(kAdj3FewAngles, ntiles / kAdj3TilesPerAngle))
                 ? 1
                 : (int)std::max<uint64_t>(
                       1, std::min<uint64_t>({(uint64_t)A, (kAdj3Workgroups + ntiles - 1) / ntiles,
