@@ -1249,14 +1249,14 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // Integer sums are exact: the result does not depend on the order of the additions. Each
 // segment is written once, in the sinogram's storage type.
 // Detector cells per segment: kGSFine where a pixel has at least kGFine cells, so that the walk's
-// lines are still about a wavefront wide, or kGFineFew where that leaves fewer than kGFineMany
-// workgroups an image; else kGS, which gives more workgroups and, at one pixel per cell, lines that
-// just fit a wavefront. 512^2 x 180, calls, us with kGS and with kGSFine (walking the chunk's pixels
-// as one flat list: third): 10 cells per pixel 141, 87 (161), 4 cells 103, 78 (110), 2 cells 82, 85
-// (97), 1 cell 77, 120 (93); 200^2 x 181 (543 workgroups) of 2 cells 39, 37 (41), 128^2 x 180 (540)
-// of 4 cells 38, 39 (40). kGS 64: 5 % more at one cell per pixel of parallel rays, 2 % less at 1.5.
+// lines are still about a wavefront wide, and that leaves kGFineMany workgroups an image; else kGS,
+// which gives more workgroups and, at one pixel per cell, lines that just fit a wavefront. Calls, us,
+// with kGS and with kGSFine (walking the chunk's pixels as one flat list: third): 512^2 x 180 of 10
+// cells per pixel 141, 87 (161), 4 cells 103, 78 (110), 2 cells 82, 85 (97), 1 cell 77, 120 (93); 640^2
+// x 17 with 2000 of 5 cells per pixel (136 workgroups of kGSFine) 46, 64 (47), x 60 with 4000 of 12
+// (960) 59, 54 (68). kGS 64: 5 % more at one cell per pixel of parallel rays, 2 % less at 1.5.
 constexpr int kGS = 62, kGSFine = 256;
-constexpr double kGFine = 1.75, kGFineFew = 4.0;
+constexpr double kGFine = 1.75;
 constexpr uint64_t kGFineMany = 1024;
 constexpr int kGSlab = 64;                                   // image lines per chunk
 constexpr int kGBits = 18;                                   // a term's bound: 2^kGBits units
@@ -1470,10 +1470,20 @@ __global__ __launch_bounds__(kMaxBlock) void k_bpT2d(typename SS::raw *__restric
             const bool in = f < NW;
             const int df = in ? f : 0;
             const float dp = (float)(dc[0] * df), ep = (float)(ec[0] * df);
-            for (int l0 = wv * per; l0 < S; l0 += 4 * per) {
-                const int m = l0 + (lane >> sh), l = min(m, S - 1);
-                const float val = to_f32<SV>(src[__shfl(at, l, 64) + df]);
-                visit(in && m < S ? val : 0.0f, dp + __shfl(dl, l, 64), ep + __shfl(el, l, 64));
+            for (int l0 = wv * per; l0 < S; l0 += 4 * per * kGBatch) {
+                float val[kGBatch];
+#pragma unroll
+                for (int q = 0; q < kGBatch; ++q) {
+                    const int l = min(l0 + 4 * per * q + (lane >> sh), S - 1);
+                    val[q] = to_f32<SV>(src[__shfl(at, l, 64) + df]);
+                }
+#pragma unroll
+                for (int q = 0; q < kGBatch; ++q) {
+                    if (l0 + 4 * per * q >= S) break;
+                    const int m = l0 + 4 * per * q + (lane >> sh), l = min(m, S - 1);
+                    visit(in && m < S ? val[q] : 0.0f, dp + __shfl(dl, l, 64),
+                          ep + __shfl(el, l, 64));
+                }
             }
             continue;
         }
@@ -2139,9 +2149,8 @@ CMI_API cmi_status cmi_backward_2d_transpose(const cmi_plan2d *plan, void *sinog
     const size_t img = (size_t)nx * ny;
     const int Wp = nx + 2 * kPad, Hp = ny + 2 * kPad;
     // (not by the batch: an image's bits do not depend on the others)
-    const bool fine = plan->cells_per_pixel >=
-                      ((uint64_t)A * ((D + kGSFine - 1) / kGSFine) >= kGFineMany ? kGFine
-                                                                                 : kGFineFew);
+    const bool fine = plan->cells_per_pixel >= kGFine &&
+                      (uint64_t)A * ((D + kGSFine - 1) / kGSFine) >= kGFineMany;
     const int gs = fine ? kGSFine : kGS;
     const uint64_t nseg = (uint64_t)(D + gs - 1) / gs;
     if ((uint64_t)A * nseg * kMaxBlock >= (1ull << 32) || batch > 65535)
