@@ -1253,8 +1253,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_fill_u64(unsigned long long *__re
 // which gives more workgroups and, at one pixel per cell, lines that just fit a wavefront. Calls, us,
 // with kGS and with kGSFine (walking the chunk's pixels as one flat list: third): 512^2 x 180 of 10
 // cells per pixel 141, 87 (161), 4 cells 103, 78 (110), 2 cells 82, 85 (97), 1 cell 77, 120 (93); 640^2
-// x 17 with 2000 of 5 cells per pixel (136 workgroups of kGSFine) 46, 64 (47), x 60 with 4000 of 12
-// (960) 59, 54 (68). kGS 64: 5 % more at one cell per pixel of parallel rays, 2 % less at 1.5.
+// x 17 with 2000 of 5 cells per pixel (136 workgroups of kGSFine) 39, 64 (47), x 60 with 4000 of 12
+// (960) 62, 54 (68). kGS 64: 5 % more at one cell per pixel of parallel rays, 2 % less at 1.5.
 constexpr int kGS = 62, kGSFine = 256;
 constexpr double kGFine = 1.75;
 constexpr uint64_t kGFineMany = 1024;
