@@ -306,3 +306,16 @@ def test_backward_3d_thin_runs(oracle, gpu, ny):
                      ("fdk", {"matched": True, "fdk": True})):
         got = cm.backward(x, geom, mode=mode)
         assert rel_l2(got, oracle.bp3d(geom, y, **kw)) <= RTOL_L2, mode
+
+
+@pytest.mark.parametrize("ny,nx,A,D", [(1, 50, 40, 60), (50, 1, 40, 60), (33, 65, 25, 90), (64, 64, 40, 300)])
+def test_adjoint_angle_groups(gpu, ny, nx, A, D):
+    """One image, whose tiles have many angle groups, and large batches, whose tiles have few: the
+    same bits, scaled data by powers of two included."""
+    n = max(ny, nx)
+    geom = as_fan_geometry(fan(nx, D, A, 2.0 * n, 3.0 * n, du=2.4 * n / D, ny=ny))
+    y = torch.tensor(np.random.RandomState(D).rand(A, D) - 0.3, dtype=torch.float32, device=gpu)
+    one = cm.adjoint(y, geom)
+    scale = torch.tensor([1.0, 4.0, 0.5], device=gpu).repeat(400)[:1000, None, None]
+    many = cm.adjoint(y * scale, geom)
+    assert torch.equal(many, one * scale)
